@@ -72,8 +72,8 @@ __device__ __forceinline__ void weight_operands(u32x4 (&a)[R], const WeightFrag<
 template <class T>
 __device__ __forceinline__ void store4(uint16_t *p, float a, float b, float c, float d) {
     u32x2 o;
-    o[0] = T::from_f32(a) | (T::from_f32(b) << 16);
-    o[1] = T::from_f32(c) | (T::from_f32(d) << 16);
+    o[0] = T::from_f32x2(a, b);
+    o[1] = T::from_f32x2(c, d);
     *reinterpret_cast<u32x2 *>(p) = o;
 }
 

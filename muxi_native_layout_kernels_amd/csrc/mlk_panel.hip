@@ -28,7 +28,7 @@
 // tiles by that XCD's L2.  K slices fold like in the row-shared kernel: fp32 partials with
 // agent-scope stores, the last workgroup to arrive adds them in slice order.
 #include "mlk_panel_loop.cuh"
-#include "mlk_panel_lds.cuh"
+#include "mlk_panel8.cuh"
 
 namespace mlk {
 
@@ -287,8 +287,8 @@ __device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)
 #pragma unroll
             for (int tb = 0; tb < 4; ++tb) {
                 u32x2 o;
-                o[0] = T::from_f32(p.alpha * acc[pr][tb][4 * g] + bias[0]) | (T::from_f32(p.alpha * acc[pr][tb][4 * g + 1] + bias[1]) << 16);
-                o[1] = T::from_f32(p.alpha * acc[pr][tb][4 * g + 2] + bias[2]) | (T::from_f32(p.alpha * acc[pr][tb][4 * g + 3] + bias[3]) << 16);
+                o[0] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g] + bias[0], p.alpha * acc[pr][tb][4 * g + 1] + bias[1]);
+                o[1] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g + 2] + bias[2], p.alpha * acc[pr][tb][4 * g + 3] + bias[3]);
                 *reinterpret_cast<u32x2 *>(buf + (tb * 32 + c32) * kP8OutPitch + row * 2) = o;
             }
         }
@@ -304,53 +304,18 @@ __device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// 256 x 256 panels of 16-bit weights: eight waves, both operands through LDS, fetched with loads that write LDS directly.
-//
-// A wave that issues v_mfma_f32_32x32x16 back to back loses matrix-core time with every other instruction it has to
-// issue in between (measured: about 20 cycles per LDS read, 24 per load); with two waves per SIMD the instructions
-// of one wave go out under the products of the other.  That needs both waves of a SIMD inside 256 registers each,
-// so nothing is staged through registers here: a k32 slab of the panel (16 weight tiles of 16 rows x 32 k, 1 KiB
-// each, as they lie in layout A; 16 chunks of 16 tokens x 32 k) is copied into LDS by 32 buffer loads with the LDS
-// bit, four per wave: the weight tiles addressed by the thread id alone (the descriptor adds 16 bytes per lane, no
-// address register), the token chunks with a per-lane offset (lane 4 t + j fetches octet j ^ (t / 4) of token t, so that
-// four lanes cover 64 consecutive bytes of a token row and the operand reads below meet no bank twice).
-// Wave w = (token half w / 4, row quarter w % 4) multiplies 64 rows x 128 tokens: per k16 step two weight operands (two
-// vertically adjacent tiles read as one 32-row operand: lane 32 g + i takes row i % 16 of tile i / 16, octet g) and four
-// token operands feed eight products.
-//
-// Ring of four slabs (128 KiB).  While slab s is multiplied, slab s + 1 is complete and published, slab s + 2 is landing
-// and the loads of slab s + 3 go out into the buffer that slab s - 1 has left; one wait (this wave's loads of slab
-// s + 2) and one barrier per slab publish slab s + 2 and retire slab s.  The operands of the first step of slab s + 1
-// are read before that barrier, so no wave stands idle behind it.  The barrier is the bare instruction: the fence that
-// comes with __syncthreads() would wait for every load in flight.
-constexpr int kP8Slab = 2048;                                  // 16-byte granules of a slab: 1024 of weights, 1024 of tokens
-constexpr size_t kP8RingBytes = (size_t)4 * kP8Slab * 16;
-
-// the four loads of one wave for slab `slab` (counted from k = 0) into ring buffer `buf`
-__device__ __forceinline__ void p8_issue(const uint8_t *a_panel, const uint16_t *b, const uint32_t (&a_soff)[2],
-                                         const uint32_t (&b_voff)[2], int wave, int slab, int buf) {
-    extern __shared__ u32x4 win[];
-    __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void *)a_panel, 16, 0xffffffffu, 1 << 23);
-    __amdgpu_buffer_rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc((void *)b, 0, 0xffffffffu, 0x00020000);
-    const int dst = buf * kP8Slab;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, win + dst + (2 * wave + i) * 64, 16, 0, a_soff[i] + slab * 1024, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, win + dst + 1024 + (2 * wave + i) * 64, 16, b_voff[i], slab * 64, 0, 0);
-}
-
+// 256 x 256 panels: the eight-wave loop of mlk_panel8.cuh.
 //
 // Grid: without K slices the workgroup ids of an XCD walk bands of p.band groups of eight row tiles in chunks of
 // p.chunk token tiles, so that the 32 workgroups an XCD runs at a time cover 8 x 4 (row tiles x token tiles) and share
 // both operands through its L2; with the token tiles of two row tiles side by side (2 x 16) the same product took
 // 17 % longer (8192 x 8192, 4096 tokens: 491 against 413 us).  A fifth slab of LDS (160 KiB) changed nothing.
-template <class T>
+template <class T, bool FP8>
 __global__ void __launch_bounds__(512) gemm_panel8_kernel(PanelArgs p) {
-    constexpr int RING = 4;
     extern __shared__ u32x4 win[];
     constexpr int PR = 2, TB = 4;
+    constexpr int WBYTES = FP8 ? 1 : 2;
+    using Loop = Panel8Loop<T, FP8, TB>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 3, wt = wave >> 2;
@@ -392,265 +357,28 @@ __global__ void __launch_bounds__(512) gemm_panel8_kernel(PanelArgs p) {
     const int nslab = 2 * ((int)((long long)(sk + 1) * nwin_total / SK) - wbeg);
 
     // sources of this wave's loads: weight tiles 2 wave, 2 wave + 1 of the panel (rows past N: a copy of the last row
-    // group, never stored), token chunks 2 wave, 2 wave + 1 (tokens past M: the last token)
-    const uint8_t *a_panel = p.A + (size_t)rgp * p.K * 32;
-    uint32_t a_soff[2], b_voff[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rg = min(rgp + 2 * wave + i, groups - 1);
-        a_soff[i] = (uint32_t)(rg - rgp) * (uint32_t)p.K * 32u;
-        const int t = lane >> 2, oct = (lane & 3) ^ ((t >> 2) & 3);
-        const int tok = min(tok0 + (2 * wave + i) * 16 + t, p.M - 1);
-        b_voff[i] = (uint32_t)tok * (uint32_t)p.K * 2u + oct * 16;
-    }
-    // operand reads (granules inside a slab, first k16 step; the second step is + 32 for weights, ^ 2 for tokens)
-    const int g = lane >> 5, i32 = lane & 31, t16 = i32 & 15, hi = i32 >> 4;
-    const int a_idx = (wr * 4 + hi) * 64 + g * 16 + t16;                                         // + 128 pr
-    const int b_idx = 1024 + (wt * 8 + hi) * 64 + 4 * t16 + (g ^ ((t16 >> 2) & 3));           // + 128 tb
-
-    f32x16 acc[PR][TB];
-#pragma unroll
-    for (int pr = 0; pr < PR; ++pr)
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[pr][tb][e] = 0.f;
-
-    u32x4 a0[PR], a1[PR], b0[TB], b1[TB];
-    auto rd = [&](u32x4 (&a)[PR], u32x4 (&b)[TB], int buf, int hs) {
-        const u32x4 *src = win + buf * kP8Slab;
-#pragma unroll
-        for (int pr = 0; pr < PR; ++pr) a[pr] = src[a_idx + 128 * pr + hs * 32];
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb) b[tb] = src[(b_idx ^ (hs * 2)) + 128 * tb];
-    };
-    auto mm = [&](const u32x4 (&a)[PR], const u32x4 (&b)[TB]) {
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int pr = 0; pr < PR; ++pr) acc[pr][tb] = T::mfma32(a[pr], b[tb], acc[pr][tb]);
-    };
-    // slabs past the end of the slice are fetched as copies of its last slab and never multiplied, which keeps the
-    // count of loads in flight the same in every trip
-    const int last = slab0 + nslab - 1;
-#pragma unroll
-    for (int i = 0; i < RING - 1; ++i) p8_issue(a_panel, p.B, a_soff, b_voff, wave, min(slab0 + i, last), i);
-    wait_vmcnt_le<4 * (RING - 3)>();                           // slabs 0 and 1 of this wave have landed
-    bare_barrier();
-    rd(a0, b0, 0, 0);
-    int cur = 0;                                               // ring buffer of slab s
-    for (int s = 0; s < nslab; ++s) {
-        const int nxt = cur == RING - 1 ? 0 : cur + 1, prv = cur == 0 ? RING - 1 : cur - 1;
-        p8_issue(a_panel, p.B, a_soff, b_voff, wave, min(slab0 + s + RING - 1, last), prv);
-        rd(a1, b1, cur, 1);
-        mm(a0, b0);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (m != 3 && m != 7) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            if (m < 4) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        rd(a0, b0, nxt, 0);
-        mm(a1, b1);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (m != 3 && m != 7) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        wait_vmcnt_le<4 * (RING - 3)>();                       // this wave's loads of slab s + 2 have landed
-        bare_barrier();
-        cur = nxt;
-    }
-    __builtin_amdgcn_s_waitcnt(0);                             // nothing may still be writing LDS when the ring is given up
-    mfma_settle();
-    __syncthreads();
-    if (SK == 1) p8_store_panel<T>(p, acc, rg0, tok0 + wt * 128, wave, lane, win);
-    else panel_finish<T, PR, TB, 8, 2>(p, acc, rg0, tok0 + wt * 128, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
-}
-
-// The same panel for soft-FP8 weights.  The fp8 tiles (512 bytes) land in a small ring of their own (three slabs of
-// 8 KiB behind the four bf16 slabs: 152 KiB in all); every wave widens the two tiles it fetched itself, two slabs ahead of
-// their use, lane by lane (8 bytes in, 16 bytes out at the same lane's place: the tile order does not change) into the
-// bf16 slab, so that each weight is widened once per workgroup and the multiplying loop is the 16-bit one.  Per slab and
-// wave: two token-chunk loads, one fp8 load (its two tiles, 32 lanes each), two 8-byte LDS reads, 32 conversion
-// instructions, two 16-byte LDS writes, sixteen products.
-constexpr int kP8RawSlab = 512;                                // granules of a slab of fp8 tiles
-constexpr size_t kP8Fp8LdsBytes = (size_t)(4 * kP8Slab + 3 * kP8RawSlab) * 16;
-
-__device__ __forceinline__ void p8_issue_fp8(const uint8_t *a_panel, const uint16_t *b, uint32_t a_voff, const uint32_t *b_voff,
-                                             int wave, int slab_b, int buf_b, int slab_a, int buf_a) {
-    extern __shared__ u32x4 win[];
-    __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void *)a_panel, 0, 0xffffffffu, 0x00020000);
-    __amdgpu_buffer_rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc((void *)b, 0, 0xffffffffu, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, win + buf_b * kP8Slab + 1024 + (2 * wave + i) * 64, 16, b_voff[i], slab_b * 64, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, win + 4 * kP8Slab + buf_a * kP8RawSlab + 2 * wave * 32, 16, a_voff, slab_a * 512, 0, 0);
-}
-
-template <class T>
-__global__ void __launch_bounds__(512) gemm_panel8_fp8_kernel(PanelArgs p) {
-    extern __shared__ u32x4 win[];
-    constexpr int PR = 2, TB = 4;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave & 3, wt = wave >> 2;
-    const int xcd = blockIdx.x & 7;
-    int u = blockIdx.x >> 3;
-    int SK, sk, tt, rt;
-    if (p.band > 0) {
-        const int TT = p.token_tiles, groups8 = (p.row_tiles + 7) >> 3, RB = p.band, TC = p.chunk;
-        const int band = u / (RB * TT);
-        const int nb = min(RB, groups8 - band * RB);
-        const int v = u - band * RB * TT;
-        const int c = v / (nb * TC);
-        const int tc = min(TC, TT - c * TC);
-        const int w = v - c * nb * TC;
-        SK = 1, sk = 0;
-        tt = c * TC + w % tc;
-        rt = (band * RB + w / tc) * 8 + xcd;
-    } else {
-        const int whole_wgs = p.whole_groups * p.token_tiles;
-        const bool sliced = u >= whole_wgs;
-        SK = sliced ? p.SK : 1;
-        if (sliced) u -= whole_wgs;
-        tt = u % p.token_tiles;
-        u /= p.token_tiles;
-        sk = u % SK;
-        rt = ((sliced ? p.whole_groups : 0) + u / SK) * 8 + xcd;
-    }
-    if (rt >= p.row_tiles) return;
-
-    const int groups = p.N >> 4;
-    const int rgp = rt * 16;
-    const int rg0 = rgp + wr * 4;
-    const int tok0 = tt * 256;
-    const int nwin_total = p.K / 64;
-    const int wbeg = (int)((long long)sk * nwin_total / SK);
-    const int slab0 = 2 * wbeg;
-    const int nslab = 2 * ((int)((long long)(sk + 1) * nwin_total / SK) - wbeg);
-    const int scale_cols = (p.K + 127) >> 7;
-
-    // this wave fetches and widens the tiles of row groups rgp + 2 wave, + 1 (rows past N: the last row group)
-    const uint8_t *a_panel = p.A + (size_t)rgp * p.K * 16;
+    // group, never stored), its token chunks (tokens past M: the last token)
+    P8Src src;
+    src.a = p.A + (size_t)rgp * p.K * 16 * WBYTES;
+    src.b = p.B;
     const int rga = min(rgp + 2 * wave, groups - 1), rgb = min(rgp + 2 * wave + 1, groups - 1);
-    const uint32_t a_voff = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * (uint32_t)p.K * 16u + (lane & 31) * 16;
-    const ScaleRow srow = load_scale_row(p.scale ? p.scale + (size_t)(rga >> 3) * scale_cols : nullptr, scale_cols, lane);
-    uint32_t b_voff[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int t = lane >> 2, oct = (lane & 3) ^ ((t >> 2) & 3);
-        const int tok = min(tok0 + (2 * wave + i) * 16 + t, p.M - 1);
-        b_voff[i] = (uint32_t)tok * (uint32_t)p.K * 2u + oct * 16;
+    ScaleRow srow;
+    if constexpr (FP8) {
+        src.a_off[0] = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * (uint32_t)p.K * 16u + (lane & 31) * 16;
+        const int scale_cols = (p.K + 127) >> 7;
+        srow = load_scale_row(p.scale ? p.scale + (size_t)(rga >> 3) * scale_cols : nullptr, scale_cols, lane);
+    } else {
+        src.a_off[0] = (uint32_t)(rga - rgp) * (uint32_t)p.K * 32u;
+        src.a_off[1] = (uint32_t)(rgb - rgp) * (uint32_t)p.K * 32u;
     }
-    const int g = lane >> 5, i32 = lane & 31, t16 = i32 & 15, hi = i32 >> 4;
-    const int a_idx = (wr * 4 + hi) * 64 + g * 16 + t16;
-    const int b_idx = 1024 + (wt * 8 + hi) * 64 + 4 * t16 + (g ^ ((t16 >> 2) & 3));
-
+#pragma unroll
+    for (int i = 0; i < Loop::NB; ++i) {
+        const int tok = min(tok0 + p8_chunk<TB>(wave, i) * 16 + (lane >> 2), p.M - 1);
+        src.b_off[i] = (uint32_t)tok * (uint32_t)p.K * 2u + p8_lane_octet(lane);
+    }
     f32x16 acc[PR][TB];
-#pragma unroll
-    for (int pr = 0; pr < PR; ++pr)
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[pr][tb][e] = 0.f;
-
-    u32x4 a0[PR], a1[PR], b0[TB], b1[TB];
-    auto rd = [&](u32x4 (&a)[PR], u32x4 (&b)[TB], int buf, int hs) {
-        const u32x4 *src = win + buf * kP8Slab;
-#pragma unroll
-        for (int pr = 0; pr < PR; ++pr) a[pr] = src[a_idx + 128 * pr + hs * 32];
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb) b[tb] = src[(b_idx ^ (hs * 2)) + 128 * tb];
-    };
-    auto mm = [&](const u32x4 (&a)[PR], const u32x4 (&b)[TB]) {
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int pr = 0; pr < PR; ++pr) acc[pr][tb] = T::mfma32(a[pr], b[tb], acc[pr][tb]);
-    };
-    // widen this wave's two tiles of slab `slab` (counted from k = 0) from raw buffer rb into bf16 slab buffer `buf`
-    auto widen = [&](int slab, int rb, int buf) {
-        const float sc = scale_at(srow, slab >> 2);
-        const u32x2 *raw = reinterpret_cast<const u32x2 *>(win + 4 * kP8Slab + rb * kP8RawSlab + 2 * wave * 32);
-        u32x4 *dst = win + buf * kP8Slab + 2 * wave * 64;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const u32x2 f = raw[i * 64 + lane];
-            uint32_t x0, x1, x2, x3;
-            fp8x4_to_bf16x4(f[0], sc, x0, x1);
-            fp8x4_to_bf16x4(f[1], sc, x2, x3);
-            dst[i * 64 + lane] = u32x4{x0, x1, x2, x3};
-        }
-    };
-    // Order of this wave's loads: chunks(0) raw(0) chunks(1) raw(1) chunks(2) raw(2) | raw(3) | then per trip s: chunks(s + 3)
-    // raw(s + 4).  Slabs past the end of the slice are fetched (and widened) as copies of its last slab and never multiplied.
-    const int last = slab0 + nslab - 1;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) p8_issue_fp8(a_panel, p.B, a_voff, b_voff, wave, min(slab0 + i, last), i, min(slab0 + i, last), i);
-    wait_vmcnt_le<3>();                                        // chunks and tiles of slabs 0 and 1 have landed
-    widen(min(slab0, last), 0, 0);
-    widen(min(slab0 + 1, last), 1, 1);
-    {   // raw(3) into the raw buffer that slab 0 has left
-        __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc((void *)a_panel, 0, 0xffffffffu, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, win + 4 * kP8Slab + 0 * kP8RawSlab + 2 * wave * 32, 16, a_voff,
-                                                 min(slab0 + 3, last) * 512, 0, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);                        // lgkmcnt(0): the widened tiles are written
-    bare_barrier();
-    rd(a0, b0, 0, 0);
-    int cur = 0, rcur = 0;                                     // ring buffer of slab s, raw buffer of slab s
-    for (int s = 0; s < nslab; ++s) {
-        const int nxt = (cur + 1) & 3, nx2 = (cur + 2) & 3, prv = (cur + 3) & 3;
-        const int r1 = rcur == 2 ? 0 : rcur + 1, r2 = rcur == 0 ? 2 : rcur - 1;      // raw buffers of slabs s + 1 (= s + 4), s + 2
-        p8_issue_fp8(a_panel, p.B, a_voff, b_voff, wave, min(slab0 + s + 3, last), prv, min(slab0 + s + 4, last), r1);
-        // the tiles of slab s + 2: everything younger than them may still be in flight (four loads in the first trip,
-        // where raw(3) went out alone; six from then on)
-        if (s == 0) wait_vmcnt_le<4>();
-        else wait_vmcnt_le<6>();
-        // the fp8 tiles are read first, widened between the products of the first half step and written after them
-        const float sc = scale_at(srow, min(slab0 + s + 2, last) >> 2);
-        const u32x2 *raw = reinterpret_cast<const u32x2 *>(win + 4 * kP8Slab + r2 * kP8RawSlab + 2 * wave * 32);
-        const u32x2 f0 = raw[lane], f1 = raw[64 + lane];
-        rd(a1, b1, cur, 1);
-        u32x4 w0, w1;
-        {
-            uint32_t x0, x1, x2, x3;
-            fp8x4_to_bf16x4(f0[0], sc, x0, x1);
-            fp8x4_to_bf16x4(f0[1], sc, x2, x3);
-            w0 = u32x4{x0, x1, x2, x3};
-            fp8x4_to_bf16x4(f1[0], sc, x0, x1);
-            fp8x4_to_bf16x4(f1[1], sc, x2, x3);
-            w1 = u32x4{x0, x1, x2, x3};
-        }
-        mm(a0, b0);
-        {
-            u32x4 *dst = win + nx2 * kP8Slab + 2 * wave * 64;
-            dst[lane] = w0;
-            dst[64 + lane] = w1;
-        }
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);       // the LDS reads
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-#pragma unroll
-        for (int m = 2; m < 8; ++m) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);   // six conversion instructions
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);       // the two LDS writes
-        __builtin_amdgcn_sched_barrier(0);
-        rd(a0, b0, nxt, 0);
-        mm(a1, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_vmcnt_le<4>();                                    // this wave's chunks of slab s + 2 have landed
-        __builtin_amdgcn_s_waitcnt(0xc07f);                    // and its widened tiles are written
-        bare_barrier();
-        cur = nxt;
-        rcur = r1;
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    mfma_settle();
+    zero_acc(acc);
+    Loop::run(acc, src, srow, slab0, nslab, wave, lane);
     __syncthreads();
     if (SK == 1) p8_store_panel<T>(p, acc, rg0, tok0 + wt * 128, wave, lane, win);
     else panel_finish<T, PR, TB, 8, 2>(p, acc, rg0, tok0 + wt * 128, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
@@ -751,7 +479,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         static bool ready_on[64] = {};                                                                             \
         bool &ready = ready_on[dev & 63];                                                                          \
         if (!ready) {                                                                                              \
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&KERNEL),                            \
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL),                            \
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)(LDS));           \
             if (e != hipSuccess) return fail(MLK_ERR_LAUNCH, hipGetErrorString(e));                                \
             ready = true;                                                                                          \
@@ -764,9 +492,9 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         // LDS: the ring, or the turn-around buffer of the output if that is larger
         constexpr size_t lds16 = kP8RingBytes > kP8OutBytes ? kP8RingBytes : kP8OutBytes;
         constexpr size_t lds8 = kP8Fp8LdsBytes > kP8OutBytes ? kP8Fp8LdsBytes : kP8OutBytes;
-        if (a_kind == MLK_FP8_E4M3) MLK_PANEL8(gemm_panel8_fp8_kernel<BF16>, lds8);
-        else if (a_kind == MLK_F16) MLK_PANEL8(gemm_panel8_kernel<F16>, lds16);
-        else MLK_PANEL8(gemm_panel8_kernel<BF16>, lds16);
+        if (a_kind == MLK_FP8_E4M3) MLK_PANEL8((gemm_panel8_kernel<BF16, true>), lds8);
+        else if (a_kind == MLK_F16) MLK_PANEL8((gemm_panel8_kernel<F16, false>), lds16);
+        else MLK_PANEL8((gemm_panel8_kernel<BF16, false>), lds16);
 #undef MLK_PANEL8
     } else if (rows == 256 && a_kind == MLK_FP8_E4M3 && (p.SK == 1 || p.whole_groups > 0)) {
         // soft-FP8, panels computed whole (or only the last round's sliced): the loop that prefetches through LDS, two
