@@ -173,6 +173,15 @@ __device__ __forceinline__ float lane_xor(float v, int mask) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, __float_as_int(v)));
 }
 
+// The lanes of one wave exchange values through LDS: the LDS unit runs a wave's accesses in program order, so
+// all that is needed between a store and the loads of other lanes is that the compiler keeps that order.  (A
+// workgroup barrier would do too, but this code also runs in a single wave of a larger workgroup.)
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Partial sums exchanged between workgroups of one kernel.  The L2 caches of the eight XCDs are
 // not coherent with each other for ordinary accesses; agent-scope atomic accesses are (they are
 // issued write-through / always-miss), and unlike an agent-scope fence they do not write back or

@@ -31,7 +31,8 @@ namespace mlk {
 
 constexpr int kMaxExperts = 256;
 constexpr int kMaxTopK = 32;
-constexpr int kMoeChunk = 256;     // tokens per expert-compute pass
+constexpr int kMoeChunk = 256;     // tokens per pass of the decode, row-shared and panel kernels
+constexpr int kMoeWideTokens = 4096, kMoeWidePairs = 16384;     // most tokens and routed pairs of a pass of the wide kernels
 static int g_moe_gemv1 = 1;        // experiment switch: GeMV-style kernels for a single token
 static int g_moe_tile = 1;         // experiment switch: row-shared kernels for tasks of more than one token block
 static inline bool moe_tile_path() { return g_moe_tile != 0; }
@@ -99,15 +100,6 @@ struct RouterLds {
     int pick_id[kMaxTopK];
     float pick_w[kMaxTopK];
 };
-
-// The lanes of one wave exchange values through LDS: the LDS unit runs a wave's accesses in program order, so
-// all that is needed between a store and the loads of other lanes is that the compiler keeps that order.  (A
-// workgroup barrier would do too, but this code also runs in a single wave of a larger workgroup.)
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Routing of one token by one wave; experts lane + 64 i live in register slot i of their lane (NE slots, so up
 // to 64 NE experts).  On return lane a < topk holds pick a (id and weight bits, in output order; the weight is
@@ -287,7 +279,7 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
                                                          int32_t *__restrict__ padded_blocks,
                                                          int32_t *__restrict__ experts_ids, int max_blocks,
                                                          MoeTask *__restrict__ tasks, int32_t *__restrict__ n_tasks,
-                                                         int cb_max) {
+                                                         int cb_max, int cb_unit) {
     constexpr int NW = 16;
     __shared__ int cnt[NW][kMaxExperts];   // per-wave counts, then per-wave write cursors
     __shared__ int start[kMaxExperts + 1]; // padded exclusive prefix
@@ -325,7 +317,7 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
     if (tid < E) {
         for (int w = 0; w < NW; ++w) total += cnt[w][tid];
         nb = (total + 15) >> 4;
-        ntk = (nb + cb_max - 1) / cb_max;
+        ntk = (nb + cb_max - 1) / cb_max;                       // cb_max is a multiple of cb_unit
         scan_pad[tid] = nb << 4;
         scan_task[tid] = ntk;
     }
@@ -349,14 +341,17 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
         start[e] = run;
         for (int b = 0; b < nb; ++b) experts_ids[(run >> 4) + b] = e;
         if (tasks) {
-            int nt = scan_task[e] - ntk;
-            for (int b = 0; b < nb; b += cb_max) {
+            // the tasks of an expert get nearly equal numbers of units of cb_unit blocks
+            const int first = scan_task[e] - ntk, units = (nb + cb_unit - 1) / cb_unit;
+            for (int i = 0; i < ntk; ++i) {
+                const int b0 = units * i / ntk * cb_unit, b1 = min(nb, units * (i + 1) / ntk * cb_unit);
                 MoeTask tk;
                 tk.expert = e;
-                tk.block0 = (run >> 4) + b;
-                tk.nblocks = min(cb_max, nb - b);
-                tk.pad = 0;
-                tasks[nt++] = tk;
+                tk.block0 = (run >> 4) + b0;
+                tk.nblocks = b1 - b0;
+                tk.first = (unsigned short)first;
+                tk.count = (unsigned short)ntk;
+                tasks[first + i] = tk;
             }
         }
         cumsum_out[e] = run + total;                    // where the reference's atomic cursor ends up
@@ -448,7 +443,7 @@ __device__ __forceinline__ void build_decode_tables(DecodeTables &t, const int32
             tk.expert = le;
             tk.block0 = nt + lane;
             tk.nblocks = 1;
-            tk.pad = 0;
+            tk.first = tk.count = 0;                        // not read by the decode kernels
             t.tasks[nt + lane] = tk;
         }
         nt += nb;
@@ -604,7 +599,7 @@ __global__ void __launch_bounds__(max_threads_for_tiles(2 * P * CB)) moe_gate_up
         }
         float h[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) h[i] = g[i] / (1.f + __expf(-g[i])) * u[i];
+        for (int i = 0; i < 4; ++i) h[i] = silu_mul(g[i], u[i]);
         const int n = (g0 + pr) * 16 + 4 * q;           // intermediate index = k of the down projection
         const size_t off = hbuf_offset(n, tk.block0 + cb, r16, p.SB);
         store4<T>(p.Hbuf + off, h[0], h[1], h[2], h[3]);
@@ -959,7 +954,7 @@ __global__ void __launch_bounds__(1024) moe_gate_up_gemv1_kernel(Moe1Args p) {
             g += red[g_local * p.WK + w][r];
             u += red[(p.G + g_local) * p.WK + w][r];
         }
-        const float h = g / (1.f + __expf(-g)) * u;
+        const float h = silu_mul(g, u);
         p.Hd[(size_t)blockIdx.y * p.I + (blockIdx.x * p.G + g_local) * 16 + r] = (uint16_t)T::from_f32(h);
     }
 }
@@ -1063,8 +1058,7 @@ __global__ void __launch_bounds__(256) moe_gate_up_tile_kernel(MoeArgs p) {
             if (cb >= tk.nblocks) continue;
             float h[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                h[i] = acc[2 * pr][cb][i] / (1.f + __expf(-acc[2 * pr][cb][i])) * acc[2 * pr + 1][cb][i];
+            for (int i = 0; i < 4; ++i) h[i] = silu_mul(acc[2 * pr][cb][i], acc[2 * pr + 1][cb][i]);
             const int n = (g0 + pr) * 16 + 4 * q;
             const size_t off = hbuf_offset(n, tk.block0 + cb, r16, p.SB);
             store4<T>(p.Hbuf + off, h[0], h[1], h[2], h[3]);
@@ -1160,11 +1154,7 @@ struct MoeWorkspace {
 
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-// Bytes of the fp32 buffer that holds the K-sliced down projections of one pass of tc tokens (defined below the
-// plan it reads).
-static size_t moe_obuf_bytes(int tc, int n_experts, int topk, int hidden, int inter);
-
-static size_t carve(uint8_t *base, int tc, int E, int K, int hidden, int inter, MoeWorkspace *ws) {
+static size_t carve(uint8_t *base, int tc, int E, int K, int hidden, int inter, size_t obuf_bytes, MoeWorkspace *ws) {
     const int n_pairs = tc * K;
     const int max_padded = n_pairs + E * 15;
     int max_blocks = (max_padded + 15) / 16;
@@ -1186,8 +1176,8 @@ static size_t carve(uint8_t *base, int tc, int E, int K, int hidden, int inter, 
     // seven spare blocks: the row-shared down kernel always fetches CB <= 8 consecutive blocks
     w.sb = max_blocks + 7;
     w.hbuf = (uint16_t *)take((size_t)inter * w.sb * 16 * 2);
-    // fp32 buffer of the K-sliced down projections, sized for the slices the plan of this pass really uses
-    w.obuf = (float *)take(moe_obuf_bytes(tc, E, K, hidden, inter));
+    // fp32 buffer of the K-sliced down projections
+    w.obuf = (float *)take(obuf_bytes);
     w.counters = (int32_t *)take(sizeof(int32_t) * (size_t)(hidden / 16));
     if (ws) *ws = w;
     return off;
@@ -1398,21 +1388,76 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
     return pl;
 }
 
-// Per routed pair and slice for the row-shared and panel kernels, per token and slice for the decode kernels,
-// nothing for the single-token kernels; the larger of the two weight kinds, since the workspace query does not
-// know which one the call will bring.
-static size_t moe_obuf_bytes(int tc, int n_experts, int topk, int hidden, int inter) {
-    size_t bytes = 256;
-    for (int fp8 = 0; fp8 < 2; ++fp8) {
-        const MoePlan pl = moe_plan(tc, n_experts, topk, hidden, inter, fp8 != 0);
-        size_t need = 0;
-        if (pl.path == kMoePathTile || pl.path == kMoePathPanel)
-            need = (size_t)tc * topk * pl.down_slices * hidden * sizeof(float);
-        else if (pl.path != kMoePathGemv1)
-            need = (size_t)tc * pl.down_slices * hidden * sizeof(float);
-        if (need > bytes) bytes = need;
+// ------------------------------------------------------------ passes
+// A call of up to kMoeChunk tokens is one pass of the kernels moe_plan() names.  A longer one goes through the wide kernels
+// (mlk_moe_wide.cuh) in passes of as many tokens as their workspace is allowed for: in passes of kMoeChunk tokens every
+// pass streams the weights of all experts again.  Measured, passes of kMoeChunk tokens -> wide kernels (us):
+//   8 experts, top-2, H 4096, I 14336, bf16      300 tokens  994 ->  590    512  1077 -> 678    2048  4287 -> 1684
+//   the same, soft-FP8                           300         659 ->  514    512   786 -> 629    2048  3098 -> 1805
+//   256 experts, top-8, H 7168, I 256, soft-FP8  300         474 ->  450    600   801 -> 535    2048  2195 ->  909
+//   128 experts, top-8, H 2048, I 768, bf16                                 512   480 -> 294    2048  1904 ->  509
+// At 256 tokens, one pass either way, the small kernels are ahead (541 / 576, 394 / 488, 282 / 428, 245 / 260 us).
+// A remainder of up to kMoeChunk tokens is a pass of the small kernels again.
+struct MoePass {
+    bool wide;
+    int tokens;
+    int cb, cb_unit;      // token blocks per task and the unit they are dealt in
+    int max_tasks;        // upper bound of the task list
+    int down_slices;
+    size_t obuf_bytes;
+    MoePlan plan;         // of a pass that is not wide
+};
+
+extern template int launch_moe_wide<BF16, false>(const MoeArgs &, int, float *, int, hipStream_t);
+extern template int launch_moe_wide<F16, false>(const MoeArgs &, int, float *, int, hipStream_t);
+extern template int launch_moe_wide<BF16, true>(const MoeArgs &, int, float *, int, hipStream_t);
+
+// K slices of the wide down projection: its panels run one per CU in rounds, so a grid of one and a half rounds wastes a
+// quarter of the chip unless the panels are cut.  In units of a k32 slab of a panel (0.75 us): a panel costs its slabs and
+// about eight more to start and to store; a slice costs the write and the read of its partial products (8 experts, bf16,
+// 1, 2, 3 slices: 677, 579, 615 us at 256 tokens, 1782, 1689, 1667 us at 2048).
+static int moe_wide_down_slices(int tokens, int n_experts, int topk, int hidden, int inter) {
+    const int cus = device_cus();
+    const double pairs = (double)tokens * topk, mean = pairs / n_experts;
+    const double tasks = ceil((mean + 0.5 * sqrt(mean)) / (16 * kWideTaskBlocks)) * (pairs < n_experts ? pairs : n_experts);
+    const double per_slice = pairs * hidden * 8 / 5e6 / 0.75;
+    int best = 1;
+    double best_cost = 0;
+    for (int skd = 1; skd <= 4 && inter / 128 / skd >= 2; ++skd) {
+        const double rounds = ceil(tasks * ((hidden + 255) / 256) * skd / cus);
+        const double cost = rounds * (inter / 32.0 / skd + 8) + per_slice * skd;
+        if (skd == 1 || cost < best_cost) best = skd, best_cost = cost;
     }
-    return bytes;
+    return best;
+}
+
+static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8) {
+    MoePass ps = {};
+    ps.wide = tokens_left > kMoeChunk;
+    if (!ps.wide) {
+        ps.tokens = tokens_left < kMoeChunk ? tokens_left : kMoeChunk;
+        ps.plan = moe_plan(ps.tokens, n_experts, topk, hidden, inter, fp8);
+        ps.cb = moe_blocks_per_task(ps.tokens, topk, n_experts);
+        ps.cb_unit = 1;
+        ps.max_tasks = ps.plan.max_tasks;
+        ps.down_slices = ps.plan.down_slices;
+        // per routed pair and slice for the row-shared and panel kernels, per token and slice for the decode kernels,
+        // nothing for the single-token kernels
+        if (ps.plan.path == kMoePathTile || ps.plan.path == kMoePathPanel)
+            ps.obuf_bytes = (size_t)ps.tokens * topk * ps.down_slices * hidden * sizeof(float);
+        else if (ps.plan.path != kMoePathGemv1)
+            ps.obuf_bytes = (size_t)ps.tokens * ps.down_slices * hidden * sizeof(float);
+        return ps;
+    }
+    const int most = kMoeWidePairs / topk < kMoeWideTokens ? kMoeWidePairs / topk : kMoeWideTokens;
+    ps.tokens = tokens_left < most ? tokens_left : most;
+    const int pairs = ps.tokens * topk;
+    ps.cb = kWideTaskBlocks;
+    ps.cb_unit = 4;
+    ps.max_tasks = (n_experts < pairs ? n_experts : pairs) + pairs / (16 * kWideTaskBlocks);
+    ps.down_slices = moe_wide_down_slices(ps.tokens, n_experts, topk, hidden, inter);
+    ps.obuf_bytes = (size_t)pairs * ps.down_slices * hidden * sizeof(float);
+    return ps;
 }
 
 }  // namespace mlk
@@ -1488,20 +1533,28 @@ extern "C" int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_
     const int max_blocks = (n_pairs + n_experts * 15 + 15) / 16;
     moe_align_kernel<<<1, 1024, 0, (hipStream_t)stream>>>(topk_ids, n_pairs, n_experts, experts_map, sorted_token_ids,
                                                           cumsum_buffer, padded_num_blocks, experts_ids, max_blocks,
-                                                          nullptr, nullptr, 1);
+                                                          nullptr, nullptr, 1, 1);
     MLK_LAUNCH_CHECK();
     return MLK_OK;
 }
 
 extern "C" size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
-    // the passes of a call share the workspace: full passes of kMoeChunk tokens and a shorter last one, whose plan
-    // (more K slices over fewer pairs) may ask for a different carving
-    const int tc = n_tokens < kMoeChunk ? n_tokens : kMoeChunk;
-    size_t bytes = carve(nullptr, tc, n_experts, topk, hidden, inter, nullptr);
-    const int last = n_tokens > kMoeChunk ? n_tokens % kMoeChunk : 0;
-    if (last > 0) {
-        const size_t b2 = carve(nullptr, last, n_experts, topk, hidden, inter, nullptr);
-        if (b2 > bytes) bytes = b2;
+    // the passes of a call share the workspace; the larger of the two weight kinds, since the query does not know which one
+    // the call will bring.  A call of more than one pass is also given what passes of kMoeChunk tokens would need.
+    size_t bytes = 0;
+    for (int fp8 = 0; fp8 < 2; ++fp8) {
+        auto cover = [&](int tokens) {
+            const MoePass ps = moe_pass(tokens, n_experts, topk, hidden, inter, fp8 != 0);
+            const size_t b = carve(nullptr, ps.tokens, n_experts, topk, hidden, inter, ps.obuf_bytes + 256, nullptr);
+            if (b > bytes) bytes = b;
+            return ps.tokens;
+        };
+        const int first = cover(n_tokens);
+        if (n_tokens > kMoeChunk) {
+            cover(kMoeChunk);
+            if (n_tokens % kMoeChunk) cover(n_tokens % kMoeChunk);
+            if (n_tokens % first) cover(n_tokens % first);
+        }
     }
     return bytes;
 }
@@ -1527,19 +1580,20 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
                 "moe: workspace too small");
     hipStream_t s = (hipStream_t)stream;
 
-    for (int t0 = 0; t0 < n_tokens; t0 += kMoeChunk) {
-        const int tc = n_tokens - t0 < kMoeChunk ? n_tokens - t0 : kMoeChunk;
+    for (int t0 = 0, tc = 0; t0 < n_tokens; t0 += tc) {
+        const MoePass ps = moe_pass(n_tokens - t0, n_experts, topk, hidden, inter, fp8);
+        const MoePlan &pl = ps.plan;
+        tc = ps.tokens;
         const int n_pairs = tc * topk;
-        const MoePlan pl = moe_plan(tc, n_experts, topk, hidden, inter, fp8);
-        const int cb = moe_blocks_per_task(tc, topk, n_experts);
+        const int cb = ps.cb;
         MoeWorkspace ws;
-        carve((uint8_t *)workspace, tc, n_experts, topk, hidden, inter, &ws);
+        carve((uint8_t *)workspace, tc, n_experts, topk, hidden, inter, ps.obuf_bytes + 256, &ws);
         const int max_padded = n_pairs + n_experts * 15;
         int max_blocks = (max_padded + 15) / 16;
         if (max_blocks < (n_pairs < kDecodePairs ? n_pairs : kDecodePairs)) max_blocks = n_pairs < kDecodePairs ? n_pairs : kDecodePairs;
-        const int max_tasks = pl.max_tasks;
+        const int max_tasks = ps.max_tasks;
         // one token: every routed pair is a GeMV with the activations in LDS
-        if (pl.path == kMoePathGemv1) {
+        if (!ps.wide && pl.path == kMoePathGemv1) {
             Moe1Args m;
             m.W1 = (const uint8_t *)w1;
             m.W2 = (const uint8_t *)w2;
@@ -1589,11 +1643,11 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
             continue;
         }
         // decode-sized batches align inside the GeMM kernels; larger ones run the alignment kernel
-        const bool inline_align = pl.path == kMoePathDecodeInline;
+        const bool inline_align = !ps.wide && pl.path == kMoePathDecodeInline;
         if (!inline_align) {
             moe_align_kernel<<<1, 1024, 0, s>>>(topk_ids + (size_t)t0 * topk, n_pairs, n_experts, experts_map,
                                                 ws.sorted, ws.cumsum, ws.padded, ws.experts_ids, max_blocks, ws.tasks,
-                                                ws.n_tasks, cb);
+                                                ws.n_tasks, cb, ps.cb_unit);
             MLK_LAUNCH_CHECK();
         }
         MoeArgs a;
@@ -1622,6 +1676,20 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
         a.counters = ws.counters;
         a.n_counters = hidden / 16;
         int rc;
+        if (ps.wide) {
+            const int skd = ps.down_slices;
+            const dim3 cgrid(tc, (hidden + 1023) / 1024);
+            if (fp8) rc = launch_moe_wide<BF16, true>(a, max_tasks, ws.obuf, skd, s);
+            else if (x_kind == MLK_F16) rc = launch_moe_wide<F16, false>(a, max_tasks, ws.obuf, skd, s);
+            else rc = launch_moe_wide<BF16, false>(a, max_tasks, ws.obuf, skd, s);
+            if (rc != MLK_OK) return rc;
+            if (x_kind == MLK_F16)
+                moe_combine_kernel<F16><<<cgrid, 256, 0, s>>>(ws.obuf, a.Y, a.topk_ids, a.experts_map, topk, hidden, n_experts, skd);
+            else
+                moe_combine_kernel<BF16><<<cgrid, 256, 0, s>>>(ws.obuf, a.Y, a.topk_ids, a.experts_map, topk, hidden, n_experts, skd);
+            MLK_LAUNCH_CHECK();
+            continue;
+        }
         if (pl.path == kMoePathPanel) {
             const int tb32 = moe_panel_tb32(cb), skd = pl.down_slices;
             const dim3 cgrid(tc, (hidden + 1023) / 1024);

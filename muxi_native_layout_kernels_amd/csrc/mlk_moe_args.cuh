@@ -8,7 +8,8 @@ namespace mlk {
 // One pass over an expert's weights: the token blocks block0 .. block0 + nblocks - 1 of the alignment
 // (16 routed pairs each) belong to `expert`.
 struct MoeTask {
-    int expert, block0, nblocks, pad;
+    int expert, block0, nblocks;
+    unsigned short first, count;      // the expert's tasks: index of the first one in the list and how many there are
 };
 
 struct MoeArgs {
@@ -37,5 +38,28 @@ struct MoeArgs {
 // [routed pair][K slice][H] for moe_combine_kernel.  Needs H % 256 == 0.
 template <class T, bool FP8>
 int launch_moe_panel(const MoeArgs &a, int tb32, int max_tasks, float *obuf, int skd, bool down_pairs, hipStream_t s);
+
+// The wide kernels (mlk_moe_wide.cuh): gate/up and down projection of tasks of up to kWideTaskBlocks blocks; same
+// intermediate and obuf as the panel kernels.
+constexpr int kWideTaskBlocks = 16;
+template <class T, bool FP8>
+int launch_moe_wide(const MoeArgs &a, int max_tasks, float *obuf, int skd, hipStream_t s);
+
+// SiLU(gate) * up
+__device__ __forceinline__ float silu_mul(float gate, float up) { return gate / (1.f + __expf(-gate)) * up; }
+
+// More than 64 KiB of dynamic LDS has to be allowed once per kernel and device.
+template <class K>
+static int panel_lds_attribute(K kernel, size_t lds, bool (&ready_on)[64]) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+    bool &ready = ready_on[dev & 63];
+    if (!ready && lds > 48 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return fail(MLK_ERR_LAUNCH, hipGetErrorString(e));
+    }
+    ready = true;
+    return MLK_OK;
+}
 
 }  // namespace mlk

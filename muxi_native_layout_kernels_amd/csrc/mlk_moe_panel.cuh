@@ -90,8 +90,7 @@ __global__ void __launch_bounds__(256, 2) moe_gate_up_panel_kernel(MoeArgs p) {
             float h[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float gate = acc[0][tb][4 * g + e], up = acc[1][tb][4 * g + e];
-                h[e] = gate / (1.f + __expf(-gate)) * up;
+                h[e] = silu_mul(acc[0][tb][4 * g + e], acc[1][tb][4 * g + e]);
             }
             store4<T>(row + 8 * g, h[0], h[1], h[2], h[3]);
         }
@@ -155,20 +154,6 @@ __global__ void __launch_bounds__(256, 2) moe_down_panel_kernel(MoeArgs p, float
                 *reinterpret_cast<f32x4 *>(row + pr * 32 + 8 * g) = v;
             }
     }
-}
-
-// More than 64 KiB of dynamic LDS has to be allowed once per kernel and device.
-template <class K>
-static int panel_lds_attribute(K kernel, size_t lds, bool (&ready_on)[64]) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    bool &ready = ready_on[dev & 63];
-    if (!ready && lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return fail(MLK_ERR_LAUNCH, hipGetErrorString(e));
-    }
-    ready = true;
-    return MLK_OK;
 }
 
 template <class T, bool FP8, int TB>

@@ -1,0 +1,229 @@
+// Fused MoE for prefill-sized batches on the eight-wave panel loop (mlk_panel8.cuh): all tokens of a pass go through the
+// two grouped products at once, so that every expert's weights are streamed once per pass and the matrix cores set the pace.
+//
+//   gate/up   panel = 128 columns of the intermediate (128 gate rows and the 128 up rows with the same index, dealt to
+//             the four row quarters of the panel as 32 + 32, so that gate and up of an element sit in the same
+//             accumulator slot of one wave) x the up to 256 routed tokens of a task.  SiLU(gate) * up goes to the
+//             intermediate, row-major [slot][I], turned around in LDS so that whole lines are stored.
+//   down      panel = 256 output rows x the same task over one K slice; products times the routing weight go to an fp32
+//             buffer [routed pair][K slice][H] for moe_combine_kernel, which adds them per token in pick order.
+//
+// A task holds up to 16 blocks of 16 routed tokens of one expert; an expert with more is split into tasks of nearly equal
+// size in units of 64 tokens (moe_align_kernel), and a panel multiplies 64, 128, 192 or 256 token columns, whichever covers
+// its task: with 512 +- 20 tokens per expert (2048 tokens, 8 experts, top-2) tasks filled to 256 first would leave a third,
+// nearly empty panel for half of the experts.
+//
+// Order of the work: the (expert, row tile, task of the expert) triples, tasks fastest, form one line that is cut into
+// eight equal runs, one per XCD (workgroup id modulo 8).  The tasks of an expert that share a row tile's weights then run
+// next to each other on one L2, and an XCD works on few experts at a time, so its token rows stay there too.
+//
+// Bound: the matrix cores (power: about 1.35 PFLOP/s in bf16, see mlk_panel.hip); fp32 partial products of the down
+// projection are 4 H bytes per routed pair and slice, written and read once.
+#pragma once
+
+#include "mlk_moe_args.cuh"
+#include "mlk_panel8.cuh"
+
+namespace mlk {
+
+constexpr int kWideOutPitch = 272;                             // gate/up turn-around buffer: bytes per token (128 columns)
+constexpr int kWideDownPitch = 144;                            // down: bytes per token (32 fp32 rows of one wave)
+constexpr size_t kWideDownOut = (size_t)8 * 128 * kWideDownPitch;
+
+// The workgroup's place on the line of n items: XCD id % 8 takes the id % 8-th run.  Returns n or more when there is none.
+__device__ __forceinline__ int wide_item(int id, int n) {
+    const int per = (n + 7) >> 3;
+    const int j = id >> 3;
+    return j < per ? (id & 7) * per + j : n;
+}
+
+template <class T, bool FP8, int TB>
+__device__ __forceinline__ void moe_gate_up_wide(const MoeArgs &p, const MoeTask &tk, int rt, int wave, int lane) {
+    extern __shared__ u32x4 win[];
+    constexpr int WB = FP8 ? 1 : 2;
+    using Loop = Panel8Loop<T, FP8, TB>;
+    const int wr = wave & 3, wt = wave >> 2;
+    const int groups_i = p.I >> 4;
+    const uint32_t tile_row = (uint32_t)p.H * 16u * WB;          // bytes of a row group
+    P8Src src;
+    src.a = p.W1 + (size_t)tk.expert * 2 * p.I * p.H * WB + (size_t)rt * 8 * tile_row;
+    src.b = p.X;
+    // tiles 2 wave, 2 wave + 1 of the panel: quarter wave / 2, its gate tiles (even waves) or up tiles (odd waves)
+    const int half = wave & 1, rg = (wave >> 1) * 2;
+    const uint32_t tile0 = (uint32_t)(half * groups_i + rg) * tile_row;
+    ScaleRow srow;
+    if constexpr (FP8) {
+        src.a_off[0] = tile0 + (lane >> 5 ? tile_row : 0u) + (lane & 31) * 16;
+        const int cols = p.H >> 7, block = (half * groups_i + rt * 8 + rg) >> 3;
+        srow = load_scale_row(p.S1 ? p.S1 + ((size_t)tk.expert * (2 * p.I >> 7) + block) * cols : nullptr, cols, lane);
+    } else {
+        src.a_off[0] = tile0;
+        src.a_off[1] = tile0 + tile_row;
+    }
+    const int slots = tk.nblocks * 16;
+    const int32_t *sorted = p.sorted + tk.block0 * 16;
+#pragma unroll
+    for (int i = 0; i < Loop::NB; ++i) {
+        // slots without a routed pair read token 0: their columns of the product are never used
+        const int slot = p8_chunk<TB>(wave, i) * 16 + (lane >> 2);
+        const int id = slot < slots ? sorted[slot] : p.n_pairs;
+        const int tok = id < p.n_pairs ? id / p.K : 0;
+        src.b_off[i] = (uint32_t)tok * (uint32_t)p.H * 2u + p8_lane_octet(lane);
+    }
+    f32x16 acc[2][TB];
+    zero_acc(acc);
+    Loop::run(acc, src, srow, 0, p.H >> 5, wave, lane);
+    __syncthreads();
+
+    // accumulator element 4 g + e of lane 32 h + c: column 8 g + 4 h + e of the wave's 32, token c of the block's 32
+    uint8_t *out = reinterpret_cast<uint8_t *>(win);
+    const int h4 = lane >> 5, c32 = lane & 31;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = silu_mul(acc[0][tb][4 * g + e], acc[1][tb][4 * g + e]);
+            u32x2 o;
+            o[0] = T::from_f32x2(h[0], h[1]);
+            o[1] = T::from_f32x2(h[2], h[3]);
+            *reinterpret_cast<u32x2 *>(out + ((wt * TB + tb) * 32 + c32) * kWideOutPitch + wr * 64 + g * 16 + h4 * 8) = o;
+        }
+    __syncthreads();
+    // sixteen lanes store the 256 bytes of a slot; slots without a routed pair are stored too (nobody reads them)
+    const int q = threadIdx.x & 15;
+    uint16_t *dst = p.Hbuf + (size_t)tk.block0 * 16 * p.I + rt * 128 + q * 8;
+#pragma unroll
+    for (int it = 0; it < 2 * TB; ++it) {
+        const int slot = it * 32 + (threadIdx.x >> 4);
+        if (slot < slots)
+            *reinterpret_cast<u32x4 *>(dst + (size_t)slot * p.I) = *reinterpret_cast<const u32x4 *>(out + slot * kWideOutPitch + q * 16);
+    }
+}
+
+template <class T, bool FP8>
+__global__ void __launch_bounds__(512) moe_gate_up_wide_kernel(MoeArgs p) {
+    const int row_tiles = p.I >> 7;
+    const int n_items = row_tiles * p.n_tasks[0];
+    const int item = wide_item(blockIdx.x, n_items);
+    if (item >= n_items) return;
+    const MoeTask t0 = p.tasks[item / row_tiles];                // some task of the item's expert
+    const int local = item - (int)t0.first * row_tiles;
+    const int rt = local / t0.count;
+    const MoeTask tk = p.tasks[t0.first + local % t0.count];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    switch ((tk.nblocks + 3) >> 2) {
+        case 1: moe_gate_up_wide<T, FP8, 1>(p, tk, rt, wave, lane); break;
+        case 2: moe_gate_up_wide<T, FP8, 2>(p, tk, rt, wave, lane); break;
+        case 3: moe_gate_up_wide<T, FP8, 3>(p, tk, rt, wave, lane); break;
+        default: moe_gate_up_wide<T, FP8, 4>(p, tk, rt, wave, lane); break;
+    }
+}
+
+template <class T, bool FP8, int TB>
+__device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restrict__ O, int skd, const MoeTask &tk, int rt, int sk,
+                                              int wave, int lane) {
+    extern __shared__ u32x4 win[];
+    constexpr int WB = FP8 ? 1 : 2;
+    using Loop = Panel8Loop<T, FP8, TB>;
+    const int wr = wave & 3, wt = wave >> 2;
+    const uint32_t tile_row = (uint32_t)p.I * 16u * WB;
+    const int groups = p.H >> 4, rgp = rt * 16;
+    P8Src src;
+    src.a = p.W2 + (size_t)tk.expert * p.H * p.I * WB + (size_t)rgp * tile_row;
+    src.b = p.Hbuf + (size_t)tk.block0 * 16 * p.I;
+    // rows past H: a copy of the last row group, never stored
+    const int rga = min(rgp + 2 * wave, groups - 1), rgb = min(rgp + 2 * wave + 1, groups - 1);
+    ScaleRow srow;
+    if constexpr (FP8) {
+        src.a_off[0] = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * tile_row + (lane & 31) * 16;
+        const int cols = p.I >> 7;
+        srow = load_scale_row(p.S2 ? p.S2 + ((size_t)tk.expert * (p.H >> 7) + (rga >> 3)) * cols : nullptr, cols, lane);
+    } else {
+        src.a_off[0] = (uint32_t)(rga - rgp) * tile_row;
+        src.a_off[1] = (uint32_t)(rgb - rgp) * tile_row;
+    }
+    const int slots = tk.nblocks * 16;
+#pragma unroll
+    for (int i = 0; i < Loop::NB; ++i) {
+        const int slot = p8_chunk<TB>(wave, i) * 16 + (lane >> 2);
+        src.b_off[i] = (uint32_t)(slot < slots ? slot : 0) * (uint32_t)p.I * 2u + p8_lane_octet(lane);
+    }
+    const int nwin = p.I >> 7;                                     // K slices are cut at multiples of 128 k
+    const int wbeg = (int)((long long)sk * nwin / skd), wend = (int)((long long)(sk + 1) * nwin / skd);
+    f32x16 acc[2][TB];
+    zero_acc(acc);
+    Loop::run(acc, src, srow, 4 * wbeg, 4 * (wend - wbeg), wave, lane);
+    __syncthreads();
+
+    // every wave turns its 32 rows x 32 TB tokens around in its own part of LDS, one row pair after the other, and stores
+    // 128 bytes of a routed pair with eight lanes
+    uint8_t *out = reinterpret_cast<uint8_t *>(win) + (size_t)wave * 128 * kWideDownPitch;
+    const int h4 = lane >> 5, c32 = lane & 31, t8 = lane >> 3, q = lane & 7;
+    const int n0 = (rgp + wr * 4) * 16;
+    if (n0 >= p.H) return;
+    const int32_t *sorted = p.sorted + tk.block0 * 16;
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<f32x4 *>(out + (tb * 32 + c32) * kWideDownPitch + g * 32 + h4 * 16) =
+                    f32x4{acc[pr][tb][4 * g], acc[pr][tb][4 * g + 1], acc[pr][tb][4 * g + 2], acc[pr][tb][4 * g + 3]};
+        wave_lds_sync();
+#pragma unroll 4
+        for (int it = 0; it < 4 * TB; ++it) {
+            const int slot = wt * TB * 32 + it * 8 + t8;
+            const int id = slot < slots ? sorted[slot] : p.n_pairs;
+            if (id < p.n_pairs) {
+                f32x4 v = *reinterpret_cast<const f32x4 *>(out + (it * 8 + t8) * kWideDownPitch + q * 16);
+                v *= T::to_f32(p.wts[id]);
+                *reinterpret_cast<f32x4 *>(O + ((size_t)id * skd + sk) * p.H + n0 + pr * 32 + q * 4) = v;
+            }
+        }
+        wave_lds_sync();
+    }
+}
+
+template <class T, bool FP8>
+__global__ void __launch_bounds__(512) moe_down_wide_kernel(MoeArgs p, float *__restrict__ O, int skd) {
+    const int row_tiles = (p.H + 255) >> 8, per_task = row_tiles * skd;
+    const int n_items = per_task * p.n_tasks[0];
+    const int item = wide_item(blockIdx.x, n_items);
+    if (item >= n_items) return;
+    const MoeTask t0 = p.tasks[item / per_task];
+    const int local = item - (int)t0.first * per_task;
+    const int rs = local / t0.count;                               // slice-major: co-running workgroups share a K window
+    const int sk = rs / row_tiles, rt = rs - sk * row_tiles;
+    const MoeTask tk = p.tasks[t0.first + local % t0.count];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    switch ((tk.nblocks + 3) >> 2) {
+        case 1: moe_down_wide<T, FP8, 1>(p, O, skd, tk, rt, sk, wave, lane); break;
+        case 2: moe_down_wide<T, FP8, 2>(p, O, skd, tk, rt, sk, wave, lane); break;
+        case 3: moe_down_wide<T, FP8, 3>(p, O, skd, tk, rt, sk, wave, lane); break;
+        default: moe_down_wide<T, FP8, 4>(p, O, skd, tk, rt, sk, wave, lane); break;
+    }
+}
+
+template <class T, bool FP8>
+int launch_moe_wide(const MoeArgs &a, int max_tasks, float *obuf, int skd, hipStream_t s) {
+    constexpr size_t ring = FP8 ? kP8Fp8LdsBytes : kP8RingBytes;
+    constexpr size_t lds_up = ring, lds_down = ring > kWideDownOut ? ring : kWideDownOut;
+    static bool ready_up[64] = {}, ready_down[64] = {};
+    int rc = panel_lds_attribute(&moe_gate_up_wide_kernel<T, FP8>, lds_up, ready_up);
+    if (rc != MLK_OK) return rc;
+    rc = panel_lds_attribute(&moe_down_wide_kernel<T, FP8>, lds_down, ready_down);
+    if (rc != MLK_OK) return rc;
+    const int items_up = (a.I >> 7) * max_tasks, items_down = ((a.H + 255) >> 8) * skd * max_tasks;
+    moe_gate_up_wide_kernel<T, FP8><<<(items_up + 7) / 8 * 8, 512, lds_up, s>>>(a);
+    MLK_LAUNCH_CHECK();
+    moe_down_wide_kernel<T, FP8><<<(items_down + 7) / 8 * 8, 512, lds_down, s>>>(a, obuf, skd);
+    MLK_LAUNCH_CHECK();
+    return MLK_OK;
+}
+
+}  // namespace mlk

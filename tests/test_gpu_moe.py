@@ -628,3 +628,23 @@ def test_fused_moe_soft_fp8_many_experts_near_a_full_pass(mlk, T):
     E = 256
     bias = randn((E,), torch.bfloat16, 0.05, 78).abs()
     _moe_case(mlk, T, E, 8, 512, 256, torch.bfloat16, 1500 + T, score="sigmoid", groups=(8, 4), bias=bias, fp8=True)
+
+
+@pytest.mark.parametrize("T,E,K,H,I,kind", [
+    (257, 2, 2, 128, 128, "bf16"),       # first size above one pass of the smaller kernels; less than one panel of rows
+    (271, 1, 1, 384, 256, "fp16"),       # 17 blocks of one expert: tasks of 128 and 143 tokens, ragged row tile
+    (530, 2, 1, 256, 384, "bf16"),       # two to three tasks per expert, 64-token units
+    (1000, 4, 2, 640, 128, "fp8"),       # tasks of 192 and 256 columns, ragged row tile, one scale block of I
+    (300, 48, 6, 256, 256, "fp8"),       # about 37 tokens per expert: panels of 64 columns
+    (300, 16, 3, 384, 2048, "fp16"),     # few row tiles and a long I: K slices
+    (700, 5, 5, 128, 512, "bf16"),       # every token on every expert
+    (4096 + 100, 4, 1, 128, 128, "bf16"),  # a full pass and a remainder on the smaller kernels
+])
+def test_fused_moe_wide_kernels(mlk, T, E, K, H, I, kind):
+    """More than 256 tokens run the wide kernels: edges of tasks, token columns, row tiles, passes and K slices."""
+    dtype = torch.float16 if kind == "fp16" else torch.bfloat16
+    emap = None
+    if K == E:
+        emap = np.arange(E, dtype=np.int32)       # every pick of a token, but for an absent expert
+        emap[-1] = -1 if E > 2 else emap[-1]
+    _moe_case(mlk, T, E, K, H, I, dtype, 7000 + T, fp8=kind == "fp8", emap=emap)
