@@ -48,18 +48,4 @@ int launch_moe_wide(const MoeArgs &a, int max_tasks, float *obuf, int skd, hipSt
 // SiLU(gate) * up
 __device__ __forceinline__ float silu_mul(float gate, float up) { return gate / (1.f + __expf(-gate)) * up; }
 
-// More than 64 KiB of dynamic LDS has to be allowed once per kernel and device.
-template <class K>
-static int panel_lds_attribute(K kernel, size_t lds, bool (&ready_on)[64]) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    bool &ready = ready_on[dev & 63];
-    if (!ready && lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return fail(MLK_ERR_LAUNCH, hipGetErrorString(e));
-    }
-    ready = true;
-    return MLK_OK;
-}
-
 }  // namespace mlk

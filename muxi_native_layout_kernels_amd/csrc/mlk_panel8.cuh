@@ -114,25 +114,6 @@ struct Panel8Loop {
 #pragma unroll
                 for (int pr = 0; pr < PR; ++pr) acc[pr][tb] = T::mfma32(a[pr], b[tb], acc[pr][tb]);
         };
-        // a step's products with the LDS reads of the next step, and the first step's with the loads, spread between them
-        auto spread = [&](int m, int n, int slots) { return ((m + 1) * n + slots - 1) / slots - (m * n + slots - 1) / slots; };
-        auto order = [&](auto loads_c) {
-            constexpr int NM = 2 * TB, ND = PR + TB, NL = decltype(loads_c)::value ? NA + NB : 0;
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                const int ds = spread(m, ND, NM);
-                if (ds == 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                if (ds == 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-                if (NL > 0) {
-                    constexpr int slots = NM < NL ? NM : (NL > 0 ? NL : 1);
-                    const int ld = m < slots ? spread(m, NL, slots) : 0;
-                    if (ld == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                    if (ld == 2) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        };
         // slabs past the end are fetched as copies of the last slab and never multiplied, which keeps the count of loads
         // in flight the same in every trip
         const int last = slab0 + nslab - 1;
@@ -148,14 +129,14 @@ struct Panel8Loop {
             int cur = 0;                                           // ring buffer of slab s
             for (int s = 0; s < nslab; ++s) {
                 const int nxt = (cur + 1) & 3, prv = (cur + 3) & 3;
+                rd(a1, b1, cur, 1);
                 issue_a(src, wave, min(slab0 + s + RING - 1, last), prv);
                 issue_b(src, wave, min(slab0 + s + RING - 1, last), prv);
-                rd(a1, b1, cur, 1);
                 mm(a0, b0);
-                order(std::true_type{});
+                spread_half_step<2 * TB, PR + TB, NA + NB>();
                 rd(a0, b0, nxt, 0);
                 mm(a1, b1);
-                order(std::false_type{});
+                spread_half_step<2 * TB, PR + TB, 0>();
                 wait_vmcnt_le<(NA + NB) * (RING - 3)>();           // this wave's loads of slab s + 2 have landed
                 bare_barrier();
                 cur = nxt;
