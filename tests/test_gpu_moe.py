@@ -114,7 +114,7 @@ def test_align_reference_example(mlk):
 
 
 @pytest.mark.parametrize("T,K,E", [(1, 2, 8), (16, 2, 8), (64, 2, 8), (256, 2, 8), (33, 8, 256), (2048, 8, 256),
-                                   (1000, 6, 64), (3, 1, 5)])
+                                   (1000, 6, 64), (3, 1, 5), (513, 3, 255), (700, 1, 1), (1025, 4, 127)])
 def test_align_random(mlk, T, K, E):
     rng = np.random.default_rng(T * 31 + K)
     ids = torch.from_numpy(np.stack([rng.choice(E, size=K, replace=False) for _ in range(T)]))
