@@ -267,14 +267,16 @@ int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_experts, in
  *   y [T, H] of x_kind (overwritten; needs no zero fill)
  *   workspace: at least mlk_moe_workspace_bytes() bytes of device scratch
  *   (alignment tables and the SiLU intermediate); contents are not preserved.
- * H % 128 == 0, I % 128 == 0, E <= 256.  Up to 256 tokens are one pass;
- * more go through the wide kernels in passes of up to min(4096, 16384 / K) tokens. */
+ * H % 128 == 0, I % 128 == 0, E <= 256.  Up to 256 tokens are one pass.  More go
+ * through the wide kernels in passes of up to min(4096, 16384 / K) tokens if the
+ * workspace has mlk_moe_wide_workspace_bytes(), else in passes of 256. */
 int mlk_fused_experts_compute(const void *w1, const void *w2, const void *x, int n_tokens, int n_experts,
                               int topk, int hidden, int inter, int w_kind, int x_kind, const int32_t *topk_ids,
                               const void *topk_weights, const int32_t *experts_map, const float *w1_scale,
                               const float *w2_scale, void *y, void *workspace, size_t workspace_bytes,
                               void *stream);
 size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter);
+size_t mlk_moe_wide_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter);
 
 /* The whole MoE layer in one call: router, alignment, both grouped GeMMs, weighted sum.  Replaces the call
  * sequence of the reference's Python entry `muxi_moe_planC.fused_moe` (muxi_layout_kernels/muxi_moe_planC.py:44-146:

@@ -1406,7 +1406,8 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
 //   256 experts, top-8, H 7168, I 256, soft-FP8  300         474 ->  450    600   801 -> 535    2048  2195 ->  909
 //   128 experts, top-8, H 2048, I 768, bf16                                 512   480 -> 294    2048  1904 ->  509
 // At 256 tokens, one pass either way, the small kernels are ahead (541 / 576, 394 / 488, 282 / 428, 245 / 260 us).
-// A remainder of up to kMoeChunk tokens is a pass of the small kernels again.
+// A remainder of up to kMoeChunk tokens is a pass of the small kernels again, and a call whose workspace only holds passes of
+// kMoeChunk tokens runs in those.
 struct MoePass {
     bool wide;
     int tokens;
@@ -1440,9 +1441,10 @@ static int moe_wide_down_slices(int tokens, int n_experts, int topk, int hidden,
     return best;
 }
 
-static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8) {
+// wide_ok: the workspace of the call is as large as the wide kernels ask for
+static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8, bool wide_ok) {
     MoePass ps = {};
-    ps.wide = tokens_left > kMoeChunk;
+    ps.wide = wide_ok && tokens_left > kMoeChunk;
     if (!ps.wide) {
         ps.tokens = tokens_left < kMoeChunk ? tokens_left : kMoeChunk;
         ps.plan = moe_plan(ps.tokens, n_experts, topk, hidden, inter, fp8);
@@ -1547,25 +1549,31 @@ extern "C" int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_
     return MLK_OK;
 }
 
-extern "C" size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
-    // the passes of a call share the workspace; the larger of the two weight kinds, since the query does not know which one
-    // the call will bring.  A call of more than one pass is also given what passes of kMoeChunk tokens would need.
+// The passes of a call share the workspace; the larger of the two weight kinds, since the query does not know which one
+// the call will bring.
+static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden, int inter, bool wide_ok) {
     size_t bytes = 0;
     for (int fp8 = 0; fp8 < 2; ++fp8) {
         auto cover = [&](int tokens) {
-            const MoePass ps = moe_pass(tokens, n_experts, topk, hidden, inter, fp8 != 0);
+            const MoePass ps = moe_pass(tokens, n_experts, topk, hidden, inter, fp8 != 0, wide_ok);
             const size_t b = carve(nullptr, ps.tokens, n_experts, topk, hidden, inter, ps.obuf_bytes + 256, nullptr);
             if (b > bytes) bytes = b;
             return ps.tokens;
         };
         const int first = cover(n_tokens);
-        if (n_tokens > kMoeChunk) {
-            cover(kMoeChunk);
-            if (n_tokens % kMoeChunk) cover(n_tokens % kMoeChunk);
-            if (n_tokens % first) cover(n_tokens % first);
-        }
+        if (n_tokens > first && n_tokens % first) cover(n_tokens % first);
     }
     return bytes;
+}
+
+extern "C" size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
+    return moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
+}
+
+extern "C" size_t mlk_moe_wide_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
+    const size_t narrow = moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
+    const size_t wide = moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
+    return wide > narrow ? wide : narrow;
 }
 
 static int experts_compute_impl(const void *w1, const void *w2, const void *x, int n_tokens, int n_experts,
@@ -1587,10 +1595,11 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
     MLK_REQUIRE(w1 && w2 && x && y && topk_ids && topk_weights && workspace, "moe: null pointer");
     MLK_REQUIRE(workspace_bytes >= mlk_moe_workspace_bytes(n_tokens, n_experts, topk, hidden, inter),
                 "moe: workspace too small");
+    const bool wide_ok = workspace_bytes >= mlk_moe_wide_workspace_bytes(n_tokens, n_experts, topk, hidden, inter);
     hipStream_t s = (hipStream_t)stream;
 
     for (int t0 = 0, tc = 0; t0 < n_tokens; t0 += tc) {
-        const MoePass ps = moe_pass(n_tokens - t0, n_experts, topk, hidden, inter, fp8);
+        const MoePass ps = moe_pass(n_tokens - t0, n_experts, topk, hidden, inter, fp8, wide_ok);
         const MoePlan &pl = ps.plan;
         tc = ps.tokens;
         const int n_pairs = tc * topk;

@@ -672,7 +672,7 @@ def experts_compute_raw(w1, w2, x, T, E, K, hidden, inter, w_kind, topk_ids, top
                         w2_scale, y):
     """Thin call of the C entry point (alignment + both grouped GeMMs + weighted sum); no checks."""
     lib = _lib.load()
-    ws = _moe_workspace(x.device, lib.mlk_moe_workspace_bytes(T, E, K, hidden, inter))
+    ws = _moe_workspace(x.device, lib.mlk_moe_wide_workspace_bytes(T, E, K, hidden, inter))
     _lib.check(lib.mlk_fused_experts_compute(_ptr(w1), _ptr(w2), _ptr(x), T, E, K, hidden, inter, w_kind,
                                              _KIND[x.dtype], _ptr(topk_ids), _ptr(topk_weights), _ptr(experts_map),
                                              _ptr(w1_scale), _ptr(w2_scale), _ptr(y), _ptr(ws), ws.numel(),
@@ -684,7 +684,7 @@ def fused_moe_raw(w1, w2, x, logits, T, E, K, hidden, inter, w_kind, score_fun, 
     """Thin call of the whole-layer entry point (router + alignment + both grouped GeMMs + weighted sum); no
     checks.  `topk_ids` / `topk_weights` receive the routing."""
     lib = _lib.load()
-    ws = _moe_workspace(x.device, lib.mlk_moe_workspace_bytes(T, E, K, hidden, inter))
+    ws = _moe_workspace(x.device, lib.mlk_moe_wide_workspace_bytes(T, E, K, hidden, inter))
     _lib.check(lib.mlk_fused_moe(_ptr(w1), _ptr(w2), _ptr(x), _ptr(logits), T, logits.size(-1), E, K, hidden, inter,
                                  w_kind, _KIND[x.dtype], score_fun, n_groups, topk_groups, _ptr(bias),
                                  int(bool(renormalize)), _ptr(experts_map), _ptr(w1_scale), _ptr(w2_scale),

@@ -648,3 +648,35 @@ def test_fused_moe_wide_kernels(mlk, T, E, K, H, I, kind):
         emap = np.arange(E, dtype=np.int32)       # every pick of a token, but for an absent expert
         emap[-1] = -1 if E > 2 else emap[-1]
     _moe_case(mlk, T, E, K, H, I, dtype, 7000 + T, fp8=kind == "fp8", emap=emap)
+
+
+@pytest.mark.parametrize("T", [300, 513])
+def test_workspace_of_256_token_passes_still_takes_longer_calls(mlk, T):
+    """A workspace of mlk_moe_workspace_bytes() (no larger than that of 256 tokens) is enough for any token count: without the
+    scratch of the wide kernels the call runs in passes of 256 tokens, with results like those of the wide kernels."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    E, K, H, I, dtype = 4, 2, 256, 512, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(77)
+    w1 = torch.randn((E, 2 * I, H), generator=g, device="cuda").mul_(H ** -0.5).to(dtype)
+    w2 = torch.randn((E, H, I), generator=g, device="cuda").mul_(I ** -0.5).to(dtype)
+    x = torch.randn((T, H), generator=g, device="cuda").to(dtype)
+    ids = torch.randint(0, E, (T, K), generator=g, device="cuda", dtype=torch.int32)
+    wts = torch.rand((T, K), generator=g, device="cuda").to(dtype)
+    w1p, w2p = mlk.pack_layout_a(w1), mlk.pack_layout_a(w2)
+    lib = _lib.load()
+    out = []
+    for need in (lib.mlk_moe_workspace_bytes(T, E, K, H, I), lib.mlk_moe_wide_workspace_bytes(T, E, K, H, I)):
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        y = torch.empty_like(x)
+        _lib.check(lib.mlk_fused_experts_compute(w1p.data_ptr(), w2p.data_ptr(), x.data_ptr(), T, E, K, H, I, 1, 1,
+                                                 ids.data_ptr(), wts.data_ptr(), None, None, None, y.data_ptr(),
+                                                 ws.data_ptr(), need, _stream()), "moe")
+        out.append(y.float().cpu())
+    _whole_tensor = torch.zeros((T, H), dtype=torch.float32, device="cuda")
+    for e in range(E):
+        gate, up = (x.float() @ w1[e].float().T).split(I, dim=1)
+        h = (torch.nn.functional.silu(gate) * up).to(dtype).float() @ w2[e].float().T
+        _whole_tensor += h * (wts.float() * (ids == e)).sum(1, keepdim=True)
+    for y in out:
+        assert_close(y, _whole_tensor.cpu().numpy(), RTOL, ATOL, "T=%d" % T)
