@@ -167,6 +167,7 @@ struct Panel8Loop {
             widen(min(slab0, last), 0, 0);
             widen(min(slab0 + 1, last), 1, 1);
             issue_a(src, wave, min(slab0 + 3, last), 0);           // raw(3) into the raw buffer that slab 0 has left
+            wait_vmcnt_le<1>();                                    // the tiles of slab 2
             __builtin_amdgcn_s_waitcnt(0xc07f);                    // lgkmcnt(0): the widened tiles are written
             bare_barrier();
             rd(a0, b0, 0, 0);
@@ -174,17 +175,15 @@ struct Panel8Loop {
             for (int s = 0; s < nslab; ++s) {
                 const int nxt = (cur + 1) & 3, nx2 = (cur + 2) & 3, prv = (cur + 3) & 3;
                 const int r1 = rcur == 2 ? 0 : rcur + 1, r2 = rcur == 0 ? 2 : rcur - 1;  // raw buffers of slabs s + 1 (= s + 4), s + 2
-                issue_b(src, wave, min(slab0 + s + 3, last), prv);
-                issue_a(src, wave, min(slab0 + s + 4, last), r1);
-                // the tiles of slab s + 2: everything younger than them may still be in flight (in the first trip raw(3), which
-                // went out alone, and this trip's loads; from then on the loads of two trips)
-                if (s == 0) wait_vmcnt_le<NB + 2>();
-                else wait_vmcnt_le<2 * (NB + 1)>();
-                // the fp8 tiles are read first, widened between the products of the first half step and written after them
+                // The fp8 tiles of slab s + 2 are read first, widened between the products of the first half step and written
+                // after them.  The loads go out behind the LDS reads, under the products (see spread_half_step); issued in front
+                // of them, right behind the barrier, every wave stood still for them: 28672 x 8192 at 1024 tokens 461 -> 451 us.
                 const float sc = scale_at(srow, min(slab0 + s + 2, last) >> 2);
                 const u32x2 *raw = reinterpret_cast<const u32x2 *>(win + 4 * kP8Slab + r2 * kP8RawSlab + 2 * wave * 32);
                 const u32x2 f0 = raw[lane], f1 = raw[64 + lane];
                 rd(a1, b1, cur, 1);
+                issue_b(src, wave, min(slab0 + s + 3, last), prv);
+                issue_a(src, wave, min(slab0 + s + 4, last), r1);
                 u32x4 w0, w1;
                 {
                     uint32_t x0, x1, x2, x3;
@@ -201,22 +200,27 @@ struct Panel8Loop {
                     dst[lane] = w0;
                     dst[64 + lane] = w1;
                 }
-                __builtin_amdgcn_sched_group_barrier(0x100, 2 + PR + TB, 0);                       // the LDS reads
                 if constexpr (TB >= 2) {
-                    constexpr int NM = 2 * TB, PER = (36 + NM - 3) / (NM - 2);                     // conversion instructions per gap
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                    constexpr int NM = 2 * TB, NR = 2 + PR + TB, PER = (36 + NM - 3) / (NM - 2);   // conversion instructions per gap
+                    constexpr int S0 = (NR + 1) / 2, LPER = (NB + 1 + NM - S0 - 1) / (NM - S0);    // first gap with loads, loads per gap
+                    __builtin_amdgcn_sched_group_barrier(0x006, 24, 0);                            // addresses
 #pragma unroll
-                    for (int m = 2; m < NM; ++m) {
-                        __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
+                    for (int m = 0; m < NM; ++m) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        if (2 * m + 1 < NR) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                        else if (2 * m < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        if (m >= 2) __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
+                        if (m >= S0 && (m - S0) * LPER < NB + 1) __builtin_amdgcn_sched_group_barrier(0x020, LPER, 0);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);                             // the two LDS writes
+                } else {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2 + PR + TB, 0);                   // the LDS reads
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 rd(a0, b0, nxt, 0);
                 mm(a1, b1);
-                __builtin_amdgcn_sched_barrier(0);
-                wait_vmcnt_le<NB + 2>();                           // this wave's chunks of slab s + 2 have landed
+                spread_half_step<2 * TB, PR + TB, 0>();
+                wait_vmcnt_le<NB + 1>();                           // this wave's chunks of slab s + 2 and tiles of slab s + 3 have landed
                 __builtin_amdgcn_s_waitcnt(0xc07f);                // and its widened tiles are written
                 bare_barrier();
                 cur = nxt;
