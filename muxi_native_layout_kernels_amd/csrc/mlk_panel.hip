@@ -268,8 +268,8 @@ __global__ void __launch_bounds__(256, 2) gemm_panel_lds_kernel(PanelArgs p) {
 // token are 8 bytes in a line that fifteen other instructions complete: 67 MB of output took 23 us that way.
 constexpr int kP8OutPitch = 144;                               // bytes per token in the turn-around buffer
 constexpr size_t kP8OutBytes = (size_t)8 * 128 * kP8OutPitch;
-template <class T>
-__device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)[2][4], int rg0, int tok0, int wave, int lane,
+template <class T, int TB>
+__device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)[2][TB], int rg0, int tok0, int wave, int lane,
                                                u32x4 *win) {
     uint8_t *buf = reinterpret_cast<uint8_t *>(win) + (size_t)wave * 128 * kP8OutPitch;
     const int half = lane >> 5, c32 = lane & 31;
@@ -285,7 +285,7 @@ __device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)
                 for (int i = 0; i < 4; ++i) bias[i] = T::to_f32(p.bias[n0 + row + i]);
             }
 #pragma unroll
-            for (int tb = 0; tb < 4; ++tb) {
+            for (int tb = 0; tb < TB; ++tb) {
                 u32x2 o;
                 o[0] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g] + bias[0], p.alpha * acc[pr][tb][4 * g + 1] + bias[1]);
                 o[1] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g + 2] + bias[2], p.alpha * acc[pr][tb][4 * g + 3] + bias[3]);
@@ -296,7 +296,7 @@ __device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)
     const int t8 = lane >> 3, q = lane & 7;
     const bool rows_ok = n0 + q * 8 < p.N;
 #pragma unroll
-    for (int it = 0; it < 16; ++it) {
+    for (int it = 0; it < 4 * TB; ++it) {
         const int token = it * 8 + t8;
         const u32x4 v = *reinterpret_cast<const u32x4 *>(buf + token * kP8OutPitch + q * 16);
         if (rows_ok && tok0 + token < p.M) *reinterpret_cast<u32x4 *>(p.C + (size_t)(tok0 + token) * p.N + n0 + q * 8) = v;
@@ -310,43 +310,15 @@ __device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)
 // p.chunk token tiles, so that the 32 workgroups an XCD runs at a time cover 8 x 4 (row tiles x token tiles) and share
 // both operands through its L2; with the token tiles of two row tiles side by side (2 x 16) the same product took
 // 17 % longer (8192 x 8192, 4096 tokens: 491 against 413 us).  A fifth slab of LDS (160 KiB) changed nothing.
-template <class T, bool FP8>
-__global__ void __launch_bounds__(512) gemm_panel8_kernel(PanelArgs p) {
+template <class T, bool FP8, int TB>
+__device__ __forceinline__ void gemm_panel8(const PanelArgs &p, int rt, int tt, int sk, int SK) {
     extern __shared__ u32x4 win[];
-    constexpr int PR = 2, TB = 4;
+    constexpr int PR = 2;
     constexpr int WBYTES = FP8 ? 1 : 2;
     using Loop = Panel8Loop<T, FP8, TB>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 3, wt = wave >> 2;
-
-    // workgroup -> (row tile, k slice, token tile), as in gemm_panel_kernel
-    const int xcd = blockIdx.x & 7;
-    int u = blockIdx.x >> 3;
-    int SK, sk, tt, rt;
-    if (p.band > 0) {
-        const int TT = p.token_tiles, groups8 = (p.row_tiles + 7) >> 3, RB = p.band, TC = p.chunk;
-        const int band = u / (RB * TT);
-        const int nb = min(RB, groups8 - band * RB);           // groups of row tiles in this band
-        const int v = u - band * RB * TT;
-        const int c = v / (nb * TC);
-        const int tc = min(TC, TT - c * TC);                   // token tiles in this chunk
-        const int w = v - c * nb * TC;
-        SK = 1, sk = 0;
-        tt = c * TC + w % tc;
-        rt = (band * RB + w / tc) * 8 + xcd;
-    } else {
-        const int whole_wgs = p.whole_groups * p.token_tiles;
-        const bool sliced = u >= whole_wgs;
-        SK = sliced ? p.SK : 1;
-        if (sliced) u -= whole_wgs;
-        tt = u % p.token_tiles;
-        u /= p.token_tiles;
-        sk = u % SK;
-        rt = ((sliced ? p.whole_groups : 0) + u / SK) * 8 + xcd;
-    }
-    if (rt >= p.row_tiles) return;
-
     const int groups = p.N >> 4;
     const int rgp = rt * 16;                                   // first row group of the panel
     const int rg0 = rgp + wr * 4;                              // of this wave
@@ -380,8 +352,47 @@ __global__ void __launch_bounds__(512) gemm_panel8_kernel(PanelArgs p) {
     zero_acc(acc);
     Loop::run(acc, src, srow, slab0, nslab, wave, lane);
     __syncthreads();
-    if (SK == 1) p8_store_panel<T>(p, acc, rg0, tok0 + wt * 128, wave, lane, win);
-    else panel_finish<T, PR, TB, 8, 2>(p, acc, rg0, tok0 + wt * 128, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
+    if (TB < 4 || SK == 1) p8_store_panel<T, TB>(p, acc, rg0, tok0 + wt * 32 * TB, wave, lane, win);
+    else if constexpr (TB == 4)
+        panel_finish<T, PR, TB, 8, 2>(p, acc, rg0, tok0 + wt * 128, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
+}
+
+template <class T, bool FP8>
+__global__ void __launch_bounds__(512) gemm_panel8_kernel(PanelArgs p) {
+    // workgroup -> (row tile, k slice, token tile), as in gemm_panel_kernel
+    const int xcd = blockIdx.x & 7;
+    int u = blockIdx.x >> 3;
+    int SK, sk, tt, rt;
+    if (p.band > 0) {
+        const int TT = p.token_tiles, groups8 = (p.row_tiles + 7) >> 3, RB = p.band, TC = p.chunk;
+        const int band = u / (RB * TT);
+        const int nb = min(RB, groups8 - band * RB);           // groups of row tiles in this band
+        const int v = u - band * RB * TT;
+        const int c = v / (nb * TC);
+        const int tc = min(TC, TT - c * TC);                   // token tiles in this chunk
+        const int w = v - c * nb * TC;
+        SK = 1, sk = 0;
+        tt = c * TC + w % tc;
+        rt = (band * RB + w / tc) * 8 + xcd;
+    } else {
+        const int whole_wgs = p.whole_groups * p.token_tiles;
+        const bool sliced = u >= whole_wgs;
+        SK = sliced ? p.SK : 1;
+        if (sliced) u -= whole_wgs;
+        tt = u % p.token_tiles;
+        u /= p.token_tiles;
+        sk = u % SK;
+        rt = ((sliced ? p.whole_groups : 0) + u / SK) * 8 + xcd;
+    }
+    if (rt >= p.row_tiles) return;
+    // The last token tile multiplies the 64, 128 or 192 token columns that cover it (28672 x 4096 bf16 at 700 tokens 196 ->
+    // 193 us, 13824 x 5120 at 3000 tokens 372 -> 367 us); the fold of K slices knows whole tiles.
+    switch (SK == 1 ? min(4, (p.M - tt * 256 + 63) >> 6) : 4) {
+        case 1: gemm_panel8<T, FP8, 1>(p, rt, tt, sk, SK); break;
+        case 2: gemm_panel8<T, FP8, 2>(p, rt, tt, sk, SK); break;
+        case 3: gemm_panel8<T, FP8, 3>(p, rt, tt, sk, SK); break;
+        default: gemm_panel8<T, FP8, 4>(p, rt, tt, sk, SK); break;
+    }
 }
 
 // Tokens per panel when the caller leaves the choice open.  Workgroups run one per CU in rounds; a 256-token panel

@@ -244,6 +244,30 @@ def test_gemm_panel_kernel_band_and_chunk_mapping(mlk, fp8):
     assert_close(c, want, RTOL, ATOL, "band / chunk mapping fp8=%s" % fp8)
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8"])
+@pytest.mark.parametrize("m", [1, 64, 65, 257, 320, 321, 384, 385, 448, 449, 512])
+def test_gemm_panel_kernel_columns_of_the_last_token_tile(mlk, kind, m):
+    """256 x 256 panels computed whole: the last token tile multiplies 64, 128, 192 or 256 columns, whichever cover it; row
+    groups past N in the last row tile."""
+    n, k = 640, 256
+    dtype = torch.float16 if kind == "fp16" else torch.bfloat16
+    b = randn((m, k), dtype, 1.0, 301)
+    params = dict(kernelParam1=4, kernelParam2=2, kernelParam3=1, kernelId=3)
+    if kind == "fp8":
+        codes = fp8_codes((n, k), 302)
+        g = torch.Generator().manual_seed(303)
+        scale = (torch.rand((n // 128, k // 128), generator=g) * 0.02 + 0.001).float()
+        c = mlk.gemm_layoutA_soft_fp8_wapper(pack_a(codes).cuda(), scale.cuda(), b.cuda(), n, m, k, **params)
+        want = ogemm.softfp8_linear_expected(codes.numpy(), scale.numpy(), b)
+    else:
+        w = randn((n, k), dtype, 0.05, 304)
+        bias = randn((1, n), dtype, 1.0, 305)
+        c = mlk.gemm_layoutA_wapper(pack_a(w).cuda(), b.cuda(), n, m, k, alpha=0.5, bias=bias.cuda(), **params)
+        want = ogemm.linear_expected(w, b, 0.5, bias)
+    assert c.shape == (m, n)
+    assert_close(c, want, RTOL, ATOL, "last token tile %s M=%d" % (kind, m))
+
+
 def test_gemm_panel_kernel_is_the_wide_default(mlk):
     """Above 64 tokens the heuristic for unscanned shapes picks the panel kernel; a K that is no
     multiple of 128 keeps the row-shared kernel, and the panel kernel refuses it when asked for by id."""
