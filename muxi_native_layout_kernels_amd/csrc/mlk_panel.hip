@@ -415,7 +415,8 @@ size_t panel_partial_bytes(int m, int n, int sk) {
 // a_kind: MLK_F16, MLK_BF16 or MLK_FP8_E4M3 (bf16 activations); width: tokens per panel (128 or 256), anything else =
 // panel_tokens(m, n); rows: weight rows per panel (128 or 256; 128 only with 128 tokens), anything else = chosen
 // from the number of panels; sk: K slices; last_round_only: slice only the panels that are left over after whole
-// rounds of one panel per CU (every panel when there is no whole round, none when nothing is left over)
+// rounds of one panel per CU (every panel when there is less than a round, none when nothing is left over or where
+// the leftover cannot be told apart and slicing everything costs more)
 int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, float alpha, const void *bias,
                  const float *scale, int width, int rows, int sk, bool last_round_only, void *counters,
                  size_t counter_bytes, void *partial, size_t partial_bytes, hipStream_t s) {
@@ -466,6 +467,18 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         MLK_REQUIRE((size_t)p.row_tiles * p.token_tiles * sizeof(int) <= counter_bytes,
                     "gemm: too many panels for the counter region");
         if (partial_bytes < panel_partial_bytes(m, n, sk)) return fail(MLK_ERR_WORKSPACE, "gemm: workspace too small");
+    }
+    // Token tiles that do not divide an XCD's CUs leave no groups that fill whole rounds, and slicing every panel of a grid of
+    // several rounds pays the fold for all of it: then the panels are computed whole, unless the slices save more rounds
+    // than their partial products cost (written and read once at about 5 TB/s; a k32 slab of a 256 x 256 panel takes 0.78 us).
+    // 11008 x 4096 fp16 at 2100 tokens (nine tiles): 374 us in two slices, 199 us whole; bf16 at 3300 tokens 495 and 286 us;
+    // soft-FP8 28672 x 8192 at 1100 tokens 739 us in three slices, 499 us whole.
+    if (last_round_only && sk > 1 && p.whole_groups == 0 && groups * p.token_tiles > device_cus() / 8) {
+        const long long cus = device_cus(), panels = (long long)p.row_tiles * p.token_tiles;
+        const double panel_us = 0.78 * (k / 32) * rows * width / 65536.;
+        const double whole_us = (double)((panels + cus - 1) / cus) * panel_us;
+        const double sliced_us = (double)((panels * sk + cus - 1) / cus) * panel_us / sk + (double)sk * m * n * 8 / 5e6;
+        if (whole_us <= sliced_us) p.SK = sk = 1;
     }
     const int grid = (p.whole_groups + (groups - p.whole_groups) * sk) * 8 * p.token_tiles;
     // one workgroup per CU (the register ring and the accumulators take a whole SIMD's file); more than 64 KiB of

@@ -191,6 +191,9 @@ def test_gemm_panel_kernel_soft_fp8(mlk, m, scaled):
     (5504, 384, 256, 2, 1, 2),       # three token tiles do not divide an XCD's CUs: every panel whole
     (2048, 1024, 256, 2, 1, 2),      # exactly one round: nothing left over, no slices
     (1024, 200, 512, 4, 1, 4),       # less than a round: every panel sliced, as with kernelId 3
+    (5504, 1152, 256, 2, 1, 2),      # nine token tiles, one and a half rounds: whole, the fold would cost more
+    (16640, 1100, 256, 4, 2, 2),     # the same with 256 x 256 panels and a ragged last token tile
+    (7424, 640, 8192, 2, 1, 4),      # five token tiles, 290 panels of a long K: four slices save more than they cost
 ])
 def test_gemm_panel_kernel_last_round_slices(mlk, n, m, k, p1, p2, p3):
     """kernelId 5: the panel kernel with K slices only on the panels left over after whole rounds of one panel per
