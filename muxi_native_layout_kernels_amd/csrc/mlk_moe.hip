@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
     if (tid < E) {
         for (int w = 0; w < NW; ++w) total += cnt[w][tid];
         nb = (total + 15) >> 4;
-        ntk = (nb + cb_max - 1) / cb_max;                       // cb_max is a multiple of cb_unit
+        ntk = (nb + cb_max - 1) / cb_max;                       // cb_max is a multiple of cb_unit (or that is 0)
         scan_pad[tid] = nb << 4;
         scan_task[tid] = ntk;
     }
@@ -351,10 +351,13 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
         start[e] = run;
         for (int b = 0; b < nb; ++b) experts_ids[(run >> 4) + b] = e;
         if (tasks) {
-            // the tasks of an expert get nearly equal numbers of units of cb_unit blocks
-            const int first = scan_task[e] - ntk, units = (nb + cb_unit - 1) / cb_unit;
+            // cb_unit 0: every task but an expert's last one gets cb_max blocks (in the row-shared kernels a block's order of
+            // summation follows from its task's number, so it does not depend on how many more tokens its expert has);
+            // else the tasks of an expert get nearly equal numbers of units of cb_unit blocks
+            const int first = scan_task[e] - ntk, units = cb_unit ? (nb + cb_unit - 1) / cb_unit : 0;
             for (int i = 0; i < ntk; ++i) {
-                const int b0 = units * i / ntk * cb_unit, b1 = min(nb, units * (i + 1) / ntk * cb_unit);
+                const int b0 = cb_unit ? units * i / ntk * cb_unit : i * cb_max;
+                const int b1 = min(nb, cb_unit ? units * (i + 1) / ntk * cb_unit : b0 + cb_max);
                 MoeTask tk;
                 tk.expert = e;
                 tk.block0 = (run >> 4) + b0;
@@ -1411,7 +1414,7 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
 struct MoePass {
     bool wide;
     int tokens;
-    int cb, cb_unit;      // token blocks per task and the unit they are dealt in
+    int cb, cb_unit;      // token blocks per task and the unit they are dealt in (0: tasks filled one after the other)
     int max_tasks;        // upper bound of the task list
     int down_slices;
     size_t obuf_bytes;
@@ -1449,7 +1452,7 @@ static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, in
         ps.tokens = tokens_left < kMoeChunk ? tokens_left : kMoeChunk;
         ps.plan = moe_plan(ps.tokens, n_experts, topk, hidden, inter, fp8);
         ps.cb = moe_blocks_per_task(ps.tokens, topk, n_experts);
-        ps.cb_unit = 1;
+        ps.cb_unit = 0;
         ps.max_tasks = ps.plan.max_tasks;
         ps.down_slices = ps.plan.down_slices;
         // per routed pair and slice for the row-shared and panel kernels, per token and slice for the decode kernels,
@@ -1544,7 +1547,7 @@ extern "C" int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_
     const int max_blocks = (n_pairs + n_experts * 15 + 15) / 16;
     moe_align_kernel<<<1, 1024, 0, (hipStream_t)stream>>>(topk_ids, n_pairs, n_experts, experts_map, sorted_token_ids,
                                                           cumsum_buffer, padded_num_blocks, experts_ids, max_blocks,
-                                                          nullptr, nullptr, 1, 1);
+                                                          nullptr, nullptr, 1, 0);
     MLK_LAUNCH_CHECK();
     return MLK_OK;
 }

@@ -256,6 +256,48 @@ def test_fused_moe_soft_fp8_panel_down_two_per_cu(mlk):
     _moe_case(mlk, T, E, K, H, I, torch.bfloat16, 2400, fp8=True)
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_row_shared_tasks_are_filled_one_after_the_other(mlk, kind):
+    """An expert with three blocks of tokens and tasks of two: its first two blocks are one task, so their 32 tokens get the
+    very bits that they get when the expert has no third block (the task's number decides the order of summation).  The second
+    half of every gate/up sum takes the first half away again, so that what is left is the rounding of that order."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    import ctypes
+    T, E, K, H, I = 256, 16, 1, 1024, 512
+    lib = _lib.load()
+    wk = 2 if kind == "fp8" else 1
+    plan = (ctypes.c_int32 * 8)()
+    assert lib.mlk_moe_plan(T, E, K, H, I, wk, ctypes.addressof(plan)) == 0 and (plan[0], plan[1]) == (3, 2), list(plan)
+    g = torch.Generator(device="cuda").manual_seed(91)
+
+    def weights(shape, std, copies=1):
+        w = torch.randn(shape[:-1] + (shape[-1] // copies,), generator=g, device="cuda").repeat(1, 1, copies)
+        return mlk.pack_layout_a((w * 16).clamp_(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8) if kind == "fp8"
+                                 else (w * std).to(torch.bfloat16))
+    w1, w2 = weights((E, 2 * I, H), H ** -0.5, 2), weights((E, H, I), I ** -0.5)
+    s1 = torch.full((E, 2 * I // 128, H // 128), H ** -0.5 / 16, device="cuda") if kind == "fp8" else None
+    s2 = torch.full((E, H // 128, I // 128), I ** -0.5 / 16, device="cuda") if kind == "fp8" else None
+    x = torch.randn((T, H // 2), generator=g, device="cuda").to(torch.bfloat16)
+    x = torch.cat([x, -x], dim=1)
+    wts = torch.ones((T, K), device="cuda", dtype=torch.bfloat16)
+    emap = torch.arange(E, device="cuda", dtype=torch.int32)
+    emap[-1] = -1                                              # the last expert is on another rank
+    ws = torch.empty(lib.mlk_moe_workspace_bytes(T, E, K, H, I), dtype=torch.uint8, device="cuda")
+    ids = (1 + torch.arange(T, device="cuda") % (E - 2)).to(torch.int32).view(T, K)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    out = []
+    for third in (0, E - 1):
+        ids[:32] = 0
+        ids[32:48] = third
+        y = torch.empty_like(x)
+        _lib.check(lib.mlk_fused_experts_compute(ptr(w1), ptr(w2), ptr(x), T, E, K, H, I, wk, 1, ptr(ids), ptr(wts), ptr(emap),
+                                                 ptr(s1), ptr(s2), ptr(y), ptr(ws), ws.numel(), _stream()), "moe")
+        out.append(y)
+    assert (out[0][:48] != 0).float().mean() > 0.9 and (out[1][32:48] == 0).all()
+    assert torch.equal(out[0][:32], out[1][:32])
+
+
 def test_fused_moe_grouped_sigmoid_bias(mlk):
     E = 64
     bias = randn((E,), torch.bfloat16, 0.05, 9).abs()
