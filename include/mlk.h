@@ -269,7 +269,8 @@ int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_experts, in
  *   (alignment tables and the SiLU intermediate); contents are not preserved.
  * H % 128 == 0, I % 128 == 0, E <= 256.  Up to 256 tokens are one pass.  More go
  * through the wide kernels in passes of up to min(4096, 16384 / K) tokens if the
- * workspace has mlk_moe_wide_workspace_bytes(), else in passes of 256. */
+ * workspace has mlk_moe_wide_workspace_bytes() and x, w1, w2 and the workspace lie
+ * on 16 bytes, else in passes of 256. */
 int mlk_fused_experts_compute(const void *w1, const void *w2, const void *x, int n_tokens, int n_experts,
                               int topk, int hidden, int inter, int w_kind, int x_kind, const int32_t *topk_ids,
                               const void *topk_weights, const int32_t *experts_map, const float *w1_scale,

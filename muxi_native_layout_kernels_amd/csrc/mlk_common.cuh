@@ -31,6 +31,10 @@ int fail(int code, const char *msg);
 // Compute units of the current device (cached per device; 256 if the runtime cannot tell).
 int device_cus();
 
+// Global loads that write LDS copy 16 bytes a lane and are only used on operands that lie on 16 bytes; plain loads go
+// through a register and take any address.
+static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
+
 #define MLK_REQUIRE(cond, msg)                                                  \
     do {                                                                        \
         if (!(cond)) return ::mlk::fail(MLK_ERR_INVALID, msg);                  \

@@ -1598,7 +1598,9 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
     MLK_REQUIRE(w1 && w2 && x && y && topk_ids && topk_weights && workspace, "moe: null pointer");
     MLK_REQUIRE(workspace_bytes >= mlk_moe_workspace_bytes(n_tokens, n_experts, topk, hidden, inter),
                 "moe: workspace too small");
-    const bool wide_ok = workspace_bytes >= mlk_moe_wide_workspace_bytes(n_tokens, n_experts, topk, hidden, inter);
+    // the wide kernels load tokens, weights and intermediate straight into LDS
+    const bool wide_ok = aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(workspace) &&
+                         workspace_bytes >= mlk_moe_wide_workspace_bytes(n_tokens, n_experts, topk, hidden, inter);
     hipStream_t s = (hipStream_t)stream;
 
     for (int t0 = 0, tc = 0; t0 < n_tokens; t0 += tc) {

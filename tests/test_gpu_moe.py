@@ -692,6 +692,29 @@ def test_fused_moe_wide_kernels(mlk, T, E, K, H, I, kind):
     _moe_case(mlk, T, E, K, H, I, dtype, 7000 + T, fp8=kind == "fp8", emap=emap)
 
 
+def test_operands_off_16_bytes_stay_off_the_wide_kernels(mlk):
+    """Tokens or weights that do not lie on 16 bytes run in passes of 256 tokens, whose kernels take any address: the very bits
+    of those passes called one by one."""
+    from muxi_native_layout_kernels_amd.moe_planC import fused_moe
+    T, E, K, H, I, dtype = 300, 8, 2, 256, 384, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(93)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+        flat[1:1 + t.numel()] = t.reshape(-1)
+        return flat[1:1 + t.numel()].view(t.shape)
+    w1 = mlk.pack_layout_a((torch.randn((E, 2 * I, H), generator=g, device="cuda") * H ** -0.5).to(dtype)).view(E, 2 * I, H)
+    w2 = mlk.pack_layout_a((torch.randn((E, H, I), generator=g, device="cuda") * I ** -0.5).to(dtype)).view(E, H, I)
+    x = torch.randn((T, H), generator=g, device="cuda").to(dtype)
+    logits = torch.randn((T, E), generator=g, device="cuda").to(dtype)
+    want = torch.cat([fused_moe(x[a:b], w1, w2, logits[a:b], K, True) for a, b in ((0, 256), (256, T))])
+    for args in ((shifted(x), w1, w2), (x, shifted(w1), w2), (x, w1, shifted(w2))):
+        assert all(t.is_contiguous() for t in args) and any(t.data_ptr() % 16 for t in args)
+        assert torch.equal(fused_moe(*args, logits, K, True), want)
+    wide = fused_moe(x, w1, w2, logits, K, True)
+    assert_close(wide, want.double().cpu().numpy(), RTOL, ATOL, "wide kernels")
+
+
 @pytest.mark.parametrize("T", [300, 513])
 def test_workspace_of_256_token_passes_still_takes_longer_calls(mlk, T):
     """A workspace of mlk_moe_workspace_bytes() (no larger than that of 256 tokens) is enough for any token count: without the
