@@ -277,6 +277,8 @@ int mlk_fused_experts_compute(const void *w1, const void *w2, const void *x, int
                               const float *w2_scale, void *y, void *workspace, size_t workspace_bytes,
                               void *stream);
 size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter);
+/* Above 256 tokens the answer holds for every shorter call too and never falls as n_tokens grows: scratch sized once for the
+ * longest prompt keeps all of them on the wide kernels.  Up to 256 tokens it is mlk_moe_workspace_bytes(). */
 size_t mlk_moe_wide_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter);
 
 /* The whole MoE layer in one call: router, alignment, both grouped GeMMs, weighted sum.  Replaces the call

@@ -24,6 +24,7 @@
 // + 2*T*H*2 + T*E*2 bytes; the SiLU intermediate (T*K*I*2 bytes, written and
 // read once) stays in L2 / Infinity Cache for decode-sized T.
 #include <math.h>
+#include <string.h>
 
 #include "mlk_moe_args.cuh"
 
@@ -1429,10 +1430,14 @@ extern template int launch_moe_wide<BF16, true>(const MoeArgs &, int, float *, i
 // quarter of the chip unless the panels are cut.  In units of a k32 slab of a panel (0.75 us): a panel costs its slabs and
 // about eight more to start and to store; a slice costs the write and the read of its partial products (8 experts, bf16,
 // 1, 2, 3 slices: 677, 579, 615 us at 256 tokens, 1782, 1689, 1667 us at 2048).
+static int moe_wide_expert_tasks(int tokens, int n_experts, int topk) {
+    const double mean = (double)tokens * topk / n_experts;
+    return (int)ceil((mean + 0.5 * sqrt(mean)) / (16 * kWideTaskBlocks));
+}
 static int moe_wide_down_slices(int tokens, int n_experts, int topk, int hidden, int inter) {
     const int cus = device_cus();
-    const double pairs = (double)tokens * topk, mean = pairs / n_experts;
-    const double tasks = ceil((mean + 0.5 * sqrt(mean)) / (16 * kWideTaskBlocks)) * (pairs < n_experts ? pairs : n_experts);
+    const double pairs = (double)tokens * topk;
+    const double tasks = moe_wide_expert_tasks(tokens, n_experts, topk) * (pairs < n_experts ? pairs : n_experts);
     const double per_slice = pairs * hidden * 8 / 5e6 / 0.75;
     int best = 1;
     double best_cost = 0;
@@ -1444,7 +1449,28 @@ static int moe_wide_down_slices(int tokens, int n_experts, int topk, int hidden,
     return best;
 }
 
-// wide_ok: the workspace of the call is as large as the wide kernels ask for
+static int moe_wide_most_tokens(int topk) { return kMoeWidePairs / topk < kMoeWideTokens ? kMoeWidePairs / topk : kMoeWideTokens; }
+
+// Routed pairs times K slices of the wide down projection, the most over all passes of kMoeChunk + 1 to `tokens` tokens.  The
+// slices drop where the tasks per expert step up, so a shorter pass can have more of both; between two steps only the
+// price of a slice grows, and the slices can only fall: one look per step.
+static size_t moe_wide_most_pair_slices(int tokens, int n_experts, int topk, int hidden, int inter) {
+    size_t most = 0;
+    for (int lo = kMoeChunk + 1; lo <= tokens;) {
+        const int per = moe_wide_expert_tasks(lo, n_experts, topk);
+        const double root = sqrt(16. * kWideTaskBlocks * per + 0.0625) - 0.25;       // of the mean load at which `per` is full
+        int hi = (int)fmin(root * root * n_experts / topk, (double)tokens);
+        while (hi > lo && moe_wide_expert_tasks(hi, n_experts, topk) > per) --hi;
+        while (hi < tokens && moe_wide_expert_tasks(hi + 1, n_experts, topk) <= per) ++hi;
+        if (hi < lo) hi = lo;
+        const size_t here = (size_t)hi * topk * moe_wide_down_slices(lo, n_experts, topk, hidden, inter);
+        if (here > most) most = here;
+        lo = hi + 1;
+    }
+    return most;
+}
+
+// wide_ok: the workspace of the call holds what the wide kernels need
 static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8, bool wide_ok) {
     MoePass ps = {};
     ps.wide = wide_ok && tokens_left > kMoeChunk;
@@ -1463,7 +1489,7 @@ static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, in
             ps.obuf_bytes = (size_t)ps.tokens * ps.down_slices * hidden * sizeof(float);
         return ps;
     }
-    const int most = kMoeWidePairs / topk < kMoeWideTokens ? kMoeWidePairs / topk : kMoeWideTokens;
+    const int most = moe_wide_most_tokens(topk);
     ps.tokens = tokens_left < most ? tokens_left : most;
     const int pairs = ps.tokens * topk;
     ps.cb = kWideTaskBlocks;
@@ -1573,9 +1599,32 @@ extern "C" size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk,
     return moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
 }
 
+// The most that a call of any 1 .. kMoeChunk tokens needs.  512 plans, about 50 us: kept per thread for the layer (and the
+// experiment switches) it was last asked for.
+static size_t moe_narrow_most(int n_experts, int topk, int hidden, int inter) {
+    const int key[11] = {n_experts, topk, hidden, inter, device_cus(), g_moe_tile, g_moe_gemv1,
+                         g_tunable[7], g_tunable[8], g_tunable[9], g_tunable[10]};
+    static thread_local int last[11] = {};
+    static thread_local size_t bytes = 0;
+    if (memcmp(key, last, sizeof key) != 0) {
+        bytes = 0;
+        for (int t = 1; t <= kMoeChunk; ++t) {
+            const size_t b = moe_workspace_of(t, n_experts, topk, hidden, inter, false);
+            if (b > bytes) bytes = b;
+        }
+        memcpy(last, key, sizeof key);
+    }
+    return bytes;
+}
+
+// Above kMoeChunk tokens: enough for every shorter call too, so that scratch sized once for the longest prompt serves the rest
+// on the same kernels.
 extern "C" size_t mlk_moe_wide_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
-    const size_t narrow = moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
-    const size_t wide = moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
+    if (n_tokens <= kMoeChunk || n_experts < 1 || topk < 1) return moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
+    const int most = moe_wide_most_tokens(topk), tokens = n_tokens < most ? n_tokens : most;
+    const size_t obuf = moe_wide_most_pair_slices(tokens, n_experts, topk, hidden, inter) * hidden * sizeof(float);
+    const size_t wide = carve(nullptr, tokens, n_experts, topk, hidden, inter, obuf + 256, nullptr);
+    const size_t narrow = moe_narrow_most(n_experts, topk, hidden, inter);
     return wide > narrow ? wide : narrow;
 }
 
@@ -1599,8 +1648,8 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
     MLK_REQUIRE(workspace_bytes >= mlk_moe_workspace_bytes(n_tokens, n_experts, topk, hidden, inter),
                 "moe: workspace too small");
     // the wide kernels load tokens, weights and intermediate straight into LDS
-    const bool wide_ok = aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(workspace) &&
-                         workspace_bytes >= mlk_moe_wide_workspace_bytes(n_tokens, n_experts, topk, hidden, inter);
+    const bool wide_ok = n_tokens > kMoeChunk && aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(workspace) &&
+                         workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
     hipStream_t s = (hipStream_t)stream;
 
     for (int t0 = 0, tc = 0; t0 < n_tokens; t0 += tc) {

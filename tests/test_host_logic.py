@@ -151,6 +151,22 @@ def test_moe_workspace_follows_the_plan():
             assert need >= lib.mlk_moe_workspace_bytes(last, E, K, H, I)
 
 
+@pytest.mark.parametrize("E,K,H,I", [(8, 2, 4096, 14336), (256, 8, 7168, 256), (1, 1, 4096, 14336), (4, 1, 4224, 2048),
+                                     (60, 5, 768, 5376), (16, 16, 1024, 2048)])
+def test_moe_wide_workspace_holds_for_every_shorter_call(E, K, H, I):
+    """Above 256 tokens the query never falls, covers every call of up to 256 tokens, and leaves room for the fp32 products of
+    at least one K slice."""
+    lib = _lib.load()
+    most = max(lib.mlk_moe_workspace_bytes(t, E, K, H, I) for t in range(1, 257))
+    before = 0
+    for t in range(257, 4400):
+        need = lib.mlk_moe_wide_workspace_bytes(t, E, K, H, I)
+        assert need >= before and need >= most and need >= min(t, 4096, 16384 // K) * K * H * 4, t
+        before = need
+    for t in (1, 16, 171, 256):
+        assert lib.mlk_moe_wide_workspace_bytes(t, E, K, H, I) == lib.mlk_moe_workspace_bytes(t, E, K, H, I)
+
+
 def test_routing_buffers_are_kept_for_every_shape_and_stream():
     from muxi_native_layout_kernels_amd import moe_planC
     cpu = torch.device("cpu")
