@@ -267,7 +267,8 @@ int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_experts, in
  *   y [T, H] of x_kind (overwritten; needs no zero fill)
  *   workspace: at least mlk_moe_workspace_bytes() bytes of device scratch
  *   (alignment tables and the SiLU intermediate); contents are not preserved.
- * H % 128 == 0, I % 128 == 0, E <= 256.  Up to 256 tokens are one pass.  More go
+ * H % 128 == 0, I % 128 == 0, E <= 256.  Up to 256 tokens are one pass.  More (but
+ * for a few above 256, where a pass of 256 and the rest are cheaper) go
  * through the wide kernels in passes of up to min(4096, 16384 / K) tokens if the
  * workspace has mlk_moe_wide_workspace_bytes() and x, w1, w2 and the workspace lie
  * on 16 bytes, else in passes of 256. */
@@ -294,8 +295,14 @@ int mlk_fused_moe(const void *w1, const void *w2, const void *x, const void *log
                   const int32_t *experts_map, const float *w1_scale, const float *w2_scale, int32_t *topk_ids,
                   void *topk_weights, void *y, void *workspace, size_t workspace_bytes, void *stream);
 
-/* How mlk_fused_experts_compute runs one pass of up to 256 tokens (a longer call has its own kernels, and only a
- * remainder of up to 256 tokens is such a pass; for it the answer is that of 256); the launch code reads the same plan.  out[0] = kernel family (0 single-token GeMV kernels, 1 decode kernels that align in-kernel, 2 decode
+/* The first pass of mlk_fused_experts_compute over operands on 16 bytes and a workspace of that size: out[0] = its tokens,
+ * out[1] = 1 if it runs the wide kernels.  For tests; no counterpart in the reference. */
+int mlk_moe_first_pass(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, size_t workspace_bytes,
+                       int32_t *out);
+
+/* How mlk_fused_experts_compute runs one pass of up to 256 tokens (for more the answer is that of 256; whether a longer call
+ * has such passes, mlk_moe_first_pass tells); the launch code reads the same plan.  out[0] = kernel family (0 single-token
+ * GeMV kernels, 1 decode kernels that align in-kernel, 2 decode
  * kernels after the alignment kernel, 3 row-shared kernels, 4 panel kernels: soft-FP8 weights with more than 64
  * tokens per pass over an expert), out[1] = token blocks per task, out[2] = upper bound of the task list,
  * out[3] = row groups per wave and out[4] = K slices of the down projection, out[5] = waves and out[6] = dynamic

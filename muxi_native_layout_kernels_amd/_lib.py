@@ -48,6 +48,7 @@ SIGNATURES = {
                               c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "mlk_moe_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "mlk_moe_wide_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "mlk_moe_first_pass": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_size_t, c_void_p]),
     "mlk_moe_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }
 

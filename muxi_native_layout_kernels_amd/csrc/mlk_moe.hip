@@ -1404,14 +1404,18 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
 // ------------------------------------------------------------ passes
 // A call of up to kMoeChunk tokens is one pass of the kernels moe_plan() names.  A longer one goes through the wide kernels
 // (mlk_moe_wide.cuh) in passes of as many tokens as their workspace is allowed for: in passes of kMoeChunk tokens every
-// pass streams the weights of all experts again.  Measured, passes of kMoeChunk tokens -> wide kernels (us):
-//   8 experts, top-2, H 4096, I 14336, bf16      300 tokens  994 ->  590    512  1077 -> 678    2048  4287 -> 1684
-//   the same, soft-FP8                           300         659 ->  514    512   786 -> 629    2048  3098 -> 1805
-//   256 experts, top-8, H 7168, I 256, soft-FP8  300         474 ->  450    600   801 -> 535    2048  2195 ->  909
-//   128 experts, top-8, H 2048, I 768, bf16                                 512   480 -> 294    2048  1904 ->  509
-// At 256 tokens, one pass either way, the small kernels are ahead (541 / 576, 394 / 488, 282 / 428, 245 / 260 us).
-// A remainder of up to kMoeChunk tokens is a pass of the small kernels again, and a call whose workspace only holds passes of
-// kMoeChunk tokens runs in those.
+// pass streams the weights of all experts it reaches again.  Measured, passes of kMoeChunk tokens -> wide kernels (us, without
+// the router):
+//                                                  tokens   257          264          272          304          512
+//   8 experts, top-2, H 4096, I 14336, bf16                 624 -> 559   894 -> 556   940 -> 555   960 -> 566  1039 -> 644
+//   the same, soft-FP8                                      440 -> 464   534 -> 462   576 -> 465   632 -> 480   735 -> 562
+//   256 experts, top-8, H 7168, I 256, bf16                 528 -> 542   657 -> 541   760 -> 543   995 -> 550   996 -> 581
+//   the same, soft-FP8                                      333 -> 491   415 -> 480   491 -> 481   625 -> 486   612 -> 508
+//   128 experts, top-8, H 2048, I 768, bf16                 243 -> 235   347 -> 234   393 -> 235   473 -> 238   439 -> 254
+//   the same, soft-FP8                                      156 -> 199   244 -> 200   277 -> 199   329 -> 200   275 -> 205
+// A few tokens above kMoeChunk, moe_two_passes_pay() keeps the pass of kMoeChunk tokens and its remainder.  A remainder of up to
+// kMoeChunk tokens is a pass of the small kernels again, and a call whose workspace only holds passes of kMoeChunk tokens, or
+// whose operands do not lie on 16 bytes, runs in those.
 struct MoePass {
     bool wide;
     int tokens;
@@ -1470,10 +1474,31 @@ static size_t moe_wide_most_pair_slices(int tokens, int n_experts, int topk, int
     return most;
 }
 
-// wide_ok: the workspace of the call holds what the wide kernels need
+// Is a pass of kMoeChunk tokens and one of the `rest` above it cheaper than one wide pass?  The small kernels stream the weights
+// at about 6.4 TB/s; the wide ones multiply at least 64 token columns per panel and reach 3.9 TB/s with soft-FP8 weights,
+// which they widen through LDS, and 6.2 TB/s with 16-bit ones.  What a byte saves that way falls with the tokens per expert,
+// as the small kernels come to be bound by their products; the remainder costs its launches and the experts it reaches once
+// more.  Where a task is one token block, the down kernel walks all tasks in every workgroup (a share per expert) and its
+// grid of 16 output rows each runs in whole rounds.  The constants (us and MB) are fitted to 24 layers of 4 to 256 experts,
+// both kinds of weights and 257 to 512 tokens: no choice costs more than 4.5 % against the better one, where going wide always
+// cost up to 56 % (256 experts, top-8, H 7168, I 2048, soft-FP8, 257 tokens: 1950 -> 3050 us).
+static bool moe_two_passes_pay(int rest, int n_experts, int topk, int hidden, int inter, bool fp8) {
+    const double miss = topk < n_experts ? 1 - (double)topk / n_experts : 0;
+    const double weights = 3e-6 * n_experts * hidden * inter * (fp8 ? 1 : 2), first = weights * (1 - pow(miss, kMoeChunk));
+    const double mean = (double)kMoeChunk * topk / n_experts;
+    double gain = first * ((fp8 ? 0.1 : 0.02) - (fp8 ? 0.0004 : 0.0008) * (mean > 8 ? mean - 8 : 0));
+    if (moe_blocks_per_task(kMoeChunk, topk, n_experts) == 1) {
+        const double rounds = hidden / 16. / device_cus();
+        gain -= (fp8 ? 0.3 : 0.1) * n_experts + (rounds > 1 ? first / 19.5 * (ceil(rounds) / rounds - 1) : 0);
+    }
+    return weights * (1 - pow(miss, rest)) / (fp8 ? 5.5 : 4) + (fp8 ? 30 : 5) < gain;
+}
+
+// wide_ok: the operands and the workspace of the call are fit for the wide kernels
 static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8, bool wide_ok) {
     MoePass ps = {};
-    ps.wide = wide_ok && tokens_left > kMoeChunk;
+    ps.wide = wide_ok && tokens_left > kMoeChunk &&
+              (tokens_left > 2 * kMoeChunk || !moe_two_passes_pay(tokens_left - kMoeChunk, n_experts, topk, hidden, inter, fp8));
     if (!ps.wide) {
         ps.tokens = tokens_left < kMoeChunk ? tokens_left : kMoeChunk;
         ps.plan = moe_plan(ps.tokens, n_experts, topk, hidden, inter, fp8);
@@ -1590,13 +1615,17 @@ static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden
             return ps.tokens;
         };
         const int first = cover(n_tokens);
-        if (n_tokens > first && n_tokens % first) cover(n_tokens % first);
+        for (int left = n_tokens > first ? n_tokens % first : 0; left > 0;) left -= cover(left);
     }
     return bytes;
 }
 
 extern "C" size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
     return moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
+}
+
+static bool moe_wide_fits(int n_tokens, int n_experts, int topk, int hidden, int inter, size_t workspace_bytes) {
+    return n_tokens > kMoeChunk && workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
 }
 
 // The most that a call of any 1 .. kMoeChunk tokens needs.  512 plans, about 50 us: kept per thread for the layer (and the
@@ -1628,6 +1657,20 @@ extern "C" size_t mlk_moe_wide_workspace_bytes(int n_tokens, int n_experts, int 
     return wide > narrow ? wide : narrow;
 }
 
+extern "C" int mlk_moe_first_pass(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, size_t workspace_bytes,
+                                  int32_t *out) {
+    MLK_REQUIRE(out != nullptr, "moe first pass: null pointer");
+    MLK_REQUIRE(n_tokens >= 1 && n_experts >= 1 && n_experts <= kMaxExperts && topk >= 1 && topk <= kMaxTopK,
+                "moe first pass: sizes out of range");
+    MLK_REQUIRE(hidden > 0 && inter > 0 && hidden % 128 == 0 && inter % 128 == 0,
+                "moe: hidden and intermediate sizes must be multiples of 128");
+    const bool wide_ok = moe_wide_fits(n_tokens, n_experts, topk, hidden, inter, workspace_bytes);
+    const MoePass ps = moe_pass(n_tokens, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3, wide_ok);
+    out[0] = ps.tokens;
+    out[1] = ps.wide;
+    return MLK_OK;
+}
+
 static int experts_compute_impl(const void *w1, const void *w2, const void *x, int n_tokens, int n_experts,
                                 int topk, int hidden, int inter, int w_kind, int x_kind,
                                 const int32_t *topk_ids, const void *topk_weights,
@@ -1648,8 +1691,8 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
     MLK_REQUIRE(workspace_bytes >= mlk_moe_workspace_bytes(n_tokens, n_experts, topk, hidden, inter),
                 "moe: workspace too small");
     // the wide kernels load tokens, weights and intermediate straight into LDS
-    const bool wide_ok = n_tokens > kMoeChunk && aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(workspace) &&
-                         workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
+    const bool wide_ok = aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(workspace) &&
+                         moe_wide_fits(n_tokens, n_experts, topk, hidden, inter, workspace_bytes);
     hipStream_t s = (hipStream_t)stream;
 
     for (int t0 = 0, tc = 0; t0 < n_tokens; t0 += tc) {

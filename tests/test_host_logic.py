@@ -151,6 +151,38 @@ def test_moe_workspace_follows_the_plan():
             assert need >= lib.mlk_moe_workspace_bytes(last, E, K, H, I)
 
 
+def _first_pass(T, E, K, H, I, kind, workspace=None):
+    """(tokens, wide) of the first pass with a workspace of the wide kernels, or of the size given."""
+    import ctypes
+    lib, out = _lib.load(), (ctypes.c_int32 * 2)()
+    need = lib.mlk_moe_wide_workspace_bytes(T, E, K, H, I) if workspace is None else workspace
+    assert lib.mlk_moe_first_pass(T, E, K, H, I, kind, need, ctypes.addressof(out)) == 0
+    return out[0], bool(out[1])
+
+
+@pytest.mark.parametrize("E,K,H,I,kind,two_passes,wide", [
+    # measured (256 CUs): the most tokens whose pass of 256 and remainder are the faster, the fewest whose wide pass is
+    (8, 2, 4096, 14336, 2, 257, 260), (256, 8, 7168, 256, 2, 264, 288), (256, 8, 7168, 2048, 2, 280, 304),
+    (128, 8, 2048, 768, 2, 257, 264), (160, 6, 5120, 1536, 2, 268, 288), (256, 2, 4096, 1024, 2, 280, 384),
+    (64, 1, 4096, 2048, 2, 280, 320), (128, 2, 4096, 2048, 1, 259, 268), (256, 8, 7168, 256, 1, 257, 264),
+    (8, 2, 4096, 14336, 1, 256, 257), (16, 4, 4096, 2048, 2, 256, 257), (64, 6, 2048, 1024, 1, 256, 257),
+    (256, 1, 2048, 512, 2, 256, 257), (256, 6, 5120, 1024, 1, 256, 257), (8, 2, 1024, 512, 2, 256, 257),
+])
+def test_moe_pass_above_256_tokens_is_the_cheaper_one(E, K, H, I, kind, two_passes, wide):
+    assert _first_pass(two_passes, E, K, H, I, kind) == (256, False)
+    assert _first_pass(wide, E, K, H, I, kind) == (wide, True)
+    most = min(4096, 16384 // K)
+    assert _first_pass(most + two_passes, E, K, H, I, kind) == (most, True)
+    # once wide, wide for every larger count; without the scratch in passes of 256
+    was = False
+    for T in range(257, 600):
+        tokens, now = _first_pass(T, E, K, H, I, kind)
+        assert now or not was, T
+        assert tokens == (T if now else 256)
+        was = now
+    assert _first_pass(600, E, K, H, I, kind, 1) == (256, False)
+
+
 @pytest.mark.parametrize("E,K,H,I", [(8, 2, 4096, 14336), (256, 8, 7168, 256), (1, 1, 4096, 14336), (4, 1, 4224, 2048),
                                      (60, 5, 768, 5376), (16, 16, 1024, 2048)])
 def test_moe_wide_workspace_holds_for_every_shorter_call(E, K, H, I):
@@ -163,6 +195,9 @@ def test_moe_wide_workspace_holds_for_every_shorter_call(E, K, H, I):
         need = lib.mlk_moe_wide_workspace_bytes(t, E, K, H, I)
         assert need >= before and need >= most and need >= min(t, 4096, 16384 // K) * K * H * 4, t
         before = need
+    for t in range(257, 4400, 7):
+        for kind in (1, 2):
+            assert _first_pass(t, E, K, H, I, kind, before) == _first_pass(t, E, K, H, I, kind), t
     for t in (1, 16, 171, 256):
         assert lib.mlk_moe_wide_workspace_bytes(t, E, K, H, I) == lib.mlk_moe_workspace_bytes(t, E, K, H, I)
 
@@ -239,5 +274,5 @@ def test_moe_plan_known_cases():
     small = _plan(256, 8, 2, 1024, 14336, 2)
     assert small["path"] == 4 and small["down_wk"] == 1
     assert _plan(256, 8, 2, 4096 + 128, 14336, 2)["path"] == 3
-    # 500 tokens run as 256 + 244: the plan of the first pass is what the query reports
+    # above 256 tokens: the plan of the passes of 256 that a call without the scratch of the wide kernels runs in
     assert _plan(500, 256, 8, 7168, 256, 2) == _plan(256, 256, 8, 7168, 256, 2)
