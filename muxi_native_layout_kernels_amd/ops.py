@@ -86,13 +86,14 @@ class WorkspacePool:
         with self._lock:
             buf = self._live.get(key)
             if buf is None or buf.numel() < nbytes:
-                if buf is not None:
-                    self._retired.append(buf)
-                grown = 0 if buf is None else buf.numel() + buf.numel() // 2      # few retirements on a growing series
+                old = buf
+                grown = 0 if old is None else old.numel() + old.numel() // 2      # few retirements on a growing series
                 size = max(int(nbytes), self.min_bytes, grown)
                 buf = torch.empty(size, dtype=torch.uint8, device=device)
                 if self.zero_prefix and prefix_bytes:
                     buf[:prefix_bytes].zero_()
+                if old is not None:                    # only now: where there is no room for more, it stays in use
+                    self._retired.append(old)
                 self._live[key] = buf
             return buf
 
@@ -581,6 +582,18 @@ def _moe_workspace(device, nbytes, stream=None):
     return _moe_pool.get(device, _stream() if stream is None else stream, nbytes)
 
 
+def _moe_scratch(device, T, E, K, hidden, inter):
+    """Scratch for T tokens: that of the wide kernels, or, where the card has no room for it, that of passes of 256 tokens
+    (8 experts, H 4096, I 14336 at 4096 tokens: 487 and 63 MiB), in which the call then runs."""
+    lib = _lib.load()
+    try:
+        return _moe_workspace(device, lib.mlk_moe_wide_workspace_bytes(T, E, K, hidden, inter))
+    except torch.OutOfMemoryError:
+        if T <= 256:
+            raise
+        return _moe_workspace(device, lib.mlk_moe_workspace_bytes(T, E, K, hidden, inter))
+
+
 def fused_experts_compute(experts_weights_matrix1, experts_weights_matrix2, activations, batch_size, expert_count,
                           dynamic_experts_per_act, topk_ids, actived_experts_weights, sorted_token_ids, cumsum_buffer,
                           padded_num_experts, experts_ids, C, y, *args, **kwargs):
@@ -672,7 +685,7 @@ def experts_compute_raw(w1, w2, x, T, E, K, hidden, inter, w_kind, topk_ids, top
                         w2_scale, y):
     """Thin call of the C entry point (alignment + both grouped GeMMs + weighted sum); no checks."""
     lib = _lib.load()
-    ws = _moe_workspace(x.device, lib.mlk_moe_wide_workspace_bytes(T, E, K, hidden, inter))
+    ws = _moe_scratch(x.device, T, E, K, hidden, inter)
     _lib.check(lib.mlk_fused_experts_compute(_ptr(w1), _ptr(w2), _ptr(x), T, E, K, hidden, inter, w_kind,
                                              _KIND[x.dtype], _ptr(topk_ids), _ptr(topk_weights), _ptr(experts_map),
                                              _ptr(w1_scale), _ptr(w2_scale), _ptr(y), _ptr(ws), ws.numel(),
@@ -684,7 +697,7 @@ def fused_moe_raw(w1, w2, x, logits, T, E, K, hidden, inter, w_kind, score_fun, 
     """Thin call of the whole-layer entry point (router + alignment + both grouped GeMMs + weighted sum); no
     checks.  `topk_ids` / `topk_weights` receive the routing."""
     lib = _lib.load()
-    ws = _moe_workspace(x.device, lib.mlk_moe_wide_workspace_bytes(T, E, K, hidden, inter))
+    ws = _moe_scratch(x.device, T, E, K, hidden, inter)
     _lib.check(lib.mlk_fused_moe(_ptr(w1), _ptr(w2), _ptr(x), _ptr(logits), T, logits.size(-1), E, K, hidden, inter,
                                  w_kind, _KIND[x.dtype], score_fun, n_groups, topk_groups, _ptr(bias),
                                  int(bool(renormalize)), _ptr(experts_map), _ptr(w1_scale), _ptr(w2_scale),

@@ -132,6 +132,33 @@ def test_workspace_pool_release():
     assert c is not b and c.numel() >= 1024
 
 
+def test_moe_scratch_falls_back_to_passes_of_256_tokens(monkeypatch):
+    """Where the card has no room for the scratch of the wide kernels the call gets that of 256-token passes; the pool keeps
+    what it had and counts it once.  Up to 256 tokens there is nothing smaller to fall back to."""
+    lib, layer = _lib.load(), (8, 2, 4096, 14336)
+    pool = ops.WorkspacePool(1024)
+    cpu = torch.device("cpu")
+    monkeypatch.setattr(ops, "_moe_workspace", lambda device, nbytes: pool.get(device, 0, nbytes))
+    small = pool.get(cpu, 0, 1 << 20)
+    narrow = lib.mlk_moe_workspace_bytes(4096, *layer)
+    real = torch.empty
+
+    def empty(size, **kw):
+        if size > room:
+            raise torch.OutOfMemoryError("no room for %d bytes" % size)
+        return real(size, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+    room = 2 * narrow
+    got = ops._moe_scratch(cpu, 4096, *layer)
+    assert got.numel() >= narrow and got.numel() < lib.mlk_moe_wide_workspace_bytes(4096, *layer)
+    assert pool.held_bytes() == small.numel() + got.numel() and any(b is small for b in pool.owned())
+    pool.release()
+    room = 1 << 20
+    with pytest.raises(torch.OutOfMemoryError):
+        ops._moe_scratch(cpu, 256, *layer)
+    assert pool.held_bytes() == 0
+
+
 def test_moe_workspace_follows_the_plan():
     """The fp32 buffer of the K-sliced down projections is sized for the slices the plan uses (not for the most
     the kernels could take), a call of several passes covers its shorter last pass, and the query grows with the
