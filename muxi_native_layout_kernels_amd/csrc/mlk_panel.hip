@@ -473,7 +473,10 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     // than their partial products cost (written and read once at about 5 TB/s; a k32 slab of a 256 x 256 panel takes 0.78 us).
     // 11008 x 4096 fp16 at 2100 tokens (nine tiles): 374 us in two slices, 199 us whole; bf16 at 3300 tokens 495 and 286 us;
     // soft-FP8 28672 x 8192 at 1100 tokens 739 us in three slices, 499 us whole.
-    if (last_round_only && sk > 1 && p.whole_groups == 0 && groups * p.token_tiles > device_cus() / 8) {
+    // Operands off 16 bytes stay sliced where the whole panels run the loop that loads straight into LDS and the sliced ones do not.
+    const bool whole_loads_lds = a_kind == MLK_FP8_E4M3 && width == 128 && rows == 256;
+    if (last_round_only && sk > 1 && p.whole_groups == 0 && groups * p.token_tiles > device_cus() / 8 &&
+        (!whole_loads_lds || (aligned16(a) && aligned16(b)))) {
         const long long cus = device_cus(), panels = (long long)p.row_tiles * p.token_tiles;
         const double panel_us = 0.78 * (k / 32) * rows * width / 65536.;
         const double whole_us = (double)((panels + cus - 1) / cus) * panel_us;

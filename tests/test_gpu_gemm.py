@@ -271,6 +271,28 @@ def test_gemm_panel_kernel_columns_of_the_last_token_tile(mlk, kind, m):
     assert_close(c, want, RTOL, ATOL, "last token tile %s M=%d" % (kind, m))
 
 
+def test_gemm_panel_kernel_id5_off_16_bytes_stays_sliced(mlk):
+    """Soft-FP8 panels of 256 x 128, eleven token tiles: computed whole by the loop that loads straight into LDS, but sliced by the
+    loop that loads through registers when the activations do not lie on 16 bytes."""
+    n, m, k = 4608, 1281, 512
+    codes = fp8_codes((n, k), 401)
+    g = torch.Generator().manual_seed(402)
+    scale = (torch.rand((n // 128, k // 128), generator=g) * 0.02 + 0.001).float().cuda()
+    a, b = pack_a(codes).cuda(), randn((m, k), torch.bfloat16, 1.0, 403).cuda()
+    flat = torch.empty(m * k + 8, dtype=b.dtype, device="cuda")
+    flat[1:1 + m * k] = b.view(-1)
+    shifted = flat[1:1 + m * k].view(m, k)
+    assert shifted.data_ptr() % 16 and shifted.is_contiguous()
+
+    def run(x, kernel_id, slices):
+        return mlk.gemm_layoutA_soft_fp8_wapper(a, scale, x, n, m, k, kernelParam1=4, kernelParam2=1, kernelParam3=slices,
+                                                kernelId=kernel_id)
+    whole, sliced = run(b, 3, 1), run(b, 3, 2)
+    assert not torch.equal(whole, sliced), "the two orders of summation cannot be told apart"
+    assert torch.equal(run(b, 5, 2), whole)
+    assert torch.equal(run(shifted, 5, 2), sliced)
+
+
 def test_gemm_panel_kernel_is_the_wide_default(mlk):
     """Above 64 tokens the heuristic for unscanned shapes picks the panel kernel; a K that is no
     multiple of 128 keeps the row-shared kernel, and the panel kernel refuses it when asked for by id."""
