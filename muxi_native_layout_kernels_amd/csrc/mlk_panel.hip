@@ -469,18 +469,31 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         if (partial_bytes < panel_partial_bytes(m, n, sk)) return fail(MLK_ERR_WORKSPACE, "gemm: workspace too small");
     }
     // Token tiles that do not divide an XCD's CUs leave no groups that fill whole rounds, and slicing every panel of a grid of
-    // several rounds pays the fold for all of it: then the panels are computed whole, unless the slices save more rounds
-    // than their partial products cost (written and read once at about 5 TB/s; a k32 slab of a 256 x 256 panel takes 0.78 us).
+    // several rounds pays the fold for all of it: then the panels are computed whole, unless the slices save more time in
+    // rounds than their partial products cost (written and read once at about 5 TB/s).  Row tiles belong to XCDs, so a round
+    // is CUs / 8 workgroups of one XCD, and the fullest XCD counts.
     // 11008 x 4096 fp16 at 2100 tokens (nine tiles): 374 us in two slices, 199 us whole; bf16 at 3300 tokens 495 and 286 us;
-    // soft-FP8 28672 x 8192 at 1100 tokens 739 us in three slices, 499 us whole.
+    // soft-FP8 28672 x 8192 at 1100 tokens 739 us in three slices, 499 us whole; but soft-FP8 4608 x 7168 at 800 tokens (35
+    // panels of 128 x 128 on half of the XCDs) 132 us in four slices, 161 us whole.  Over the 294 grids of this kind that the
+    // shipped tables lead to, at their fewest, middle and most tokens, twice, the choice is within 7 % of the better one, and within
+    // 3 % on all but 11 of 1764 (rounds counted over the whole chip and a panel's time taken as rows times tokens: up to 53 %).
     // Operands off 16 bytes stay sliced where the whole panels run the loop that loads straight into LDS and the sliced ones do not.
     const bool whole_loads_lds = a_kind == MLK_FP8_E4M3 && width == 128 && rows == 256;
     if (last_round_only && sk > 1 && p.whole_groups == 0 && groups * p.token_tiles > device_cus() / 8 &&
         (!whole_loads_lds || (aligned16(a) && aligned16(b)))) {
-        const long long cus = device_cus(), panels = (long long)p.row_tiles * p.token_tiles;
-        const double panel_us = 0.78 * (k / 32) * rows * width / 65536.;
-        const double whole_us = (double)((panels + cus - 1) / cus) * panel_us;
-        const double sliced_us = (double)((panels * sk + cus - 1) / cus) * panel_us / sk + (double)sk * m * n * 8 / 5e6;
+        const int per_xcd = groups * p.token_tiles, round = device_cus() / 8;
+        // us per k32 slab of a round of panels (whole soft-FP8 panels of 256 x 128 run two per CU: 0.65 us for a full round of
+        // those, 0.5 us for half a one), and what a round takes to start and to store: 6 us whole, 2 us sliced and 5 us for the fold
+        const double slab_us = width == 256 ? 0.8 : rows == 256 ? 0.57 : a_kind == MLK_FP8_E4M3 ? 0.35 : 0.29;
+        const double slabs = k / 32;
+        const double whole_rounds = (per_xcd + round - 1) / round, sliced_rounds = (double)(((long long)per_xcd * sk + round - 1) / round);
+        double whole_us = whole_rounds * slab_us * slabs;
+        if (whole_loads_lds) {
+            const int left = per_xcd % (2 * round);
+            whole_us = (per_xcd / (2 * round) * 0.65 + (left > round ? 0.65 : left > 0 ? 0.5 : 0.)) * slabs;
+        }
+        whole_us += whole_rounds * 6;
+        const double sliced_us = sliced_rounds * (slab_us * slabs / sk + 2) + (double)sk * m * n * 8 / 5e6 + 5;
         if (whole_us <= sliced_us) p.SK = sk = 1;
     }
     const int grid = (p.whole_groups + (groups - p.whole_groups) * sk) * 8 * p.token_tiles;

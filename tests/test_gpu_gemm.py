@@ -271,6 +271,36 @@ def test_gemm_panel_kernel_columns_of_the_last_token_tile(mlk, kind, m):
     assert_close(c, want, RTOL, ATOL, "last token tile %s M=%d" % (kind, m))
 
 
+@pytest.mark.parametrize("kind,n,m,k,p1,p2,p3,whole", [
+    ("fp8", 4608, 800, 7168, 2, 1, 4, False),    # 252 panels, but 35 of them on half of the XCDs: a second round for three
+    ("fp8", 4608, 2112, 7168, 4, 1, 4, True),    # 256 x 128 panels, two per CU when whole
+    ("fp8", 4608, 1856, 7168, 4, 1, 2, True),
+    ("bf16", 4608, 800, 7168, 2, 1, 4, False),
+    ("bf16", 11008, 2100, 4096, 4, 2, 2, True),
+])
+def test_gemm_panel_kernel_id5_slices_where_it_pays(mlk, kind, n, m, k, p1, p2, p3, whole):
+    """Token tiles that do not divide an XCD's CUs, several rounds: which of the two orders of summation kernelId 5 takes (both
+    measured) shows in the bits."""
+    g = torch.Generator(device="cuda").manual_seed(411)
+    b = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((n, k), generator=g, device="cuda")
+    if kind == "fp8":
+        a = mlk.pack_layout_a((w * 16).clamp_(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8))
+        scale = (torch.rand((n // 128, k // 128), generator=g, device="cuda") + 0.5) * (k ** -0.5 / 16)
+    else:
+        a, scale = mlk.pack_layout_a((w * k ** -0.5).to(torch.bfloat16)), None
+
+    def run(kernel_id, slices):
+        kw = dict(kernelParam1=p1, kernelParam2=p2, kernelParam3=slices, kernelId=kernel_id)
+        if kind == "fp8":
+            return mlk.gemm_layoutA_soft_fp8_wapper(a, scale, b, n, m, k, **kw)
+        return mlk.gemm_layoutA_wapper(a, b, n, m, k, **kw)
+    orders = {True: run(3, 1), False: run(3, p3)}
+    assert not torch.equal(orders[True], orders[False]), "the two orders of summation cannot be told apart"
+    assert_close(orders[True], orders[False].double().cpu().numpy(), RTOL, ATOL, "whole and sliced panels")
+    assert torch.equal(run(5, p3), orders[whole])
+
+
 def test_gemm_panel_kernel_id5_off_16_bytes_stays_sliced(mlk):
     """Soft-FP8 panels of 256 x 128, eleven token tiles: computed whole by the loop that loads straight into LDS, but sliced by the
     loop that loads through registers when the activations do not lie on 16 bytes."""
