@@ -306,14 +306,16 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
         if (experts_map) e = experts_map[e];
         return (e >= 0 && e < E) ? e : -1;
     };
-    // the expert ids of kAlignBatch tiles are fetched together: one trip to memory per batch instead of one per tile
+    // the expert ids of kAlignBatch tiles are fetched together: one trip to memory per batch instead of one per tile; tiles past
+    // the wave's last one are passed over (worked through empty they cost a call of 48 tokens and 8 experts 1.1 of 5.4 us)
     auto each_tile = [&](auto body) {
         for (int t0 = t_beg; t0 < t_end; t0 += kAlignBatch) {
             int e[kAlignBatch];
 #pragma unroll
             for (int j = 0; j < kAlignBatch; ++j) e[j] = t0 + j < t_end ? local_expert((t0 + j) * 64 + lane) : -1;
 #pragma unroll
-            for (int j = 0; j < kAlignBatch; ++j) body((t0 + j) * 64 + lane, e[j]);
+            for (int j = 0; j < kAlignBatch; ++j)
+                if (t0 + j < t_end) body((t0 + j) * 64 + lane, e[j]);
         }
     };
     each_tile([&](int, int e) {
