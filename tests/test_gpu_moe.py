@@ -203,7 +203,7 @@ def test_fused_moe_soft_fp8(mlk, T):
 
 @pytest.mark.parametrize("T,E,K,H,I", [
     (256, 8, 2, 256, 384),      # six token blocks per task: panels of 96 tokens
-    (300, 4, 2, 512, 384),      # eight blocks (panels of 128 tokens), then a pass of 44 tokens on the row-shared kernels
+    (256, 4, 2, 512, 384),      # eight blocks: panels of 128 tokens
     (200, 2, 1, 768, 128),      # one k window per slice boundary case: I = 128
     (256, 3, 3, 256, 1024),     # every token on every expert: tasks of 256 tokens in two panels each
 ])
@@ -666,7 +666,8 @@ def test_reference_grid_soft_fp8(mlk, m, n, k, e):
 @pytest.mark.parametrize("T", [171, 172, 244, 256, 500])
 def test_fused_moe_soft_fp8_many_experts_near_a_full_pass(mlk, T):
     """256 experts, top-8, soft-FP8 with 170 to 256 tokens in a pass: one token block per task, so the decode down
-    kernel runs with an output tile of up to 256 tokens; the rows per wave are chosen so that it fits the LDS."""
+    kernel runs with an output tile of up to 256 tokens; the rows per wave are chosen so that it fits the LDS.  (500 tokens
+    are one pass of the wide kernels.)"""
     E = 256
     bias = randn((E,), torch.bfloat16, 0.05, 78).abs()
     _moe_case(mlk, T, E, 8, 512, 256, torch.bfloat16, 1500 + T, score="sigmoid", groups=(8, 4), bias=bias, fp8=True)
@@ -715,33 +716,50 @@ def test_operands_off_16_bytes_stay_off_the_wide_kernels(mlk):
     assert_close(wide, want.double().cpu().numpy(), RTOL, ATOL, "wide kernels")
 
 
-@pytest.mark.parametrize("T", [300, 513])
-def test_workspace_of_256_token_passes_still_takes_longer_calls(mlk, T):
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+@pytest.mark.parametrize("T", [513, 556])
+def test_workspace_of_256_token_passes_still_takes_longer_calls(mlk, T, kind):
     """A workspace of mlk_moe_workspace_bytes() (no larger than that of 256 tokens) is enough for any token count: without the
-    scratch of the wide kernels the call runs in passes of 256 tokens, with results like those of the wide kernels."""
+    scratch of the wide kernels the call runs in passes of 256 tokens (row-shared or, with soft-FP8 weights, panel kernels) and a
+    remainder of one token or 44, with results like those of the wide kernels."""
     from muxi_native_layout_kernels_amd import _lib
     from muxi_native_layout_kernels_amd.ops import _stream
-    E, K, H, I, dtype = 4, 2, 256, 512, torch.bfloat16
+    import ctypes
+    E, K, H, I, dtype = 4, 2, 512, 384, torch.bfloat16
+    wk = 2 if kind == "fp8" else 1
     g = torch.Generator(device="cuda").manual_seed(77)
-    w1 = torch.randn((E, 2 * I, H), generator=g, device="cuda").mul_(H ** -0.5).to(dtype)
-    w2 = torch.randn((E, H, I), generator=g, device="cuda").mul_(I ** -0.5).to(dtype)
+
+    def weights(rows, k):
+        """(packed, scales or None, float32 values)"""
+        w = torch.randn((E, rows, k), generator=g, device="cuda")
+        if kind != "fp8":
+            w = (w * k ** -0.5).to(dtype)
+            return mlk.pack_layout_a(w), None, w.float()
+        codes = (w * 16).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        scale = torch.exp2(torch.randint(-10, -8, (E, rows // 128, k // 128), generator=g, device="cuda").float())
+        return (mlk.pack_layout_a(codes.view(torch.uint8)), scale,
+                codes.float() * scale.repeat_interleave(128, 1).repeat_interleave(128, 2))
+    (w1p, s1, w1), (w2p, s2, w2) = weights(2 * I, H), weights(H, I)
     x = torch.randn((T, H), generator=g, device="cuda").to(dtype)
     ids = torch.randint(0, E, (T, K), generator=g, device="cuda", dtype=torch.int32)
     wts = torch.rand((T, K), generator=g, device="cuda").to(dtype)
-    w1p, w2p = mlk.pack_layout_a(w1), mlk.pack_layout_a(w2)
+    ptr = lambda t: None if t is None else t.data_ptr()
     lib = _lib.load()
     out = []
-    for need in (lib.mlk_moe_workspace_bytes(T, E, K, H, I), lib.mlk_moe_wide_workspace_bytes(T, E, K, H, I)):
+    first, plan = (ctypes.c_int32 * 2)(), (ctypes.c_int32 * 8)()
+    assert lib.mlk_moe_plan(256, E, K, H, I, wk, ctypes.addressof(plan)) == 0 and plan[0] == (4 if kind == "fp8" else 3)
+    for need, want in ((lib.mlk_moe_workspace_bytes(T, E, K, H, I), [256, 0]),
+                       (lib.mlk_moe_wide_workspace_bytes(T, E, K, H, I), [T, 1])):
+        assert lib.mlk_moe_first_pass(T, E, K, H, I, wk, need, ctypes.addressof(first)) == 0 and list(first) == want
         ws = torch.empty(need, dtype=torch.uint8, device="cuda")
         y = torch.empty_like(x)
-        _lib.check(lib.mlk_fused_experts_compute(w1p.data_ptr(), w2p.data_ptr(), x.data_ptr(), T, E, K, H, I, 1, 1,
-                                                 ids.data_ptr(), wts.data_ptr(), None, None, None, y.data_ptr(),
-                                                 ws.data_ptr(), need, _stream()), "moe")
+        _lib.check(lib.mlk_fused_experts_compute(ptr(w1p), ptr(w2p), ptr(x), T, E, K, H, I, wk, 1, ptr(ids), ptr(wts), None,
+                                                 ptr(s1), ptr(s2), ptr(y), ptr(ws), need, _stream()), "moe")
         out.append(y.float().cpu())
-    _whole_tensor = torch.zeros((T, H), dtype=torch.float32, device="cuda")
+    want = torch.zeros((T, H), dtype=torch.float32, device="cuda")
     for e in range(E):
-        gate, up = (x.float() @ w1[e].float().T).split(I, dim=1)
-        h = (torch.nn.functional.silu(gate) * up).to(dtype).float() @ w2[e].float().T
-        _whole_tensor += h * (wts.float() * (ids == e)).sum(1, keepdim=True)
+        gate, up = (x.float() @ w1[e].T).split(I, dim=1)
+        h = (torch.nn.functional.silu(gate) * up).to(dtype).float() @ w2[e].T
+        want += h * (wts.float() * (ids == e)).sum(1, keepdim=True)
     for y in out:
-        assert_close(y, _whole_tensor.cpu().numpy(), RTOL, ATOL, "T=%d" % T)
+        assert_close(y, want.cpu().numpy(), RTOL, ATOL, "T=%d" % T)
