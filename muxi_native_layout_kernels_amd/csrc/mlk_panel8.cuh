@@ -167,7 +167,7 @@ struct Panel8Loop {
             widen(min(slab0, last), 0, 0);
             widen(min(slab0 + 1, last), 1, 1);
             issue_a(src, wave, min(slab0 + 3, last), 0);           // raw(3) into the raw buffer that slab 0 has left
-            wait_vmcnt_le<1>();                                    // the tiles of slab 2
+            if constexpr (TB > 1) wait_vmcnt_le<1>();              // the tiles of slab 2
             __builtin_amdgcn_s_waitcnt(0xc07f);                    // lgkmcnt(0): the widened tiles are written
             bare_barrier();
             rd(a0, b0, 0, 0);
@@ -175,15 +175,28 @@ struct Panel8Loop {
             for (int s = 0; s < nslab; ++s) {
                 const int nxt = (cur + 1) & 3, nx2 = (cur + 2) & 3, prv = (cur + 3) & 3;
                 const int r1 = rcur == 2 ? 0 : rcur + 1, r2 = rcur == 0 ? 2 : rcur - 1;  // raw buffers of slabs s + 1 (= s + 4), s + 2
+                auto issue = [&]() {
+                    issue_b(src, wave, min(slab0 + s + 3, last), prv);
+                    issue_a(src, wave, min(slab0 + s + 4, last), r1);
+                };
+                // With 64 token columns a slab has four products to hide anything under and latency sets the pace: the loads go
+                // out first, the operands are read in front of the products, and the tiles of slab s + 2 are waited for only
+                // here, a trip later than with more columns (the loads of two trips may be in flight; in the first one raw(3),
+                // which went out alone, and this trip's).  256 experts top-8, I 256, at 300 tokens: 487 -> 467 us.
+                if constexpr (TB == 1) {
+                    issue();
+                    if (s == 0) wait_vmcnt_le<NB + 2>();
+                    else wait_vmcnt_le<2 * (NB + 1)>();
+                }
                 // The fp8 tiles of slab s + 2 are read first, widened between the products of the first half step and written
-                // after them.  The loads go out behind the LDS reads, under the products (see spread_half_step); issued in front
-                // of them, right behind the barrier, every wave stood still for them: 28672 x 8192 at 1024 tokens 461 -> 451 us.
+                // after them.  From 128 columns on the loads go out behind the LDS reads, under the products (see
+                // spread_half_step); issued in front of them, right behind the barrier, every wave stood still for them:
+                // 28672 x 8192 at 1024 tokens 454 -> 444 us.
                 const float sc = scale_at(srow, min(slab0 + s + 2, last) >> 2);
                 const u32x2 *raw = reinterpret_cast<const u32x2 *>(win + 4 * kP8Slab + r2 * kP8RawSlab + 2 * wave * 32);
                 const u32x2 f0 = raw[lane], f1 = raw[64 + lane];
                 rd(a1, b1, cur, 1);
-                issue_b(src, wave, min(slab0 + s + 3, last), prv);
-                issue_a(src, wave, min(slab0 + s + 4, last), r1);
+                if constexpr (TB > 1) issue();
                 u32x4 w0, w1;
                 {
                     uint32_t x0, x1, x2, x3;
@@ -219,8 +232,10 @@ struct Panel8Loop {
                 __builtin_amdgcn_sched_barrier(0);
                 rd(a0, b0, nxt, 0);
                 mm(a1, b1);
-                spread_half_step<2 * TB, PR + TB, 0>();
-                wait_vmcnt_le<NB + 1>();                           // this wave's chunks of slab s + 2 and tiles of slab s + 3 have landed
+                if constexpr (TB > 1) spread_half_step<2 * TB, PR + TB, 0>();
+                else __builtin_amdgcn_sched_barrier(0);
+                // this wave's chunks of slab s + 2 have landed, and (but for 64 token columns) its tiles of slab s + 3
+                wait_vmcnt_le<TB == 1 ? NB + 2 : NB + 1>();
                 __builtin_amdgcn_s_waitcnt(0xc07f);                // and its widened tiles are written
                 bare_barrier();
                 cur = nxt;
