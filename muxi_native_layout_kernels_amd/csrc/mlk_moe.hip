@@ -20,6 +20,12 @@
 //               un-permute: no atomics, no intermediate [pairs, H] buffer, fixed
 //               summation order.
 //
+// That is the decode form of the two GeMMs.  One token has GeMV kernels of its own; tasks of
+// more than one token block run row-shared kernels (below) or, with soft-FP8 weights, panel
+// kernels (mlk_moe_panel.cuh), and calls of more than 256 tokens the wide kernels
+// (mlk_moe_wide.cuh); those three write fp32 products per routed pair, which
+// moe_combine_kernel adds per token in pick order.
+//
 // Algorithmic traffic per layer: active experts * 3*I*H*sizeof(W) (+ scales)
 // + 2*T*H*2 + T*E*2 bytes; the SiLU intermediate (T*K*I*2 bytes, written and
 // read once) stays in L2 / Infinity Cache for decode-sized T.
@@ -1408,13 +1414,13 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
 // (mlk_moe_wide.cuh) in passes of as many tokens as their workspace is allowed for: in passes of kMoeChunk tokens every
 // pass streams the weights of all experts it reaches again.  Measured, passes of kMoeChunk tokens -> wide kernels (us, without
 // the router):
-//                                                  tokens   257          264          272          304          512
-//   8 experts, top-2, H 4096, I 14336, bf16                 624 -> 559   894 -> 556   940 -> 555   960 -> 566  1039 -> 644
-//   the same, soft-FP8                                      440 -> 464   534 -> 462   576 -> 465   632 -> 480   735 -> 562
-//   256 experts, top-8, H 7168, I 256, bf16                 528 -> 542   657 -> 541   760 -> 543   995 -> 550   996 -> 581
-//   the same, soft-FP8                                      333 -> 491   415 -> 480   491 -> 481   625 -> 486   612 -> 508
-//   128 experts, top-8, H 2048, I 768, bf16                 243 -> 235   347 -> 234   393 -> 235   473 -> 238   439 -> 254
-//   the same, soft-FP8                                      156 -> 199   244 -> 200   277 -> 199   329 -> 200   275 -> 205
+//                                                  tokens   257          264          272          320
+//   8 experts, top-2, H 4096, I 14336, bf16                 624 -> 559   940 -> 547   942 -> 550   972 -> 561
+//   the same, soft-FP8                                      454 -> 461   579 -> 453   577 -> 468   637 -> 482
+//   256 experts, top-8, H 7168, I 256, bf16                 527 -> 542   651 -> 543   762 -> 541  1022 -> 551
+//   the same, soft-FP8                                      332 -> 468   413 -> 458   475 -> 459   664 -> 469
+//   128 experts, top-8, H 2048, I 768, bf16                 242 -> 240   346 -> 235   398 -> 236   476 -> 240
+//   the same, soft-FP8                                      158 -> 192   235 -> 193   276 -> 196   336 -> 194
 // A few tokens above kMoeChunk, moe_two_passes_pay() keeps the pass of kMoeChunk tokens and its remainder.  A remainder of up to
 // kMoeChunk tokens is a pass of the small kernels again, and a call whose workspace only holds passes of kMoeChunk tokens, or
 // whose operands do not lie on 16 bytes, runs in those.
@@ -1482,18 +1488,18 @@ static size_t moe_wide_most_pair_slices(int tokens, int n_experts, int topk, int
 // as the small kernels come to be bound by their products; the remainder costs its launches and the experts it reaches once
 // more.  Where a task is one token block, the down kernel walks all tasks in every workgroup (a share per expert) and its
 // grid of 16 output rows each runs in whole rounds.  The constants (us and MB) are fitted to 24 layers of 4 to 256 experts,
-// both kinds of weights and 257 to 512 tokens: no choice costs more than 4.5 % against the better one, where going wide always
-// cost up to 56 % (256 experts, top-8, H 7168, I 2048, soft-FP8, 257 tokens: 1950 -> 3050 us).
+// both kinds of weights and 257 to 320 tokens: three of 572 choices cost more than 3 % against the better one (4, 5 and 7.5 %),
+// where going wide always cost up to 52 % (256 experts, top-8, H 7168, I 2048, soft-FP8, 257 tokens: 1940 -> 2960 us).
 static bool moe_two_passes_pay(int rest, int n_experts, int topk, int hidden, int inter, bool fp8) {
     const double miss = topk < n_experts ? 1 - (double)topk / n_experts : 0;
     const double weights = 3e-6 * n_experts * hidden * inter * (fp8 ? 1 : 2), first = weights * (1 - pow(miss, kMoeChunk));
     const double mean = (double)kMoeChunk * topk / n_experts;
-    double gain = first * ((fp8 ? 0.1 : 0.02) - (fp8 ? 0.0004 : 0.0008) * (mean > 8 ? mean - 8 : 0));
+    double gain = first * ((fp8 ? 0.09 : 0.014) - (fp8 ? 0.0006 : 0.0008) * (mean > 8 ? mean - 8 : 0));
     if (moe_blocks_per_task(kMoeChunk, topk, n_experts) == 1) {
         const double rounds = hidden / 16. / device_cus();
         gain -= (fp8 ? 0.3 : 0.1) * n_experts + (rounds > 1 ? first / 19.5 * (ceil(rounds) / rounds - 1) : 0);
     }
-    return weights * (1 - pow(miss, rest)) / (fp8 ? 5.5 : 4) + (fp8 ? 30 : 5) < gain;
+    return weights * (1 - pow(miss, rest)) / (fp8 ? 5.5 : 6) + (fp8 ? 25 : 5) < gain;
 }
 
 // wide_ok: the operands and the workspace of the call are fit for the wide kernels
@@ -1630,7 +1636,7 @@ static bool moe_wide_fits(int n_tokens, int n_experts, int topk, int hidden, int
     return n_tokens > kMoeChunk && workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
 }
 
-// The most that a call of any 1 .. kMoeChunk tokens needs.  512 plans, about 50 us: kept per thread for the layer (and the
+// The most that a call of any 1 .. kMoeChunk tokens needs.  512 plans, about 25 us: kept per thread for the layer (and the
 // experiment switches) it was last asked for.
 static size_t moe_narrow_most(int n_experts, int topk, int hidden, int inter) {
     const int key[11] = {n_experts, topk, hidden, inter, device_cus(), g_moe_tile, g_moe_gemv1,
