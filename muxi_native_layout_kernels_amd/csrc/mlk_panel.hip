@@ -541,7 +541,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     } else if (rows == 256 && a_kind == MLK_FP8_E4M3 && (p.SK == 1 || p.whole_groups > 0)) {
         // soft-FP8, panels computed whole (or only the last round's sliced): the loop that prefetches through LDS, two
         // workgroups per CU (28672 x 8192 at 1024 tokens: 616 -> 474 us); fully sliced grids and 16-bit weights stay on
-        // the register-ring loop, which is ahead there
+        // the register-ring loop, which was ahead there (compared while the fold of this kernel still spilled)
 #define MLK_PANEL_LDS(TT, F8, RING)                                                                                    \
     do {                                                                                                           \
         constexpr size_t lds = PanelLdsShape<F8, 4, RING>::lds_bytes;                                              \
