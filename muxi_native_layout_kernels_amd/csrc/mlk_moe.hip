@@ -1614,6 +1614,7 @@ extern "C" int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_
 // The passes of a call share the workspace; the larger of the two weight kinds, since the query does not know which one
 // the call will bring.
 static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden, int inter, bool wide_ok) {
+    if (n_tokens < 1 || n_experts < 1 || topk < 1) return 0;       // nothing to run
     size_t bytes = 0;
     for (int fp8 = 0; fp8 < 2; ++fp8) {
         auto cover = [&](int tokens) {

@@ -1,5 +1,7 @@
 """CPU: host-side logic of the operator mirror that needs no GPU - argument parsing of the overloaded
 `fused_experts_compute`, `fused_moe` argument errors, launch-parameter guards, workspace sizing."""
+import os
+
 import pytest
 import torch
 
@@ -66,6 +68,18 @@ def test_workspace_sizes_from_the_library():
     huge = lib.mlk_moe_workspace_bytes(4096, 8, 2, 4096, 14336)
     assert 0 < small < big == huge          # tokens are processed in passes of 256
     assert lib.mlk_gemm_counter_bytes() == 65536
+
+
+def test_workspace_of_an_empty_batch():
+    """No tokens need no scratch (the calls themselves return at once); the queries ended the process with a division by zero.
+    Asked in a process of its own."""
+    import subprocess
+    import sys
+    code = ("from muxi_native_layout_kernels_amd import _lib\nlib = _lib.load()\n"
+            "print(lib.mlk_moe_workspace_bytes(0, 8, 2, 4096, 14336), lib.mlk_moe_wide_workspace_bytes(0, 8, 2, 4096, 14336))")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert out.returncode == 0 and out.stdout.split() == ["0", "0"], out.stderr
 
 
 def test_beta_must_be_zero():
