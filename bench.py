@@ -367,7 +367,7 @@ def main():
         b = torch.randn((m, k), generator=gen, device=dev).to(DT[xk])
         scale = block_scales((n // 128, k // 128)) if kind == 2 else None
         table = "layoutA_soft_fp8_gemm" if kind == 2 else ("layout_gemm" if native else "layoutA_gemm")
-        kid, p1, p2, p3 = mlk.ops._gemm_guard(arg_selector.selector(table).get_args((n, m, k)), n)
+        kid, p1, p2, p3 = mlk.ops._gemm_args(table, n, m, k, kind)
         if native:
             b_in = mlk.layoutB(b)
             c = torch.empty((n // 32, m // 16, 4, 16, 8), dtype=DT[xk], device=dev)
@@ -381,7 +381,7 @@ def main():
                 st = torch.cuda.current_stream().cuda_stream
                 ws_ptr, ws_len = 0, 0
                 if p3 > 1:      # per-stream scratch of the K split (allocated by the warm-up calls, before the capture)
-                    ws = mlk.ops._workspace(dev, lib.mlk_gemm_workspace_bytes(m, n, p1, p3), lib.mlk_gemm_counter_bytes(), st)
+                    ws = mlk.ops._workspace(dev, mlk.ops._gemm_workspace_bytes(lib, n, m, k, kid, p1, p2, p3), lib.mlk_gemm_counter_bytes(), st)
                     ws_ptr, ws_len = ws.data_ptr(), ws.numel()
                 _lib.check(lib.mlk_gemm_layout_a(a.data_ptr(), b_in.data_ptr(), c.data_ptr(), m, n, k, kind, xk,
                                                  1 if native else 0, 1 if native else 0, 1.0, 0,

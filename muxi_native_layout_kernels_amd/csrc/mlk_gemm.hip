@@ -53,6 +53,11 @@ extern template int launch_modes<BF16, true>(const GemmArgs &, int, int, int, in
 
 // kernel id 3 (mlk_panel.hip)
 size_t panel_partial_bytes(int m, int n, int sk);
+size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int sk);
+void panel8_plan(int m, int n, int k, bool fp8, int32_t *p1, int32_t *p2, int32_t *p3);
+int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, bool b_native, bool c_native,
+                       float alpha, const void *bias, const float *scale, int pr, int tb, int sk, int whole_groups, void *partial,
+                       size_t partial_bytes, hipStream_t s);
 int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, float alpha, const void *bias,
                  const float *scale, int width, int rows, int sk, bool last_round_only, void *counters,
                  size_t counter_bytes, void *partial, size_t partial_bytes, hipStream_t s);
@@ -77,6 +82,21 @@ extern "C" size_t mlk_gemm_workspace_bytes(int m, int n, int p1, int p3) {
     return kCounterBytes + bytes;
 }
 
+extern "C" size_t mlk_gemm_panel_workspace_bytes(int m, int n, int k, int p1, int p2, int p3) {
+    if (m <= 0 || n <= 0 || k < 64 || (p1 != 2 && p1 != 4) || p2 < 1 || p2 > 4 || p3 <= 1) return 0;
+    const size_t bytes = panel8_partial_bytes(m, n, k, p1 / 2, p2, p3);
+    return bytes ? kCounterBytes + bytes : 0;
+}
+
+extern "C" int mlk_gemm_panel_plan(int m, int n, int k, int a_kind, int32_t *out) {
+    MLK_REQUIRE(out != nullptr, "gemm: null pointer");
+    MLK_REQUIRE(m > 0 && n > 0 && n % 16 == 0 && k > 0 && k % 128 == 0, "gemm: the panel kernel needs N % 16 == 0 and K % 128 == 0");
+    MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
+    out[0] = 8;
+    panel8_plan(m, n, k, a_kind == MLK_FP8_E4M3, out + 1, out + 2, out + 3);
+    return MLK_OK;
+}
+
 extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, int x_kind,
                                  int b_mode, int c_mode, float alpha, const void *bias, const float *scale,
                                  int kernel_id, int p1, int p2, int p3, void *workspace, size_t workspace_bytes,
@@ -84,12 +104,12 @@ extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, i
     MLK_REQUIRE(m >= 0 && n >= 0 && k >= 0, "gemm: negative size");
     MLK_REQUIRE(n % 16 == 0, "gemm: N % 16 must be 0");
     MLK_REQUIRE(k % 32 == 0, "gemm: K % 32 must be 0");
-    MLK_REQUIRE(kernel_id == 1 || kernel_id == 2 || kernel_id == 3 || kernel_id == 4 || kernel_id == 5 || kernel_id == 12 || kernel_id == 14 || kernel_id == 16 ||
+    MLK_REQUIRE(kernel_id == 1 || kernel_id == 2 || kernel_id == 3 || kernel_id == 4 || kernel_id == 5 || kernel_id == 8 || kernel_id == 12 || kernel_id == 14 || kernel_id == 16 ||
                     kernel_id == 18,
                 "gemm: unknown kernel id");
     MLK_REQUIRE(p1 == 1 || p1 == 2 || p1 == 4 || p1 == 8, "gemm: row groups per wave (p1) must be 1, 2, 4 or 8");
-    MLK_REQUIRE(kernel_id == 3 || kernel_id == 5 || (n / 16) % p1 == 0, "gemm: row groups per wave (p1) must divide N/16");
-    MLK_REQUIRE(p2 == 1 || p2 == 2 || p2 == 4 || p2 == 8 || p2 == 16, "gemm: waves per workgroup (p2) must be 1, 2, 4, 8 or 16");
+    MLK_REQUIRE(kernel_id == 3 || kernel_id == 5 || kernel_id == 8 || (n / 16) % p1 == 0, "gemm: row groups per wave (p1) must divide N/16");
+    MLK_REQUIRE((p2 == 3 && kernel_id == 8) || p2 == 1 || p2 == 2 || p2 == 4 || p2 == 8 || p2 == 16, "gemm: waves per workgroup (p2) must be 1, 2, 4, 8 or 16");
     MLK_REQUIRE(p3 >= 1 && p3 <= 64, "gemm: K splits across workgroups (p3) must be 1..64");
     MLK_REQUIRE(x_kind == MLK_F16 || x_kind == MLK_BF16, "gemm: activations must be fp16 or bf16");
     MLK_REQUIRE(b_mode == MLK_B_ROWMAJOR || b_mode == MLK_B_NATIVE, "gemm: bad activation placement");
@@ -119,6 +139,22 @@ extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, i
         return launch_panel(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, alpha, bias, scale, p2 == 1 ? 128 : (p2 == 2 ? 256 : 0),
                             p1 == 2 ? 128 : (p1 == 4 ? 256 : 0), m > 64 ? p3 : 1, kernel_id == 5, ws, kCounterBytes,
                             ws ? ws + kCounterBytes : nullptr, ws ? part_bytes : 0, (hipStream_t)stream);
+    }
+    if (kernel_id == 8) {
+        // eight-wave panels; p1 = row groups per wave pair (2: 128-row panels, 4: 256-row panels), p2 = tokens per panel / 64, p3 = K slices.
+        // Their loads write LDS and their stores move 16 bytes: operands off 16 bytes take the kernels that go through registers.
+        MLK_REQUIRE((p1 == 2 || p1 == 4) && p2 <= 4, "gemm: kernel 8 takes p1 = 2 or 4 and p2 = 1 to 4");
+        MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
+        uint8_t *ws = (uint8_t *)workspace;
+        const size_t part_bytes = workspace_bytes > kCounterBytes ? workspace_bytes - kCounterBytes : 0;
+        if (aligned16(a) && aligned16(b) && aligned16(c) && aligned16(workspace))
+            return launch_panel8_gemm(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, b_mode == MLK_B_NATIVE, c_mode == MLK_C_NATIVE,
+                                      alpha, bias, scale, p1 / 2, p2, p3, -1, ws ? ws + kCounterBytes : nullptr, ws ? part_bytes : 0,
+                                      (hipStream_t)stream);
+        if (b_mode == MLK_B_ROWMAJOR && c_mode == MLK_C_ROWMAJOR)
+            return launch_panel(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, alpha, bias, scale, 128, 128, 1, false, nullptr, 0, nullptr, 0,
+                                (hipStream_t)stream);
+        kernel_id = 1, p1 = 1, p2 = 4, p3 = 1;
     }
     int sk = p3;
     if (sk > k / 32) sk = k / 32 > 0 ? k / 32 : 1;
@@ -179,7 +215,7 @@ extern "C" int mlk_gemm_layout_a_noalloc(const void *a, const void *b, void *c, 
     void *ws = nullptr;
     if (p3 > 1) {
         MLK_REQUIRE(m >= 0 && n >= 0 && n % 16 == 0, "gemm: N % 16 must be 0");
-        if (mlk_gemm_workspace_bytes(m, n, p1, p3) > kStaticScratchBytes)
+        if ((kernel_id == 8 ? mlk_gemm_panel_workspace_bytes(m, n, k, p1, p2, p3) : mlk_gemm_workspace_bytes(m, n, p1, p3)) > kStaticScratchBytes)
             return fail(MLK_ERR_WORKSPACE,
                         "gemm: this K split needs more than the 16 MiB of built-in scratch; use fewer splits (p3) "
                         "or mlk_gemm_layout_a with a caller-owned workspace");

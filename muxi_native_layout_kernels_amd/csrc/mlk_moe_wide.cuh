@@ -27,7 +27,7 @@
 #pragma once
 
 #include "mlk_moe_args.cuh"
-#include "mlk_panel8.cuh"
+#include "mlk_panel8_small.cuh"
 
 namespace mlk {
 
@@ -46,15 +46,16 @@ template <class T, bool FP8, int TB>
 __device__ __forceinline__ void moe_gate_up_wide(const MoeArgs &p, const MoeTask &tk, int rt, int wave, int lane) {
     extern __shared__ u32x4 win[];
     constexpr int WB = FP8 ? 1 : 2;
-    using Loop = Panel8Loop<T, FP8, TB>;
+    using Loop = typename Panel8<T, FP8, TB, 2>::Loop;
     const int wr = wave & 3, wt = wave >> 2;
     const int groups_i = p.I >> 4;
     const uint32_t tile_row = (uint32_t)p.H * 16u * WB;          // bytes of a row group
     P8Src src;
     src.a = p.W1 + (size_t)tk.expert * 2 * p.I * p.H * WB + (size_t)rt * 8 * tile_row;
     src.b = p.X;
-    // tiles 2 wave, 2 wave + 1 of the panel: quarter wave / 2, its gate tiles (even waves) or up tiles (odd waves)
-    const int half = wave & 1, rg = (wave >> 1) * 2;
+    // tiles 2 pair, 2 pair + 1 of the panel: quarter pair / 2, its gate tiles (even pairs) or up tiles (odd pairs)
+    const int pair = FP8 ? Loop::pair(wave) : Loop::tile(wave, 0) >> 1;
+    const int half = pair & 1, rg = (pair >> 1) * 2;
     const uint32_t tile0 = (uint32_t)(half * groups_i + rg) * tile_row;
     ScaleRow srow;
     if constexpr (FP8) {
@@ -67,16 +68,12 @@ __device__ __forceinline__ void moe_gate_up_wide(const MoeArgs &p, const MoeTask
     }
     const int slots = tk.nblocks * 16;
     const int32_t *sorted = p.sorted + tk.block0 * 16;
-#pragma unroll
-    for (int i = 0; i < Loop::NB; ++i) {
+    p8_token_rows<Loop>(src, (uint32_t)p.H * 2u, wave, lane, [&](int slot) {
         // slots without a routed pair read token 0: their columns of the product are never used
-        const int slot = p8_chunk<TB>(wave, i) * 16 + (lane >> 2);
         const int id = slot < slots ? sorted[slot] : p.n_pairs;
-        const int tok = id < p.n_pairs ? id / p.K : 0;
-        src.b_off[i] = (uint32_t)tok * (uint32_t)p.H * 2u + p8_lane_octet(lane);
-    }
+        return id < p.n_pairs ? id / p.K : 0;
+    });
     f32x16 acc[2][TB];
-    zero_acc(acc);
     Loop::run(acc, src, srow, 0, p.H >> 5, wave, lane);
     __syncthreads();
 
@@ -132,7 +129,7 @@ __device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restric
                                               int wave, int lane) {
     extern __shared__ u32x4 win[];
     constexpr int WB = FP8 ? 1 : 2;
-    using Loop = Panel8Loop<T, FP8, TB>;
+    using Loop = typename Panel8<T, FP8, TB, 2>::Loop;
     const int wr = wave & 3, wt = wave >> 2;
     const uint32_t tile_row = (uint32_t)p.I * 16u * WB;
     const int groups = p.H >> 4, rgp = rt * 16;
@@ -140,7 +137,8 @@ __device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restric
     src.a = p.W2 + (size_t)tk.expert * p.H * p.I * WB + (size_t)rgp * tile_row;
     src.b = p.Hbuf + (size_t)tk.block0 * 16 * p.I;
     // rows past H: a copy of the last row group, never stored
-    const int rga = min(rgp + 2 * wave, groups - 1), rgb = min(rgp + 2 * wave + 1, groups - 1);
+    const int tile = FP8 ? 2 * Loop::pair(wave) : Loop::tile(wave, 0);
+    const int rga = min(rgp + tile, groups - 1), rgb = min(rgp + tile + 1, groups - 1);
     ScaleRow srow;
     if constexpr (FP8) {
         src.a_off[0] = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * tile_row + (lane & 31) * 16;
@@ -151,15 +149,10 @@ __device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restric
         src.a_off[1] = (uint32_t)(rgb - rgp) * tile_row;
     }
     const int slots = tk.nblocks * 16;
-#pragma unroll
-    for (int i = 0; i < Loop::NB; ++i) {
-        const int slot = p8_chunk<TB>(wave, i) * 16 + (lane >> 2);
-        src.b_off[i] = (uint32_t)(slot < slots ? slot : 0) * (uint32_t)p.I * 2u + p8_lane_octet(lane);
-    }
+    p8_token_rows<Loop>(src, (uint32_t)p.I * 2u, wave, lane, [&](int slot) { return slot < slots ? slot : 0; });
     const int nwin = p.I >> 7;                                     // K slices are cut at multiples of 128 k
     const int wbeg = (int)((long long)sk * nwin / skd), wend = (int)((long long)(sk + 1) * nwin / skd);
     f32x16 acc[2][TB];
-    zero_acc(acc);
     Loop::run(acc, src, srow, 4 * wbeg, 4 * (wend - wbeg), wave, lane);
     __syncthreads();
 
@@ -216,7 +209,7 @@ __global__ void __launch_bounds__(512) moe_down_wide_kernel(MoeArgs p, float *__
 
 template <class T, bool FP8>
 int launch_moe_wide(const MoeArgs &a, int max_tasks, float *obuf, int skd, hipStream_t s) {
-    constexpr size_t ring = FP8 ? kP8Fp8LdsBytes : kP8RingBytes;
+    constexpr size_t ring = p8_ring_bytes<FP8, 2, 4>();
     constexpr size_t lds_up = ring, lds_down = ring > kWideDownOut ? ring : kWideDownOut;
     static bool ready_up[64] = {}, ready_down[64] = {};
     int rc = panel_lds_attribute(&moe_gate_up_wide_kernel<T, FP8>, lds_up, ready_up);

@@ -28,123 +28,9 @@
 // tiles by that XCD's L2.  K slices fold like in the row-shared kernel: fp32 partials with
 // agent-scope stores, the last workgroup to arrive adds them in slice order.
 #include "mlk_panel_loop.cuh"
-#include "mlk_panel8.cuh"
+#include "mlk_panel8_gemm.cuh"
 
 namespace mlk {
-
-struct PanelArgs {
-    const uint8_t *A;
-    const uint16_t *B;
-    uint16_t *C;
-    const uint16_t *bias;
-    const float *scale;
-    f32x4 *partial;      // [SK][sliced tiles][4 waves][quads of a wave][two planes of 64 x 8 bytes]
-    int *counters;       // [sliced tiles], zero between calls
-    int M, N, K;
-    int SK;              // K slices of the row tiles from whole_groups * 8 on
-    int whole_groups;    // groups of eight row tiles in front that are not sliced (0: every row tile has SK slices)
-    int row_tiles, token_tiles;
-    int band, chunk;     // gemm_panel8_kernel: groups of row tiles and token tiles that neighbouring workgroups of an XCD cover
-    float alpha;
-};
-
-// What happens to the accumulators of a panel: scaled and stored, or (K slices) handed over as fp32 partials that the
-// last workgroup to arrive adds in slice order.  acc[pr][tb] covers the row groups rg0 + 2 pr, + 1 and the 32 tokens from
-// tok0 + 32 tb on; NWAVES waves per workgroup, each with PR x TB accumulators; the fold fetches FB accumulators at a time.
-template <class T, int PR, int TB, int NWAVES, int FB>
-__device__ __forceinline__ void panel_finish(const PanelArgs &p, f32x16 (&acc)[PR][TB], int rg0, int tok0, int SK, int sk,
-                                             int rt, int tt, int wave, int lane, int *s_last) {
-    const int groups = p.N >> 4;
-    // accumulator element 4 g + e of lane 32 h + c: weight row 8 g + 4 h + e of the pair's 32, token c of the block's 32
-    const int half = lane >> 5, c32 = lane & 31;
-    auto epilogue = [&](int pr, int tb, int g, f32x4 v) {
-        const int n = (rg0 + 2 * pr) * 16 + 8 * g + 4 * half;
-        const int tok = tok0 + tb * 32 + c32;
-        if ((n >> 4) >= groups || tok >= p.M) return;
-        float o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o[i] = p.alpha * v[i];
-            if (p.bias) o[i] += T::to_f32(p.bias[n + i]);
-        }
-        store4<T>(p.C + (size_t)tok * p.N + n, o[0], o[1], o[2], o[3]);
-    };
-    auto quad = [&](const f32x16 &v, int g) { return f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}; };
-    if (SK == 1) {
-#pragma unroll
-        for (int pr = 0; pr < PR; ++pr)
-#pragma unroll
-            for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) epilogue(pr, tb, g, quad(acc[pr][tb], g));
-        return;
-    }
-    const int tile = (rt - p.whole_groups * 8) * p.token_tiles + tt;               // among the sliced tiles
-    const int tiles = (p.row_tiles - p.whole_groups * 8) * p.token_tiles;
-    // 64-lane group of quad jj of this wave in slice s (two planes of 8-byte halves, see st_agent_planar)
-    auto group_at = [&](int s, int jj) -> f32x4 * {
-        return p.partial + ((((size_t)s * tiles + tile) * NWAVES + wave) * (PR * TB * 4) + jj) * 64;
-    };
-    // partials travel as agent-scope (write-through / always-miss) accesses, like in the narrow kernels; a release /
-    // acquire fence pair around ordinary stores was measured slower (it writes back and invalidates a whole L2)
-#pragma unroll
-    for (int pr = 0; pr < PR; ++pr)
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) st_agent_planar(group_at(sk, (pr * TB + tb) * 4 + g), 64, lane, quad(acc[pr][tb], g));
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int prev = __hip_atomic_fetch_add(&p.counters[tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *s_last = (prev == SK - 1);
-        if (*s_last) __hip_atomic_store(&p.counters[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!*s_last) return;
-    // slice order; the loads of the next slice are in flight while the current one is added (a round trip to
-    // memory per slice would otherwise be paid in full: these loads bypass the caches).  FB accumulators are fetched,
-    // added and stored at a time (all of a row pair's where the registers allow it), in registers of their own: the
-    // published accumulators are dead, and summing into them kept all of them alive to the end, at 256 registers and a
-    // hundred spilled ones in the eight-wave kernels (now 234 and none: 4096 x 11008 at 1024 tokens in four slices, fp16 134 ->
-    // 108 us, bf16 131 -> 105 us; 8192 x 8192 fp16 at 512 tokens in two 148 -> 122 us).
-    static_assert(TB % FB == 0, "fetch groups are whole accumulators of one row pair");
-#pragma unroll
-    for (int pr = 0; pr < PR; ++pr) {
-#pragma unroll
-        for (int t0b = 0; t0b < TB; t0b += FB) {
-            f32x16 sum[FB];
-#pragma unroll
-            for (int tb = 0; tb < FB; ++tb)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) sum[tb][e] = 0.f;
-            f32x4 t0[FB * 4], t1[FB * 4];
-            auto fetch = [&](f32x4 (&t)[FB * 4], int sl) {
-#pragma unroll
-                for (int jj = 0; jj < FB * 4; ++jj) t[jj] = ld_agent_planar(group_at(sl, (pr * TB + t0b) * 4 + jj), 64, lane);
-            };
-            auto add = [&](const f32x4 (&t)[FB * 4]) {
-#pragma unroll
-                for (int tb = 0; tb < FB; ++tb)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) sum[tb][e] += t[tb * 4 + (e >> 2)][e & 3];
-            };
-            fetch(t0, 0);
-            for (int sl = 0; sl < SK; sl += 2) {
-                if (sl + 1 < SK) fetch(t1, sl + 1);
-                add(t0);
-                if (sl + 1 < SK) {
-                    if (sl + 2 < SK) fetch(t0, sl + 2);
-                    add(t1);
-                }
-            }
-#pragma unroll
-            for (int tb = 0; tb < FB; ++tb)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) epilogue(pr, t0b + tb, g, quad(sum[tb], g));
-        }
-    }
-}
 
 template <class T, bool FP8, int TB, int PR>
 __global__ void __launch_bounds__(256, 1) gemm_panel_kernel(PanelArgs p) {
@@ -264,137 +150,145 @@ __global__ void __launch_bounds__(256, 2) gemm_panel_lds_kernel(PanelArgs p) {
     panel_finish<T, PR, TB, kTileWaves, 2>(p, acc, rg0, tok0, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
 }
 
-// Output of an eight-wave panel that is computed whole: every wave turns its 64 rows x 128 tokens around in LDS (the ring
-// is free by then; 144 bytes per token, so that the 8-byte pieces of 32 tokens meet each bank at most twice) and stores
-// whole 128-byte lines, eight tokens per instruction.  Stored straight from the accumulators, a lane's four rows of one
-// token are 8 bytes in a line that fifteen other instructions complete: 67 MB of output took 23 us that way.
-constexpr int kP8OutPitch = 144;                               // bytes per token in the turn-around buffer
-constexpr size_t kP8OutBytes = (size_t)8 * 128 * kP8OutPitch;
-template <class T, int TB>
-__device__ __forceinline__ void p8_store_panel(const PanelArgs &p, f32x16 (&acc)[2][TB], int rg0, int tok0, int wave, int lane,
-                                               u32x4 *win) {
-    uint8_t *buf = reinterpret_cast<uint8_t *>(win) + (size_t)wave * 128 * kP8OutPitch;
-    const int half = lane >> 5, c32 = lane & 31;
-    const int n0 = rg0 * 16;                                   // first of the wave's 64 rows
-#pragma unroll
-    for (int pr = 0; pr < 2; ++pr)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int row = pr * 32 + 8 * g + 4 * half;        // of the wave's 64
-            float bias[4] = {0.f, 0.f, 0.f, 0.f};
-            if (p.bias && n0 + row < p.N) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) bias[i] = T::to_f32(p.bias[n0 + row + i]);
-            }
-#pragma unroll
-            for (int tb = 0; tb < TB; ++tb) {
-                u32x2 o;
-                o[0] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g] + bias[0], p.alpha * acc[pr][tb][4 * g + 1] + bias[1]);
-                o[1] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g + 2] + bias[2], p.alpha * acc[pr][tb][4 * g + 3] + bias[3]);
-                *reinterpret_cast<u32x2 *>(buf + (tb * 32 + c32) * kP8OutPitch + row * 2) = o;
-            }
+extern template int launch_panel8<BF16, false>(const Panel8Args &, int, int, hipStream_t);
+extern template int launch_panel8<F16, false>(const Panel8Args &, int, int, hipStream_t);
+extern template int launch_panel8<BF16, true>(const Panel8Args &, int, int, hipStream_t);
+
+// Lines, whole and dealt panels of m x n x k in panels of 128 pr rows x 64 tb tokens.  sk = 1: every panel whole; 2 .. 63: in that
+// many slices of K; kP8Deal: dealt evenly to one workgroup per CU.  With more panels than CUs only those that are left over after
+// whole rounds of one panel per CU are sliced or dealt, unless the caller says how many groups of eight row tiles are not (kernel ids
+// 3 and 5 on panels of 256 x 256).
+constexpr int kP8Deal = 64;
+static void panel8_shape(Panel8Args &p, int m, int n, int k, int pr, int tb, int sk, int whole_groups = -1) {
+    const int cus = device_cus(), windows = k / 64;
+    p.M = m;
+    p.N = n;
+    p.K = k;
+    p.row_tiles = (n + 128 * pr - 1) / (128 * pr);
+    p.token_tiles = (m + 64 * tb - 1) / (64 * tb);
+    const int panels = p.row_tiles * p.token_tiles;
+    const bool bands = whole_groups > 0 || (whole_groups < 0 || sk <= 1 ? panels > cus : false);
+    p.band = bands ? 8 : 0;
+    p.chunk = 4;
+    p.panels = bands ? (p.row_tiles + 7) / 8 * p.token_tiles : panels;
+    p.whole = p.panels;
+    p.deal = 0;
+    p.slots = 1;
+    if (sk <= 1) return;
+    const int round = bands ? cus / 8 : cus;                 // workgroups of a line that run at a time
+    const int whole = whole_groups >= 0 ? whole_groups * p.token_tiles : (bands ? p.panels / round * round : 0), rest = p.panels - whole;
+    if (rest == 0) return;
+    p.whole = whole;
+    if (sk < kP8Deal) {
+        p.deal = rest * (sk < windows ? sk : windows);
+    } else {
+        p.deal = round < rest * windows ? round : rest * windows;
+        p.slots = 2;
+    }
+}
+static size_t panel8_partial_bytes(const Panel8Args &p, int pr, int tb) {
+    return (size_t)(p.band > 0 ? 8 : 1) * p.deal * p.slots * pr * tb * 32768;
+}
+size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int sk) {
+    Panel8Args p = {};
+    panel8_shape(p, m, n, k, pr, tb, sk);
+    return panel8_partial_bytes(p, pr, tb);
+}
+
+// Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
+// rounds).  Fitted to the times of all shapes of this kernel on 24 weight shapes (512 to 32000 rows, K 640 to 18944) at 19 token counts from
+// 20 to 3000, bf16 and soft-FP8: the shape it picks is 1.8 % (soft-FP8 1.1 %) slower than the best one in the geometric mean, 11 % (7 %) at the
+// 95th percentile, of which the greater part is scatter of the single measurements.
+struct P8Cost {
+    // up to one panel per CU: start, store (256 x 256), fold = fold + fold_slice per slice + fold_mb per MB of slots; a k32 slab of a panel
+    // on an idle chip, what a workgroup on every CU adds to it, and the share of that which weights shared by token tiles keep
+    float start, store, fold, fold_slice, fold_mb, shared, slab[2][4], busy[2][4];
+    // several rounds: start, end of a round (256 x 256), what a last round that is not full saves of its empty part, fold, per MB; a slab
+    float r_start, r_end, r_empty, r_fold, r_fold_mb, r_slab[2][4];
+};
+static const P8Cost kP8Cost16 = {3.6f, 3.0f, 2.65f, 0.09f, 0.215f, 0.32f,
+                                 {{0.105f, 0.178f, 0.257f, 0.341f}, {0.171f, 0.299f, 0.362f, 0.503f}},
+                                 {{0.222f, 0.223f, 0.210f, 0.229f}, {0.487f, 0.401f, 0.470f, 0.548f}},
+                                 4.5f, 7.2f, 0.47f, 3.6f, 0.244f,
+                                 {{0.207f, 0.290f, 0.398f, 0.498f}, {0.315f, 0.476f, 0.649f, 0.808f}}};
+static const P8Cost kP8Cost8 = {5.3f, 2.8f, 3.0f, 0.1f, 0.197f, 0.68f,
+                                {{0.113f, 0.162f, 0.229f, 0.390f}, {0.196f, 0.257f, 0.531f, 0.462f}},
+                                {{0.096f, 0.136f, 0.152f, 0.152f}, {0.172f, 0.274f, 0.192f, 0.438f}},
+                                5.8f, 8.7f, 0.47f, 4.6f, 0.197f,
+                                {{0.192f, 0.281f, 0.381f, 0.564f}, {0.322f, 0.471f, 0.730f, 0.844f}}};
+static double panel8_us(const P8Cost &f, int m, int n, int k, int pr, int tb, int sk) {
+    const int cus = device_cus(), rows = (n + 128 * pr - 1) / (128 * pr), tokens = (m + 64 * tb - 1) / (64 * tb), windows = k / 64;
+    const int narrow = (m - (tokens - 1) * 64 * tb + 63) / 64;                   // columns / 64 of the last token tile
+    const long long panels = (long long)rows * tokens;
+    if (panels <= cus) {
+        const int t = tokens == 1 ? narrow : tb;
+        const double wgs = (double)panels * sk, busy = wgs < cus ? wgs / cus : 1;
+        const double slab = f.slab[pr - 1][t - 1] + f.busy[pr - 1][t - 1] * busy * (f.shared + (1 - f.shared) / tokens);
+        double us = f.start + f.store * pr * t / 8 + 2 * ((windows + sk - 1) / sk) * slab;
+        if (sk > 1) us += f.fold + f.fold_slice * sk + f.fold_mb * wgs * pr * t * 0.032768;
+        return us;
+    }
+    // row tiles belong to XCDs, and the fullest one counts
+    const int groups = (rows + 7) / 8, round = cus / 8;
+    const long long per_xcd = (long long)groups * tokens, rounds = (per_xcd + round - 1) / round;
+    const long long full = (long long)groups * (narrow < tb ? tokens - 1 : tokens);              // panels of all 64 tb columns
+    const double slabs = 2. * windows, end = f.r_end * pr * tb / 8;
+    const double t_full = f.r_slab[pr - 1][tb - 1] * slabs, t_narrow = f.r_slab[pr - 1][narrow - 1] * slabs;
+    const double even = (full * t_full + (per_xcd - full) * t_narrow) / round;                   // dealt out evenly
+    if (sk == 1) {
+        const double dealt = even + (double)per_xcd / round * end;
+        const double whole = (rounds - 1) * t_full + (full > round * (rounds - 1) ? t_full : t_narrow) + rounds * end;
+        return f.r_start + dealt + (whole - dealt) * (1 - f.r_empty);
+    }
+    if (per_xcd % round == 0) return 1e30;                                                       // nothing is left over
+    // 3 % in favour of whole panels, which are as good where the two come out alike
+    return 1.03 * (f.r_start + even + (per_xcd / round + 1.2) * end + f.r_fold + f.r_fold_mb * cus * pr * tb * 0.032768);
+}
+
+// Shape of kernel id 8 for m tokens x n rows x k: row groups per wave, tokens / 64 of a panel and K slices as the id takes them.
+void panel8_plan(int m, int n, int k, bool fp8, int32_t *p1, int32_t *p2, int32_t *p3) {
+    const P8Cost &f = fp8 ? kP8Cost8 : kP8Cost16;
+    double best = 1e30;
+    *p1 = 2, *p2 = 1, *p3 = 1;
+    for (int pr = 1; pr <= 2; ++pr)
+        for (int tb = 1; tb <= 4; ++tb) {
+            if (tb > 1 && m <= 64 * (tb - 1)) break;
+            const long long panels = (long long)((n + 128 * pr - 1) / (128 * pr)) * ((m + 64 * tb - 1) / (64 * tb));
+            auto consider = [&](int sk) {
+                const double us = panel8_us(f, m, n, k, pr, tb, sk);
+                if (us < best) best = us, *p1 = 2 * pr, *p2 = tb, *p3 = sk;
+            };
+            consider(1);
+            if (panels > device_cus()) consider(kP8Deal);
+            else
+                // slices of at least four slabs that one workgroup per CU takes
+                for (int sk = 2; sk <= 32 && panels * sk <= device_cus() && k / 64 / sk >= 2; ++sk) consider(sk);
         }
-    // lane 8 t + q: 16 bytes (8 rows) q of token t of each group of eight tokens
-    const int t8 = lane >> 3, q = lane & 7;
-    const bool rows_ok = n0 + q * 8 < p.N;
-#pragma unroll
-    for (int it = 0; it < 4 * TB; ++it) {
-        const int token = it * 8 + t8;
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(buf + token * kP8OutPitch + q * 16);
-        if (rows_ok && tok0 + token < p.M) *reinterpret_cast<u32x4 *>(p.C + (size_t)(tok0 + token) * p.N + n0 + q * 8) = v;
-    }
 }
 
-// ---------------------------------------------------------------------------------------------------------------
-// 256 x 256 panels: the eight-wave loop of mlk_panel8.cuh.
-//
-// Grid: without K slices the workgroup ids of an XCD walk bands of p.band groups of eight row tiles in chunks of
-// p.chunk token tiles, so that the 32 workgroups an XCD runs at a time cover 8 x 4 (row tiles x token tiles) and share
-// both operands through its L2; with the token tiles of two row tiles side by side (2 x 16) the same product took
-// 17 % longer (8192 x 8192, 4096 tokens: 491 against 413 us).  A fifth slab of LDS (160 KiB) changed nothing.
-template <class T, bool FP8, int TB>
-__device__ __forceinline__ void gemm_panel8(const PanelArgs &p, int rt, int tt, int sk, int SK) {
-    extern __shared__ u32x4 win[];
-    constexpr int PR = 2;
-    constexpr int WBYTES = FP8 ? 1 : 2;
-    using Loop = Panel8Loop<T, FP8, TB>;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave & 3, wt = wave >> 2;
-    const int groups = p.N >> 4;
-    const int rgp = rt * 16;                                   // first row group of the panel
-    const int rg0 = rgp + wr * 4;                              // of this wave
-    const int tok0 = tt * 256;
-    const int nwin_total = p.K / 64;                           // slices are cut in windows of 64 k, as the host counts them
-    const int wbeg = (int)((long long)sk * nwin_total / SK);
-    const int slab0 = 2 * wbeg;
-    const int nslab = 2 * ((int)((long long)(sk + 1) * nwin_total / SK) - wbeg);
-
-    // sources of this wave's loads: weight tiles 2 wave, 2 wave + 1 of the panel (rows past N: a copy of the last row
-    // group, never stored), its token chunks (tokens past M: the last token)
-    P8Src src;
-    src.a = p.A + (size_t)rgp * p.K * 16 * WBYTES;
-    src.b = p.B;
-    const int rga = min(rgp + 2 * wave, groups - 1), rgb = min(rgp + 2 * wave + 1, groups - 1);
-    ScaleRow srow;
-    if constexpr (FP8) {
-        src.a_off[0] = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * (uint32_t)p.K * 16u + (lane & 31) * 16;
-        const int scale_cols = (p.K + 127) >> 7;
-        srow = load_scale_row(p.scale ? p.scale + (size_t)(rga >> 3) * scale_cols : nullptr, scale_cols, lane);
-    } else {
-        src.a_off[0] = (uint32_t)(rga - rgp) * (uint32_t)p.K * 32u;
-        src.a_off[1] = (uint32_t)(rgb - rgp) * (uint32_t)p.K * 32u;
+int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, bool b_native, bool c_native,
+                       float alpha, const void *bias, const float *scale, int pr, int tb, int sk, int whole_groups, void *partial,
+                       size_t partial_bytes, hipStream_t s) {
+    MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
+    MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
+    Panel8Args p = {};
+    p.A = (const uint8_t *)a;
+    p.B = (const uint16_t *)b;
+    p.C = (uint16_t *)c;
+    p.bias = (const uint16_t *)bias;
+    p.scale = scale;
+    p.partial = (f32x4 *)partial;
+    p.alpha = alpha;
+    p.b_native = b_native;
+    p.c_native = c_native;
+    panel8_shape(p, m, n, k, pr, tb, sk, whole_groups);
+    if (p.deal > 0) {
+        MLK_REQUIRE(partial != nullptr, "gemm: a K split across workgroups needs a workspace");
+        if (partial_bytes < panel8_partial_bytes(p, pr, tb)) return fail(MLK_ERR_WORKSPACE, "gemm: workspace too small");
     }
-#pragma unroll
-    for (int i = 0; i < Loop::NB; ++i) {
-        const int tok = min(tok0 + p8_chunk<TB>(wave, i) * 16 + (lane >> 2), p.M - 1);
-        src.b_off[i] = (uint32_t)tok * (uint32_t)p.K * 2u + p8_lane_octet(lane);
-    }
-    f32x16 acc[PR][TB];
-    zero_acc(acc);
-    Loop::run(acc, src, srow, slab0, nslab, wave, lane);
-    __syncthreads();
-    if (TB < 4 || SK == 1) p8_store_panel<T, TB>(p, acc, rg0, tok0 + wt * 32 * TB, wave, lane, win);
-    else if constexpr (TB == 4)
-        panel_finish<T, PR, TB, 8, 2>(p, acc, rg0, tok0 + wt * 128, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
-}
-
-template <class T, bool FP8>
-__global__ void __launch_bounds__(512) gemm_panel8_kernel(PanelArgs p) {
-    // workgroup -> (row tile, k slice, token tile), as in gemm_panel_kernel
-    const int xcd = blockIdx.x & 7;
-    int u = blockIdx.x >> 3;
-    int SK, sk, tt, rt;
-    if (p.band > 0) {
-        const int TT = p.token_tiles, groups8 = (p.row_tiles + 7) >> 3, RB = p.band, TC = p.chunk;
-        const int band = u / (RB * TT);
-        const int nb = min(RB, groups8 - band * RB);           // groups of row tiles in this band
-        const int v = u - band * RB * TT;
-        const int c = v / (nb * TC);
-        const int tc = min(TC, TT - c * TC);                   // token tiles in this chunk
-        const int w = v - c * nb * TC;
-        SK = 1, sk = 0;
-        tt = c * TC + w % tc;
-        rt = (band * RB + w / tc) * 8 + xcd;
-    } else {
-        const int whole_wgs = p.whole_groups * p.token_tiles;
-        const bool sliced = u >= whole_wgs;
-        SK = sliced ? p.SK : 1;
-        if (sliced) u -= whole_wgs;
-        tt = u % p.token_tiles;
-        u /= p.token_tiles;
-        sk = u % SK;
-        rt = ((sliced ? p.whole_groups : 0) + u / SK) * 8 + xcd;
-    }
-    if (rt >= p.row_tiles) return;
-    // The last token tile multiplies the 64, 128 or 192 token columns that cover it (28672 x 4096 bf16 at 700 tokens 196 ->
-    // 193 us, 13824 x 5120 at 3000 tokens 372 -> 367 us); the fold of K slices knows whole tiles.
-    switch (SK == 1 ? min(4, (p.M - tt * 256 + 63) >> 6) : 4) {
-        case 1: gemm_panel8<T, FP8, 1>(p, rt, tt, sk, SK); break;
-        case 2: gemm_panel8<T, FP8, 2>(p, rt, tt, sk, SK); break;
-        case 3: gemm_panel8<T, FP8, 3>(p, rt, tt, sk, SK); break;
-        default: gemm_panel8<T, FP8, 4>(p, rt, tt, sk, SK); break;
-    }
+    if (a_kind == MLK_FP8_E4M3) return launch_panel8<BF16, true>(p, pr, tb, s);
+    if (a_kind == MLK_F16) return launch_panel8<F16, false>(p, pr, tb, s);
+    return launch_panel8<BF16, false>(p, pr, tb, s);
 }
 
 // Tokens per panel when the caller leaves the choice open.  Workgroups run one per CU in rounds; a 256-token panel
@@ -435,6 +329,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     p.K = k;
     p.alpha = alpha;
     if (width != 128 && width != 256) width = panel_tokens(m, n, a_kind == MLK_FP8_E4M3);
+    if (width == 256) rows = 256;
     p.token_tiles = (m + width - 1) / width;
     MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
     MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
@@ -444,7 +339,6 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     p.SK = sk;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    if (width == 256) rows = 256;
     if (rows != 128 && rows != 256) {
         const int cus = device_cus();
         // few panels: 128-row panels put twice as many CUs to work (a 128-row panel takes two thirds of the time of
@@ -498,6 +392,9 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         const double sliced_us = sliced_rounds * (slab_us * slabs / sk + 2) + (double)sk * m * n * 8 / 5e6 + 5;
         if (whole_us <= sliced_us) p.SK = sk = 1;
     }
+    if (width == 256)
+        return launch_panel8_gemm(a, b, c, m, n, k, a_kind, false, false, alpha, bias, scale, 2, 4, p.SK, p.whole_groups, partial,
+                                  partial_bytes, s);
     const int grid = (p.whole_groups + (groups - p.whole_groups) * sk) * 8 * p.token_tiles;
     // one workgroup per CU (the register ring and the accumulators take a whole SIMD's file); more than 64 KiB of
     // dynamic LDS has to be requested once per kernel
@@ -514,31 +411,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         }                                                                                                          \
         gemm_panel_kernel<TT, F8, TBB, PRR><<<grid, 256, lds, s>>>(p);                                                  \
     } while (0)
-    if (width == 256) {
-        // eight waves, operands through LDS
-#define MLK_PANEL8(KERNEL, LDS)                                                                                        \
-    do {                                                                                                           \
-        static bool ready_on[64] = {};                                                                             \
-        bool &ready = ready_on[dev & 63];                                                                          \
-        if (!ready) {                                                                                              \
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(KERNEL),                            \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)(LDS));           \
-            if (e != hipSuccess) return fail(MLK_ERR_LAUNCH, hipGetErrorString(e));                                \
-            ready = true;                                                                                          \
-        }                                                                                                          \
-        KERNEL<<<grid, 512, LDS, s>>>(p);                                                                          \
-    } while (0)
-        const bool whole = p.SK == 1 && p.whole_groups == 0;
-        p.band = whole ? 8 : 0;
-        p.chunk = 4;
-        // LDS: the ring, or the turn-around buffer of the output if that is larger
-        constexpr size_t lds16 = kP8RingBytes > kP8OutBytes ? kP8RingBytes : kP8OutBytes;
-        constexpr size_t lds8 = kP8Fp8LdsBytes > kP8OutBytes ? kP8Fp8LdsBytes : kP8OutBytes;
-        if (a_kind == MLK_FP8_E4M3) MLK_PANEL8((gemm_panel8_kernel<BF16, true>), lds8);
-        else if (a_kind == MLK_F16) MLK_PANEL8((gemm_panel8_kernel<F16, false>), lds16);
-        else MLK_PANEL8((gemm_panel8_kernel<BF16, false>), lds16);
-#undef MLK_PANEL8
-    } else if (rows == 256 && a_kind == MLK_FP8_E4M3 && (p.SK == 1 || p.whole_groups > 0)) {
+    if (rows == 256 && a_kind == MLK_FP8_E4M3 && (p.SK == 1 || p.whole_groups > 0)) {
         // soft-FP8, panels computed whole (or only the last round's sliced): the loop that prefetches through LDS, two
         // workgroups per CU (28672 x 8192 at 1024 tokens: 616 -> 474 us); fully sliced grids and 16-bit weights stay on
         // the register-ring loop, which was ahead there (compared while the fold of this kernel still spilled)

@@ -9,6 +9,7 @@ stream.  PyTorch is used for device memory and streams only.
 Reference naming: `m` = weight rows (output features), `k` = reduction,
 `n` = activation rows (tokens).
 """
+import ctypes
 import threading
 
 import torch
@@ -335,7 +336,7 @@ def _gemm_call(A, A_Scale, B, m, n, k, alpha, beta, bias, b_mode, c_mode, kernel
     ws = None
     ws_bytes = 0
     if p3 > 1:
-        ws_bytes = lib.mlk_gemm_workspace_bytes(n, m, int(p1), int(p3))
+        ws_bytes = _gemm_workspace_bytes(lib, m, n, k, int(kernel_id), int(p1), int(p2), int(p3))
         ws = _workspace(B.device, ws_bytes, lib.mlk_gemm_counter_bytes())
         ws_bytes = ws.numel()
     _lib.check(lib.mlk_gemm_layout_a(_ptr(A), _ptr(B), _ptr(C), n, m, k, a_kind, _KIND[B.dtype], b_mode, c_mode,
@@ -344,13 +345,35 @@ def _gemm_call(A, A_Scale, B, m, n, k, alpha, beta, bias, b_mode, c_mode, kernel
     return C
 
 
+def _gemm_workspace_bytes(lib, m, n, k, kid, p1, p2, p3):
+    if kid == 8:
+        return lib.mlk_gemm_panel_workspace_bytes(n, m, k, p1, p2, p3)
+    return lib.mlk_gemm_workspace_bytes(n, m, p1, p3)
+
+
 def _gemm_guard(args, m):
     kid, p1, p2, p3 = args
+    if kid == 8:
+        return args if p1 in (2, 4) and p2 in (1, 2, 3, 4) and 1 <= p3 <= 64 else (1, 1, 4, 1)
     if kid not in (1, 2, 3, 4, 5, 12, 14, 16, 18) or p1 not in (1, 2, 4, 8) or \
             (kid not in (3, 5) and (m // 16) % p1 != 0) or \
             p2 not in (1, 2, 4, 8, 16) or p3 < 1:
         return (1, 1, 4, 1)
     return args
+
+
+def _gemm_args(table, m, n, k, a_kind):
+    """Launch parameters of a table-driven GeMM call: the table's row of this very shape, else, above 64 tokens, the eight-wave
+    panels in the shape that the library expects to be fastest (`mlk_gemm_panel_plan`), else what the selector makes of
+    it.  The shipped tables hold no rows above 64 tokens: on 24 weight shapes at 14 token counts from 65 to 3000 the
+    panels were 1.3 (bf16) to 1.43 (soft-FP8) times as fast as the rows that had been scanned for the older panel kernels (geometric
+    mean; 0.98 at worst, 3.2 at best), and in native layouts, where those do not run, up to ten times."""
+    sel = arg_selector.selector(table)
+    if n > 64 and k % 128 == 0 and n * k < 1 << 31 and (m, n, k) not in sel.table():
+        plan = (ctypes.c_int32 * 4)()
+        if _lib.load().mlk_gemm_panel_plan(n, m, k, a_kind, plan) == 0:
+            return tuple(plan)
+    return _gemm_guard(sel.get_args((m, n, k)), m)
 
 
 def _gemm_eager(tag, table, checked, A, A_Scale, B, alpha, beta, bias, b_mode, c_mode):
@@ -379,9 +402,9 @@ def _gemm_eager(tag, table, checked, A, A_Scale, B, alpha, beta, bias, b_mode, c
     lib = _lib.load()
     m, k = A.size(0) * 16, A.size(1) * 8
     n = B.size(0) if b_mode == _B_ROWMAJOR else B.size(1) * 16
-    kid, p1, p2, p3 = _gemm_guard(arg_selector.selector(table).get_args((m, n, k)), m)
+    kid, p1, p2, p3 = _gemm_args(table, m, n, k, _kind(A))
     _plans[key] = (m, n, k, _kind(A), _KIND[B.dtype], kid, p1, p2, p3,
-                   lib.mlk_gemm_workspace_bytes(n, m, int(p1), int(p3)) if p3 > 1 else 0, lib.mlk_gemm_counter_bytes(),
+                   _gemm_workspace_bytes(lib, m, n, k, kid, p1, p2, p3) if p3 > 1 else 0, lib.mlk_gemm_counter_bytes(),
                    _is_fp8(A) and A_Scale is not None, tuple(C.shape), lib.mlk_gemm_layout_a)
     return C
 
@@ -417,7 +440,7 @@ def _gemm_layoutA_checked(A, B, alpha=1, beta=0, bias=None):
     k = a_k
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
-    kid, p1, p2, p3 = _gemm_guard(arg_selector.selector("layoutA_gemm").get_args((m, n, k)), m)
+    kid, p1, p2, p3 = _gemm_args("layoutA_gemm", m, n, k, _kind(A))
     return gemm_layoutA_wapper(A, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 
@@ -447,7 +470,7 @@ def _gemm_layoutA_soft_fp8_checked(A, A_Scale, B, alpha=1, beta=0, bias=None):
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
     _check(B.dtype == torch.bfloat16, "soft-FP8 weights need bf16 activations")
-    kid, p1, p2, p3 = _gemm_guard(arg_selector.selector("layoutA_soft_fp8_gemm").get_args((m, n, k)), m)
+    kid, p1, p2, p3 = _gemm_args("layoutA_soft_fp8_gemm", m, n, k, _kind(A))
     return gemm_layoutA_soft_fp8_wapper(A, A_Scale, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 
@@ -488,7 +511,7 @@ def _gemm_layoutAB_ContinuousC_checked(A, B, alpha=1, beta=0, bias=None):
     k = a_k
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
-    kid, p1, p2, p3 = _gemm_guard(arg_selector.selector("continuous_gemm").get_args((m, n, k)), m)
+    kid, p1, p2, p3 = _gemm_args("continuous_gemm", m, n, k, _kind(A))
     return gemm_layoutAB_ContinuousC_wapper(A, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 
@@ -515,7 +538,7 @@ def _gemm_layoutABC_checked(A, B, alpha=1, beta=0, bias=None):
     k = a_k
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
-    kid, p1, p2, p3 = _gemm_guard(arg_selector.selector("layout_gemm").get_args((m, n, k)), m)
+    kid, p1, p2, p3 = _gemm_args("layout_gemm", m, n, k, _kind(A))
     return gemm_layoutABC_wapper(A, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 

@@ -568,3 +568,85 @@ def test_gemm_repeated_calls_take_the_launch_plan_and_keep_the_checks(mlk):
     wide = torch.zeros((m, 2 * k), dtype=torch.float16, device="cuda")
     with pytest.raises(RuntimeError, match="contiguous"):
         mlk.gemm_layoutA(a, wide[:, ::2])
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8"])
+@pytest.mark.parametrize("p1,p2", [(p1, p2) for p1 in (2, 4) for p2 in (1, 2, 3, 4)])
+@pytest.mark.parametrize("n,m,k,p3", [
+    (128, 1, 128, 1),           # the smallest call: one panel, four slabs
+    (272, 65, 384, 1),          # rows that end inside a panel, a token tile of one token
+    (400, 130, 640, 3),         # ten k windows in three slices
+    (528, 257, 1152, 64),       # k windows dealt to as many workgroups: runs that end inside a panel
+    (1040, 192, 2048, 16),      # two windows per slice
+])
+def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3):
+    """kernelId 8 in every panel shape: remainders of rows, tokens and k, whole, sliced and dealt; row-major operands against the
+    oracle, layout-B activations and layout-C output against the row-major run, whose sums have the same order."""
+    dtype = torch.float16 if kind == "fp16" else torch.bfloat16
+    x = randn((m, k), dtype, 1.0, 31)
+    bias = randn((1, n), dtype, 1.0, 32)
+    kw = dict(alpha=0.5, bias=bias.cuda(), kernelParam1=p1, kernelParam2=p2, kernelParam3=p3, kernelId=8)
+    if kind == "fp8":
+        w = fp8_codes((n, k), 33)
+        scale = (torch.rand(((n + 127) // 128, k // 128), generator=torch.Generator().manual_seed(34)) * 0.02 + 0.001).float()
+        c = mlk.gemm_layoutA_soft_fp8_wapper(pack_a(w).cuda(), scale.cuda(), x.cuda(), n, m, k, **kw)
+        want = ogemm.softfp8_linear_expected(w, scale, x, 0.5, bias)
+        assert_close(c, want, RTOL, ATOL, "soft-FP8 panels")
+        return
+    w = randn((n, k), dtype, k ** -0.5, 33)
+    a = pack_a(w).cuda()
+    c = mlk.gemm_layoutA_wapper(a, x.cuda(), n, m, k, **kw)
+    assert_close(c, ogemm.linear_expected(w, x, 0.5, bias), RTOL, ATOL, "panels")
+    if m % 16 == 0 and n % 32 == 0:
+        xb = mlk.layoutB(x.cuda())
+        assert torch.equal(bits(mlk.gemm_layoutAB_ContinuousC_wapper(a, xb, n, m, k, **kw)), bits(c))
+        assert torch.equal(bits(mlk.reLayoutC(mlk.gemm_layoutABC_wapper(a, xb, n, m, k, **kw))), bits(c))
+
+
+@pytest.mark.parametrize("n,m,k,p1,p2", [(4352, 4100, 256, 4, 4), (2304, 1984, 256, 2, 1), (8448, 1000, 128, 2, 2)])
+def test_gemm_eight_wave_panels_several_rounds(mlk, n, m, k, p1, p2):
+    """More panels than CUs: the bands' order of the panels, and the panels left over after whole rounds dealt or sliced."""
+    g = torch.Generator(device="cuda").manual_seed(35)
+    w = (torch.randn((n, k), generator=g, device="cuda") * k ** -0.5).to(torch.bfloat16)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    a = mlk.pack_layout_a(w)
+    want = (x.float() @ w.float().t()).double().cpu().numpy()
+    for p3 in (1, 2, 64):
+        c = mlk.gemm_layoutA_wapper(a, x, n, m, k, kernelParam1=p1, kernelParam2=p2, kernelParam3=p3, kernelId=8)
+        assert_close(c, want, RTOL, ATOL, "several rounds, p3 = %d" % p3)
+
+
+@pytest.mark.parametrize("native", [False, True])
+def test_gemm_eight_wave_panels_off_16_bytes(mlk, native):
+    """Operands that do not lie on 16 bytes run the kernels that load through registers."""
+    n, m, k = 640, 80, 512
+    w, x = randn((n, k), torch.bfloat16, 0.05, 36), randn((m, k), torch.bfloat16, 1.0, 37)
+    a = pack_a(w).cuda()
+    b = pack_b(x).cuda() if native else x.cuda()
+    flat = torch.empty(m * k + 8, dtype=b.dtype, device="cuda")
+    flat[1:1 + m * k] = b.view(-1)
+    shifted = flat[1:1 + m * k].view(b.shape)
+    assert shifted.data_ptr() % 16
+    c = mlk.gemm_layoutAB_ContinuousC(a, shifted) if native else mlk.gemm_layoutA(a, shifted)
+    assert_close(c, ogemm.linear_expected(w, x), RTOL, ATOL, "off 16 bytes")
+
+
+def test_gemm_eight_wave_panels_replayed_from_a_graph(mlk):
+    """The second launch of a sliced product under capture: every replay equals the eager result."""
+    n, m, k = 1024, 100, 4096
+    w, x = randn((n, k), torch.bfloat16, 0.02, 38), randn((m, k), torch.bfloat16, 1.0, 39).cuda()
+    a = pack_a(w).cuda()
+    want = mlk.gemm_layoutA(a, x)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        mlk.gemm_layoutA(a, x)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            c = mlk.gemm_layoutA(a, x)
+    for _ in range(3):
+        c.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want)
+        assert torch.equal(mlk.gemm_layoutA(a, x), want)

@@ -317,3 +317,34 @@ def test_moe_plan_known_cases():
     assert _plan(256, 8, 2, 4096 + 128, 14336, 2)["path"] == 3
     # above 256 tokens: the plan of the passes of 256 that a call without the scratch of the wide kernels runs in
     assert _plan(500, 256, 8, 7168, 256, 2) == _plan(256, 256, 8, 7168, 256, 2)
+
+
+def test_panel_plan_is_a_shape_the_kernel_takes():
+    """The eight-wave panels' plan over odd and ordinary shapes: launch parameters that the guard passes, K slices of at least two k
+    windows, a workspace exactly where panels are split, and table rows of the very shape in front of it."""
+    import ctypes
+    import random
+    from muxi_native_layout_kernels_amd import _lib, arg_selector
+    lib = _lib.load()
+    rng = random.Random(7)
+    for _ in range(300):
+        n, k, m = 128 * rng.randint(1, 250), 128 * rng.randint(1, 140), rng.choice([1, 33, 64, 65, 100, 256, 257, 777, 4096])
+        out = (ctypes.c_int32 * 4)()
+        assert lib.mlk_gemm_panel_plan(m, n, k, rng.choice([0, 2]), out) == 0
+        kid, p1, p2, p3 = out
+        assert kid == 8 and ops._gemm_guard(tuple(out), n) == tuple(out)
+        panels = -(-n // (64 * p1)) * -(-m // (64 * p2))
+        assert p3 == 1 or (p3 == 64 and panels > 256) or (panels * p3 <= 256 and k // 64 // p3 >= 2)
+        assert (lib.mlk_gemm_panel_workspace_bytes(m, n, k, p1, p2, p3) > 0) == (p3 > 1)
+    assert lib.mlk_gemm_panel_plan(100, 128, 96, 0, out) != 0          # K % 128
+    assert lib.mlk_gemm_panel_plan(1 << 24, 128, 128, 0, out) != 0     # activations beyond 32-bit offsets
+    assert ops._gemm_args("layoutA_gemm", 4224, 300, 1024, 1)[0] == 8
+    assert ops._gemm_args("layout_gemm", 4224, 304, 1024, 1)[0] == 8
+    assert ops._gemm_args("layoutA_gemm", 4224, 300, 1088, 1)[0] == 2  # K % 128
+    assert ops._gemm_args("layoutA_gemm", 4224, 64, 1024, 1)[0] != 8
+    table = arg_selector.selector("layoutA_gemm").table()
+    table[(4224, 300, 1024)] = (3, 4, 1, 1)
+    try:
+        assert ops._gemm_args("layoutA_gemm", 4224, 300, 1024, 1) == (3, 4, 1, 1)
+    finally:
+        del table[(4224, 300, 1024)]
