@@ -126,6 +126,12 @@ class _Selector:
             return above[0]
         return same[-1] if same else None
 
+    def near(self, key):
+        """Whether a row of the same weight shape can be borrowed for this key."""
+        self.table()                            # read before the lock is taken, which reading takes too
+        with self._lock:
+            return self.neighbours and self._neighbour(tuple(int(v) for v in key)) is not None
+
     def get_args(self, key):
         key = tuple(int(v) for v in key)
         hit = self.table().get(key)
