@@ -1376,6 +1376,11 @@ struct MoePlan {
     int down_wk;      // decode down kernel: waves per workgroup; panel down kernel: workgroups per CU
     size_t down_lds;  // decode down kernel: dynamic LDS bytes
 };
+static void moe_plan_tile(MoePlan *pl, int hidden, int inter) {
+    pl->path = kMoePathTile;
+    pl->down_r = moe_tile_down_rows(pl->cb, hidden);
+    pl->down_slices = moe_tile_down_slices(pl->cb, hidden, inter, pl->max_tasks);
+}
 static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, bool fp8) {
     MoePlan pl = {};
     const int n_pairs = tc * topk;
@@ -1398,9 +1403,7 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
         return pl;
     }
     if (!inline_align && pl.cb >= 2 && (moe_tile_path() || pl.cb > 4)) {
-        pl.path = kMoePathTile;
-        pl.down_r = moe_tile_down_rows(pl.cb, hidden);
-        pl.down_slices = moe_tile_down_slices(pl.cb, hidden, inter, pl.max_tasks);
+        moe_plan_tile(&pl, hidden, inter);
         return pl;
     }
     pl.path = inline_align ? kMoePathDecodeInline : kMoePathDecode;
@@ -1502,8 +1505,38 @@ static bool moe_two_passes_pay(int rest, int n_experts, int topk, int hidden, in
     return weights * (1 - pow(miss, rest)) / (fp8 ? 5.5 : 6) + (fp8 ? 25 : 5) < gain;
 }
 
-// wide_ok: the operands and the workspace of the call are fit for the wide kernels
-static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8, bool wide_ok) {
+// The decode kernels take tasks of one token block; their down kernel deals its 16 waves to the tasks in turn, every workgroup
+// walking all of them, so that many experts are a long serial chain per workgroup.  The row-shared kernels give every task
+// workgroups of its own.  Above 48 experts in reach they are the faster ones even where a task of theirs (two blocks, so that
+// a hot expert is one pass) is half empty.  Decode -> row-shared kernels, us:
+//                                                tokens     8           12          24          64         200
+//   256 experts, top-8, H 7168, I 256, bf16            143 -> 108  165 -> 132  231 -> 193  335 -> 268  507 -> 346
+//   the same, soft-FP8                                 104 -> 109  119 -> 116  173 -> 147  242 -> 198  439 -> 234
+//   128 experts, top-8, H 2048, I 768, bf16            124 -> 101  149 -> 122  216 -> 171  260 -> 203
+//   the same, soft-FP8                                 104 ->  76  119 ->  87  168 -> 113  201 -> 129
+//   64 experts, top-6, H 2048, I 1024, soft-FP8         80 ->  69 (48 pairs)  117 -> 94  128 -> 96
+//   256 experts, top-1, H 4096, I 512, soft-FP8                    39 ->  39   60 ->  67  106 ->  92
+//   48 experts, top-8, H 4096, I 1024, bf16            158 -> 173  190 -> 198  209 -> 214  219 -> 219
+//   32 experts, top-4, H 4096, I 1024, bf16             98 -> 114  122 -> 126  137 -> 142  152 -> 152
+//   20 experts, top-2, H 4096, I 2048, soft-FP8         65 ->  65   71 ->  88   99 -> 117  110 -> 121
+// Soft-FP8 weights ask for three workgroups on two CUs as well: with one per CU (256 experts, 8 tokens: 64 tasks of 4) the
+// walk over H sets the pace, which the decode kernels split over waves.
+constexpr int kMoeWalkExperts = 48;
+static void moe_share_rows(MoePass *ps, int n_experts, int topk, int hidden, int inter, bool fp8) {
+    const int n_pairs = ps->tokens * topk, active = n_experts < n_pairs ? n_experts : n_pairs;
+    if ((ps->plan.path != kMoePathDecode && ps->plan.path != kMoePathDecodeInline) || ps->cb != 1 || active <= kMoeWalkExperts) return;
+    if (!moe_tile_path() || g_tunable[8] == 1) return;
+    if (fp8 && active * (inter / 64) * 2 < 3 * device_cus()) return;
+    MoePlan pl = {};
+    ps->cb = pl.cb = 2;
+    pl.max_tasks = active + n_pairs / (16 * pl.cb);
+    moe_plan_tile(&pl, hidden, inter);
+    ps->plan = pl;
+}
+
+// wide_ok: the operands and the workspace of the call are fit for the wide kernels; share_ok: the workspace holds what
+// moe_share_rows() needs (fp32 products per routed pair, where the decode kernels hold them per token)
+static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, int inter, bool fp8, bool wide_ok, bool share_ok) {
     MoePass ps = {};
     ps.wide = wide_ok && tokens_left > kMoeChunk &&
               (tokens_left > 2 * kMoeChunk || !moe_two_passes_pay(tokens_left - kMoeChunk, n_experts, topk, hidden, inter, fp8));
@@ -1511,6 +1544,7 @@ static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, in
         ps.tokens = tokens_left < kMoeChunk ? tokens_left : kMoeChunk;
         ps.plan = moe_plan(ps.tokens, n_experts, topk, hidden, inter, fp8);
         ps.cb = moe_blocks_per_task(ps.tokens, topk, n_experts);
+        if (share_ok) moe_share_rows(&ps, n_experts, topk, hidden, inter, fp8);
         ps.cb_unit = 0;
         ps.max_tasks = ps.plan.max_tasks;
         ps.down_slices = ps.plan.down_slices;
@@ -1613,12 +1647,12 @@ extern "C" int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_
 
 // The passes of a call share the workspace; the larger of the two weight kinds, since the query does not know which one
 // the call will bring.
-static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden, int inter, bool wide_ok) {
+static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden, int inter, bool wide_ok, bool share_ok) {
     if (n_tokens < 1 || n_experts < 1 || topk < 1) return 0;       // nothing to run
     size_t bytes = 0;
     for (int fp8 = 0; fp8 < 2; ++fp8) {
         auto cover = [&](int tokens) {
-            const MoePass ps = moe_pass(tokens, n_experts, topk, hidden, inter, fp8 != 0, wide_ok);
+            const MoePass ps = moe_pass(tokens, n_experts, topk, hidden, inter, fp8 != 0, wide_ok, share_ok);
             const size_t b = carve(nullptr, ps.tokens, n_experts, topk, hidden, inter, ps.obuf_bytes + 256, nullptr);
             if (b > bytes) bytes = b;
             return ps.tokens;
@@ -1630,14 +1664,16 @@ static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden
 }
 
 extern "C" size_t mlk_moe_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
-    return moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
+    const size_t least = moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false, false);
+    const size_t shared = moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false, true);
+    return shared > least ? shared : least;
 }
 
 static bool moe_wide_fits(int n_tokens, int n_experts, int topk, int hidden, int inter, size_t workspace_bytes) {
-    return n_tokens > kMoeChunk && workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true);
+    return n_tokens > kMoeChunk && workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, true, false);
 }
 
-// The most that a call of any 1 .. kMoeChunk tokens needs.  512 plans, about 25 us: kept per thread for the layer (and the
+// The most that a call of any 1 .. kMoeChunk tokens needs.  1024 plans, about 50 us: kept per thread for the layer (and the
 // experiment switches) it was last asked for.
 static size_t moe_narrow_most(int n_experts, int topk, int hidden, int inter) {
     const int key[11] = {n_experts, topk, hidden, inter, device_cus(), g_moe_tile, g_moe_gemv1,
@@ -1647,7 +1683,7 @@ static size_t moe_narrow_most(int n_experts, int topk, int hidden, int inter) {
     if (memcmp(key, last, sizeof key) != 0) {
         bytes = 0;
         for (int t = 1; t <= kMoeChunk; ++t) {
-            const size_t b = moe_workspace_of(t, n_experts, topk, hidden, inter, false);
+            const size_t b = mlk_moe_workspace_bytes(t, n_experts, topk, hidden, inter);
             if (b > bytes) bytes = b;
         }
         memcpy(last, key, sizeof key);
@@ -1658,7 +1694,7 @@ static size_t moe_narrow_most(int n_experts, int topk, int hidden, int inter) {
 // Above kMoeChunk tokens: enough for every shorter call too, so that scratch sized once for the longest prompt serves the rest
 // on the same kernels.
 extern "C" size_t mlk_moe_wide_workspace_bytes(int n_tokens, int n_experts, int topk, int hidden, int inter) {
-    if (n_tokens <= kMoeChunk || n_experts < 1 || topk < 1) return moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false);
+    if (n_tokens <= kMoeChunk || n_experts < 1 || topk < 1) return mlk_moe_workspace_bytes(n_tokens, n_experts, topk, hidden, inter);
     const int most = moe_wide_most_tokens(topk), tokens = n_tokens < most ? n_tokens : most;
     const size_t obuf = moe_wide_most_pair_slices(tokens, n_experts, topk, hidden, inter) * hidden * sizeof(float);
     const size_t wide = carve(nullptr, tokens, n_experts, topk, hidden, inter, obuf + 256, nullptr);
@@ -1674,7 +1710,7 @@ extern "C" int mlk_moe_first_pass(int n_tokens, int n_experts, int topk, int hid
     MLK_REQUIRE(hidden > 0 && inter > 0 && hidden % 128 == 0 && inter % 128 == 0,
                 "moe: hidden and intermediate sizes must be multiples of 128");
     const bool wide_ok = moe_wide_fits(n_tokens, n_experts, topk, hidden, inter, workspace_bytes);
-    const MoePass ps = moe_pass(n_tokens, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3, wide_ok);
+    const MoePass ps = moe_pass(n_tokens, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3, wide_ok, false);
     out[0] = ps.tokens;
     out[1] = ps.wide;
     return MLK_OK;
@@ -1697,15 +1733,16 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
     else MLK_REQUIRE(w_kind == x_kind, "moe: weights and activations must have the same 16-bit type");
     if (n_tokens == 0) return MLK_OK;
     MLK_REQUIRE(w1 && w2 && x && y && topk_ids && topk_weights && workspace, "moe: null pointer");
-    MLK_REQUIRE(workspace_bytes >= mlk_moe_workspace_bytes(n_tokens, n_experts, topk, hidden, inter),
+    MLK_REQUIRE(workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, false, false),
                 "moe: workspace too small");
     // the wide kernels load tokens, weights and intermediate straight into LDS
     const bool wide_ok = aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(workspace) &&
                          moe_wide_fits(n_tokens, n_experts, topk, hidden, inter, workspace_bytes);
+    const bool share_ok = workspace_bytes >= moe_workspace_of(n_tokens, n_experts, topk, hidden, inter, wide_ok, true);
     hipStream_t s = (hipStream_t)stream;
 
     for (int t0 = 0, tc = 0; t0 < n_tokens; t0 += tc) {
-        const MoePass ps = moe_pass(n_tokens - t0, n_experts, topk, hidden, inter, fp8, wide_ok);
+        const MoePass ps = moe_pass(n_tokens - t0, n_experts, topk, hidden, inter, fp8, wide_ok, share_ok);
         const MoePlan &pl = ps.plan;
         tc = ps.tokens;
         const int n_pairs = tc * topk;

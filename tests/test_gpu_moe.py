@@ -763,3 +763,67 @@ def test_workspace_of_256_token_passes_still_takes_longer_calls(mlk, T, kind):
         want += h * (wts.float() * (ids == e)).sum(1, keepdim=True)
     for y in out:
         assert_close(y, want.cpu().numpy(), RTOL, ATOL, "T=%d" % T)
+
+
+@pytest.mark.parametrize("T,E,K,H,I,kind,shared", [
+    (7, 64, 7, 256, 384, "bf16", True),       # 49 pairs: one more than the decode kernels keep, without the alignment kernel there
+    (8, 64, 6, 256, 384, "bf16", False),      # 48 pairs
+    (17, 48, 4, 256, 384, "fp16", False),     # 48 experts
+    (17, 49, 4, 1152, 256, "fp16", True),     # output rows of one tile and an eighth
+    (200, 64, 1, 512, 128, "bf16", True),     # the routing below gives 100 tokens to one expert: seven blocks, four tasks
+    (33, 256, 8, 128, 128, "bf16", True),
+    (48, 256, 1, 256, 384, "bf16", False),
+    (12, 64, 8, 256, 384, "fp8", True),       # 64 tasks of 6 workgroups: three on two CUs of 256
+    (12, 63, 8, 256, 384, "fp8", False),      # just fewer
+    (16, 64, 4, 256, 1024, "fp8", True),      # K slices of the down projection
+])
+def test_many_experts_of_one_block_share_rows(mlk, T, E, K, H, I, kind, shared):
+    """More than 48 experts in reach with one token block per task: the row-shared kernels, which need scratch per routed pair.
+    A workspace that only holds the decode kernels' sums keeps the call on those; nothing behind it is written."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    dtype = torch.float16 if kind == "fp16" else torch.bfloat16
+    wk, xk = {"fp16": (0, 0), "bf16": (1, 1), "fp8": (2, 1)}[kind]
+    g = torch.Generator(device="cuda").manual_seed(5 + T)
+
+    def weights(rows, k):
+        w = torch.randn((E, rows, k), generator=g, device="cuda")
+        if kind != "fp8":
+            w = (w * k ** -0.5).to(dtype)
+            return mlk.pack_layout_a(w), None, w.float()
+        codes = (w * 16).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        scale = torch.exp2(torch.randint(-10, -8, (E, rows // 128, k // 128), generator=g, device="cuda").float())
+        return (mlk.pack_layout_a(codes.view(torch.uint8)), scale,
+                codes.float() * scale.repeat_interleave(128, 1).repeat_interleave(128, 2))
+    (w1p, s1, w1), (w2p, s2, w2) = weights(2 * I, H), weights(H, I)
+    x = torch.randn((T, H), generator=g, device="cuda").to(dtype)
+    ids = torch.rand((T, E), generator=g, device="cuda").topk(K, dim=1).indices.to(torch.int32)
+    if K == 1:
+        ids[: T // 2] = 3
+    emap = torch.arange(E, device="cuda", dtype=torch.int32)
+    emap[1] = -1                                               # on another rank
+    wts = (0.5 + torch.rand((T, K), generator=g, device="cuda")).to(dtype)
+    want = torch.zeros((T, H), dtype=torch.float32, device="cuda")
+    for e in range(E):
+        if e != 1:
+            gate, up = (x.float() @ w1[e].T).split(I, dim=1)
+            h = (torch.nn.functional.silu(gate) * up).to(dtype).float() @ w2[e].T
+            want += h * (wts.float() * (ids == e)).sum(1, keepdim=True)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    lib = _lib.load()
+    full = lib.mlk_moe_workspace_bytes(T, E, K, H, I)
+    lib.mlk_moe_set_tile_path(0)
+    try:
+        least = lib.mlk_moe_workspace_bytes(T, E, K, H, I)     # of the decode kernels
+    finally:
+        lib.mlk_moe_set_tile_path(1)
+    assert full >= least and (full > least or not shared or K == 1)      # one pick: the decode kernels' K slices need as much
+    for size in (full, least):
+        ws = torch.full((full + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
+        y = torch.empty_like(x)
+        _lib.check(lib.mlk_fused_experts_compute(ptr(w1p), ptr(w2p), ptr(x), T, E, K, H, I, wk, xk, ptr(ids), ptr(wts), ptr(emap),
+                                                 ptr(s1), ptr(s2), ptr(y), ptr(ws), size, _stream()), "moe")
+        assert (ws[size:] == 0xAB).all()
+        if size > least:
+            assert bool((ws[least:size] != 0xAB).any()) == shared
+        assert_close(y, want.cpu().numpy(), RTOL, ATOL, "T=%d" % T)
