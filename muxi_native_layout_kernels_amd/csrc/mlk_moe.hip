@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
                                                          int32_t *__restrict__ padded_blocks,
                                                          int32_t *__restrict__ experts_ids, int max_blocks,
                                                          MoeTask *__restrict__ tasks, int32_t *__restrict__ n_tasks,
-                                                         int cb_max, int cb_unit) {
+                                                         int cb_max, int cb_unit, int32_t *__restrict__ queues) {
     constexpr int NW = 16;
     __shared__ int cnt[NW][kMaxExperts];   // per-wave counts, then per-wave write cursors
     __shared__ int start[kMaxExperts + 1]; // padded exclusive prefix
@@ -298,6 +298,7 @@ __global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t *__restri
 
     for (int i = tid; i < NW * kMaxExperts; i += 1024) (&cnt[0][0])[i] = 0;
     for (int i = tid; i < max_padded; i += 1024) sorted_ids[i] = n_pairs;   // sentinel everywhere
+    if (queues && tid < kWideQueues) queues[tid * kWideQueueStep] = 0;
     for (int i = tid; i < max_blocks; i += 1024) experts_ids[i] = 0;
     __syncthreads();
 
@@ -1168,6 +1169,7 @@ struct MoeWorkspace {
     int32_t *n_tasks;
     int32_t *sorted, *cumsum, *padded, *experts_ids;
     uint16_t *hbuf;
+    int32_t *queues;
     float *obuf;
     int32_t *counters;
     int sb;          // token blocks the intermediate is dimensioned for
@@ -1197,6 +1199,8 @@ static size_t carve(uint8_t *base, int tc, int E, int K, int hidden, int inter, 
     // seven spare blocks: the row-shared down kernel always fetches CB <= 8 consecutive blocks
     w.sb = max_blocks + 7;
     w.hbuf = (uint16_t *)take((size_t)inter * w.sb * 16 * 2);
+    w.queues = (int32_t *)(w.hbuf + (size_t)inter * max_blocks * 16);      // of the wide kernels, which leave the spare blocks alone
+    static_assert(kWideQueues * kWideQueueStep * 4 <= 7 * 128 * 32, "seven blocks of the smallest intermediate");
     // fp32 buffer of the K-sliced down projections
     w.obuf = (float *)take(obuf_bytes);
     w.counters = (int32_t *)take(sizeof(int32_t) * (size_t)(hidden / 16));
@@ -1640,7 +1644,7 @@ extern "C" int mlk_moe_align_tokens(const int32_t *topk_ids, int n_pairs, int n_
     const int max_blocks = (n_pairs + n_experts * 15 + 15) / 16;
     moe_align_kernel<<<1, 1024, 0, (hipStream_t)stream>>>(topk_ids, n_pairs, n_experts, experts_map, sorted_token_ids,
                                                           cumsum_buffer, padded_num_blocks, experts_ids, max_blocks,
-                                                          nullptr, nullptr, 1, 0);
+                                                          nullptr, nullptr, 1, 0, nullptr);
     MLK_LAUNCH_CHECK();
     return MLK_OK;
 }
@@ -1808,7 +1812,7 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
         if (!inline_align) {
             moe_align_kernel<<<1, 1024, 0, s>>>(topk_ids + (size_t)t0 * topk, n_pairs, n_experts, experts_map,
                                                 ws.sorted, ws.cumsum, ws.padded, ws.experts_ids, max_blocks, ws.tasks,
-                                                ws.n_tasks, cb, ps.cb_unit);
+                                                ws.n_tasks, cb, ps.cb_unit, ps.wide ? ws.queues : nullptr);
             MLK_LAUNCH_CHECK();
         }
         MoeArgs a;
@@ -1823,6 +1827,7 @@ static int experts_compute_impl(const void *w1, const void *w2, const void *x, i
         a.sorted = ws.sorted;
         a.tasks = ws.tasks;
         a.n_tasks = ws.n_tasks;
+        a.queues = ws.queues;
         a.T = tc;
         a.K = topk;
         a.H = hidden;

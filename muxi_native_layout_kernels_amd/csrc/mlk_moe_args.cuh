@@ -12,6 +12,9 @@ struct MoeTask {
     unsigned short first, count;      // the expert's tasks: index of the first one in the list and how many there are
 };
 
+// The queues of the wide kernels: each in a cache line of its own, all in the spare blocks of the intermediate.
+constexpr int kWideQueues = 16, kWideQueueStep = 32;
+
 struct MoeArgs {
     const uint8_t *W1;        // [E][2I][H] layout-A slabs
     const uint8_t *W2;        // [E][H][I]
@@ -30,6 +33,7 @@ struct MoeArgs {
     float *part;              // down projection with K slices: fp32 partial output tiles [slice][workgroup][T][16R]
     int32_t *counters;        // arrival counters, one per down workgroup column (zeroed by the gate/up kernel)
     int n_counters;
+    int32_t *queues;          // wide kernels: items taken of the eight runs of gate/up, then of down (zeroed by moe_align_kernel)
 };
 
 // Panel kernels for tasks of more than one token block (mlk_moe_panel.cuh): gate/up and down projection of every

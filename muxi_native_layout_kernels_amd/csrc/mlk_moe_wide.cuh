@@ -15,16 +15,22 @@
 //
 // Order of the work: the (expert, row tile, task of the expert) triples, tasks fastest, form one line that is cut into
 // eight equal runs, one per XCD (workgroup id modulo 8).  The tasks of an expert that share a row tile's weights then run
-// next to each other on one L2, and an XCD works on few experts at a time, so its token rows stay there too.
+// next to each other on one L2, and an XCD works on few experts at a time, so its token rows stay there too.  Equal runs are unequal
+// work where tasks differ in width; there one workgroup per CU fetches its items from queues (wide_queue_pays).  One workgroup per
+// item -> queues, 8 experts, top-2, H 4096, I 14336, whole layer: bf16 658 -> 606 us at 420 tokens, 1079 -> 963 at 1100,
+// 1587 -> 1529 at 2048; soft-FP8 556 -> 474, 1039 -> 965, 1621 -> 1540; 256 experts, top-8, H 7168, I 256 at 2048 tokens bf16
+// 836 -> 798, soft-FP8 770 -> 710.
 //
 // What bounds it: neither the matrix cores' peak nor memory.  8 experts, top-2, H 4096, I 14336, bf16, 2048 tokens: gate/up 962
-// GFLOP in 1066 us (0.90 PFLOP/s), down 481 GFLOP in 599 us (0.80), where the same loop reaches 1.36 PFLOP/s on a dense 8192 x
+// GFLOP in 1066 us (0.90 PFLOP/s), down 481 GFLOP in 599 us (0.80) with a workgroup per item, where the same loop reaches 1.36 PFLOP/s on a dense 8192 x
 // 8192 product of 4096 tokens.  Counted: 7.8 % of the products are columns that pad a task; the matrix cores are busy 51 % (down:
 // 42 %) of the cycles, at a clock that power holds at 1.8 to 1.95 GHz; a shader engine holds waves 85 % of the time and a CU 79 %
-// (73 %), since the XCDs get equal numbers of items of unequal widths and a workgroup's first slabs and its epilogue have nothing
+// (73 %), since the XCDs got equal numbers of items of unequal widths and a workgroup's first slabs and its epilogue have nothing
 // beside them on the CU; the L2s serve 78 % of the requests.  fp32 partial products of the down projection are 4 H bytes per
 // routed pair and slice, written and read once (the sum over them: 26 us).
 #pragma once
+
+#include <math.h>
 
 #include "mlk_moe_args.cuh"
 #include "mlk_panel8_small.cuh"
@@ -35,15 +41,57 @@ constexpr int kWideOutPitch = 272;                             // gate/up turn-a
 constexpr int kWideDownPitch = 144;                            // down: bytes per token (32 fp32 rows of one wave)
 constexpr size_t kWideDownOut = (size_t)8 * 128 * kWideDownPitch;
 
-// The workgroup's place on the line of n items: XCD id % 8 takes the id % 8-th run.  Returns n or more when there is none.
+// The line of n items is cut into eight equal runs, one per XCD (workgroup id modulo 8).  Without queues every item has a workgroup of
+// its own.  With them (wide_queue_pays) a workgroup per CU starts with item id / 8 of its run and goes on: queue[x] counts the items
+// that have been taken from run x since, and where a run has ended its CUs help the run that has most left.
 __device__ __forceinline__ int wide_item(int id, int n) {
     const int per = (n + 7) >> 3;
     const int j = id >> 3;
     return j < per ? (id & 7) * per + j : n;
 }
+__device__ __forceinline__ int wide_run(int n, int x) {
+    const int per = (n + 7) >> 3;
+    return max(0, min(per, n - x * per));
+}
+__device__ __forceinline__ int wide_ticket(int32_t *queue, int x, int lane) {
+    int got = 0;
+    if (lane == 0) got = __hip_atomic_fetch_add(queue + x * kWideQueueStep, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return got + ((int)(gridDim.x + 7 - x) >> 3);
+}
+// One wave: the item of a ticket of run x (valid in lane 0), or, when that run has ended, the next one of the run that has most
+// left; -1 when all have ended.  A ticket that comes too late leaves its run ended for good, so there are eight attempts at most.
+__device__ __forceinline__ int wide_next(int32_t *queue, int n, int x, int ticket, int lane) {
+    for (;;) {
+        ticket = __builtin_amdgcn_readfirstlane(ticket);
+        if (ticket < wide_run(n, x)) return x * ((n + 7) >> 3) + ticket;
+        int best = 0;
+        if (lane < 8) {
+            const int taken = __hip_atomic_load(queue + lane * kWideQueueStep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) +
+                              ((int)(gridDim.x + 7 - lane) >> 3);
+            const int left = wide_run(n, lane) - taken;
+            if (left > 0) best = left * 8 + lane;
+        }
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) best = max(best, __shfl_xor(best, off));
+        best = __builtin_amdgcn_readfirstlane(best);
+        if (best == 0) return -1;
+        x = best & 7;
+        ticket = wide_ticket(queue, x, lane);
+    }
+}
+// The kernel's arguments (MoeArgs come first) and the place in the workgroup, taken afresh for every item: what the compiler works out
+// from them in front of the loop over items is spilled there (soft-FP8 gate/up: 17 vector registers).
+__device__ __forceinline__ const MoeArgs &wide_args(int &lane, int &wave) {
+    auto at = __builtin_amdgcn_kernarg_segment_ptr();
+    int tid = threadIdx.x;
+    asm volatile("" : "+s"(at), "+v"(tid));
+    lane = tid & 63;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    return *(const MoeArgs *)at;
+}
 
-template <class T, bool FP8, int TB>
-__device__ __forceinline__ void moe_gate_up_wide(const MoeArgs &p, const MoeTask &tk, int rt, int wave, int lane) {
+template <class T, bool FP8, bool QUEUE, int TB>
+__device__ __forceinline__ int moe_gate_up_wide(const MoeArgs &p, const MoeTask &tk, int rt, int wave, int lane) {
     extern __shared__ u32x4 win[];
     constexpr int WB = FP8 ? 1 : 2;
     using Loop = typename Panel8<T, FP8, TB, 2>::Loop;
@@ -76,6 +124,7 @@ __device__ __forceinline__ void moe_gate_up_wide(const MoeArgs &p, const MoeTask
     f32x16 acc[2][TB];
     Loop::run(acc, src, srow, 0, p.H >> 5, wave, lane);
     __syncthreads();
+    const int ticket = QUEUE && wave == 0 ? wide_ticket(p.queues, blockIdx.x & 7, lane) : 0;      // of the next item
 
     // accumulator element 4 g + e of lane 32 h + c: column 8 g + 4 h + e of the wave's 32, token c of the block's 32
     uint8_t *out = reinterpret_cast<uint8_t *>(win);
@@ -94,39 +143,58 @@ __device__ __forceinline__ void moe_gate_up_wide(const MoeArgs &p, const MoeTask
         }
     __syncthreads();
     // sixteen lanes store the 256 bytes of a slot; slots without a routed pair are stored too (nobody reads them)
-    const int q = threadIdx.x & 15;
+    const int tid = wave * 64 + lane, q = tid & 15;
     uint16_t *dst = p.Hbuf + (size_t)tk.block0 * 16 * p.I + rt * 128 + q * 8;
 #pragma unroll
     for (int it = 0; it < 2 * TB; ++it) {
-        const int slot = it * 32 + (threadIdx.x >> 4);
+        const int slot = it * 32 + (tid >> 4);
         if (slot < slots)
             *reinterpret_cast<u32x4 *>(dst + (size_t)slot * p.I) = *reinterpret_cast<const u32x4 *>(out + slot * kWideOutPitch + q * 16);
+    }
+    return ticket;
+}
+
+template <class T, bool FP8, bool QUEUE>
+__device__ __forceinline__ int moe_gate_up_wide_item(const MoeArgs &p, int row_tiles, int item, int wave, int lane) {
+    const MoeTask t0 = p.tasks[item / row_tiles];                // some task of the item's expert
+    const int local = item - (int)t0.first * row_tiles;
+    const int rt = local / t0.count;
+    const MoeTask tk = p.tasks[t0.first + local % t0.count];
+    switch ((tk.nblocks + 3) >> 2) {
+        case 1: return moe_gate_up_wide<T, FP8, QUEUE, 1>(p, tk, rt, wave, lane);
+        case 2: return moe_gate_up_wide<T, FP8, QUEUE, 2>(p, tk, rt, wave, lane);
+        case 3: return moe_gate_up_wide<T, FP8, QUEUE, 3>(p, tk, rt, wave, lane);
+        default: return moe_gate_up_wide<T, FP8, QUEUE, 4>(p, tk, rt, wave, lane);
     }
 }
 
 template <class T, bool FP8>
 __global__ void __launch_bounds__(512) moe_gate_up_wide_kernel(MoeArgs p) {
-    const int row_tiles = p.I >> 7;
-    const int n_items = row_tiles * p.n_tasks[0];
+    const int row_tiles = p.I >> 7, n_items = row_tiles * p.n_tasks[0];
     const int item = wide_item(blockIdx.x, n_items);
     if (item >= n_items) return;
-    const MoeTask t0 = p.tasks[item / row_tiles];                // some task of the item's expert
-    const int local = item - (int)t0.first * row_tiles;
-    const int rt = local / t0.count;
-    const MoeTask tk = p.tasks[t0.first + local % t0.count];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    switch ((tk.nblocks + 3) >> 2) {
-        case 1: moe_gate_up_wide<T, FP8, 1>(p, tk, rt, wave, lane); break;
-        case 2: moe_gate_up_wide<T, FP8, 2>(p, tk, rt, wave, lane); break;
-        case 3: moe_gate_up_wide<T, FP8, 3>(p, tk, rt, wave, lane); break;
-        default: moe_gate_up_wide<T, FP8, 4>(p, tk, rt, wave, lane); break;
+    moe_gate_up_wide_item<T, FP8, false>(p, row_tiles, item, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+}
+
+template <class T, bool FP8>
+__global__ void __launch_bounds__(512) moe_gate_up_queue_kernel(MoeArgs) {
+    __shared__ int s_item;
+    int ticket = blockIdx.x >> 3;
+    for (;;) {
+        int lane, wave;
+        const MoeArgs &p = wide_args(lane, wave);
+        const int row_tiles = p.I >> 7, n_items = row_tiles * p.n_tasks[0];
+        if (wave == 0) s_item = wide_next(p.queues, n_items, blockIdx.x & 7, ticket, lane);
+        __syncthreads();                                         // also: LDS is free again
+        const int item = __builtin_amdgcn_readfirstlane(s_item);
+        if (item < 0) return;
+        ticket = moe_gate_up_wide_item<T, FP8, true>(p, row_tiles, item, wave, lane);
     }
 }
 
-template <class T, bool FP8, int TB>
-__device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restrict__ O, int skd, const MoeTask &tk, int rt, int sk,
-                                              int wave, int lane) {
+template <class T, bool FP8, bool QUEUE, int TB>
+__device__ __forceinline__ int moe_down_wide(const MoeArgs &p, float *__restrict__ O, int skd, const MoeTask &tk, int rt, int sk,
+                                             int wave, int lane) {
     extern __shared__ u32x4 win[];
     constexpr int WB = FP8 ? 1 : 2;
     using Loop = typename Panel8<T, FP8, TB, 2>::Loop;
@@ -155,13 +223,14 @@ __device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restric
     f32x16 acc[2][TB];
     Loop::run(acc, src, srow, 4 * wbeg, 4 * (wend - wbeg), wave, lane);
     __syncthreads();
+    const int ticket = QUEUE && wave == 0 ? wide_ticket(p.queues + 8 * kWideQueueStep, blockIdx.x & 7, lane) : 0;  // of the next item
 
     // every wave turns its 32 rows x 32 TB tokens around in its own part of LDS, one row pair after the other, and stores
     // 128 bytes of a routed pair with eight lanes
     uint8_t *out = reinterpret_cast<uint8_t *>(win) + (size_t)wave * 128 * kWideDownPitch;
     const int h4 = lane >> 5, c32 = lane & 31, t8 = lane >> 3, q = lane & 7;
     const int n0 = (rgp + wr * 4) * 16;
-    if (n0 >= p.H) return;
+    if (n0 >= p.H) return ticket;
     const int32_t *sorted = p.sorted + tk.block0 * 16;
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
@@ -184,42 +253,77 @@ __device__ __forceinline__ void moe_down_wide(const MoeArgs &p, float *__restric
         }
         wave_lds_sync();
     }
+    return ticket;
 }
 
-template <class T, bool FP8>
-__global__ void __launch_bounds__(512) moe_down_wide_kernel(MoeArgs p, float *__restrict__ O, int skd) {
-    const int row_tiles = (p.H + 255) >> 8, per_task = row_tiles * skd;
-    const int n_items = per_task * p.n_tasks[0];
-    const int item = wide_item(blockIdx.x, n_items);
-    if (item >= n_items) return;
+template <class T, bool FP8, bool QUEUE>
+__device__ __forceinline__ int moe_down_wide_item(const MoeArgs &p, float *__restrict__ O, int skd, int row_tiles, int item, int wave,
+                                                  int lane) {
+    const int per_task = row_tiles * skd;
     const MoeTask t0 = p.tasks[item / per_task];
     const int local = item - (int)t0.first * per_task;
     const int rs = local / t0.count;                               // slice-major: co-running workgroups share a K window
     const int sk = rs / row_tiles, rt = rs - sk * row_tiles;
     const MoeTask tk = p.tasks[t0.first + local % t0.count];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     switch ((tk.nblocks + 3) >> 2) {
-        case 1: moe_down_wide<T, FP8, 1>(p, O, skd, tk, rt, sk, wave, lane); break;
-        case 2: moe_down_wide<T, FP8, 2>(p, O, skd, tk, rt, sk, wave, lane); break;
-        case 3: moe_down_wide<T, FP8, 3>(p, O, skd, tk, rt, sk, wave, lane); break;
-        default: moe_down_wide<T, FP8, 4>(p, O, skd, tk, rt, sk, wave, lane); break;
+        case 1: return moe_down_wide<T, FP8, QUEUE, 1>(p, O, skd, tk, rt, sk, wave, lane);
+        case 2: return moe_down_wide<T, FP8, QUEUE, 2>(p, O, skd, tk, rt, sk, wave, lane);
+        case 3: return moe_down_wide<T, FP8, QUEUE, 3>(p, O, skd, tk, rt, sk, wave, lane);
+        default: return moe_down_wide<T, FP8, QUEUE, 4>(p, O, skd, tk, rt, sk, wave, lane);
     }
+}
+
+template <class T, bool FP8>
+__global__ void __launch_bounds__(512) moe_down_wide_kernel(MoeArgs p, float *__restrict__ O, int skd) {
+    const int row_tiles = (p.H + 255) >> 8, n_items = row_tiles * skd * p.n_tasks[0];
+    const int item = wide_item(blockIdx.x, n_items);
+    if (item >= n_items) return;
+    moe_down_wide_item<T, FP8, false>(p, O, skd, row_tiles, item, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+}
+
+template <class T, bool FP8>
+__global__ void __launch_bounds__(512) moe_down_queue_kernel(MoeArgs, float *__restrict__ O, int skd) {
+    __shared__ int s_item;
+    int ticket = blockIdx.x >> 3;
+    for (;;) {
+        int lane, wave;
+        const MoeArgs &p = wide_args(lane, wave);
+        const int row_tiles = (p.H + 255) >> 8, n_items = row_tiles * skd * p.n_tasks[0];
+        if (wave == 0) s_item = wide_next(p.queues + 8 * kWideQueueStep, n_items, blockIdx.x & 7, ticket, lane);
+        __syncthreads();                                           // also: LDS is free again
+        const int item = __builtin_amdgcn_readfirstlane(s_item);
+        if (item < 0) return;
+        ticket = moe_down_wide_item<T, FP8, true>(p, O, skd, row_tiles, item, wave, lane);
+    }
+}
+
+// Do at most n items of `slabs` k32 slabs each go through the queues?  They cost about 2 us a kernel (a ticket behind every item, a
+// look at all runs at the end: with queues everywhere layers of 64 and 128 experts of H 2048 lost 1 to 3 %, at 120 to 300 us) and win
+// where the XCDs' equal runs are unequal work, which takes panels of unequal widths: experts
+// whose loads, three standard deviations of an even routing either way, do not all need the same columns; and enough
+// rounds of long enough items to share out.
+static inline bool wide_queue_pays(const MoeArgs &a, int n, int slabs) {
+    const double mean = (double)a.n_pairs / a.E, spread = 3 * sqrt(mean);
+    if (ceil(fmax(mean - spread, 1) / 64) == ceil((mean + spread) / 64)) return false;
+    return n > device_cus() && (double)n / device_cus() * (slabs + 8) >= 350;
 }
 
 template <class T, bool FP8>
 int launch_moe_wide(const MoeArgs &a, int max_tasks, float *obuf, int skd, hipStream_t s) {
     constexpr size_t ring = p8_ring_bytes<FP8, 2, 4>();
     constexpr size_t lds_up = ring, lds_down = ring > kWideDownOut ? ring : kWideDownOut;
-    static bool ready_up[64] = {}, ready_down[64] = {};
-    int rc = panel_lds_attribute(&moe_gate_up_wide_kernel<T, FP8>, lds_up, ready_up);
-    if (rc != MLK_OK) return rc;
-    rc = panel_lds_attribute(&moe_down_wide_kernel<T, FP8>, lds_down, ready_down);
-    if (rc != MLK_OK) return rc;
+    static bool ready_up[2][64] = {}, ready_down[2][64] = {};
     const int items_up = (a.I >> 7) * max_tasks, items_down = ((a.H + 255) >> 8) * skd * max_tasks;
-    moe_gate_up_wide_kernel<T, FP8><<<(items_up + 7) / 8 * 8, 512, lds_up, s>>>(a);
+    const bool queue_up = wide_queue_pays(a, items_up, a.H >> 5), queue_down = wide_queue_pays(a, items_down, (a.I >> 5) / skd);
+    const auto up = queue_up ? &moe_gate_up_queue_kernel<T, FP8> : &moe_gate_up_wide_kernel<T, FP8>;
+    const auto down = queue_down ? &moe_down_queue_kernel<T, FP8> : &moe_down_wide_kernel<T, FP8>;
+    int rc = panel_lds_attribute(up, lds_up, ready_up[queue_up]);
+    if (rc != MLK_OK) return rc;
+    rc = panel_lds_attribute(down, lds_down, ready_down[queue_down]);
+    if (rc != MLK_OK) return rc;
+    up<<<queue_up ? device_cus() : (items_up + 7) / 8 * 8, 512, lds_up, s>>>(a);
     MLK_LAUNCH_CHECK();
-    moe_down_wide_kernel<T, FP8><<<(items_down + 7) / 8 * 8, 512, lds_down, s>>>(a, obuf, skd);
+    down<<<queue_down ? device_cus() : (items_down + 7) / 8 * 8, 512, lds_down, s>>>(a, obuf, skd);
     MLK_LAUNCH_CHECK();
     return MLK_OK;
 }

@@ -827,3 +827,63 @@ def test_many_experts_of_one_block_share_rows(mlk, T, E, K, H, I, kind, shared):
         if size > least:
             assert bool((ws[least:size] != 0xAB).any()) == shared
         assert_close(y, want.cpu().numpy(), RTOL, ATOL, "T=%d" % T)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+@pytest.mark.parametrize("picks", ["even", "skewed", "four experts", "none here"])
+def test_wide_kernels_share_out_items_through_queues(mlk, picks, kind):
+    """Sizes at which both wide kernels fetch their items from the queues (44 tasks at most, several rounds of long items), loads that
+    leave some XCDs' runs short, long or empty, output rows of sixteen and a half tiles; the same bits in every run."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    T, E, K, H, I = 2048, 12, 4, 4224, 4096
+    g = torch.Generator(device="cuda").manual_seed(11)
+    x = torch.randn((T, H), generator=g, device="cuda").to(torch.bfloat16)
+    score = torch.rand((T, E), generator=g, device="cuda")
+    if picks == "skewed":
+        score[: T // 2, :4] += 1
+    elif picks == "four experts":
+        score[:, 4:8] += 1
+    ids = score.topk(K, dim=1).indices.to(torch.int32)
+    wts = (0.5 + torch.rand((T, K), generator=g, device="cuda")).to(torch.bfloat16)
+    emap = torch.arange(E, device="cuda", dtype=torch.int32)
+    emap[1] = -1                                               # on another rank
+    if picks == "none here":
+        emap[:] = -1
+    want = torch.zeros((T, H), dtype=torch.float32, device="cuda")
+
+    def weights(rows, k):
+        packed = torch.empty((E, rows, k), dtype=torch.uint8 if kind == "fp8" else torch.bfloat16, device="cuda")
+        scales = torch.empty((E, rows // 128, k // 128), device="cuda") if kind == "fp8" else None
+        return packed, scales
+
+    def fill(dst, scales, e):
+        w = torch.randn(dst.shape[1:], generator=g, device="cuda")
+        if kind == "bf16":
+            w = (w * w.shape[1] ** -0.5).to(torch.bfloat16)
+            dst[e] = mlk.pack_layout_a(w).view(w.shape)
+            return w.float()
+        codes = (w * 16).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        # the intermediate stays below 16: its bf16 may round the other way (2 ** -4) on sums in another order, which moves an output by
+        # up to 2 ** -4 times a weight (0.05) times a routing weight (1.5); at twice these scales it is beyond 50 and 0.04
+        scales[e] = torch.exp2(torch.randint(-11, -9, scales.shape[1:], generator=g, device="cuda").float())
+        dst[e] = mlk.pack_layout_a(codes.view(torch.uint8)).view(w.shape)
+        return codes.float() * scales[e].repeat_interleave(128, 0).repeat_interleave(128, 1)
+    (w1p, s1), (w2p, s2) = weights(2 * I, H), weights(H, I)
+    for e in range(E):
+        w1, w2 = fill(w1p, s1, e), fill(w2p, s2, e)
+        if emap[e] >= 0:
+            gate, up = (x.float() @ w1.T).split(I, dim=1)
+            want += (torch.nn.functional.silu(gate) * up).to(torch.bfloat16).float() @ w2.T * (wts.float() * (ids == e)).sum(1, keepdim=True)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    lib = _lib.load()
+    size = lib.mlk_moe_wide_workspace_bytes(T, E, K, H, I)
+    ws = torch.full((size,), 0xAB, dtype=torch.uint8, device="cuda")
+    out = []
+    for _ in range(2):
+        y = torch.empty_like(x)
+        _lib.check(lib.mlk_fused_experts_compute(ptr(w1p), ptr(w2p), ptr(x), T, E, K, H, I, 2 if kind == "fp8" else 1, 1, ptr(ids),
+                                                 ptr(wts), ptr(emap), ptr(s1), ptr(s2), ptr(y), ptr(ws), size, _stream()), "moe")
+        out.append(y)
+    assert torch.equal(out[0], out[1])
+    assert_close(out[0], want.cpu().numpy(), RTOL, ATOL, picks)
