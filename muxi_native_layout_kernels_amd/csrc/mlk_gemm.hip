@@ -53,10 +53,10 @@ extern template int launch_modes<BF16, true>(const GemmArgs &, int, int, int, in
 
 // kernel id 3 (mlk_panel.hip)
 size_t panel_partial_bytes(int m, int n, int sk);
-size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int sk);
+size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int p3);
 void gemm_plan(int m, int n, int k, bool fp8, int32_t *out);
 int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, bool b_native, bool c_native,
-                       float alpha, const void *bias, const float *scale, int pr, int tb, int sk, int whole_groups, void *partial,
+                       float alpha, const void *bias, const float *scale, int pr, int tb, int p3, int whole_groups, void *partial,
                        size_t partial_bytes, hipStream_t s);
 int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, float alpha, const void *bias,
                  const float *scale, int width, int rows, int sk, bool last_round_only, void *counters,

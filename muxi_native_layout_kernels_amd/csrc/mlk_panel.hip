@@ -156,11 +156,13 @@ extern template int launch_panel8<BF16, false>(const Panel8Args &, int, int, hip
 extern template int launch_panel8<F16, false>(const Panel8Args &, int, int, hipStream_t);
 extern template int launch_panel8<BF16, true>(const Panel8Args &, int, int, hipStream_t);
 
-// Lines, whole and dealt panels of m x n x k in panels of 128 pr rows x 64 tb tokens.  sk = 1: every panel whole; 2 .. 63: in that
+// Lines, whole and dealt panels of m x n x k in panels of 128 pr rows x 64 tb tokens.  sk = 1: every panel whole; from 2 on: in that
 // many slices of K; kP8Deal: dealt evenly to one workgroup per CU.  With more panels than CUs only those that are left over after
 // whole rounds of one panel per CU are sliced or dealt, unless the caller says how many groups of eight row tiles are not (kernel ids
 // 3 and 5 on panels of 256 x 256).
-constexpr int kP8Deal = 64;
+// kP8Deal is no count that a caller can ask for: kernel id 8 says it as p3 = 64, but ids 3 and 5 take p3 = 64 for as many slices, and
+// their workspace holds those.
+constexpr int kP8Deal = 1 << 20, kP8DealP3 = 64;
 static void panel8_shape(Panel8Args &p, int m, int n, int k, int pr, int tb, int sk, int whole_groups = -1) {
     const int cus = device_cus(), windows = k / 64;
     p.M = m;
@@ -181,7 +183,7 @@ static void panel8_shape(Panel8Args &p, int m, int n, int k, int pr, int tb, int
     const int whole = whole_groups >= 0 ? whole_groups * p.token_tiles : (bands ? p.panels / round * round : 0), rest = p.panels - whole;
     if (rest == 0) return;
     p.whole = whole;
-    if (sk < kP8Deal) {
+    if (sk != kP8Deal) {
         p.deal = rest * (sk < windows ? sk : windows);
     } else {
         p.deal = round < rest * windows ? round : rest * windows;
@@ -191,9 +193,11 @@ static void panel8_shape(Panel8Args &p, int m, int n, int k, int pr, int tb, int
 static size_t panel8_partial_bytes(const Panel8Args &p, int pr, int tb) {
     return (size_t)(p.band > 0 ? 8 : 1) * p.deal * p.slots * pr * tb * 32768;
 }
-size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int sk) {
+// p3: as kernel id 8 takes it
+static int panel8_slices(int p3) { return p3 == kP8DealP3 ? kP8Deal : p3; }
+size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int p3) {
     Panel8Args p = {};
-    panel8_shape(p, m, n, k, pr, tb, sk);
+    panel8_shape(p, m, n, k, pr, tb, panel8_slices(p3));
     return panel8_partial_bytes(p, pr, tb);
 }
 
@@ -293,7 +297,7 @@ void gemm_plan(int m, int n, int k, bool fp8, int32_t *out) {
             if (tb > 1 && m <= 64 * (tb - 1)) break;
             const long long panels = (long long)((n + 128 * pr - 1) / (128 * pr)) * ((m + 64 * tb - 1) / (64 * tb));
             offer(panel8_us(f, m, n, k, pr, tb, 1), 8, 2 * pr, tb, 1);
-            if (panels > device_cus()) offer(panel8_us(f, m, n, k, pr, tb, kP8Deal), 8, 2 * pr, tb, kP8Deal);
+            if (panels > device_cus()) offer(panel8_us(f, m, n, k, pr, tb, kP8Deal), 8, 2 * pr, tb, kP8DealP3);
             else
                 // slices of at least four slabs that one workgroup per CU takes
                 for (int sk = 2; sk <= 32 && panels * sk <= device_cus() && k / 64 / sk >= 2; ++sk)
@@ -314,8 +318,9 @@ void gemm_plan(int m, int n, int k, bool fp8, int32_t *out) {
                     offer(narrow_us(fp8, m, n, k, 1, p1, p2, p3), 1, p1, p2, p3);
 }
 
+// whole_groups < 0: kernel id 8, p3 as it takes it; else kernel ids 3 and 5, p3 = K slices of the row tiles behind those groups
 int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, bool b_native, bool c_native,
-                       float alpha, const void *bias, const float *scale, int pr, int tb, int sk, int whole_groups, void *partial,
+                       float alpha, const void *bias, const float *scale, int pr, int tb, int p3, int whole_groups, void *partial,
                        size_t partial_bytes, hipStream_t s) {
     MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
     MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
@@ -329,7 +334,7 @@ int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int 
     p.alpha = alpha;
     p.b_native = b_native;
     p.c_native = c_native;
-    panel8_shape(p, m, n, k, pr, tb, sk, whole_groups);
+    panel8_shape(p, m, n, k, pr, tb, whole_groups < 0 ? panel8_slices(p3) : p3, whole_groups);
     if (p.deal > 0) {
         MLK_REQUIRE(partial != nullptr, "gemm: a K split across workgroups needs a workspace");
         if (partial_bytes < panel8_partial_bytes(p, pr, tb)) return fail(MLK_ERR_WORKSPACE, "gemm: workspace too small");

@@ -616,6 +616,29 @@ def test_gemm_eight_wave_panels_several_rounds(mlk, n, m, k, p1, p2):
         assert_close(c, want, RTOL, ATOL, "several rounds, p3 = %d" % p3)
 
 
+@pytest.mark.parametrize("kid", [3, 5])
+@pytest.mark.parametrize("n,m,k,p3", [
+    (256, 256, 4096, 63), (256, 256, 4096, 64),     # one panel, as many k windows as slices
+    (512, 300, 8192, 64),                           # four panels, two windows a slice
+    (256, 256, 1024, 64),                           # fewer windows than slices
+])
+def test_gemm_panel_ids_3_and_5_take_64_slices(mlk, kid, n, m, k, p3):
+    """p3 = 64 is a slice count of kernel ids 3 and 5 like any other (kernel id 8 gives it a meaning of its own): panels of 256 x 256
+    run on the workspace that mlk_gemm_workspace_bytes() answers, and nothing behind it is written."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    lib = _lib.load()
+    w, x = randn((n, k), torch.bfloat16, k ** -0.5, 41), randn((m, k), torch.bfloat16, 1.0, 42)
+    a, b, c = pack_a(w).cuda(), x.cuda(), torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+    size = lib.mlk_gemm_workspace_bytes(m, n, 4, p3)
+    ws = torch.full((size + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
+    ws[:lib.mlk_gemm_counter_bytes()].zero_()
+    _lib.check(lib.mlk_gemm_layout_a(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, 1, 1, 0, 0, 1.0, None, None, kid, 4, 2, p3,
+                                     ws.data_ptr(), size, _stream()), "gemm")
+    assert_close(c, ogemm.linear_expected(w, x), RTOL, ATOL, "p3 = %d" % p3)
+    assert (ws[size:] == 0xAB).all()
+
+
 @pytest.mark.parametrize("native", [False, True])
 def test_gemm_eight_wave_panels_off_16_bytes(mlk, native):
     """Operands that do not lie on 16 bytes run the kernels that load through registers."""
