@@ -383,6 +383,10 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     p.alpha = alpha;
     if (width != 128 && width != 256) width = panel_tokens(m, n, a_kind == MLK_FP8_E4M3);
     if (width == 256) rows = 256;
+    // the loops that fetch straight into LDS take operands on 16 bytes, and panels of 256 tokens store 16 bytes at a time; others
+    // run panels of 128 tokens that fetch through registers
+    const bool loads_on16 = aligned16(a) && aligned16(b);
+    if (width == 256 && !(loads_on16 && aligned16(c) && aligned16(partial))) width = 128;
     p.token_tiles = (m + width - 1) / width;
     MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
     MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
@@ -428,8 +432,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     // 3 % on all but 11 of 1764 (rounds counted over the whole chip and a panel's time taken as rows times tokens: up to 53 %).
     // Operands off 16 bytes stay sliced where the whole panels run the loop that loads straight into LDS and the sliced ones do not.
     const bool whole_loads_lds = a_kind == MLK_FP8_E4M3 && width == 128 && rows == 256;
-    if (last_round_only && sk > 1 && p.whole_groups == 0 && groups * p.token_tiles > device_cus() / 8 &&
-        (!whole_loads_lds || (aligned16(a) && aligned16(b)))) {
+    if (last_round_only && sk > 1 && p.whole_groups == 0 && groups * p.token_tiles > device_cus() / 8 && (!whole_loads_lds || loads_on16)) {
         const int per_xcd = groups * p.token_tiles, round = device_cus() / 8;
         // us per k32 slab of a round of panels (whole soft-FP8 panels of 256 x 128 run two per CU: 0.65 us for a full round of
         // those, 0.5 us for half a one), and what a round takes to start and to store: 6 us whole, 2 us sliced and 5 us for the fold
@@ -464,7 +467,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         }                                                                                                          \
         gemm_panel_kernel<TT, F8, TBB, PRR><<<grid, 256, lds, s>>>(p);                                                  \
     } while (0)
-    if (rows == 256 && a_kind == MLK_FP8_E4M3 && (p.SK == 1 || p.whole_groups > 0)) {
+    if (rows == 256 && a_kind == MLK_FP8_E4M3 && (p.SK == 1 || p.whole_groups > 0) && loads_on16) {
         // soft-FP8, panels computed whole (or only the last round's sliced): the loop that prefetches through LDS, two
         // workgroups per CU (28672 x 8192 at 1024 tokens: 616 -> 474 us); fully sliced grids and 16-bit weights stay on
         // the register-ring loop, which was ahead there (compared while the fold of this kernel still spilled)

@@ -639,6 +639,36 @@ def test_gemm_panel_ids_3_and_5_take_64_slices(mlk, kid, n, m, k, p3):
     assert (ws[size:] == 0xAB).all()
 
 
+@pytest.mark.parametrize("kid,p3", [(3, 1), (3, 2), (5, 2)])
+@pytest.mark.parametrize("kind", ["fp16", "fp8"])
+@pytest.mark.parametrize("n,m,k", [(256, 300, 512), (2304, 520, 256)])
+def test_gemm_panel_ids_3_and_5_off_16_bytes(mlk, n, m, k, kind, kid, p3):
+    """Weights, activations or both off 16 bytes: panels of 128 tokens through registers, also where 256 were asked for."""
+    dtype = torch.float16 if kind == "fp16" else torch.bfloat16
+    x = randn((m, k), dtype, 1.0, 43)
+    if kind == "fp8":
+        w = fp8_codes((n, k), 44)
+        scale = (torch.rand((n // 128, k // 128), generator=torch.Generator().manual_seed(45)) * 0.02 + 0.001).float()
+        want = ogemm.softfp8_linear_expected(w.numpy(), scale.numpy(), x)
+    else:
+        w = randn((n, k), dtype, k ** -0.5, 44)
+        want = ogemm.linear_expected(w, x)
+
+    def shifted(t):
+        at = 1 if t.element_size() == 2 else 8
+        flat = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+        flat[at:at + t.numel()] = t.reshape(-1)
+        out = flat[at:at + t.numel()].view(t.shape)
+        assert out.data_ptr() % 16 and out.is_contiguous()
+        return out
+    a, b = pack_a(w).cuda(), x.cuda()
+    kw = dict(kernelParam1=4, kernelParam2=2, kernelParam3=p3, kernelId=kid)
+    for aa, bb in ((a, shifted(b)), (shifted(a), b), (shifted(a), shifted(b))):
+        c = mlk.gemm_layoutA_soft_fp8_wapper(aa, scale.cuda(), bb, n, m, k, **kw) if kind == "fp8" else \
+            mlk.gemm_layoutA_wapper(aa, bb, n, m, k, **kw)
+        assert_close(c, want, RTOL, ATOL, "off 16 bytes")
+
+
 @pytest.mark.parametrize("native", [False, True])
 def test_gemm_eight_wave_panels_off_16_bytes(mlk, native):
     """Operands that do not lie on 16 bytes run the kernels that load through registers."""
