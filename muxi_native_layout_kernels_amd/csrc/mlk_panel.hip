@@ -170,6 +170,7 @@ static void panel8_shape(Panel8Args &p, int m, int n, int k, int pr, int tb, int
     p.K = k;
     p.row_tiles = (n + 128 * pr - 1) / (128 * pr);
     p.token_tiles = (m + 64 * tb - 1) / (64 * tb);
+    p.cols = p.token_tiles == 1 ? (m + 15) / 16 * 16 : 64 * tb;
     const int panels = p.row_tiles * p.token_tiles;
     const bool bands = whole_groups > 0 || (whole_groups < 0 || sk <= 1 ? panels > cus : false);
     p.band = bands ? 8 : 0;
@@ -190,15 +191,15 @@ static void panel8_shape(Panel8Args &p, int m, int n, int k, int pr, int tb, int
         p.slots = 2;
     }
 }
-static size_t panel8_partial_bytes(const Panel8Args &p, int pr, int tb) {
-    return (size_t)(p.band > 0 ? 8 : 1) * p.deal * p.slots * pr * tb * 32768;
+static size_t panel8_partial_bytes(const Panel8Args &p, int pr) {
+    return (size_t)(p.band > 0 ? 8 : 1) * p.deal * p.slots * pr * p.cols * 512;
 }
 // p3: as kernel id 8 takes it
 static int panel8_slices(int p3) { return p3 == kP8DealP3 ? kP8Deal : p3; }
 size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int p3) {
     Panel8Args p = {};
     panel8_shape(p, m, n, k, pr, tb, panel8_slices(p3));
-    return panel8_partial_bytes(p, pr, tb);
+    return panel8_partial_bytes(p, pr);
 }
 
 // Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
@@ -337,7 +338,7 @@ int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int 
     panel8_shape(p, m, n, k, pr, tb, whole_groups < 0 ? panel8_slices(p3) : p3, whole_groups);
     if (p.deal > 0) {
         MLK_REQUIRE(partial != nullptr, "gemm: a K split across workgroups needs a workspace");
-        if (partial_bytes < panel8_partial_bytes(p, pr, tb)) return fail(MLK_ERR_WORKSPACE, "gemm: workspace too small");
+        if (partial_bytes < panel8_partial_bytes(p, pr)) return fail(MLK_ERR_WORKSPACE, "gemm: workspace too small");
     }
     if (a_kind == MLK_FP8_E4M3) return launch_panel8<BF16, true>(p, pr, tb, s);
     if (a_kind == MLK_F16) return launch_panel8<F16, false>(p, pr, tb, s);

@@ -33,9 +33,11 @@ struct Panel8Args {
     uint16_t *C;
     const uint16_t *bias;
     const float *scale;
-    f32x4 *partial;      // [line][deal][slots] of [8 waves][4 pr tb quads][64 lanes]
+    f32x4 *partial;      // [line][deal][slots] of slots of 128 pr rows x cols tokens (p8_slot_quad)
     int M, N, K;
     int row_tiles, token_tiles;
+    int cols;            // tokens of a slot: 64 tb, or the call's tokens in blocks of 16 where one token tile holds them all (32 to 48
+                         // tokens in slices are then no larger than the narrow kernels' partial sums)
     int band, chunk;     // groups of eight row tiles and token tiles that neighbouring workgroups of an XCD cover
     int panels;          // of the longest line
     int whole, deal;     // of one line
@@ -61,6 +63,12 @@ __device__ __forceinline__ bool p8_panel(const Panel8Args &p, int line, int u, i
     rt = u / p.token_tiles;
     tt = u - rt * p.token_tiles;
     return rt < p.row_tiles;
+}
+
+// Where accumulator quad g of a lane (rows 8 g + 4 (lane / 32) .. + 3 of row pair `pair` of the panel, token block + lane % 32) lies in
+// a panel's sums of `cols` tokens.  A block of 32 tokens is one run per row pair, 1 KiB per quad; the last block may have 16 tokens.
+__device__ __forceinline__ int p8_slot_quad(int cols, int pair, int block, int width, int g, int lane) {
+    return (pair * cols + block) * 8 + (2 * g + (lane >> 5)) * width + (lane & 31);
 }
 
 // Element offset of 8 rows n .. n + 7 (n % 8 == 0) of token tok in a layout-C output of m tokens.
@@ -278,15 +286,18 @@ __device__ __forceinline__ void gemm_panel8(const Panel8Args &p, int rt, int tt,
         p8_store_panel<T, PR, TB>(p, acc, rg0, tok0 + wt * 32 * TB, wave, lane, win);
         return;
     }
-    slot += (size_t)wave * (PR * TB * 4) * 64 + lane;
+    const int cols = min(p.cols, 64 * TB);
 #pragma unroll
-    for (int pr = 0; pr < PR; ++pr)
+    for (int tb = 0; tb < TB; ++tb) {
+        const int block = (wt * TB + tb) * 32, width = min(32, cols - block);
+        if ((lane & 31) >= width) continue;
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
+        for (int pr = 0; pr < PR; ++pr)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                slot[((pr * TB + tb) * 4 + g) * 64] =
+                slot[p8_slot_quad(cols, wr * PR + pr, block, width, g, lane)] =
                     f32x4{acc[pr][tb][4 * g], acc[pr][tb][4 * g + 1], acc[pr][tb][4 * g + 2], acc[pr][tb][4 * g + 3]};
+    }
 }
 
 // Token columns / 64 that token tile tt multiplies: the last tile those that cover it (28672 x 4096 bf16 at 700 tokens 196 ->
@@ -315,7 +326,7 @@ __global__ void __launch_bounds__(512) gemm_panel8_kernel(Panel8Args p) {
         const int panel = at / windows, w0 = at - panel * windows, n = min(windows - w0, end - at);
         int rt, tt;
         if (p8_panel(p, line, panel, rt, tt)) {
-            f32x4 *slot = n == windows ? nullptr : p.partial + ((size_t)(line * p.deal + j) * p.slots + seg) * (8 * PR * MAXTB * 4 * 64);
+            f32x4 *slot = n == windows ? nullptr : p.partial + ((size_t)(line * p.deal + j) * p.slots + seg) * (32 * PR * p.cols);
             const int tb = p8_columns(p.M, tt, MAXTB);
             if (MAXTB == 1 || tb == 1) gemm_panel8<T, FP8, PR, 1, MAXTB>(p, rt, tt, 2 * w0, 2 * n, slot);
             if constexpr (MAXTB >= 2)
@@ -345,24 +356,26 @@ __global__ void __launch_bounds__(256) gemm_panel8_fold_kernel(Panel8Args p, int
     if (i >= 16 * pr_n * tb_n) return;
     const int gp = (i & 1) * 2;
     i >>= 1;
-    const int quad0 = i * 4 + gp;                              // of the slot: i counts (wave, row pair, token block)
     const int tb = i % tb_n, pr = i / tb_n % pr_n, wave = i / (tb_n * pr_n);
+    const int cols = min(p.cols, 64 * tb_n), block = ((wave >> 2) * tb_n + tb) * 32, width = min(32, cols - block);     // of the panel's tokens
+    if ((lane & 31) >= width) return;
 
     const int windows = p.K >> 6, total = (p.panels - p.whole) * windows, first = local * windows;
     auto owner = [&](int at) { return (int)((((long long)at + 1) * p.deal - 1) / total); };
     const int j0 = owner(first), j1 = owner(first + windows - 1);
     if (j0 == j1) return;                                      // one workgroup computed and stored it
     const bool j0_starts = (int)((long long)j0 * total / p.deal) == first;
-    const size_t slot_quads = (size_t)8 * pr_n * maxtb * 4 * 64;
+    const size_t slot_quads = (size_t)32 * pr_n * p.cols;
+    const int quad = p8_slot_quad(cols, (wave & 3) * pr_n + pr, block, width, gp, lane);
     auto at = [&](int j) {
-        return p.partial + ((size_t)(line * p.deal + j) * p.slots + (j == j0 && !j0_starts)) * slot_quads + (size_t)quad0 * 64 + lane;
+        return p.partial + ((size_t)(line * p.deal + j) * p.slots + (j == j0 && !j0_starts)) * slot_quads + quad;
     };
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
     for (int j = j0; j <= j1; j += 8) {                        // eight slots in flight: a round trip each if fetched one by one
         f32x4 t[8][2];
 #pragma unroll
         for (int d = 0; d < 8; ++d)
-            if (j + d <= j1) t[d][0] = at(j + d)[0], t[d][1] = at(j + d)[64];
+            if (j + d <= j1) t[d][0] = at(j + d)[0], t[d][1] = at(j + d)[2 * width];
 #pragma unroll
         for (int d = 0; d < 8; ++d)
             if (j + d <= j1) s0 += t[d][0], s1 += t[d][1];
@@ -377,7 +390,7 @@ __global__ void __launch_bounds__(256) gemm_panel8_fold_kernel(Panel8Args p, int
         o[4 + e] = __uint_as_float(x[1]);
     }
     const int n = (rt * 8 * pr_n + (wave & 3) * 2 * pr_n + 2 * pr) * 16 + 8 * (gp + (lane >> 5));
-    const int tok = tt * 64 * maxtb + (wave >> 2) * 32 * tb_n + tb * 32 + (lane & 31);
+    const int tok = tt * 64 * maxtb + block + (lane & 31);
     if (n >= p.N || tok >= p.M) return;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {

@@ -639,6 +639,33 @@ def test_gemm_panel_ids_3_and_5_take_64_slices(mlk, kid, n, m, k, p3):
     assert (ws[size:] == 0xAB).all()
 
 
+@pytest.mark.parametrize("m,p1,p2,p3", [(1, 2, 1, 3), (16, 2, 1, 6), (33, 2, 1, 6), (48, 4, 1, 5), (40, 2, 2, 4), (64, 2, 1, 7)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_gemm_eight_wave_slices_fit_the_workspace_of_the_other_ids(mlk, kind, m, p1, p2, p3):
+    """Up to 64 tokens the K slices of kernel id 8 run on what mlk_gemm_workspace_bytes() answers, as those of every row of the
+    tables do, and write nothing behind what mlk_gemm_panel_workspace_bytes() says."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    lib = _lib.load()
+    n, k = 512, 1152
+    x = randn((m, k), torch.bfloat16, 1.0, 46)
+    if kind == "fp8":
+        w = fp8_codes((n, k), 47)
+        scale = (torch.rand((n // 128, k // 128), generator=torch.Generator().manual_seed(48)) * 0.02 + 0.001).float()
+        want, sc = ogemm.softfp8_linear_expected(w.numpy(), scale.numpy(), x), scale.cuda()
+    else:
+        w = randn((n, k), torch.bfloat16, k ** -0.5, 47)
+        want, sc = ogemm.linear_expected(w, x), None
+    a, b, c = pack_a(w).cuda(), x.cuda(), torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+    size, need = lib.mlk_gemm_workspace_bytes(m, n, p1, p3), lib.mlk_gemm_panel_workspace_bytes(m, n, k, p1, p2, p3)
+    assert need <= size
+    ws = torch.full((size + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.mlk_gemm_layout_a(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, 2 if kind == "fp8" else 1, 1, 0, 0, 1.0, None,
+                                     None if sc is None else sc.data_ptr(), 8, p1, p2, p3, ws.data_ptr(), size, _stream()), "gemm")
+    assert_close(c, want, RTOL, ATOL, "m = %d" % m)
+    assert (ws[need:] == 0xAB).all()
+
+
 @pytest.mark.parametrize("kid,p3", [(3, 1), (3, 2), (5, 2)])
 @pytest.mark.parametrize("kind", ["fp16", "fp8"])
 @pytest.mark.parametrize("n,m,k", [(256, 300, 512), (2304, 520, 256)])

@@ -352,3 +352,19 @@ def test_panel_plan_is_a_shape_the_kernel_takes():
         assert ops._gemm_args("layoutA_gemm", 4224, 300, 1024, 1) == (3, 4, 1, 1)
     finally:
         del table[(4224, 300, 1024)]
+
+
+def test_shipped_panel_rows_fit_the_documented_workspace():
+    """A C caller sizes the K split of a table row with mlk_gemm_workspace_bytes(): enough for the rows of kernel id 8 too, at their own
+    token count and at every smaller one that borrows them."""
+    from muxi_native_layout_kernels_amd import _lib, arg_selector
+    lib = _lib.load()
+    rows = 0
+    for name in ("layout_gemm", "continuous_gemm", "layoutA_gemm", "layoutA_soft_fp8_gemm"):
+        for (n, m, k), (kid, p1, p2, p3) in arg_selector.selector(name).table().items():
+            if kid == 8:
+                rows += 1
+                for tokens in range(max(1, m - 31), m + 1):
+                    assert lib.mlk_gemm_panel_workspace_bytes(tokens, n, k, p1, p2, p3) <= lib.mlk_gemm_workspace_bytes(tokens, n, p1, p3), \
+                        (name, n, tokens, k)
+    assert rows > 0
