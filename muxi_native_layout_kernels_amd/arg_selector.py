@@ -10,8 +10,9 @@ one-time warning and a fallback that is remembered for the rest of the process
 miss memo is kept under a lock.  Where the reference falls back to fixed
 arguments, a GEMM shape whose table holds the same weight shape at other token
 counts borrows the row of the nearest scanned count in the same kernel range
-(up to 64 tokens, or above), and only a weight shape that was never scanned
-gets arguments from a rule of thumb.
+(up to 64 tokens, or above).  A shape that can borrow none (above 64 tokens the
+packaged tables hold no rows) gets what the library expects to be fastest
+(`mlk_gemm_plan`), and where that has no answer arguments from a rule of thumb.
 
 What the columns select on gfx950 (the rows are produced by the scripts in
 `kernel_args_scan/`):
@@ -126,19 +127,16 @@ class _Selector:
             return above[0]
         return same[-1] if same else None
 
-    def near(self, key):
-        """Whether a row of the same weight shape can be borrowed for this key."""
-        self.table()                            # read before the lock is taken, which reading takes too
-        with self._lock:
-            return self.neighbours and self._neighbour(tuple(int(v) for v in key)) is not None
-
-    def get_args(self, key):
+    def get_args(self, key, plan=None):
+        """Launch parameters of a shape.  `plan` is asked for those of a shape that has no row and can borrow none; where it has no
+        answer (None) they come from the rule of thumb."""
         key = tuple(int(v) for v in key)
         hit = self.table().get(key)
         if hit is not None:
             return hit
         with self._lock:
-            memo = self._memo.get(key)
+            memo_key = (key, plan is not None)
+            memo = self._memo.get(memo_key)
             if memo is not None:
                 return memo
             near = self._neighbour(key) if self.neighbours else None
@@ -147,12 +145,14 @@ class _Selector:
                 sys.stderr.write(" Warning: No matching arguments found for %s shape: %s. Borrowing the args of %d "
                                  "tokens: %s\n" % (self.label, ", ".join(str(v) for v in key), near[0],
                                                    ",".join(str(v) for v in args)))
-                self._memo[key] = args
+                self._memo[memo_key] = args
                 return args
-            args = self.heuristic(*key) if self.heuristic is not None else self.fallback
+            args = plan() if plan is not None else None
+            if args is None:
+                args = self.heuristic(*key) if self.heuristic is not None else self.fallback
             sys.stderr.write(" Warning: No matching arguments found for %s shape: %s. Fallback args to %s\n" %
                              (self.label, ", ".join(str(v) for v in key), ",".join(str(v) for v in args)))
-            self._memo[key] = args
+            self._memo[memo_key] = args
             return args
 
 

@@ -363,18 +363,18 @@ def _gemm_guard(args, m):
 
 
 def _gemm_args(table, m, n, k, a_kind):
-    """Launch parameters of a table-driven GeMM call: the table's row of this very shape; up to 64 tokens the row of a nearby token
-    count; else what the library expects to be fastest (`mlk_gemm_plan`: a fitted cost of every launch it considers), else what the
-    selector makes of it.  The shipped tables hold no rows above 64 tokens: on 24 weight shapes at 14 token counts from 65 to
+    """Launch parameters of a table-driven GeMM call: the table's row of this very shape; else the row of a nearby token count (up to
+    64 tokens, or above); else what the library expects to be fastest (`mlk_gemm_plan`: a fitted cost of every launch it considers),
+    else what the selector makes of it.  The packaged tables hold no rows above 64 tokens: on 24 weight shapes at 14 token counts from 65 to
     3000 the eight-wave panels were 1.29 (bf16) to 1.40 (soft-FP8) times as fast as the rows that had been scanned for the older panel
     kernels (geometric mean), and in native layouts, where those do not run, up to fifteen times.  Weight shapes outside the tables
     at up to 64 tokens: 1.37 times the fixed launch parameters they had."""
-    sel = arg_selector.selector(table)
-    if (m, n, k) not in sel.table() and k % 128 == 0 and n * k < 1 << 31 and (n > 64 or not sel.near((m, n, k))):
-        plan = (ctypes.c_int32 * 4)()
-        if _lib.load().mlk_gemm_plan(n, m, k, a_kind, plan) == 0:
-            return tuple(plan)
-    return _gemm_guard(sel.get_args((m, n, k)), m)
+    def plan():
+        out = (ctypes.c_int32 * 4)()
+        if k % 128 or n * k >= 1 << 31 or _lib.load().mlk_gemm_plan(n, m, k, a_kind, out) != 0:
+            return None
+        return tuple(out)
+    return _gemm_guard(arg_selector.selector(table).get_args((m, n, k), plan), m)
 
 
 def _gemm_eager(tag, table, checked, A, A_Scale, B, alpha, beta, bias, b_mode, c_mode):

@@ -368,3 +368,25 @@ def test_shipped_panel_rows_fit_the_documented_workspace():
                     assert lib.mlk_gemm_panel_workspace_bytes(tokens, n, k, p1, p2, p3) <= lib.mlk_gemm_workspace_bytes(tokens, n, p1, p3), \
                         (name, n, tokens, k)
     assert rows > 0
+
+
+def test_rows_above_64_tokens_are_borrowed_and_misses_are_named(capsys, tmp_path, monkeypatch):
+    """Rows that a user has scanned above 64 tokens serve nearby counts above 64, in front of the library's plan and never below; a shape
+    without any gets the plan.  Either is named on stderr once."""
+    from muxi_native_layout_kernels_amd import arg_selector
+    p = tmp_path / "t.csv"
+    p.write_text("m,n,k,kernelId,kernelParam1,kernelParam2,kernelParam3\n"
+                 "4224,32,1024,1,2,4,1\n4224,256,1024,3,4,1,2\n4224,1024,1024,5,4,2,2\n4352,32,1024,1,2,4,1\n")
+    sel = arg_selector._Selector(str(p), 3, arg_selector.GEMM_FALLBACK, "tmp", lambda n, m, k: (1, 1, 8, 1), True)
+    sel.path = lambda: str(p)
+    monkeypatch.setattr(arg_selector, "selector", lambda name: sel)
+    for _ in range(2):
+        assert ops._gemm_args("layoutA_gemm", 4224, 256, 1024, 1) == (3, 4, 1, 2)
+        assert ops._gemm_args("layoutA_gemm", 4224, 65, 1024, 1) == (3, 4, 1, 2)
+        assert ops._gemm_args("layoutA_gemm", 4224, 300, 1024, 1) == (5, 4, 2, 2)
+        assert ops._gemm_args("layoutA_gemm", 4224, 4096, 1024, 1) == (5, 4, 2, 2)
+        assert ops._gemm_args("layoutA_gemm", 4224, 64, 1024, 1) == (1, 2, 4, 1)
+        assert ops._gemm_args("layoutA_gemm", 4352, 300, 1024, 1)[0] == 8          # no row above 64 tokens: planned
+        assert ops._gemm_args("layoutA_gemm", 4224, 300, 1088, 1) == (1, 1, 8, 1)  # K % 128: no plan
+    err = capsys.readouterr().err
+    assert err.count("Borrowing the args of") == 4 and err.count("Fallback args to") == 2
