@@ -367,7 +367,7 @@ def main():
         b = torch.randn((m, k), generator=gen, device=dev).to(DT[xk])
         scale = block_scales((n // 128, k // 128)) if kind == 2 else None
         table = "layoutA_soft_fp8_gemm" if kind == 2 else ("layout_gemm" if native else "layoutA_gemm")
-        kid, p1, p2, p3 = mlk.ops._gemm_args(table, n, m, k, kind)
+        kid, p1, p2, p3 = mlk.ops._gemm_args(table, n, m, k, kind, 1 if native else 0)
         if native:
             b_in = mlk.layoutB(b)
             c = torch.empty((n // 32, m // 16, 4, 16, 8), dtype=DT[xk], device=dev)

@@ -12,7 +12,7 @@ arguments, a GEMM shape whose table holds the same weight shape at other token
 counts borrows the row of the nearest scanned count in the same kernel range
 (up to 64 tokens, or above).  A shape that can borrow none (above 64 tokens the
 packaged tables hold no rows) gets what the library expects to be fastest
-(`mlk_gemm_plan`), and where that has no answer arguments from a rule of thumb.
+(`mlk_gemm_plan_placed`), and where that has no answer arguments from a rule of thumb.
 
 What the columns select on gfx950 (the rows are produced by the scripts in
 `kernel_args_scan/`):

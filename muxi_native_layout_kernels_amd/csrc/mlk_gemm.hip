@@ -54,7 +54,7 @@ extern template int launch_modes<BF16, true>(const GemmArgs &, int, int, int, in
 // kernel id 3 (mlk_panel.hip)
 size_t panel_partial_bytes(int m, int n, int sk);
 size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int p3);
-void gemm_plan(int m, int n, int k, bool fp8, int32_t *out);
+void gemm_plan(int m, int n, int k, bool fp8, bool b_native, int32_t *out);
 int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, bool b_native, bool c_native,
                        float alpha, const void *bias, const float *scale, int pr, int tb, int p3, int whole_groups, void *partial,
                        size_t partial_bytes, hipStream_t s);
@@ -88,12 +88,17 @@ extern "C" size_t mlk_gemm_panel_workspace_bytes(int m, int n, int k, int p1, in
     return bytes ? kCounterBytes + bytes : 0;
 }
 
-extern "C" int mlk_gemm_plan(int m, int n, int k, int a_kind, int32_t *out) {
+extern "C" int mlk_gemm_plan_placed(int m, int n, int k, int a_kind, int b_mode, int32_t *out) {
     MLK_REQUIRE(out != nullptr, "gemm: null pointer");
     MLK_REQUIRE(m > 0 && n > 0 && n % 16 == 0 && k > 0 && k % 128 == 0, "gemm: the panel kernel needs N % 16 == 0 and K % 128 == 0");
     MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
-    gemm_plan(m, n, k, a_kind == MLK_FP8_E4M3, out);
+    MLK_REQUIRE(b_mode == MLK_B_ROWMAJOR || b_mode == MLK_B_NATIVE, "gemm: bad activation placement");
+    gemm_plan(m, n, k, a_kind == MLK_FP8_E4M3, b_mode == MLK_B_NATIVE, out);
     return MLK_OK;
+}
+
+extern "C" int mlk_gemm_plan(int m, int n, int k, int a_kind, int32_t *out) {
+    return mlk_gemm_plan_placed(m, n, k, a_kind, MLK_B_ROWMAJOR, out);
 }
 
 extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, int x_kind,

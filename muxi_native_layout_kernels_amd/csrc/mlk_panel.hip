@@ -287,7 +287,7 @@ static double narrow_us(bool fp8, int m, int n, int k, int id, int p1, int p2, i
 }
 
 // Launch parameters (kernel id, p1, p2, p3) that are expected to be fastest for m tokens x n rows x k.
-void gemm_plan(int m, int n, int k, bool fp8, int32_t *out) {
+void gemm_plan(int m, int n, int k, bool fp8, bool b_native, int32_t *out) {
     const P8Cost &f = fp8 ? kP8Cost8 : kP8Cost16;
     double best = 1e30;
     auto offer = [&](double us, int id, int p1, int p2, int p3) {
@@ -310,7 +310,8 @@ void gemm_plan(int m, int n, int k, bool fp8, int32_t *out) {
     int r = m > 32 || groups % 2 ? 1 : 2, waves = 1;
     while (waves < 16 && (long long)groups / r * waves < 8 * cus) waves *= 2;
     offer(0.96 * narrow_us(fp8, m, n, k, 1, r, waves, 1), 1, r, waves, 1);
-    if (groups > cus && groups <= cus * (fp8 ? 8 : 4) && (!fp8 || m > 16))
+    // kernel 4 exists from two token blocks on with soft-FP8 weights and with layout-B activations
+    if (groups > cus && groups <= cus * (fp8 ? 8 : 4) && ((!fp8 && !b_native) || m > 16))
         for (int p2 = 4; p2 <= 8; p2 *= 2) offer(narrow_us(fp8, m, n, k, 4, 1, p2, 1), 4, 1, p2, 1);
     for (int p1 = 1; p1 <= 4; p1 *= 2)
         for (int p2 = 4; groups % p1 == 0 && p2 <= 16; p2 *= 2)

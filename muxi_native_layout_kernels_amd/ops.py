@@ -362,16 +362,16 @@ def _gemm_guard(args, m):
     return args
 
 
-def _gemm_args(table, m, n, k, a_kind):
+def _gemm_args(table, m, n, k, a_kind, b_mode=_B_ROWMAJOR):
     """Launch parameters of a table-driven GeMM call: the table's row of this very shape; else the row of a nearby token count (up to
-    64 tokens, or above); else what the library expects to be fastest (`mlk_gemm_plan`: a fitted cost of every launch it considers),
+    64 tokens, or above); else what the library expects to be fastest (`mlk_gemm_plan_placed`: a fitted cost of every launch it considers),
     else what the selector makes of it.  The packaged tables hold no rows above 64 tokens: on 24 weight shapes at 14 token counts from 65 to
     3000 the eight-wave panels were 1.29 (bf16) to 1.40 (soft-FP8) times as fast as the rows that had been scanned for the older panel
     kernels (geometric mean), and in native layouts, where those do not run, up to fifteen times.  Weight shapes outside the tables
     at up to 64 tokens: 1.37 times the fixed launch parameters they had."""
     def plan():
         out = (ctypes.c_int32 * 4)()
-        if k % 128 or n * k >= 1 << 31 or _lib.load().mlk_gemm_plan(n, m, k, a_kind, out) != 0:
+        if k % 128 or n * k >= 1 << 31 or _lib.load().mlk_gemm_plan_placed(n, m, k, a_kind, b_mode, out) != 0:
             return None
         return tuple(out)
     return _gemm_guard(arg_selector.selector(table).get_args((m, n, k), plan), m)
@@ -403,7 +403,7 @@ def _gemm_eager(tag, table, checked, A, A_Scale, B, alpha, beta, bias, b_mode, c
     lib = _lib.load()
     m, k = A.size(0) * 16, A.size(1) * 8
     n = B.size(0) if b_mode == _B_ROWMAJOR else B.size(1) * 16
-    kid, p1, p2, p3 = _gemm_args(table, m, n, k, _kind(A))
+    kid, p1, p2, p3 = _gemm_args(table, m, n, k, _kind(A), b_mode)
     _plans[key] = (m, n, k, _kind(A), _KIND[B.dtype], kid, p1, p2, p3,
                    _gemm_workspace_bytes(lib, m, n, k, kid, p1, p2, p3) if p3 > 1 else 0, lib.mlk_gemm_counter_bytes(),
                    _is_fp8(A) and A_Scale is not None, tuple(C.shape), lib.mlk_gemm_layout_a)
@@ -441,7 +441,7 @@ def _gemm_layoutA_checked(A, B, alpha=1, beta=0, bias=None):
     k = a_k
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
-    kid, p1, p2, p3 = _gemm_args("layoutA_gemm", m, n, k, _kind(A))
+    kid, p1, p2, p3 = _gemm_args("layoutA_gemm", m, n, k, _kind(A), _B_ROWMAJOR)
     return gemm_layoutA_wapper(A, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 
@@ -471,7 +471,7 @@ def _gemm_layoutA_soft_fp8_checked(A, A_Scale, B, alpha=1, beta=0, bias=None):
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
     _check(B.dtype == torch.bfloat16, "soft-FP8 weights need bf16 activations")
-    kid, p1, p2, p3 = _gemm_args("layoutA_soft_fp8_gemm", m, n, k, _kind(A))
+    kid, p1, p2, p3 = _gemm_args("layoutA_soft_fp8_gemm", m, n, k, _kind(A), _B_ROWMAJOR)
     return gemm_layoutA_soft_fp8_wapper(A, A_Scale, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 
@@ -512,7 +512,7 @@ def _gemm_layoutAB_ContinuousC_checked(A, B, alpha=1, beta=0, bias=None):
     k = a_k
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
-    kid, p1, p2, p3 = _gemm_args("continuous_gemm", m, n, k, _kind(A))
+    kid, p1, p2, p3 = _gemm_args("continuous_gemm", m, n, k, _kind(A), _B_NATIVE)
     return gemm_layoutAB_ContinuousC_wapper(A, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 
@@ -539,7 +539,7 @@ def _gemm_layoutABC_checked(A, B, alpha=1, beta=0, bias=None):
     k = a_k
     _check(m % 128 == 0, "GEMM m % 128 == 0, currently, will be revised soon")
     _check(k % 128 == 0, "GEMM k % 128 must be 0")
-    kid, p1, p2, p3 = _gemm_args("layout_gemm", m, n, k, _kind(A))
+    kid, p1, p2, p3 = _gemm_args("layout_gemm", m, n, k, _kind(A), _B_NATIVE)
     return gemm_layoutABC_wapper(A, B, m, n, k, alpha, beta, p1, p2, p3, kid, bias)
 
 

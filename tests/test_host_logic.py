@@ -390,3 +390,25 @@ def test_rows_above_64_tokens_are_borrowed_and_misses_are_named(capsys, tmp_path
         assert ops._gemm_args("layoutA_gemm", 4224, 300, 1088, 1) == (1, 1, 8, 1)  # K % 128: no plan
     err = capsys.readouterr().err
     assert err.count("Borrowing the args of") == 4 and err.count("Fallback args to") == 2
+
+
+def test_plan_of_native_activations_names_kernels_that_take_them():
+    """Layout-B activations of one token block have no kernel id 4: the plan leaves it out there (a launch that asks for it runs kernel id 1
+    with the least of everything), offers it from 17 tokens on, and is the row-major one wherever that names another kernel."""
+    import ctypes
+    from muxi_native_layout_kernels_amd import _lib
+    lib = _lib.load()
+    met = 0
+    for n in range(128, 32768, 384):
+        for k in (512, 2688, 4096, 7168, 14336):
+            for m in (16, 32, 64):
+                row, nat = (ctypes.c_int32 * 4)(), (ctypes.c_int32 * 4)()
+                assert lib.mlk_gemm_plan_placed(m, n, k, 1, 0, row) == 0 and lib.mlk_gemm_plan_placed(m, n, k, 1, 1, nat) == 0
+                if m == 16 and row[0] == 4:
+                    met += 1
+                    assert nat[0] in (1, 8) and (n // 16) % nat[1] == 0
+                else:
+                    assert list(nat) == list(row)
+    assert met > 0
+    assert lib.mlk_gemm_plan_placed(16, 128, 128, 1, 2, nat) != 0
+    assert ops._gemm_args("layout_gemm", 9344, 16, 2688, 1, 1)[0] != 4
