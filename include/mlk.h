@@ -196,7 +196,8 @@ int mlk_gemv_layout_a(const void *a, const void *x, void *y, int m, int n, int k
  *                whole; 2 to 63: K slices; 64: the k windows dealt evenly to one workgroup per CU.  With more panels than CUs p3
  *                applies to those left over after whole rounds of one per CU.  fp32 sums of panels that were not computed
  *                whole are added in the order of k by a second launch; workspace: mlk_gemm_panel_workspace_bytes().  Operands
- *                off 16 bytes run kernel 3 (native B or C: kernel 1) instead.  mlk_gemm_plan_placed() picks p1, p2, p3
+ *                off 16 bytes run kernel 3 (up to 64 tokens and with native B or C: 1 or 4) instead, in as many K slices as the
+ *                workspace holds.  mlk_gemm_plan_placed() picks p1, p2, p3
  *   kernel_id 12, 14, 16, 18  kernel 1 with 2, 4, 6 or 8 k tiles in flight per wave instead of the
  *                default depth; honoured for up to 16 tokens with row-major B and C, otherwise
  *                the same as kernel 1
@@ -218,6 +219,9 @@ size_t mlk_gemm_panel_workspace_bytes(int m, int n, int k, int p1, int p2, int p
 int mlk_gemm_plan(int m, int n, int k, int a_kind, int32_t *out);
 /* the same for activations in the layout that b_mode says (mlk_gemm_plan: row-major) */
 int mlk_gemm_plan_placed(int m, int n, int k, int a_kind, int b_mode, int32_t *out);
+/* out[4] = kernel id, p1, p2, p3 of the launch that kernel id 8 stands for with operands off 16 bytes, for callers that keep launch
+ * parameters (workspace: mlk_gemm_workspace_bytes()) */
+int mlk_gemm_plan_off16(int m, int n, int k, int a_kind, int b_mode, int c_mode, int32_t *out);
 size_t mlk_gemm_counter_bytes(void);
 
 /* mlk_gemm_layout_a for callers that can neither allocate device memory nor bring a workspace (code under

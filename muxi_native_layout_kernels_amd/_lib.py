@@ -38,6 +38,7 @@ SIGNATURES = {
     "mlk_gemm_panel_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "mlk_gemm_plan": (c_int, [c_int, c_int, c_int, c_int, c_void_p]),
     "mlk_gemm_plan_placed": (c_int, [c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "mlk_gemm_plan_off16": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "mlk_gemm_counter_bytes": (c_size_t, []),
     "mlk_fused_routing_gate": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                        c_void_p, c_void_p, c_void_p]),

@@ -55,6 +55,7 @@ extern template int launch_modes<BF16, true>(const GemmArgs &, int, int, int, in
 size_t panel_partial_bytes(int m, int n, int sk);
 size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int p3);
 void gemm_plan(int m, int n, int k, bool fp8, bool b_native, int32_t *out);
+void gemm_plan_off16(int m, int n, int k, bool fp8, bool b_native, bool c_native, size_t partial_bytes, int32_t *out);
 int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, bool b_native, bool c_native,
                        float alpha, const void *bias, const float *scale, int pr, int tb, int p3, int whole_groups, void *partial,
                        size_t partial_bytes, hipStream_t s);
@@ -101,6 +102,13 @@ extern "C" int mlk_gemm_plan(int m, int n, int k, int a_kind, int32_t *out) {
     return mlk_gemm_plan_placed(m, n, k, a_kind, MLK_B_ROWMAJOR, out);
 }
 
+extern "C" int mlk_gemm_plan_off16(int m, int n, int k, int a_kind, int b_mode, int c_mode, int32_t *out) {
+    MLK_REQUIRE(out != nullptr, "gemm: null pointer");
+    MLK_REQUIRE(m > 0 && n > 0 && n % 16 == 0 && k > 0 && k % 128 == 0, "gemm: the panel kernel needs N % 16 == 0 and K % 128 == 0");
+    gemm_plan_off16(m, n, k, a_kind == MLK_FP8_E4M3, b_mode == MLK_B_NATIVE, c_mode == MLK_C_NATIVE, (size_t)-1, out);
+    return MLK_OK;
+}
+
 extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, int n, int k, int a_kind, int x_kind,
                                  int b_mode, int c_mode, float alpha, const void *bias, const float *scale,
                                  int kernel_id, int p1, int p2, int p3, void *workspace, size_t workspace_bytes,
@@ -130,6 +138,21 @@ extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, i
     }
     if (m == 0 || n == 0) return MLK_OK;
     MLK_REQUIRE(a && b && c, "gemm: null pointer");
+    if (kernel_id == 8) {
+        // eight-wave panels; p1 = row groups per wave pair (2: 128-row panels, 4: 256-row panels), p2 = tokens per panel / 64, p3 = K slices.
+        // Their loads write LDS and their stores move 16 bytes: operands off 16 bytes take the kernels that go through registers.
+        MLK_REQUIRE((p1 == 2 || p1 == 4) && p2 <= 4, "gemm: kernel 8 takes p1 = 2 or 4 and p2 = 1 to 4");
+        MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
+        uint8_t *ws = (uint8_t *)workspace;
+        const size_t part_bytes = ws && workspace_bytes > kCounterBytes ? workspace_bytes - kCounterBytes : 0;
+        if (aligned16(a) && aligned16(b) && aligned16(c) && aligned16(workspace))
+            return launch_panel8_gemm(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, b_mode == MLK_B_NATIVE, c_mode == MLK_C_NATIVE,
+                                      alpha, bias, scale, p1 / 2, p2, p3, -1, ws ? ws + kCounterBytes : nullptr, part_bytes,
+                                      (hipStream_t)stream);
+        int32_t plan[4];
+        gemm_plan_off16(m, n, k, fp8, b_mode == MLK_B_NATIVE, c_mode == MLK_C_NATIVE, aligned16(workspace) ? part_bytes : 0, plan);
+        kernel_id = plan[0], p1 = plan[1], p2 = plan[2], p3 = plan[3];
+    }
     if (kernel_id == 3 || kernel_id == 5) {
         // panel kernel: any number of tokens in one launch; kernel id 5 slices only the panels of the last, partial
         // round of one panel per CU; p1 = row groups per wave (2: 128-row panels, 4: 256-row
@@ -143,22 +166,6 @@ extern "C" int mlk_gemm_layout_a(const void *a, const void *b, void *c, int m, i
         return launch_panel(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, alpha, bias, scale, p2 == 1 ? 128 : (p2 == 2 ? 256 : 0),
                             p1 == 2 ? 128 : (p1 == 4 ? 256 : 0), m > 64 ? p3 : 1, kernel_id == 5, ws, kCounterBytes,
                             ws ? ws + kCounterBytes : nullptr, ws ? part_bytes : 0, (hipStream_t)stream);
-    }
-    if (kernel_id == 8) {
-        // eight-wave panels; p1 = row groups per wave pair (2: 128-row panels, 4: 256-row panels), p2 = tokens per panel / 64, p3 = K slices.
-        // Their loads write LDS and their stores move 16 bytes: operands off 16 bytes take the kernels that go through registers.
-        MLK_REQUIRE((p1 == 2 || p1 == 4) && p2 <= 4, "gemm: kernel 8 takes p1 = 2 or 4 and p2 = 1 to 4");
-        MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
-        uint8_t *ws = (uint8_t *)workspace;
-        const size_t part_bytes = workspace_bytes > kCounterBytes ? workspace_bytes - kCounterBytes : 0;
-        if (aligned16(a) && aligned16(b) && aligned16(c) && aligned16(workspace))
-            return launch_panel8_gemm(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, b_mode == MLK_B_NATIVE, c_mode == MLK_C_NATIVE,
-                                      alpha, bias, scale, p1 / 2, p2, p3, -1, ws ? ws + kCounterBytes : nullptr, ws ? part_bytes : 0,
-                                      (hipStream_t)stream);
-        if (b_mode == MLK_B_ROWMAJOR && c_mode == MLK_C_ROWMAJOR)
-            return launch_panel(a, b, c, m, n, k, fp8 ? MLK_FP8_E4M3 : x_kind, alpha, bias, scale, 128, 128, 1, false, nullptr, 0, nullptr, 0,
-                                (hipStream_t)stream);
-        kernel_id = 1, p1 = 1, p2 = 4, p3 = 1;
     }
     int sk = p3;
     if (sk > k / 32) sk = k / 32 > 0 ? k / 32 : 1;

@@ -202,6 +202,12 @@ size_t panel8_partial_bytes(int m, int n, int k, int pr, int tb, int p3) {
     return panel8_partial_bytes(p, pr);
 }
 
+size_t panel_partial_bytes(int m, int n, int sk) {
+    const size_t row_tiles = (n + kPanelRowsPerWg - 1) / kPanelRowsPerWg;
+    const size_t tokens = (size_t)((m + 255) / 256) * 256;       // covers both panel widths
+    return (size_t)sk * row_tiles * kPanelRowsPerWg * tokens * 4;
+}
+
 // Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
 // rounds).  Fitted to the times of all shapes of this kernel on 24 weight shapes (512 to 32000 rows, K 640 to 18944) at 19 token counts from
 // 20 to 3000, bf16 and soft-FP8: the shape it picks is 1.8 % (soft-FP8 1.1 %) slower than the best one in the geometric mean, 11 % (7 %) at the
@@ -286,6 +292,25 @@ static double narrow_us(bool fp8, int m, int n, int k, int id, int p1, int p2, i
     return id == 4 ? us * f.even : us;
 }
 
+// Launches of the narrow kernels (ids 1 and 4) for up to 64 tokens, whose partial sums of K slices take at most `row_blocks` KiB per
+// token block.
+template <class Offer>
+static void narrow_offers(int m, int n, int k, bool fp8, bool b_native, size_t row_blocks, Offer offer) {
+    const int groups = n / 16, cus = device_cus();
+    // the plain launch: two row groups up to 32 tokens, waves until the chip has eight per CU; 4 % in its favour
+    int r = m > 32 || groups % 2 ? 1 : 2, waves = 1;
+    while (waves < 16 && (long long)groups / r * waves < 8 * cus) waves *= 2;
+    offer(0.96 * narrow_us(fp8, m, n, k, 1, r, waves, 1), 1, r, waves, 1);
+    // kernel 4 exists from two token blocks on with soft-FP8 weights and with layout-B activations
+    if (groups > cus && groups <= cus * (fp8 ? 8 : 4) && ((!fp8 && !b_native) || m > 16))
+        for (int p2 = 4; p2 <= 8; p2 *= 2) offer(narrow_us(fp8, m, n, k, 4, 1, p2, 1), 4, 1, p2, 1);
+    for (int p1 = 1; p1 <= 4; p1 *= 2)
+        for (int p2 = 4; groups % p1 == 0 && p2 <= 16; p2 *= 2)
+            for (int p3 = 1; p3 <= 8; p3 *= 2)
+                if (groups / p1 * (long long)p3 <= 4 * cus && (p3 == 1 || (groups / p1 <= 300 && (size_t)p3 * groups <= row_blocks)) && k / 32 / p3 / p2 >= 1)
+                    offer(narrow_us(fp8, m, n, k, 1, p1, p2, p3), 1, p1, p2, p3);
+}
+
 // Launch parameters (kernel id, p1, p2, p3) that are expected to be fastest for m tokens x n rows x k.
 void gemm_plan(int m, int n, int k, bool fp8, bool b_native, int32_t *out) {
     const P8Cost &f = fp8 ? kP8Cost8 : kP8Cost16;
@@ -304,20 +329,31 @@ void gemm_plan(int m, int n, int k, bool fp8, bool b_native, int32_t *out) {
                 for (int sk = 2; sk <= 32 && panels * sk <= device_cus() && k / 64 / sk >= 2; ++sk)
                     offer(panel8_us(f, m, n, k, pr, tb, sk), 8, 2 * pr, tb, sk);
         }
-    if (m > 64) return;
-    const int groups = n / 16, cus = device_cus();
-    // the plain launch: two row groups up to 32 tokens, waves until the chip has eight per CU; 4 % in its favour
-    int r = m > 32 || groups % 2 ? 1 : 2, waves = 1;
-    while (waves < 16 && (long long)groups / r * waves < 8 * cus) waves *= 2;
-    offer(0.96 * narrow_us(fp8, m, n, k, 1, r, waves, 1), 1, r, waves, 1);
-    // kernel 4 exists from two token blocks on with soft-FP8 weights and with layout-B activations
-    if (groups > cus && groups <= cus * (fp8 ? 8 : 4) && ((!fp8 && !b_native) || m > 16))
-        for (int p2 = 4; p2 <= 8; p2 *= 2) offer(narrow_us(fp8, m, n, k, 4, 1, p2, 1), 4, 1, p2, 1);
-    for (int p1 = 1; p1 <= 4; p1 *= 2)
-        for (int p2 = 4; groups % p1 == 0 && p2 <= 16; p2 *= 2)
-            for (int p3 = 1; p3 <= 8; p3 *= 2)
-                if (groups / p1 * (long long)p3 <= 4 * cus && (p3 == 1 || groups / p1 <= 300) && k / 32 / p3 / p2 >= 1)
-                    offer(narrow_us(fp8, m, n, k, 1, p1, p2, p3), 1, p1, p2, p3);
+    if (m <= 64) narrow_offers(m, n, k, fp8, b_native, (size_t)-1, offer);
+}
+
+// The same for operands that the panels cannot take (off 16 bytes), with up to `partial_bytes` of partial sums: kernel id 3 on
+// row-major operands above 64 tokens, else ids 1 and 4, in passes of up to 64 tokens.
+void gemm_plan_off16(int m, int n, int k, bool fp8, bool b_native, bool c_native, size_t partial_bytes, int32_t *out) {
+    double best = 1e30;
+    out[0] = 1, out[1] = 1, out[2] = 4, out[3] = 1;
+    auto offer = [&](double us, int id, int p1, int p2, int p3) {
+        if (us < best) best = us, out[0] = id, out[1] = p1, out[2] = p2, out[3] = p3;
+    };
+    if (m <= 64 || b_native || c_native) {
+        const int blocks = (m + 15) / 16;                      // the kernels ask for sums of up to eight token blocks
+        narrow_offers(m < 64 ? m : 64, n, k, fp8, b_native, partial_bytes / 1024 / (blocks < 8 ? blocks : 8), offer);
+        return;
+    }
+    // 128-row panels put twice as many CUs to work while there are few; K slices of four windows at least that one workgroup per CU
+    // takes
+    const int cus = device_cus();
+    const long long tokens = (m + 127) / 128;
+    const bool small = (n + 255) / 256 * tokens * 8 <= (long long)cus * 3;
+    const long long panels = (small ? (n + 127) / 128 : (n + 255) / 256) * tokens;
+    int sk = 4;
+    while (sk > 1 && (panels * sk > cus || k / 128 / sk < 4 || panel_partial_bytes(m, n, sk) > partial_bytes)) sk >>= 1;
+    out[0] = 3, out[1] = small ? 2 : 4, out[2] = 1, out[3] = sk;
 }
 
 // whole_groups < 0: kernel id 8, p3 as it takes it; else kernel ids 3 and 5, p3 = K slices of the row tiles behind those groups
@@ -355,12 +391,6 @@ int panel_tokens(int m, int n, bool fp8) {
     const long long rounds128 = (row_tiles * ((m + 127) / 128) + cus - 1) / cus;
     const long long rounds256 = (row_tiles * ((m + 255) / 256) + cus - 1) / cus;
     return rounds256 * (fp8 ? 184 : 140) < rounds128 * 100 ? 256 : 128;
-}
-
-size_t panel_partial_bytes(int m, int n, int sk) {
-    const size_t row_tiles = (n + kPanelRowsPerWg - 1) / kPanelRowsPerWg;
-    const size_t tokens = (size_t)((m + 255) / 256) * 256;       // covers both panel widths
-    return (size_t)sk * row_tiles * kPanelRowsPerWg * tokens * 4;
 }
 
 // a_kind: MLK_F16, MLK_BF16 or MLK_FP8_E4M3 (bf16 activations); width: tokens per panel (128 or 256), anything else =

@@ -711,6 +711,30 @@ def test_gemm_eight_wave_panels_off_16_bytes(mlk, native):
     assert_close(c, ogemm.linear_expected(w, x), RTOL, ATOL, "off 16 bytes")
 
 
+@pytest.mark.parametrize("native", [0, 1, 2])
+@pytest.mark.parametrize("n,m,k,split", [(512, 112, 8192, True), (512, 32, 8192, True), (4352, 64, 512, False), (8448, 1040, 256, False)])
+def test_gemm_eight_wave_panels_off_16_bytes_fill_the_chip(mlk, n, m, k, split, native):
+    """Off 16 bytes a call for the eight-wave panels gets launch parameters for the kernels that take it: K slices where it has few
+    rows (they write partial sums into the workspace), row-major, with layout-B activations and with layout-C output too."""
+    from muxi_native_layout_kernels_amd import _lib
+    from muxi_native_layout_kernels_amd.ops import _stream
+    lib = _lib.load()
+    w, x = randn((n, k), torch.bfloat16, k ** -0.5, 49), randn((m, k), torch.bfloat16, 1.0, 50)
+    a, b = pack_a(w).cuda(), pack_b(x).cuda() if native else x.cuda()
+    flat = torch.empty(m * k + 8, dtype=b.dtype, device="cuda")
+    flat[1:1 + m * k] = b.view(-1)
+    c = torch.empty((n // 32, m // 16, 4, 16, 8) if native == 2 else (m, n), dtype=b.dtype, device="cuda")
+    counters = lib.mlk_gemm_counter_bytes()
+    for size in (counters + (4 << 20), 0):
+        ws = torch.full((size + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
+        ws[:counters if size else 0].zero_()
+        _lib.check(lib.mlk_gemm_layout_a(a.data_ptr(), flat.data_ptr() + 2, c.data_ptr(), m, n, k, 1, 1, int(native > 0), int(native == 2),
+                                         1.0, None, None, 8, 4, 2, 1, ws.data_ptr() if size else None, size, _stream()), "gemm")
+        assert_close(mlk.reLayoutC(c) if native == 2 else c, ogemm.linear_expected(w, x), RTOL, ATOL, "off 16 bytes")
+        assert bool((ws[counters:size] != 0xAB).any()) == (split and size > 0)
+        assert (ws[size:] == 0xAB).all() and not ws[:counters if size else 0].any()
+
+
 def test_gemm_eight_wave_panels_replayed_from_a_graph(mlk):
     """The second launch of a sliced product under capture: every replay equals the eager result."""
     n, m, k = 1024, 100, 4096

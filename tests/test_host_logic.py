@@ -412,3 +412,23 @@ def test_plan_of_native_activations_names_kernels_that_take_them():
     assert met > 0
     assert lib.mlk_gemm_plan_placed(16, 128, 128, 1, 2, nat) != 0
     assert ops._gemm_args("layout_gemm", 9344, 16, 2688, 1, 1)[0] != 4
+
+
+def test_launches_off_16_bytes_are_planned():
+    """What kernel id 8 stands for with operands off 16 bytes: kernel 3 on row-major operands above 64 tokens, with as many K slices as
+    put a workgroup on every CU, else kernels 1 and 4; never the panels, and always parameters the library takes."""
+    import random
+    rng = random.Random(9)
+    for _ in range(300):
+        m, k, n = 128 * rng.randint(1, 250), 128 * rng.randint(1, 140), rng.choice([1, 16, 33, 64, 65, 100, 256, 777, 4096])
+        kind, native = rng.choice([0, 2]), rng.randint(0, 2)
+        if native and (kind == 2 or n % 16):
+            continue
+        kid, p1, p2, p3, ws = ops._off16_plan(m, n, k, kind, int(native > 0), int(native == 2))
+        assert ops._gemm_guard((kid, p1, p2, p3), m) == (kid, p1, p2, p3) and (ws > 0) == (p3 > 1)
+        assert kid == 3 if n > 64 and not native else kid in (1, 4)
+        if kid == 3:
+            panels = -(-m // (64 * p1)) * -(-n // 128)
+            assert p2 == 1 and (p3 == 1 or panels * p3 <= 256)
+    assert ops._off16_plan(4096, 100, 4096, 1, 0, 0)[:4] == (3, 2, 1, 4)
+    assert ops._off_panels(8, 0x1002) and not ops._off_panels(8, 0x1010) and not ops._off_panels(3, 0x1002)
