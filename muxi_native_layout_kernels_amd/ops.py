@@ -143,6 +143,14 @@ def _workspace(device, nbytes, counter_bytes, stream=None):
     return _gemm_pool.get(device, _stream() if stream is None else stream, nbytes, counter_bytes)
 
 
+def _split_scratch(device, stream, nbytes, counter_bytes):
+    """The same, or None where the card has no room: every kernel also runs in one slice, which needs none."""
+    try:
+        return _gemm_pool.get(device, stream, nbytes, counter_bytes)
+    except torch.OutOfMemoryError:
+        return None
+
+
 # ------------------------------------------------------------------ relayout
 def pack_layout_a(weight):
     """[N, K] or [E, N, K] (16-bit or 1-byte elements) -> layout-A [.., N/16, K/8, 16, 8].
@@ -342,9 +350,12 @@ def _gemm_call(A, A_Scale, B, m, n, k, alpha, beta, bias, b_mode, c_mode, kernel
         else:
             kernel_id, p1, p2, p3, _ = _off16_plan(m, n, k, a_kind, b_mode, c_mode)
     if p3 > 1:
-        ws_bytes = _gemm_workspace_bytes(lib, m, n, k, int(kernel_id), int(p1), int(p2), int(p3))
-        ws = _workspace(B.device, ws_bytes, lib.mlk_gemm_counter_bytes())
-        ws_bytes = ws.numel()
+        ws = _split_scratch(B.device, _stream(), _gemm_workspace_bytes(lib, m, n, k, int(kernel_id), int(p1), int(p2), int(p3)),
+                            lib.mlk_gemm_counter_bytes())
+        if ws is None:
+            p3 = 1
+        else:
+            ws_bytes = ws.numel()
     _lib.check(lib.mlk_gemm_layout_a(_ptr(A), _ptr(B), _ptr(C), n, m, k, a_kind, _KIND[B.dtype], b_mode, c_mode,
                                      float(alpha), _ptr(bias), _ptr(A_Scale), int(kernel_id), int(p1), int(p2),
                                      int(p3), _ptr(ws), ws_bytes, _stream()), what)
@@ -432,8 +443,11 @@ def _gemm_eager(tag, table, checked, A, A_Scale, B, alpha, beta, bias, b_mode, c
                 kid, p1, p2, p3, ws_need = _off16_plan(m, n, k, a_kind, b_mode, c_mode)
         ws_ptr = ws_len = 0
         if p3 > 1:
-            ws = _gemm_pool.get(B.device, stream, ws_need, counter_bytes)
-            ws_ptr, ws_len = ws.data_ptr(), ws.numel()
+            ws = _split_scratch(B.device, stream, ws_need, counter_bytes)
+            if ws is None:
+                p3 = 1
+            else:
+                ws_ptr, ws_len = ws.data_ptr(), ws.numel()
         rc = fn(a_ptr, b_ptr, C.data_ptr(), n, m, k, a_kind, x_kind, b_mode, c_mode, float(alpha),
                 0 if bias is None else bias.data_ptr(), A_Scale.data_ptr() if use_scale else 0, kid, p1, p2, p3,
                 ws_ptr, ws_len, stream)

@@ -735,6 +735,39 @@ def test_gemm_eight_wave_panels_off_16_bytes_fill_the_chip(mlk, n, m, k, split, 
         assert (ws[size:] == 0xAB).all() and not ws[:counters if size else 0].any()
 
 
+@pytest.mark.parametrize("native", [False, True])
+@pytest.mark.parametrize("n,m,k,dealt", [(512, 112, 4096, False), (512, 48, 4096, False), (2304, 1984, 256, True)])
+def test_gemm_without_room_for_scratch_runs_in_one_slice(mlk, monkeypatch, n, m, k, dealt, native):
+    """A card without room for the scratch of K slices or dealt panels: the call runs whole panels (or one slice) on its first pass and from
+    the launch plan, and takes the slices again once there is room."""
+    from muxi_native_layout_kernels_amd import ops
+    w, x = randn((n, k), torch.bfloat16, k ** -0.5, 56), randn((m, k), torch.bfloat16, 1.0, 57)
+    a, b = pack_a(w).cuda(), pack_b(x).cuda() if native else x.cuda()
+    kid, p1, p2, p3 = (8, 2, 1, 64) if dealt else \
+        ops._gemm_args("continuous_gemm" if native else "layoutA_gemm", n, m, k, 1, int(native))
+    assert p3 > 1
+
+    def run(slices):
+        fn = mlk.gemm_layoutAB_ContinuousC_wapper if native else mlk.gemm_layoutA_wapper
+        return fn(a, b, n, m, k, kernelParam1=p1, kernelParam2=p2, kernelParam3=slices, kernelId=kid)
+
+    def call():
+        return run(p3) if dealt else (mlk.gemm_layoutAB_ContinuousC if native else mlk.gemm_layoutA)(a, b)
+    whole = run(1)
+
+    def full(device, stream, nbytes, prefix_bytes=0):
+        raise torch.OutOfMemoryError("no room for %d bytes" % nbytes)
+    with monkeypatch.context() as patch:
+        patch.setattr(ops._gemm_pool, "get", full)
+        for _ in range(2):
+            assert torch.equal(call(), whole)
+    want = ogemm.linear_expected(w, x)
+    assert_close(whole, want, RTOL, ATOL, "no scratch")
+    split = call()
+    assert_close(split, want, RTOL, ATOL, "scratch")
+    assert not torch.equal(split, whole), "the two orders of summation cannot be told apart"
+
+
 def test_gemm_eight_wave_panels_replayed_from_a_graph(mlk):
     """The second launch of a sliced product under capture: every replay equals the eager result."""
     n, m, k = 1024, 100, 4096
