@@ -319,8 +319,9 @@ int mlk_moe_first_pass(int n_tokens, int n_experts, int topk, int hidden, int in
                        int32_t *out);
 
 /* How mlk_fused_experts_compute runs one pass of up to 256 tokens (for more the answer is that of 256; whether a longer call
- * has such passes, mlk_moe_first_pass tells); the launch code reads the same plan, and runs one of family 1 or 2 that reaches
- * more than 48 experts with one token block per task in family 3 with two.  out[0] = kernel family (0 single-token
+ * has such passes, mlk_moe_first_pass tells) on the least scratch it takes; the launch code reads the same plan.  With more scratch one
+ * of family 1 or 2 that reaches more than 48 experts with one token block per task runs family 3 with two: mlk_moe_pass_plan()
+ * tells what runs on a workspace of a given size.  out[0] = kernel family (0 single-token
  * GeMV kernels, 1 decode kernels that align in-kernel, 2 decode
  * kernels after the alignment kernel, 3 row-shared kernels, 4 panel kernels: soft-FP8 weights with more than 64
  * tokens per pass over an expert), out[1] = token blocks per task, out[2] = upper bound of the task list,
@@ -332,6 +333,9 @@ int mlk_moe_first_pass(int n_tokens, int n_experts, int topk, int hidden, int in
  * where there is no GPU, so a plan made on a host without a GPU can name another slice count than a launch on a
  * device with a different CU count uses.  For tests and the tuning scripts; no counterpart in the reference. */
 int mlk_moe_plan(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, int32_t *out);
+/* The same for a workspace of that size (with mlk_moe_workspace_bytes() of scratch: what a call of up to 256 tokens runs). */
+int mlk_moe_pass_plan(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, size_t workspace_bytes,
+                      int32_t *out);
 
 #ifdef __cplusplus
 }

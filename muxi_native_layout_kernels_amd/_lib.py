@@ -54,6 +54,7 @@ SIGNATURES = {
     "mlk_moe_wide_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "mlk_moe_first_pass": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_size_t, c_void_p]),
     "mlk_moe_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "mlk_moe_pass_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_size_t, c_void_p]),
 }
 
 _lock = threading.Lock()

@@ -1368,7 +1368,7 @@ static int moe_panel_tb32(int cb) { return (cb + 1) / 2 > 4 ? 4 : (cb + 1) / 2; 
 // Experiment switch 9: 1 keeps the row-shared kernels.
 static bool moe_panel_path(int cb, int hidden, bool fp8) { return fp8 && cb >= 5 && hidden % 256 == 0 && g_tunable[9] != 1; }
 
-// How one pass of up to kMoeChunk tokens is run.  The launch code below and mlk_moe_plan() both read it.
+// How one pass of up to kMoeChunk tokens is run.  The launch code below and mlk_moe_plan() both read it, through moe_pass().
 enum { kMoePathGemv1 = 0, kMoePathDecodeInline = 1, kMoePathDecode = 2, kMoePathTile = 3, kMoePathPanel = 4 };
 struct MoePlan {
     int path;         // kMoePath*
@@ -1575,14 +1575,17 @@ static MoePass moe_pass(int tokens_left, int n_experts, int topk, int hidden, in
 
 using namespace mlk;
 
-extern "C" int mlk_moe_plan(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, int32_t *out) {
+static size_t moe_workspace_of(int n_tokens, int n_experts, int topk, int hidden, int inter, bool wide_ok, bool share_ok);
+
+static int moe_plan_out(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, const size_t *workspace_bytes, int32_t *out) {
     MLK_REQUIRE(out != nullptr, "moe plan: null pointer");
     MLK_REQUIRE(n_tokens >= 1 && n_experts >= 1 && n_experts <= kMaxExperts && topk >= 1 && topk <= kMaxTopK,
                 "moe plan: sizes out of range");
     MLK_REQUIRE(hidden > 0 && inter > 0 && hidden % 128 == 0 && inter % 128 == 0,
                 "moe: hidden and intermediate sizes must be multiples of 128");
     const int tc = n_tokens < kMoeChunk ? n_tokens : kMoeChunk;
-    const MoePlan pl = moe_plan(tc, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3);
+    const bool share_ok = workspace_bytes && *workspace_bytes >= moe_workspace_of(tc, n_experts, topk, hidden, inter, false, true);
+    const MoePlan pl = moe_pass(tc, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3, false, share_ok).plan;
     out[0] = pl.path;
     out[1] = pl.cb;
     out[2] = pl.max_tasks;
@@ -1592,6 +1595,15 @@ extern "C" int mlk_moe_plan(int n_tokens, int n_experts, int topk, int hidden, i
     out[6] = (int32_t)pl.down_lds;
     out[7] = (int32_t)sizeof(DecodeTables);
     return MLK_OK;
+}
+
+extern "C" int mlk_moe_plan(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, int32_t *out) {
+    return moe_plan_out(n_tokens, n_experts, topk, hidden, inter, w_kind, nullptr, out);
+}
+
+extern "C" int mlk_moe_pass_plan(int n_tokens, int n_experts, int topk, int hidden, int inter, int w_kind, size_t workspace_bytes,
+                                 int32_t *out) {
+    return moe_plan_out(n_tokens, n_experts, topk, hidden, inter, w_kind, &workspace_bytes, out);
 }
 
 extern "C" void mlk_moe_set_tile_path(int on) {
@@ -1714,7 +1726,7 @@ extern "C" int mlk_moe_first_pass(int n_tokens, int n_experts, int topk, int hid
     MLK_REQUIRE(hidden > 0 && inter > 0 && hidden % 128 == 0 && inter % 128 == 0,
                 "moe: hidden and intermediate sizes must be multiples of 128");
     const bool wide_ok = moe_wide_fits(n_tokens, n_experts, topk, hidden, inter, workspace_bytes);
-    const MoePass ps = moe_pass(n_tokens, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3, wide_ok, false);
+    const MoePass ps = moe_pass(n_tokens, n_experts, topk, hidden, inter, w_kind == MLK_FP8_E4M3, wide_ok, true);
     out[0] = ps.tokens;
     out[1] = ps.wide;
     return MLK_OK;

@@ -780,6 +780,7 @@ def test_workspace_of_256_token_passes_still_takes_longer_calls(mlk, T, kind):
 def test_many_experts_of_one_block_share_rows(mlk, T, E, K, H, I, kind, shared):
     """More than 48 experts in reach with one token block per task: the row-shared kernels, which need scratch per routed pair.
     A workspace that only holds the decode kernels' sums keeps the call on those; nothing behind it is written."""
+    import ctypes
     from muxi_native_layout_kernels_amd import _lib
     from muxi_native_layout_kernels_amd.ops import _stream
     dtype = torch.float16 if kind == "fp16" else torch.bfloat16
@@ -818,7 +819,10 @@ def test_many_experts_of_one_block_share_rows(mlk, T, E, K, H, I, kind, shared):
     finally:
         lib.mlk_moe_set_tile_path(1)
     assert full >= least and (full > least or not shared or K == 1)      # one pick: the decode kernels' K slices need as much
+    plan = (ctypes.c_int32 * 8)()
     for size in (full, least):
+        assert lib.mlk_moe_pass_plan(T, E, K, H, I, wk, size, plan) == 0
+        assert (plan[0] == 3) == (shared and (size > least or full == least))
         ws = torch.full((full + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
         y = torch.empty_like(x)
         _lib.check(lib.mlk_fused_experts_compute(ptr(w1p), ptr(w2p), ptr(x), T, E, K, H, I, wk, xk, ptr(ids), ptr(wts), ptr(emap),

@@ -432,3 +432,31 @@ def test_launches_off_16_bytes_are_planned():
             assert p2 == 1 and (p3 == 1 or panels * p3 <= 256)
     assert ops._off16_plan(4096, 100, 4096, 1, 0, 0)[:4] == (3, 2, 1, 4)
     assert ops._off_panels(8, 0x1002) and not ops._off_panels(8, 0x1010) and not ops._off_panels(3, 0x1002)
+
+
+def test_moe_pass_plan_names_what_runs():
+    """One token block per task: with all the scratch it asks for a pass above 48 experts in reach (soft-FP8 weights: and three workgroups
+    on two CUs) is the row-shared kernels, two blocks per task, else the decode kernels; on the scratch of the decode kernels, and
+    everywhere else, it is what mlk_moe_plan() says."""
+    import ctypes
+    lib, out = _lib.load(), (ctypes.c_int32 * 8)()
+
+    def pass_plan(T, E, K, H, I, kind, size):
+        assert lib.mlk_moe_pass_plan(T, E, K, H, I, kind, size, out) == 0
+        return list(out)
+
+    def plan(T, E, K, H, I, kind):
+        assert lib.mlk_moe_plan(T, E, K, H, I, kind, out) == 0
+        return list(out)
+    for T, E, K, H, I, kind, shared in [(7, 64, 7, 256, 384, 1, True), (8, 64, 6, 256, 384, 1, False), (17, 48, 4, 256, 384, 0, False),
+                                        (17, 49, 4, 1152, 256, 0, True), (12, 64, 8, 256, 384, 2, True), (12, 63, 8, 256, 384, 2, False),
+                                        (16, 256, 8, 7168, 256, 2, True), (244, 256, 8, 7168, 256, 2, True), (1, 256, 8, 7168, 256, 1, False),
+                                        (64, 8, 2, 4096, 14336, 1, False), (256, 8, 2, 4096, 14336, 2, False)]:
+        full = lib.mlk_moe_workspace_bytes(T, E, K, H, I)
+        got, decode = pass_plan(T, E, K, H, I, kind, full), plan(T, E, K, H, I, kind)
+        if shared:
+            assert decode[0] in (1, 2) and got[:3] == [3, 2, min(E, T * K) + T * K // 32]
+            assert pass_plan(T, E, K, H, I, kind, full // 2) == decode
+        else:
+            assert got == decode
+    assert lib.mlk_moe_pass_plan(16, 8, 2, 4096, 100, 1, 0, out) != 0
