@@ -1422,12 +1422,12 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
 // pass streams the weights of all experts it reaches again.  Measured, passes of kMoeChunk tokens -> wide kernels (us, without
 // the router):
 //                                                  tokens   257          264          272          320
-//   8 experts, top-2, H 4096, I 14336, bf16                 624 -> 559   940 -> 547   942 -> 550   972 -> 561
-//   the same, soft-FP8                                      454 -> 461   579 -> 453   577 -> 468   637 -> 482
-//   256 experts, top-8, H 7168, I 256, bf16                 527 -> 542   651 -> 543   762 -> 541  1022 -> 551
-//   the same, soft-FP8                                      332 -> 468   413 -> 458   475 -> 459   664 -> 469
-//   128 experts, top-8, H 2048, I 768, bf16                 242 -> 240   346 -> 235   398 -> 236   476 -> 240
-//   the same, soft-FP8                                      158 -> 192   235 -> 193   276 -> 196   336 -> 194
+//   8 experts, top-2, H 4096, I 14336, bf16                 645 -> 524   887 -> 523   940 -> 523   964 -> 538
+//   the same, soft-FP8                                      424 -> 365   550 -> 332   578 -> 374   632 -> 393
+//   256 experts, top-8, H 7168, I 256, bf16                 524 -> 555   603 -> 543   676 -> 543   915 -> 552
+//   the same, soft-FP8                                      327 -> 388   407 -> 385   442 -> 389   578 -> 396
+//   128 experts, top-8, H 2048, I 768, bf16                 240 -> 239   313 -> 234   345 -> 234   417 -> 236
+//   the same, soft-FP8                                      156 -> 163   200 -> 163   225 -> 164   261 -> 165
 // A few tokens above kMoeChunk, moe_two_passes_pay() keeps the pass of kMoeChunk tokens and its remainder.  A remainder of up to
 // kMoeChunk tokens is a pass of the small kernels again, and a call whose workspace only holds passes of kMoeChunk tokens, or
 // whose operands do not lie on 16 bytes, runs in those.
@@ -1489,26 +1489,6 @@ static size_t moe_wide_most_pair_slices(int tokens, int n_experts, int topk, int
     return most;
 }
 
-// Is a pass of kMoeChunk tokens and one of the `rest` above it cheaper than one wide pass?  The small kernels stream the weights
-// at about 6.4 TB/s; the wide ones multiply at least 64 token columns per panel and reach 3.9 TB/s with soft-FP8 weights,
-// which they widen through LDS, and 6.2 TB/s with 16-bit ones.  What a byte saves that way falls with the tokens per expert,
-// as the small kernels come to be bound by their products; the remainder costs its launches and the experts it reaches once
-// more.  Where a task is one token block, the down kernel walks all tasks in every workgroup (a share per expert) and its
-// grid of 16 output rows each runs in whole rounds.  The constants (us and MB) are fitted to 24 layers of 4 to 256 experts,
-// both kinds of weights and 257 to 320 tokens: three of 572 choices cost more than 3 % against the better one (4, 5 and 7.5 %),
-// where going wide always cost up to 52 % (256 experts, top-8, H 7168, I 2048, soft-FP8, 257 tokens: 1940 -> 2960 us).
-static bool moe_two_passes_pay(int rest, int n_experts, int topk, int hidden, int inter, bool fp8) {
-    const double miss = topk < n_experts ? 1 - (double)topk / n_experts : 0;
-    const double weights = 3e-6 * n_experts * hidden * inter * (fp8 ? 1 : 2), first = weights * (1 - pow(miss, kMoeChunk));
-    const double mean = (double)kMoeChunk * topk / n_experts;
-    double gain = first * ((fp8 ? 0.09 : 0.014) - (fp8 ? 0.0006 : 0.0008) * (mean > 8 ? mean - 8 : 0));
-    if (moe_blocks_per_task(kMoeChunk, topk, n_experts) == 1) {
-        const double rounds = hidden / 16. / device_cus();
-        gain -= (fp8 ? 0.3 : 0.1) * n_experts + (rounds > 1 ? first / 19.5 * (ceil(rounds) / rounds - 1) : 0);
-    }
-    return weights * (1 - pow(miss, rest)) / (fp8 ? 5.5 : 6) + (fp8 ? 25 : 5) < gain;
-}
-
 // The decode kernels take tasks of one token block; their down kernel deals its 16 waves to the tasks in turn, every workgroup
 // walking all of them, so that many experts are a long serial chain per workgroup.  The row-shared kernels give every task
 // workgroups of its own.  Above 48 experts in reach they are the faster ones even where a task of theirs (two blocks, so that
@@ -1526,16 +1506,53 @@ static bool moe_two_passes_pay(int rest, int n_experts, int topk, int hidden, in
 // Soft-FP8 weights ask for three workgroups on two CUs as well: with one per CU (256 experts, 8 tokens: 64 tasks of 4) the
 // walk over H sets the pace, which the decode kernels split over waves.
 constexpr int kMoeWalkExperts = 48;
+static bool moe_sharing_pays(int active, int inter, bool fp8) {
+    if (active <= kMoeWalkExperts || !moe_tile_path() || g_tunable[8] == 1) return false;
+    return !fp8 || active * (inter / 64) * 2 >= 3 * device_cus();
+}
 static void moe_share_rows(MoePass *ps, int n_experts, int topk, int hidden, int inter, bool fp8) {
     const int n_pairs = ps->tokens * topk, active = n_experts < n_pairs ? n_experts : n_pairs;
-    if ((ps->plan.path != kMoePathDecode && ps->plan.path != kMoePathDecodeInline) || ps->cb != 1 || active <= kMoeWalkExperts) return;
-    if (!moe_tile_path() || g_tunable[8] == 1) return;
-    if (fp8 && active * (inter / 64) * 2 < 3 * device_cus()) return;
+    if ((ps->plan.path != kMoePathDecode && ps->plan.path != kMoePathDecodeInline) || ps->cb != 1) return;
+    if (!moe_sharing_pays(active, inter, fp8)) return;
     MoePlan pl = {};
     ps->cb = pl.cb = 2;
     pl.max_tasks = active + n_pairs / (16 * pl.cb);
     moe_plan_tile(&pl, hidden, inter);
     ps->plan = pl;
+}
+
+// Is a pass of kMoeChunk tokens and one of the `rest` above it cheaper than one wide pass?  The small kernels stream the weights
+// faster, and a wide layer pays the start and the end of every panel.  What a byte saves that way falls with the tokens per expert,
+// as the small kernels come to be bound by their products; the remainder costs its launches and the experts it reaches once
+// more.  Where a task is one token block and the decode kernels run it, the down kernel walks all tasks in every workgroup (a share per
+// expert) and its grid of 16 output rows each runs in whole rounds.  The constants (us and MB) are fitted to 44 layers of 8 to 256 experts,
+// both kinds of weights and 257 to 320 tokens (twelve small layers to 512): of 832 choices twelve cost more than 3 % against the better one (10 % at
+// most; 0.1 % in the mean).  Fitted before tasks of one block had the row-shared kernels and the wide kernels their short panels, the choice was
+// wrong by more than 3 % 74 times, by up to 40 % (soft-FP8, 32 experts, top-1, H 4096, I 2048, 268 tokens: two passes 232 us, wide 166 us;
+// 256 experts, top-1, H 2048, I 512, 257 tokens: 129 and 154 us).
+struct MoeTwoPasses {
+    float per_mb, per_mb_mean;     // us that a MB of weights saves in the pass of kMoeChunk tokens; less per token above eight of an expert
+    float per_panel;               // us per wide panel on a CU
+    float bandwidth, start;        // the remainder: MB/us, us
+};
+static bool moe_two_passes_pay(int rest, int n_experts, int topk, int hidden, int inter, bool fp8) {
+    constexpr MoeTwoPasses kBlocks[2] = {{0.014f, 0.0008f, 0.f, 6.f, 5.f}, {0.026f, 0.0006f, 0.4f, 3.7f, 5.f}};      // 16-bit, soft-FP8
+    constexpr MoeTwoPasses kShared[2] = {{0.005f, 0.f, 0.46f, 8.4f, 5.f}, {0.044f, 0.f, 0.83f, 2.9f, 15.f}};         // one block per task
+    constexpr MoeTwoPasses kWalk[2] = {{0.014f, 0.f, 0.f, 6.f, 5.f}, {0.09f, 0.f, 0.f, 5.5f, 25.f}};
+    const bool one_block = moe_blocks_per_task(kMoeChunk, topk, n_experts) == 1;
+    const int pairs = kMoeChunk * topk;
+    const bool walk = one_block && !moe_sharing_pays(n_experts < pairs ? n_experts : pairs, inter, fp8);
+    const MoeTwoPasses &f = (walk ? kWalk : one_block ? kShared : kBlocks)[fp8];
+    const double miss = topk < n_experts ? 1 - (double)topk / n_experts : 0;
+    const double weights = 3e-6 * n_experts * hidden * inter * (fp8 ? 1 : 2), first = weights * (1 - pow(miss, kMoeChunk));
+    const double mean = (double)pairs / n_experts;
+    const double panels = (double)n_experts * (inter / 128. + hidden / 256.) / device_cus();
+    double gain = first * (f.per_mb - f.per_mb_mean * (mean > 8 ? mean - 8 : 0)) + f.per_panel * panels;
+    if (walk) {
+        const double rounds = hidden / 16. / device_cus();
+        gain -= (fp8 ? 0.3 : 0.1) * n_experts + (rounds > 1 ? first / 19.5 * (ceil(rounds) / rounds - 1) : 0);
+    }
+    return weights * (1 - pow(miss, rest)) / f.bandwidth + f.start < gain;
 }
 
 // wide_ok: the operands and the workspace of the call are fit for the wide kernels; share_ok: the workspace holds what
