@@ -44,6 +44,10 @@ What the columns select on gfx950 (the rows are produced by the scripts in
                                  and kernelParam3 are not used; otherwise the same as 1)
                              5 = kernel 3 with the K slices (kernelParam3) applied only to the panels left
                                  over after whole rounds of one panel per CU
+                             8 = eight-wave panels, any token count, row-major or native
+                                 operands (K % 128 == 0): kernelParam1 = 2 / 4: 128 / 256 rows,
+                                 kernelParam2 = 1 to 4: tokens / 64, kernelParam3 = 1: whole,
+                                 2 to 63: K slices, 64: k windows dealt evenly to the CUs
                              12, 14, 16, 18 = kernel 1 with 2, 4, 6, 8 k tiles in flight per
                                  wave (up to 16 tokens, row-major activations and output;
                                  otherwise the same as 1)

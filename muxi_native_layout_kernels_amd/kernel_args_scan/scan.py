@@ -231,6 +231,21 @@ def scan_gemv(table, shapes, iters, progress=None):
     return rows
 
 
+def panel_grid(n, m, k, cus=256):
+    """Launches of the eight-wave panels (kernel 8): 128 or 256 rows x 64 to 256 tokens, whole, in K slices of at least two k windows that one
+    workgroup per CU takes, or (more panels than CUs) dealt; all that the library's own plan chooses from."""
+    grid = []
+    for p1 in (2, 4):
+        for p2 in range(1, min(4, (m + 63) // 64) + 1):
+            panels = -(-n // (64 * p1)) * -(-m // (64 * p2))
+            grid.append((8, p1, p2, 1))
+            if panels > cus:
+                grid.append((8, p1, p2, 64))
+            else:
+                grid += [(8, p1, p2, sk) for sk in range(2, 33) if panels * sk <= cus and k // 64 // sk >= 2]
+    return grid
+
+
 def scan_gemm(table, shapes, tokens, iters, progress=None, known=(), kernel_ids=None):
     mode, dtype = GEMM_TABLES[table]
     fp8 = mode == "fp8"
@@ -278,6 +293,8 @@ def scan_gemm(table, shapes, tokens, iters, progress=None, known=(), kernel_ids=
                 grid += [(3, rg, w, sk) for rg, w in ((2, 1), (4, 1), (4, 2)) for sk in (1, 2, 4) if (k // 128) // sk >= 2]
                 # kernel 5: the same with only the panels of the last, partial round sliced
                 grid += [(5, rg, w, sk) for rg, w in ((2, 1), (4, 1), (4, 2)) for sk in (2, 3, 4) if (k // 128) // sk >= 2]
+            # kernel 8: the eight-wave panels, which serve every call above 64 tokens that has no row
+            grid += panel_grid(n, m, k)
             for kid, p1, p2, p3 in grid:
                 if (n // 16) % p1 or (kernel_ids is not None and kid not in kernel_ids):
                     continue

@@ -461,3 +461,23 @@ def test_moe_pass_plan_names_what_runs():
         else:
             assert got == decode
     assert lib.mlk_moe_pass_plan(16, 8, 2, 4096, 100, 1, 0, out) != 0
+
+
+def test_scan_grid_holds_what_the_plan_chooses_from():
+    """A scan tries every launch of the eight-wave panels that the library's plan can answer and that the packaged tables hold, so that a
+    scanned row in front of the plan is no slower for want of having been tried."""
+    import ctypes
+    import random
+    from muxi_native_layout_kernels_amd import arg_selector
+    from muxi_native_layout_kernels_amd.kernel_args_scan import scan
+    lib, out, rng, met = _lib.load(), (ctypes.c_int32 * 4)(), random.Random(11), 0
+    for _ in range(300):
+        n, k, m = 128 * rng.randint(1, 250), 128 * rng.randint(1, 140), rng.choice([1, 33, 64, 65, 100, 256, 300, 777, 4096])
+        assert lib.mlk_gemm_plan(m, n, k, rng.choice([0, 2]), out) == 0
+        if out[0] == 8:
+            met += 1
+            assert tuple(out) in scan.panel_grid(n, m, k)
+    assert met > 100
+    for name in ("layout_gemm", "continuous_gemm", "layoutA_gemm", "layoutA_soft_fp8_gemm"):
+        for (n, m, k), args in arg_selector.selector(name).table().items():
+            assert args[0] != 8 or args in scan.panel_grid(n, m, k)
