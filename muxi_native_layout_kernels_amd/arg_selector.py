@@ -201,8 +201,8 @@ def panel_shape(n, m, k, cus=256):
 
 
 def _gemm_default_rowmajor(n, m, k):
-    """Row-major activations and output: above 64 tokens the panel kernel (id 3) takes over (measured ahead of
-    the row-shared kernel from 72 tokens on; panel width left to the library)."""
+    """Row-major activations and output: above 64 tokens the panel kernel (id 3; panel width left to the library).  Asked
+    only where the library has no plan; with activations beyond 32-bit offsets that kernel refuses the call."""
     if m > 64 and k % 128 == 0:
         rg, sk = panel_shape(n, m, k)
         return (3, rg, 4, sk)

@@ -324,19 +324,24 @@ def test_gemm_panel_kernel_id5_off_16_bytes_stays_sliced(mlk):
 
 
 def test_gemm_panel_kernel_is_the_wide_default(mlk):
-    """Above 64 tokens the heuristic for unscanned shapes picks the panel kernel; a K that is no
-    multiple of 128 keeps the row-shared kernel, and the panel kernel refuses it when asked for by id."""
-    from muxi_native_layout_kernels_amd import arg_selector
+    """Above 64 tokens unscanned shapes run the eight-wave panels; the rule of thumb for shapes that the library has no plan for names the
+    older panel kernel, which computes the same, but for a K that is no multiple of 128, which keeps the row-shared kernel and which
+    the panel kernel refuses when asked for by id."""
+    from muxi_native_layout_kernels_amd import arg_selector, ops
     # 4224 rows: a weight shape that no packaged table holds
     assert arg_selector.selector("layoutA_gemm").get_args((4224, 300, 1024))[0] == 3
     assert arg_selector.selector("layoutA_soft_fp8_gemm").get_args((4224, 300, 1024))[0] == 3
     assert arg_selector.selector("layoutA_gemm").get_args((4224, 300, 1088))[0] == 2
     assert arg_selector.selector("layout_gemm").get_args((4224, 304, 1024))[0] == 2       # native operands
     n, k, m = 4224, 1024, 300
+    assert ops._gemm_args("layoutA_gemm", n, m, k, 1)[0] == 8 and ops._gemm_args("layoutA_soft_fp8_gemm", n, m, k, 2)[0] == 8
     w = randn((n, k), torch.bfloat16, 0.02, 98)
     b = randn((m, k), torch.bfloat16, 1.0, 99)
     c = mlk.gemm_layoutA_linear(pack_a(w).cuda(), b.cuda())
     assert_close(c, ogemm.linear_expected(w, b), RTOL, ATOL, "panel default")
+    _, p1, p2, p3 = arg_selector.selector("layoutA_gemm").get_args((n, m, k))
+    c = mlk.gemm_layoutA_wapper(pack_a(w).cuda(), b.cuda(), n, m, k, kernelParam1=p1, kernelParam2=p2, kernelParam3=p3, kernelId=3)
+    assert_close(c, ogemm.linear_expected(w, b), RTOL, ATOL, "kernel 3")
     with pytest.raises(RuntimeError, match="K % 128"):
         mlk.gemm_layoutA_wapper(pack_a(w[:, :960].contiguous()).cuda(), b[:, :960].contiguous().cuda(), n, m, 960,
                                 kernelParam1=1, kernelParam2=1, kernelParam3=1, kernelId=3)
@@ -494,6 +499,20 @@ def test_native_chain_config(mlk):
     assert_close(c2, ogemm.linear_expected(w2, c.cpu()), RTOL, ATOL, "chained")
 
 
+@pytest.mark.parametrize("n,k,kid", [(8704, 512, 1), (9728, 256, 1), (640, 1152, 1)])
+def test_native_chain_planned(mlk, n, k, kid):
+    """Sixteen tokens in layout B on weight shapes that no table holds: launch parameters of a kernel that takes them (the first of these shapes
+    has kernel 4 with row-major activations), both outputs."""
+    from muxi_native_layout_kernels_amd import ops
+    m = 16
+    w, x = randn((n, k), torch.bfloat16, k ** -0.5, 23), randn((m, k), torch.bfloat16, 1.0, 24)
+    assert ops._gemm_args("layout_gemm", n, m, k, 1, 1)[0] == kid
+    a, xb = pack_a(w).cuda(), mlk.layoutB(x.cuda())
+    c = mlk.gemm_layoutAB_ContinuousC(a, xb)
+    assert_close(c, ogemm.linear_expected(w, x), RTOL, ATOL, "planned")
+    assert torch.equal(mlk.reLayoutC(mlk.gemm_layoutABC(a, xb)), c)
+
+
 @pytest.mark.parametrize("m", [1, 4, 16, 33])
 @pytest.mark.parametrize("scaled", [False, True])
 def test_gemm_soft_fp8(mlk, m, scaled):
@@ -572,14 +591,19 @@ def test_gemm_repeated_calls_take_the_launch_plan_and_keep_the_checks(mlk):
 
 @pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8"])
 @pytest.mark.parametrize("p1,p2", [(p1, p2) for p1 in (2, 4) for p2 in (1, 2, 3, 4)])
-@pytest.mark.parametrize("n,m,k,p3", [
-    (128, 1, 128, 1),           # the smallest call: one panel, four slabs
-    (272, 65, 384, 1),          # rows that end inside a panel, a token tile of one token
-    (400, 130, 640, 3),         # ten k windows in three slices
-    (528, 257, 1152, 64),       # k windows dealt to as many workgroups: runs that end inside a panel
-    (1040, 192, 2048, 16),      # two windows per slice
+@pytest.mark.parametrize("n,m,k,p3,native", [
+    (128, 1, 128, 1, False),           # the smallest call: one panel, four slabs
+    (272, 65, 384, 1, False),          # rows that end inside a panel, a token tile of one token
+    (400, 130, 640, 3, False),         # ten k windows in three slices
+    (528, 257, 1152, 64, False),       # k windows dealt to as many workgroups: runs that end inside a panel
+    (1040, 192, 2048, 16, False),      # two windows per slice
+    (416, 80, 384, 1, True),           # the same remainders in native layouts: whole,
+    (544, 272, 1152, 64, True),        # dealt,
+    (416, 144, 640, 3, True),          # sliced, the last token tile narrower than the others
+    (1056, 192, 2048, 16, True),
+    (160, 48, 512, 4, True),           # slots of 48 tokens
 ])
-def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3):
+def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3, native):
     """kernelId 8 in every panel shape: remainders of rows, tokens and k, whole, sliced and dealt; row-major operands against the
     oracle, layout-B activations and layout-C output against the row-major run, whose sums have the same order."""
     dtype = torch.float16 if kind == "fp16" else torch.bfloat16
@@ -597,22 +621,33 @@ def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3):
     a = pack_a(w).cuda()
     c = mlk.gemm_layoutA_wapper(a, x.cuda(), n, m, k, **kw)
     assert_close(c, ogemm.linear_expected(w, x, 0.5, bias), RTOL, ATOL, "panels")
-    if m % 16 == 0 and n % 32 == 0:
+    if native:
         xb = mlk.layoutB(x.cuda())
-        assert torch.equal(bits(mlk.gemm_layoutAB_ContinuousC_wapper(a, xb, n, m, k, **kw)), bits(c))
-        assert torch.equal(bits(mlk.reLayoutC(mlk.gemm_layoutABC_wapper(a, xb, n, m, k, **kw))), bits(c))
+        assert torch.equal(mlk.gemm_layoutAB_ContinuousC_wapper(a, xb, n, m, k, **kw), c)
+        assert torch.equal(mlk.reLayoutC(mlk.gemm_layoutABC_wapper(a, xb, n, m, k, **kw)), c)
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
 @pytest.mark.parametrize("n,m,k,p1,p2", [(4352, 4100, 256, 4, 4), (2304, 1984, 256, 2, 1), (8448, 1000, 128, 2, 2)])
-def test_gemm_eight_wave_panels_several_rounds(mlk, n, m, k, p1, p2):
+def test_gemm_eight_wave_panels_several_rounds(mlk, kind, n, m, k, p1, p2):
     """More panels than CUs: the bands' order of the panels, and the panels left over after whole rounds dealt or sliced."""
     g = torch.Generator(device="cuda").manual_seed(35)
-    w = (torch.randn((n, k), generator=g, device="cuda") * k ** -0.5).to(torch.bfloat16)
+    w = torch.randn((n, k), generator=g, device="cuda") * k ** -0.5
     x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
-    a = mlk.pack_layout_a(w)
-    want = (x.float() @ w.float().t()).double().cpu().numpy()
+    kw = dict(kernelParam1=p1, kernelParam2=p2, kernelId=8)
+    if kind == "fp8":
+        codes = (w * 256).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        # powers of two: the widened weight is the bf16 that the reference multiplies
+        scale = torch.exp2(torch.randint(-9, -6, (n // 128, k // 128), generator=g, device="cuda").float())
+        a, w = mlk.pack_layout_a(codes.view(torch.uint8)), codes.float() * scale.repeat_interleave(128, 0).repeat_interleave(128, 1)
+    else:
+        a, w = mlk.pack_layout_a(w.to(torch.bfloat16)), w.to(torch.bfloat16).float()
+    want = (x.float() @ w.t()).double().cpu().numpy()
     for p3 in (1, 2, 64):
-        c = mlk.gemm_layoutA_wapper(a, x, n, m, k, kernelParam1=p1, kernelParam2=p2, kernelParam3=p3, kernelId=8)
+        if kind == "fp8":
+            c = mlk.gemm_layoutA_soft_fp8_wapper(a, scale, x, n, m, k, kernelParam3=p3, **kw)
+        else:
+            c = mlk.gemm_layoutA_wapper(a, x, n, m, k, kernelParam3=p3, **kw)
         assert_close(c, want, RTOL, ATOL, "several rounds, p3 = %d" % p3)
 
 

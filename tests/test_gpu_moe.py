@@ -891,3 +891,24 @@ def test_wide_kernels_share_out_items_through_queues(mlk, picks, kind):
         out.append(y)
     assert torch.equal(out[0], out[1])
     assert_close(out[0], want.cpu().numpy(), RTOL, ATOL, picks)
+    if picks != "skewed":
+        return
+    # from a graph, with eager calls on the same scratch in between: every replay clears the queues for itself
+    s, y = torch.cuda.Stream(), torch.empty_like(x)
+    s.wait_stream(torch.cuda.current_stream())
+
+    def call():
+        _lib.check(lib.mlk_fused_experts_compute(ptr(w1p), ptr(w2p), ptr(x), T, E, K, H, I, 2 if kind == "fp8" else 1, 1, ptr(ids),
+                                                 ptr(wts), ptr(emap), ptr(s1), ptr(s2), ptr(y), ptr(ws), size, _stream()), "moe")
+    with torch.cuda.stream(s):
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            call()
+        for _ in range(3):
+            for run in (graph.replay, call):
+                y.zero_()
+                run()
+                torch.cuda.synchronize()
+                assert torch.equal(y, out[0])
