@@ -80,7 +80,11 @@ __device__ __forceinline__ int wide_next(int32_t *queue, int n, int x, int ticke
     }
 }
 // The kernel's arguments (MoeArgs come first) and the place in the workgroup, taken afresh for every item: what the compiler works out
-// from them in front of the loop over items is spilled there (soft-FP8 gate/up: 17 vector registers).
+// from them in front of the loop over items is spilled there (soft-FP8 gate/up: 17 vector registers).  A kernel that calls this takes
+// MoeArgs as its first argument: first_is_moe_args() is asserted where it is launched.
+template <class... Rest>
+constexpr bool first_is_moe_args(void (*)(MoeArgs, Rest...)) { return true; }
+constexpr bool first_is_moe_args(...) { return false; }
 __device__ __forceinline__ const MoeArgs &wide_args(int &lane, int &wave) {
     auto at = __builtin_amdgcn_kernarg_segment_ptr();
     int tid = threadIdx.x;
@@ -315,6 +319,8 @@ int launch_moe_wide(const MoeArgs &a, int max_tasks, float *obuf, int skd, hipSt
     static bool ready_up[2][64] = {}, ready_down[2][64] = {};
     const int items_up = (a.I >> 7) * max_tasks, items_down = ((a.H + 255) >> 8) * skd * max_tasks;
     const bool queue_up = wide_queue_pays(a, items_up, a.H >> 5), queue_down = wide_queue_pays(a, items_down, (a.I >> 5) / skd);
+    static_assert(first_is_moe_args(moe_gate_up_queue_kernel<T, FP8>) && first_is_moe_args(moe_down_queue_kernel<T, FP8>),
+                  "wide_args() reads MoeArgs where the kernel's arguments begin");
     const auto up = queue_up ? &moe_gate_up_queue_kernel<T, FP8> : &moe_gate_up_wide_kernel<T, FP8>;
     const auto down = queue_down ? &moe_down_queue_kernel<T, FP8> : &moe_down_wide_kernel<T, FP8>;
     int rc = panel_lds_attribute(up, lds_up, ready_up[queue_up]);
