@@ -1,11 +1,13 @@
-// Kernel id 3: panel GeMM for more than 64 tokens over layout-A weights (row-major activations and
-// output), where the product is bound by the matrix cores and no longer by the weight stream.
+// Kernel ids 3 and 5: panel GeMM for more than 64 tokens over layout-A weights (row-major activations and
+// output), where the product is bound by the matrix cores and no longer by the weight stream; and the launch plan and entry of kernel
+// id 8 (mlk_panel8_gemm.cuh), which serves calls that name no launch parameters.  Calls and table rows that ask for ids 3 and 5 run
+// here, and operands off 16 bytes above 64 tokens (gemm_plan_off16).
 //
 // A workgroup of four waves computes a panel of 256 weight rows x 128 tokens over one of SK slices
 // of K with v_mfma_f32_32x32x16 (one wave per SIMD issues the 16x16x32 form at little more than half
 // rate; the 32x32 form runs at nine tenths of peak from a single wave).  Every wave owns four row
 // groups (two pairs of 32 rows) and all four blocks of 32 tokens: eight 32x32 accumulators.  Two other
-// shapes exist: 256 rows x 256 tokens (sixteen accumulators, k windows of 64 instead of 128) when that
+// shapes exist: 256 rows x 256 tokens (the eight-wave panels of mlk_panel8_gemm.cuh) when that
 // makes fewer rounds of one workgroup per CU, and 128 rows x 128 tokens (one pair of row groups per
 // wave) while panels are too few to give every CU one.
 //
@@ -97,7 +99,7 @@ __global__ void __launch_bounds__(256, 1) gemm_panel_kernel(PanelArgs p) {
     for (int pr = 0; pr < PR; ++pr) srows[pr] = srow;          // the row groups of a wave lie in one 128-row block
     PanelLoop<T, FP8, TB, PR>::run(acc, abase, srows, p.B, boff, wbeg, nwin, win);
 
-    panel_finish<T, PR, TB, kTileWaves, TB>(p, acc, rg0, tok0, SK, sk, rt, tt, wave, lane, &s_last);
+    panel_finish<T, PR, TB, TB>(p, acc, rg0, tok0, SK, sk, rt, tt, wave, lane, &s_last);
 }
 
 // 256 x 128 panels on the loop of mlk_panel_lds.cuh (four waves, LDS as the prefetch buffer; soft-FP8: two workgroups
@@ -149,7 +151,7 @@ __global__ void __launch_bounds__(256, 2) gemm_panel_lds_kernel(PanelArgs p) {
             for (int e = 0; e < 16; ++e) acc[pr][tb][e] = 0.f;
     PanelLoopLds<T, FP8, TB, RING>::run(acc, abase, srows, p.B, row_off, 4 * wbeg, 4 * nwin, win);
     __syncthreads();                                           // the ring is given up: its first word takes the fold's flag
-    panel_finish<T, PR, TB, kTileWaves, 2>(p, acc, rg0, tok0, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
+    panel_finish<T, PR, TB, 2>(p, acc, rg0, tok0, SK, sk, rt, tt, wave, lane, reinterpret_cast<int *>(win));
 }
 
 extern template int launch_panel8<BF16, false>(const Panel8Args &, int, int, hipStream_t);
@@ -459,8 +461,8 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     // is CUs / 8 workgroups of one XCD, and the fullest XCD counts.
     // 11008 x 4096 fp16 at 2100 tokens (nine tiles): 374 us in two slices, 199 us whole; bf16 at 3300 tokens 495 and 286 us;
     // soft-FP8 28672 x 8192 at 1100 tokens 739 us in three slices, 499 us whole; but soft-FP8 4608 x 7168 at 800 tokens (35
-    // panels of 128 x 128 on half of the XCDs) 132 us in four slices, 161 us whole.  Over the 294 grids of this kind that the
-    // shipped tables lead to, at their fewest, middle and most tokens, twice, the choice is within 7 % of the better one, and within
+    // panels of 128 x 128 on half of the XCDs) 132 us in four slices, 161 us whole.  Over 294 grids of this kind (weight
+    // shapes of the tables, 65 to 4096 tokens), each at three token counts, twice, the choice is within 7 % of the better one, and within
     // 3 % on all but 11 of 1764 (rounds counted over the whole chip and a panel's time taken as rows times tokens: up to 53 %).
     // Operands off 16 bytes stay sliced where the whole panels run the loop that loads straight into LDS and the sliced ones do not.
     const bool whole_loads_lds = a_kind == MLK_FP8_E4M3 && width == 128 && rows == 256;

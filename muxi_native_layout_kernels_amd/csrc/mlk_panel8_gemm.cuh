@@ -78,8 +78,8 @@ __device__ __forceinline__ size_t native_c_offset(int n, int tok, int m) {
 
 // What happens to the accumulators of a panel: scaled and stored, or (K slices) handed over as fp32 partials that the
 // last workgroup to arrive adds in slice order.  acc[pr][tb] covers the row groups rg0 + 2 pr, + 1 and the 32 tokens from
-// tok0 + 32 tb on; NWAVES waves per workgroup, each with PR x TB accumulators; the fold fetches FB accumulators at a time.
-template <class T, int PR, int TB, int NWAVES, int FB>
+// tok0 + 32 tb on; kTileWaves waves per workgroup, each with PR x TB accumulators; the fold fetches FB accumulators at a time.
+template <class T, int PR, int TB, int FB>
 __device__ __forceinline__ void panel_finish(const PanelArgs &p, f32x16 (&acc)[PR][TB], int rg0, int tok0, int SK, int sk,
                                              int rt, int tt, int wave, int lane, int *s_last) {
     const int groups = p.N >> 4;
@@ -111,7 +111,7 @@ __device__ __forceinline__ void panel_finish(const PanelArgs &p, f32x16 (&acc)[P
     const int tiles = (p.row_tiles - p.whole_groups * 8) * p.token_tiles;
     // 64-lane group of quad jj of this wave in slice s (two planes of 8-byte halves, see st_agent_planar)
     auto group_at = [&](int s, int jj) -> f32x4 * {
-        return p.partial + ((((size_t)s * tiles + tile) * NWAVES + wave) * (PR * TB * 4) + jj) * 64;
+        return p.partial + ((((size_t)s * tiles + tile) * kTileWaves + wave) * (PR * TB * 4) + jj) * 64;
     };
     // partials travel as agent-scope (write-through / always-miss) accesses, like in the narrow kernels; a release /
     // acquire fence pair around ordinary stores was measured slower (it writes back and invalidates a whole L2)
@@ -132,10 +132,8 @@ __device__ __forceinline__ void panel_finish(const PanelArgs &p, f32x16 (&acc)[P
     if (!*s_last) return;
     // slice order; the loads of the next slice are in flight while the current one is added (a round trip to
     // memory per slice would otherwise be paid in full: these loads bypass the caches).  FB accumulators are fetched,
-    // added and stored at a time (all of a row pair's where the registers allow it), in registers of their own: the
-    // published accumulators are dead, and summing into them kept all of them alive to the end, at 256 registers and a
-    // hundred spilled ones in the eight-wave kernels (now 234 and none: 4096 x 11008 at 1024 tokens in four slices, fp16 134 ->
-    // 108 us, bf16 131 -> 105 us; 8192 x 8192 fp16 at 512 tokens in two 148 -> 122 us).
+    // added and stored at a time, in registers of their own: the published accumulators are dead, and summing into them would
+    // keep all of them alive to the end.
     static_assert(TB % FB == 0, "fetch groups are whole accumulators of one row pair");
 #pragma unroll
     for (int pr = 0; pr < PR; ++pr) {
