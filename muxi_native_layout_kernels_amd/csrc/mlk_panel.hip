@@ -420,7 +420,8 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     // the loops that fetch straight into LDS take operands on 16 bytes, and panels of 256 tokens store 16 bytes at a time; others
     // run panels of 128 tokens that fetch through registers
     const bool loads_on16 = aligned16(a) && aligned16(b);
-    if (width == 256 && !(loads_on16 && aligned16(c) && aligned16(partial))) width = 128;
+    const bool narrowed = width == 256 && !(loads_on16 && aligned16(c) && aligned16(partial));
+    if (narrowed) width = 128;
     p.token_tiles = (m + width - 1) / width;
     MLK_REQUIRE(k % 128 == 0, "gemm: the panel kernel needs K % 128 == 0");
     MLK_REQUIRE((long long)m * k < (1ll << 31), "gemm: the panel kernel indexes activations with 32 bits");
@@ -449,6 +450,8 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
         }
         if (p.whole_groups == groups) p.whole_groups = 0, p.SK = sk = 1;    // nothing left over
     }
+    // twice as many panels as the call asked for may be more than have a counter
+    if (narrowed && (size_t)p.row_tiles * p.token_tiles * sizeof(int) > counter_bytes) p.whole_groups = 0, p.SK = sk = 1;
     if (sk > 1) {
         MLK_REQUIRE(partial != nullptr && counters != nullptr, "gemm: a K split across workgroups needs a workspace");
         MLK_REQUIRE((size_t)p.row_tiles * p.token_tiles * sizeof(int) <= counter_bytes,

@@ -481,3 +481,19 @@ def test_scan_grid_holds_what_the_plan_chooses_from():
     for name in ("layout_gemm", "continuous_gemm", "layoutA_gemm", "layoutA_soft_fp8_gemm"):
         for (n, m, k), args in arg_selector.selector(name).table().items():
             assert args[0] != 8 or args in scan.panel_grid(n, m, k)
+
+
+def test_panels_off_16_bytes_have_a_counter_each_or_run_whole():
+    """Kernel ids 3 and 5 asked for 256 x 256 panels in K slices with operands off 16 bytes run twice as many panels of 128 tokens: where those are
+    more than there are counters for, the call runs whole panels and is not refused (here it gets as far as the launch, which has no GPU)."""
+    import torch
+    from muxi_native_layout_kernels_amd import _lib
+    if torch.cuda.is_available():
+        pytest.skip("the operands are addresses of nothing")
+    lib = _lib.load()
+    n, m, k, at = 131072, 8192, 256, 1 << 40                  # 512 x 32 panels of 256 x 256: as many as there are counters
+    size = lib.mlk_gemm_workspace_bytes(m, n, 4, 2)
+    for kid in (3, 5):
+        for shift in (0, 2):
+            rc = lib.mlk_gemm_layout_a(at, at + shift, at, m, n, k, 1, 1, 0, 0, 1.0, None, None, kid, 4, 2, 2, at, size, None)
+            assert rc != 0 and b"counter region" not in lib.mlk_last_error() and b"workspace" not in lib.mlk_last_error()
