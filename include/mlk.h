@@ -204,7 +204,7 @@ int mlk_gemv_layout_a(const void *a, const void *x, void *y, int m, int n, int k
  *   p1 = row groups per wave (1, 2, 4 or 8; 8 means 4 when more than 16 tokens meet a native B or C);
  *   p3 = K splits across workgroups (>= 1; > 1 needs
  *   `workspace`).
- * workspace: device scratch of at least mlk_gemm_workspace_bytes() bytes, only
+ * workspace: device scratch of at least mlk_gemm_workspace_bytes() bytes (kernel id 8 above 64 tokens: mlk_gemm_panel_workspace_bytes()), only
  * read and written inside the call (contents need not be preserved, but the
  * first `mlk_gemm_counter_bytes()` bytes must be zero before the first call and
  * are left zero by every call).  May be NULL when p3 == 1. */
@@ -228,7 +228,8 @@ size_t mlk_gemm_counter_bytes(void);
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the
  * reference.  Same arguments, kernels and results as mlk_gemm_layout_a; the scratch of a K split across
  * workgroups (p3 > 1) lives in a device array built into the library, mlk_gemm_noalloc_scratch_bytes() =
- * 16 MiB per GPU, held until the process ends.  A call whose mlk_gemm_workspace_bytes(m, n, p1, p3) exceeds
+ * 16 MiB per GPU, held until the process ends.  A call whose mlk_gemm_workspace_bytes(m, n, p1, p3) (kernel id 8:
+ * mlk_gemm_panel_workspace_bytes()) exceeds
  * that returns MLK_ERR_WORKSPACE and launches nothing.  The call allocates and frees nothing.  All calls on
  * one GPU share the array: calls that may overlap (different streams, or graphs replayed side by side) race;
  * order them on one stream.  The first call on a GPU looks up the array's address; nothing is cleared: the

@@ -212,8 +212,10 @@ size_t panel_partial_bytes(int m, int n, int sk) {
 
 // Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
 // rounds).  Fitted to the times of all shapes of this kernel on 24 weight shapes (512 to 32000 rows, K 640 to 18944) at 19 token counts from
-// 20 to 3000, bf16 and soft-FP8: the shape it picks is 1.8 % (soft-FP8 1.1 %) slower than the best one in the geometric mean, 11 % (7 %) at the
-// 95th percentile, of which the greater part is scatter of the single measurements.
+// 20 to 3000, bf16 and soft-FP8.  On 950 other products of 65 to 4096 tokens the launch it picks is 1.8 % (soft-FP8 1.2 %) slower than the best one in
+// the geometric mean, 11 % (8 %) at the 95th percentile.  What it does not know: 16-bit panels of 192 and 256 tokens are slower where all token tiles have one length
+// (bf16 4096 x 7936 in panels of 256 x 256: 174 us at 2048 tokens, 141 us at 2049; likely because they walk in step and ask for the same weights at the
+// same time, which a shorter last tile, running ahead, has fetched for the others; 22016 x 4096 at 368 tokens 89 us in the panels of 192 tokens that it picks, 74 us in those of 256).
 struct P8Cost {
     // up to one panel per CU: start, store (256 x 256), fold = fold + fold_slice per slice + fold_mb per MB of slots; a k32 slab of a panel
     // on an idle chip, what a workgroup on every CU adds to it, and the share of that which weights shared by token tiles keep
