@@ -2,9 +2,11 @@
 """Benchmark of the native-layout hot path on one MI355X.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--quick] [--case TEXT] [--no-cpu] [--case-steps S]
-                    [--no-eager] [--no-blas] [--counters]
+                    [--no-eager] [--no-blas] [--counters] [--details FILE]
 
-Prints ONE JSON line.  The headline workload is the fp16 narrow GeMM of the
+Prints ONE JSON line on stdout, short enough to be read whole from a log that keeps the last 8 KB: of the other
+configurations the time, the fraction of the bound, the vendor BLAS and the CPU baseline.  The same line with everything that was
+measured goes to stderr, and to a file with --details.  The headline workload is the fp16 narrow GeMM of the
 second benchmark configuration (`gemm_layoutA`, weights 11008 x 4096 in
 layout-A, 16 tokens); one step is one call.  Inputs are synthetic, seeded and
 resident in HBM before the timed region.  Every call of a timed region reads a
@@ -90,6 +92,7 @@ def main():
                          "crashed the profiler), no settle replays, --steps calls per case after --warmup calls, no "
                          "yardsticks, no vendor BLAS, no CPU legs, no eager-call lines; the headline runs only if "
                          "--case names it; timings of such a run are not benchmark numbers")
+    ap.add_argument("--details", metavar="FILE", help="write the JSON line with every measured number to this file too")
     ap.add_argument("--no-eager", action="store_true", help="skip the eager-call lines (public Python API, wall clock)")
     ap.add_argument("--tunable", action="append", default=[], metavar="ID=VALUE",
                     help="set an experiment switch of the library (mlk_set_tunable) before anything runs; repeatable")
@@ -782,7 +785,29 @@ def main():
         "eager_calls": eager,
         "per_config": per_config,
     }
-    print(json.dumps(line))
+    full = json.dumps(line)
+    print(full, file=sys.stderr)
+    if args.details:
+        with open(args.details, "w") as f:
+            f.write(full + "\n")
+    line["per_config"] = [brief(row) for row in per_config]
+    line["eager_calls"] = [{k: row[k] for k in ("name", "eager_us", "graph_us", "host_us_per_call") if row.get(k) is not None}
+                           for row in eager]
+    print(json.dumps(line, separators=(",", ":")), flush=True)
+
+
+def brief(row):
+    """A per_config row on the short line: microseconds, the fraction of its bound, and what else was timed for it."""
+    out = {"name": row["name"], "us": round(row["us"], 2)}
+    for key in ("frac", "mfma_frac"):
+        if row.get(key) is not None:
+            out[key] = round(row[key], 3)
+    if row.get("blas_us") is not None:
+        out["blas_us"] = round(row["blas_us"], 1)
+    base = row.get("cpu_baseline")
+    if base and base.get("us_scaled_to_full") is not None:
+        out["cpu_us"] = round(base["us_scaled_to_full"])
+    return out
 
 
 if __name__ == "__main__":
