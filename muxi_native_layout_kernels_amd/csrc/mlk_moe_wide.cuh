@@ -110,11 +110,17 @@ __device__ __forceinline__ int moe_gate_up_wide(const MoeArgs &p, const MoeTask 
     const int pair = FP8 ? Loop::pair(wave) : Loop::tile(wave, 0) >> 1;
     const int half = pair & 1, rg = (pair >> 1) * 2;
     const uint32_t tile0 = (uint32_t)(half * groups_i + rg) * tile_row;
-    ScaleRow srow;
+    // block scales: of the half that the wave multiplies, or of the gate rows and the up rows
+    constexpr int NS = Panel8<T, FP8, TB, 2>::SMALL ? 1 : 2;
+    ScaleRow srow[NS];
     if constexpr (FP8) {
         src.a_off[0] = tile0 + (lane >> 5 ? tile_row : 0u) + (lane & 31) * 16;
-        const int cols = p.H >> 7, block = (half * groups_i + rt * 8 + rg) >> 3;
-        srow = load_scale_row(p.S1 ? p.S1 + ((size_t)tk.expert * (2 * p.I >> 7) + block) * cols : nullptr, cols, lane);
+        const int cols = p.H >> 7;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const int block = ((NS == 2 ? i : half) * groups_i + rt * 8) >> 3;
+            srow[i] = load_scale_row(p.S1 ? p.S1 + ((size_t)tk.expert * (2 * p.I >> 7) + block) * cols : nullptr, cols, lane);
+        }
     } else {
         src.a_off[0] = tile0;
         src.a_off[1] = tile0 + tile_row;
@@ -126,26 +132,22 @@ __device__ __forceinline__ int moe_gate_up_wide(const MoeArgs &p, const MoeTask 
         const int id = slot < slots ? sorted[slot] : p.n_pairs;
         return id < p.n_pairs ? id / p.K : 0;
     });
-    f32x16 acc[2][TB];
+    typename Loop::Acc acc;
     Loop::run(acc, src, srow, 0, p.H >> 5, wave, lane);
     __syncthreads();
     const int ticket = QUEUE && wave == 0 ? wide_ticket(p.queues, blockIdx.x & 7, lane) : 0;      // of the next item
 
-    // accumulator element 4 g + e of lane 32 h + c: column 8 g + 4 h + e of the wave's 32, token c of the block's 32
+    // the first half of the wave's rows: gate, the second: up, of its 32 columns
     uint8_t *out = reinterpret_cast<uint8_t *>(win);
-    const int h4 = lane >> 5, c32 = lane & 31;
+    acc.each_half(lane, [&](int col, int token, f32x4 gate, f32x4 up) {
+        float h[4];
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = silu_mul(acc[0][tb][4 * g + e], acc[1][tb][4 * g + e]);
-            u32x2 o;
-            o[0] = T::from_f32x2(h[0], h[1]);
-            o[1] = T::from_f32x2(h[2], h[3]);
-            *reinterpret_cast<u32x2 *>(out + ((wt * TB + tb) * 32 + c32) * kWideOutPitch + wr * 64 + g * 16 + h4 * 8) = o;
-        }
+        for (int e = 0; e < 4; ++e) h[e] = silu_mul(gate[e], up[e]);
+        u32x2 o;
+        o[0] = T::from_f32x2(h[0], h[1]);
+        o[1] = T::from_f32x2(h[2], h[3]);
+        *reinterpret_cast<u32x2 *>(out + (wt * TB * 32 + token) * kWideOutPitch + wr * 64 + col * 2) = o;
+    });
     __syncthreads();
     // sixteen lanes store the 256 bytes of a slot; slots without a routed pair are stored too (nobody reads them)
     const int tid = wave * 64 + lane, q = tid & 15;
@@ -212,11 +214,12 @@ __device__ __forceinline__ int moe_down_wide(const MoeArgs &p, float *__restrict
     // rows past H: a copy of the last row group, never stored
     const int tile = FP8 ? 2 * Loop::pair(wave) : Loop::tile(wave, 0);
     const int rga = min(rgp + tile, groups - 1), rgb = min(rgp + tile + 1, groups - 1);
-    ScaleRow srow;
+    ScaleRow srow[1];
     if constexpr (FP8) {
         src.a_off[0] = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * tile_row + (lane & 31) * 16;
         const int cols = p.I >> 7;
-        srow = load_scale_row(p.S2 ? p.S2 + ((size_t)tk.expert * (p.H >> 7) + (rga >> 3)) * cols : nullptr, cols, lane);
+        const int rgs = min(rgp + Loop::scale_tile(wave), groups - 1);
+        srow[0] = load_scale_row(p.S2 ? p.S2 + ((size_t)tk.expert * (p.H >> 7) + (rgs >> 3)) * cols : nullptr, cols, lane);
     } else {
         src.a_off[0] = (uint32_t)(rga - rgp) * tile_row;
         src.a_off[1] = (uint32_t)(rgb - rgp) * tile_row;
@@ -225,7 +228,7 @@ __device__ __forceinline__ int moe_down_wide(const MoeArgs &p, float *__restrict
     p8_token_rows<Loop>(src, (uint32_t)p.I * 2u, wave, lane, [&](int slot) { return slot < slots ? slot : 0; });
     const int nwin = p.I >> 7;                                     // K slices are cut at multiples of 128 k
     const int wbeg = (int)((long long)sk * nwin / skd), wend = (int)((long long)(sk + 1) * nwin / skd);
-    f32x16 acc[2][TB];
+    typename Loop::Acc acc;
     Loop::run(acc, src, srow, 4 * wbeg, 4 * (wend - wbeg), wave, lane);
     __syncthreads();
     const int ticket = QUEUE && wave == 0 ? wide_ticket(p.queues + 8 * kWideQueueStep, blockIdx.x & 7, lane) : 0;  // of the next item
@@ -233,18 +236,15 @@ __device__ __forceinline__ int moe_down_wide(const MoeArgs &p, float *__restrict
     // every wave turns its 32 rows x 32 TB tokens around in its own part of LDS, one row pair after the other, and stores
     // 128 bytes of a routed pair with eight lanes
     uint8_t *out = reinterpret_cast<uint8_t *>(win) + (size_t)wave * 128 * kWideDownPitch;
-    const int h4 = lane >> 5, c32 = lane & 31, t8 = lane >> 3, q = lane & 7;
+    const int t8 = lane >> 3, q = lane & 7;
     const int n0 = (rgp + wr * 4) * 16;
     if (n0 >= p.H) return ticket;
     const int32_t *sorted = p.sorted + tk.block0 * 16;
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<f32x4 *>(out + (tb * 32 + c32) * kWideDownPitch + g * 32 + h4 * 16) =
-                    f32x4{acc[pr][tb][4 * g], acc[pr][tb][4 * g + 1], acc[pr][tb][4 * g + 2], acc[pr][tb][4 * g + 3]};
+        acc.each(lane, [&](int row, int token, f32x4 v) {
+            if (row >> 5 == pr) *reinterpret_cast<f32x4 *>(out + token * kWideDownPitch + (row & 31) * 4) = v;
+        });
         wave_lds_sync();
 #pragma unroll 4
         for (int it = 0; it < 4 * TB; ++it) {

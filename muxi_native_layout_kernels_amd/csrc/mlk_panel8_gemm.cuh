@@ -65,10 +65,10 @@ __device__ __forceinline__ bool p8_panel(const Panel8Args &p, int line, int u, i
     return rt < p.row_tiles;
 }
 
-// Where accumulator quad g of a lane (rows 8 g + 4 (lane / 32) .. + 3 of row pair `pair` of the panel, token block + lane % 32) lies in
-// a panel's sums of `cols` tokens.  A block of 32 tokens is one run per row pair, 1 KiB per quad; the last block may have 16 tokens.
-__device__ __forceinline__ int p8_slot_quad(int cols, int pair, int block, int width, int g, int lane) {
-    return (pair * cols + block) * 8 + (2 * g + (lane >> 5)) * width + (lane & 31);
+// Where the four sums of rows 4 quad .. + 3 (quad < 8) of row pair `pair` of the panel and token block + t lie in
+// a panel's sums of `cols` tokens.  A block of 32 tokens is one run per row pair; the last block may have 16 tokens.
+__device__ __forceinline__ int p8_slot_quad(int cols, int pair, int block, int width, int quad, int t) {
+    return (pair * cols + block) * 8 + quad * width + t;
 }
 
 // Element offset of 8 rows n .. n + 7 (n % 8 == 0) of token tok in a layout-C output of m tokens.
@@ -184,31 +184,23 @@ constexpr size_t p8_lds_bytes() {
     const size_t ring = p8_ring_bytes<FP8, PR, TB>(), out = (size_t)8 * 32 * TB * p8_out_pitch(PR);
     return ring > out ? ring : out;
 }
-template <class T, int PR, int TB>
-__device__ __forceinline__ void p8_store_panel(const Panel8Args &p, f32x16 (&acc)[PR][TB], int rg0, int tok0, int wave, int lane,
+template <class T, int PR, int TB, class Acc>
+__device__ __forceinline__ void p8_store_panel(const Panel8Args &p, const Acc &acc, int rg0, int tok0, int wave, int lane,
                                                u32x4 *win) {
     constexpr int PITCH = p8_out_pitch(PR);
     uint8_t *buf = reinterpret_cast<uint8_t *>(win) + (size_t)wave * 32 * TB * PITCH;
-    const int half = lane >> 5, c32 = lane & 31;
     const int n0 = rg0 * 16;                                   // first of the wave's 32 PR rows
+    acc.each(lane, [&](int row, int token, f32x4 v) {
+        float bias[4] = {0.f, 0.f, 0.f, 0.f};
+        if (p.bias && n0 + row < p.N) {
 #pragma unroll
-    for (int pr = 0; pr < PR; ++pr)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int row = pr * 32 + 8 * g + 4 * half;        // of the wave's rows
-            float bias[4] = {0.f, 0.f, 0.f, 0.f};
-            if (p.bias && n0 + row < p.N) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) bias[i] = T::to_f32(p.bias[n0 + row + i]);
-            }
-#pragma unroll
-            for (int tb = 0; tb < TB; ++tb) {
-                u32x2 o;
-                o[0] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g] + bias[0], p.alpha * acc[pr][tb][4 * g + 1] + bias[1]);
-                o[1] = T::from_f32x2(p.alpha * acc[pr][tb][4 * g + 2] + bias[2], p.alpha * acc[pr][tb][4 * g + 3] + bias[3]);
-                *reinterpret_cast<u32x2 *>(buf + (tb * 32 + c32) * PITCH + row * 2) = o;
-            }
+            for (int e = 0; e < 4; ++e) bias[e] = T::to_f32(p.bias[n0 + row + e]);
         }
+        u32x2 o;
+        o[0] = T::from_f32x2(p.alpha * v[0] + bias[0], p.alpha * v[1] + bias[1]);
+        o[1] = T::from_f32x2(p.alpha * v[2] + bias[2], p.alpha * v[3] + bias[3]);
+        *reinterpret_cast<u32x2 *>(buf + token * PITCH + row * 2) = o;
+    });
     if (p.c_native) {
         // lane 16 q + t: octet q of token t of each block of 16 tokens x 32 rows
         const int t16 = lane & 15, q = lane >> 4;
@@ -249,7 +241,11 @@ __device__ __forceinline__ void gemm_panel8(const Panel8Args &p, int rt, int tt,
     extern __shared__ u32x4 win[];
     constexpr int WBYTES = FP8 ? 1 : 2;
     using Loop = typename Panel8<T, FP8, TB, PR>::Loop;
-    const int tid = threadIdx.x, lane = tid & 63;
+    // taken afresh for every run: what the compiler works out from it in front of the loop over runs is spilled there (soft-FP8 256 x 256:
+    // 20 vector registers)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 3, wt = wave >> 2;
     const int groups = p.N >> 4;
@@ -262,13 +258,14 @@ __device__ __forceinline__ void gemm_panel8(const Panel8Args &p, int rt, int tt,
     P8Src src;
     src.a = p.A + (size_t)rgp * p.K * 16 * WBYTES;
     src.b = p.B;
-    ScaleRow srow;
+    ScaleRow srow[1];
     if constexpr (FP8) {
         const int t0 = 2 * Loop::pair(wave);
         const int rga = min(rgp + t0, groups - 1), rgb = min(rgp + t0 + 1, groups - 1);
         src.a_off[0] = (uint32_t)((lane >> 5 ? rgb : rga) - rgp) * (uint32_t)p.K * 16u + (lane & 31) * 16;
         const int scale_cols = (p.K + 127) >> 7;
-        srow = load_scale_row(p.scale ? p.scale + (size_t)(rga >> 3) * scale_cols : nullptr, scale_cols, lane);
+        const int rgs = min(rgp + Loop::scale_tile(wave), groups - 1);
+        srow[0] = load_scale_row(p.scale ? p.scale + (size_t)(rgs >> 3) * scale_cols : nullptr, scale_cols, lane);
     } else {
 #pragma unroll
         for (int i = 0; i < PR; ++i)
@@ -277,7 +274,7 @@ __device__ __forceinline__ void gemm_panel8(const Panel8Args &p, int rt, int tt,
     auto token_of = [&](int slot) { return min(tok0 + slot, p.M - 1); };
     if (p.b_native) p8_token_native<Loop>(src, p.M, wave, lane, token_of);
     else p8_token_rows<Loop>(src, (uint32_t)p.K * 2u, wave, lane, token_of);
-    f32x16 acc[PR][TB];
+    typename Loop::Acc acc;
     Loop::run(acc, src, srow, slab0, nslab, wave, lane);
     if (slot == nullptr) {
         __syncthreads();
@@ -285,17 +282,10 @@ __device__ __forceinline__ void gemm_panel8(const Panel8Args &p, int rt, int tt,
         return;
     }
     const int cols = min(p.cols, 64 * TB);
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb) {
-        const int block = (wt * TB + tb) * 32, width = min(32, cols - block);
-        if ((lane & 31) >= width) continue;
-#pragma unroll
-        for (int pr = 0; pr < PR; ++pr)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                slot[p8_slot_quad(cols, wr * PR + pr, block, width, g, lane)] =
-                    f32x4{acc[pr][tb][4 * g], acc[pr][tb][4 * g + 1], acc[pr][tb][4 * g + 2], acc[pr][tb][4 * g + 3]};
-    }
+    acc.each(lane, [&](int row, int token, f32x4 v) {
+        const int block = (wt * TB + (token >> 5)) * 32, width = min(32, cols - block);
+        if ((token & 31) < width) slot[p8_slot_quad(cols, wr * PR + (row >> 5), block, width, (row & 31) >> 2, token & 31)] = v;
+    });
 }
 
 // Token columns / 64 that token tile tt multiplies: the last tile those that cover it (28672 x 4096 bf16 at 700 tokens 196 ->
@@ -364,7 +354,7 @@ __global__ void __launch_bounds__(256) gemm_panel8_fold_kernel(Panel8Args p, int
     if (j0 == j1) return;                                      // one workgroup computed and stored it
     const bool j0_starts = (int)((long long)j0 * total / p.deal) == first;
     const size_t slot_quads = (size_t)32 * pr_n * p.cols;
-    const int quad = p8_slot_quad(cols, (wave & 3) * pr_n + pr, block, width, gp, lane);
+    const int quad = p8_slot_quad(cols, (wave & 3) * pr_n + pr, block, width, 2 * gp + (lane >> 5), lane & 31);
     auto at = [&](int j) {
         return p.partial + ((size_t)(line * p.deal + j) * p.slots + (j == j0 && !j0_starts)) * slot_quads + quad;
     };

@@ -627,6 +627,30 @@ def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3, native):
         assert torch.equal(mlk.reLayoutC(mlk.gemm_layoutABC_wapper(a, xb, n, m, k, **kw)), c)
 
 
+@pytest.mark.parametrize("kind", ["fp16", "fp8"])
+@pytest.mark.parametrize("p1,p2", [(p1, p2) for p1 in (2, 4) for p2 in (1, 2, 3, 4)])
+@pytest.mark.parametrize("k,p3", [(128, 2), (256, 1), (384, 2), (640, 1), (768, 5), (896, 1), (1152, 1), (1664, 3), (1920, 1)])
+def test_gemm_eight_wave_rings(mlk, kind, p1, p2, k, p3):
+    """kernelId 8 on full panels: K, and slices of it, shorter than the rings of every shape (one to six pairs of k32 slabs), as long, and
+    longer by every remainder.  The weights of neighbouring slabs differ in scale, so that a slab multiplied twice or by its
+    neighbour's tokens shows; whole numbers, so that sums of up to 2^24 have one value in any order."""
+    n, m = 64 * p1, 64 * p2
+    g = torch.Generator().manual_seed(36)
+    x = torch.randint(-3, 4, (m, k), generator=g).to(torch.float16 if kind == "fp16" else torch.bfloat16)
+    w = torch.randint(-2, 3, (n, k), generator=g) * (1 + torch.arange(k) // 32 % 3)
+    want = x.double() @ w.double().t()
+    kw = dict(kernelParam1=p1, kernelParam2=p2, kernelParam3=p3, kernelId=8)
+    if kind == "fp8":
+        # one scale per 128 x 128 block, powers of two: widened exactly
+        scale = torch.exp2(torch.randint(-2, 3, ((n + 127) // 128, k // 128), generator=g).float())
+        want = x.double() @ (w * scale.repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)).double().t()
+        a = pack_a(w.float().to(torch.float8_e4m3fn).view(torch.uint8)).cuda()
+        c = mlk.gemm_layoutA_soft_fp8_wapper(a, scale.cuda(), x.cuda(), n, m, k, **kw)
+    else:
+        c = mlk.gemm_layoutA_wapper(pack_a(w.to(x.dtype)).cuda(), x.cuda(), n, m, k, **kw)
+    assert torch.equal(c.cpu(), want.float().to(x.dtype))
+
+
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 @pytest.mark.parametrize("n,m,k,p1,p2", [(4352, 4100, 256, 4, 4), (2304, 1984, 256, 2, 1), (8448, 1000, 128, 2, 2)])
 def test_gemm_eight_wave_panels_several_rounds(mlk, kind, n, m, k, p1, p2):
