@@ -40,6 +40,7 @@ struct P8Src {
     const uint16_t *b;     // base of the token rows
     uint32_t b_off[4];     // per-lane byte offsets of this lane's 16 bytes of the wave's chunks at k = 0
     uint32_t b_step;       // bytes from one pair of slabs to the next: of a token row, or of all tokens in layout B
+    bool b_runs;           // layout B
 };
 
 // The sums of a wave, its 32 PR rows x 32 TB tokens, as its loop leaves them.  each(lane, f): f(row, token, the sums of rows row .. row + 3),
@@ -91,7 +92,9 @@ struct P8Acc32 {
 };
 
 // Tokens of two slabs: chunks of 8 tokens x 64 k (128 bytes of a token row, a whole line), TB per wave.  Lane 8 r + j of a chunk's load
-// fetches octet j ^ t of token t = r ^ (chunk & 1), so that the operand reads of 16 tokens meet 16 different bank groups.
+// fetches octet j ^ t of token t = r ^ (chunk & 1), so that the operand reads of 16 tokens meet 16 different bank groups.  Activations in
+// layout B lie as operands already: a chunk is one run of 1 KiB, 16 tokens of one slab, block j of slab e chunk 2 j + e.  (What a CU
+// pulls out of L2: 125 GB/s in runs of 1 KiB, 78 GB/s of loads that gather two pieces or more.)
 template <int TB>
 struct P8TokenPairs {
     static constexpr int NB = TB, B_PAIR = 512 * TB;                    // granules of a pair of slabs
@@ -99,15 +102,18 @@ struct P8TokenPairs {
     __device__ static __forceinline__ int token_in_chunk(int wave, int i, int lane) { return (lane >> 3) ^ (chunk(wave, i) & 1); }
     __device__ static __forceinline__ int token(int wave, int i, int lane) { return chunk(wave, i) * 8 + token_in_chunk(wave, i, lane); }
     __device__ static __forceinline__ int octet(int wave, int i, int lane) { return (lane & 7) ^ token_in_chunk(wave, i, lane); }
-    // granule of token lane % 16 of a block of 16 tokens, octet lane / 16 of the first slab; the second is at ^ 4, block j at + 128 j
-    __device__ static __forceinline__ int operand16(int lane) {
+    // Granules of a wave's operands; block j of 16 tokens is at + 128 j.
+    // 16x16x32: token lane % 16, octet lane / 16 of slab e.
+    __device__ static __forceinline__ int operand16(const P8Src &src, int e, int lane) {
+        if (src.b_runs) return 64 * e + lane;
         const int t = lane & 7, c = (lane >> 3) & 1;
-        return c * 64 + (t ^ c) * 8 + ((lane >> 4) ^ t);
+        return c * 64 + (t ^ c) * 8 + (((lane >> 4) + 4 * e) ^ t);
     }
-    // granule of token lane % 32 of a block of 32 tokens, octet lane / 32; octet 2 h + lane / 32 is at ^ (2 h), block tb at + 256 tb
-    __device__ static __forceinline__ int operand32(int lane) {
+    // 32x32x16: token lane % 32 of a block of 32, octet 2 h + lane / 32 of the pair
+    __device__ static __forceinline__ int operand32(const P8Src &src, int h, int lane) {
         const int i = lane & 31, t = i & 7, c = i >> 3;
-        return c * 64 + (t ^ (c & 1)) * 8 + ((lane >> 5) ^ t);
+        if (src.b_runs) return (c >> 1) * 128 + 32 * h + (lane >> 5) * 16 + (i & 15);
+        return c * 64 + (t ^ (c & 1)) * 8 + ((2 * h + (lane >> 5)) ^ t);
     }
     __device__ static __forceinline__ void issue1(const P8Src &src, int wave, u32x4 *dst, int pair, int i) {
         __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)src.b, 0, 0xffffffffu, 0x00020000);
@@ -173,14 +179,14 @@ struct Panel8Loop16 : P8TokenPairs<TB> {
                                                int wave, int lane) {
         extern __shared__ u32x4 win[];
         const int wr = wave & 3, wt = wave >> 2;
-        const int a_idx = wr * RT * 64 + lane, b_idx = B_AT + Tok::operand16(lane) + wt * TT * 128;
+        const int a_idx = wr * RT * 64 + lane, b_idx[2] = {B_AT + Tok::operand16(src, 0, lane) + wt * TT * 128, B_AT + Tok::operand16(src, 1, lane) + wt * TT * 128};
         struct Frags {
             u32x4 a[RT], b[TT];
         } f0, f1;
         // read r of a slab: its row tiles first
         auto rd = [&](Frags &f, int abuf, int bbuf, int odd, int r) {
             if (r < RT) f.a[r] = win[abuf * A_SLAB + a_idx + r * 64];
-            else f.b[r - RT] = win[bbuf * Tok::B_PAIR + (b_idx ^ (4 * odd)) + (r - RT) * 128];
+            else f.b[r - RT] = win[bbuf * Tok::B_PAIR + b_idx[odd] + (r - RT) * 128];
         };
         constexpr int NR = RT + TT, NM = RT * TT, SIZE = NM % 8 ? 4 : 8, BLOCKS = NM / SIZE;
         // slabs past the end are fetched as copies of the last one and never multiplied, which keeps the count of loads in flight
@@ -287,12 +293,12 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
         extern __shared__ u32x4 win[];
         const int wr = wave & 3, wt = wave >> 2;
         const int a_idx = wr * RT * 64 + lane;                     // 8-byte units; row tile i + 64 i, second slab + 512 PR
-        const int b_idx = RAW_PAIR + Tok::operand16(lane) + wt * TT * 128;
+        const int b_idx[2] = {RAW_PAIR + Tok::operand16(src, 0, lane) + wt * TT * 128, RAW_PAIR + Tok::operand16(src, 1, lane) + wt * TT * 128};
         u32x4 a[2][RT], b[2][TT];
         u32x2 raw[RT];
         float sc[NS];
         auto rd_raw = [&](int buf, int odd, int i) { raw[i] = reinterpret_cast<const u32x2 *>(win + buf * SLOT)[a_idx + odd * 512 * PR + i * 64]; };
-        auto rd_b = [&](u32x4 (&f)[TT], int buf, int odd, int j) { f[j] = win[buf * SLOT + (b_idx ^ (4 * odd)) + j * 128]; };
+        auto rd_b = [&](u32x4 (&f)[TT], int buf, int odd, int j) { f[j] = win[buf * SLOT + b_idx[odd] + j * 128]; };
         auto widen = [&](u32x4 &o, int i) {
             const float s = sc[NS == 2 ? i / PR : 0];
             uint32_t x0, x1, x2, x3;

@@ -53,8 +53,9 @@ struct Panel8SmallFp8 : P8TokenPairs<TB> {
         extern __shared__ u32x4 win[];
         const int half = wave >> 2;
         const int a_idx = ((lane >> 4) & 1) * 64 + (lane >> 5) * 16 + (lane & 15);    // 8-byte units; second k16 step + 32, second slab + 128
-        const int b_idx = RAW_PAIR + Tok::operand32(lane);
-        const int b_flip = PR == 1 ? 4 * half : 0;                                    // PR = 1: the slab of the pair that is this wave's
+        int b_idx[NH];                                                                // PR = 1: of the slab of the pair that is this wave's
+#pragma unroll
+        for (int h = 0; h < NH; ++h) b_idx[h] = RAW_PAIR + Tok::operand32(src, (PR == 1 ? 2 * half : 0) + h, lane);
         u32x2 raw[2];                                                                 // tiles of the next two steps
         u32x4 op[2], b[2][TB2];
         f32x16 sum[TB2];
@@ -67,7 +68,7 @@ struct Panel8SmallFp8 : P8TokenPairs<TB> {
         };
         auto rd_b = [&](u32x4 (&f)[TB2], int buf, int h) {
 #pragma unroll
-            for (int tb = 0; tb < TB2; ++tb) f[tb] = win[buf * SLOT + (b_idx ^ (b_flip + 2 * h)) + 256 * tb];
+            for (int tb = 0; tb < TB2; ++tb) f[tb] = win[buf * SLOT + b_idx[h] + 256 * tb];
         };
         auto widen = [&](u32x4 &o, const u32x2 &r, float sc) {
             uint32_t x0, x1, x2, x3;
@@ -171,6 +172,7 @@ constexpr size_t p8_ring_bytes() {
 template <class Loop, class TokenOf>
 __device__ __forceinline__ void p8_token_rows(P8Src &src, uint32_t row_bytes, int wave, int lane, TokenOf token_of) {
     src.b_step = 128;
+    src.b_runs = false;
 #pragma unroll
     for (int i = 0; i < Loop::NB; ++i)
         src.b_off[i] = (uint32_t)token_of(Loop::token(wave, i, lane)) * row_bytes + Loop::octet(wave, i, lane) * 16;
@@ -179,10 +181,11 @@ __device__ __forceinline__ void p8_token_rows(P8Src &src, uint32_t row_bytes, in
 template <class Loop, class TokenOf>
 __device__ __forceinline__ void p8_token_native(P8Src &src, int m, int wave, int lane, TokenOf token_of) {
     src.b_step = (uint32_t)m * 128u;
+    src.b_runs = true;
 #pragma unroll
     for (int i = 0; i < Loop::NB; ++i) {
-        const uint32_t tok = token_of(Loop::token(wave, i, lane)), oct = Loop::octet(wave, i, lane);
-        src.b_off[i] = (oct >> 2) * ((uint32_t)m * 64u) + (tok >> 4) * 1024u + (oct & 3) * 256u + (tok & 15) * 16u;
+        const int chunk = Loop::chunk(wave, i);
+        src.b_off[i] = (uint32_t)(chunk & 1) * ((uint32_t)m * 64u) + ((uint32_t)token_of((chunk >> 1) * 16) >> 4) * 1024u + lane * 16u;
     }
 }
 
