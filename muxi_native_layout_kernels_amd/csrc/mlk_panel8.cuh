@@ -72,6 +72,14 @@ struct P8Acc16 {
 template <int PR, int TB>
 struct P8Acc32 {
     f32x16 acc[PR][TB];                                        // v_mfma_f32_32x32x16: row pairs, blocks of 32 tokens
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int pr = 0; pr < PR; ++pr)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[pr][tb][e] = 0.f;
+    }
     __device__ static __forceinline__ f32x4 quad(const f32x16 &v, int g) { return f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}; }
     template <class F>
     __device__ __forceinline__ void each(int lane, F f) const {
@@ -286,19 +294,31 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
     }
 
     // As Panel8Loop16::run; srow[0]: block scales of the wave's rows, srow[1] (NS = 2): of its second half of row tiles
-    using Acc = P8Acc16<PR, TB>;
+    // 256 rows: the 32 x 32 form, which leaves the vector unit more issue slots for the widening (11008 x 4096 at 512 tokens 89 -> 76 us,
+    // 28672 x 8192 at 1024 454 -> 431, 8192 x 8192 at 4096, where power counts, 445 -> 449).  128 rows, half as many weights a product: the
+    // 16 x 16 form (8192 x 8192 at 2048 tokens 275 -> 246).
+    static constexpr bool M32 = PR == 2;
+    using Acc = std::conditional_t<M32, P8Acc32<PR, TB>, P8Acc16<PR, TB>>;
     template <int NS>
     __device__ static __forceinline__ void run(Acc &out, const P8Src &src, const ScaleRow (&srow)[NS], int slab0, int nslab,
                                                int wave, int lane) {
         extern __shared__ u32x4 win[];
         const int wr = wave & 3, wt = wave >> 2;
-        const int a_idx = wr * RT * 64 + lane;                     // 8-byte units; row tile i + 64 i, second slab + 512 PR
-        const int b_idx[2] = {RAW_PAIR + Tok::operand16(src, 0, lane) + wt * TT * 128, RAW_PAIR + Tok::operand16(src, 1, lane) + wt * TT * 128};
+        // operands of a slab: row tiles and blocks of 16 tokens, or (M32) those of row pair or block of 32 i / 2, k16 step i % 2
+        const int a_idx = wr * RT * 64 + (M32 ? ((lane >> 4) & 1) * 64 + (lane >> 5) * 16 + (lane & 15) : lane);    // 8-byte units; second slab + 512 PR
+        int b_idx[M32 ? 4 : 2];
+#pragma unroll
+        for (int h = 0; h < (M32 ? 4 : 2); ++h)
+            b_idx[h] = RAW_PAIR + (M32 ? Tok::operand32(src, h, lane) : Tok::operand16(src, h, lane)) + wt * TT * 128;
         u32x4 a[2][RT], b[2][TT];
         u32x2 raw[RT];
         float sc[NS];
-        auto rd_raw = [&](int buf, int odd, int i) { raw[i] = reinterpret_cast<const u32x2 *>(win + buf * SLOT)[a_idx + odd * 512 * PR + i * 64]; };
-        auto rd_b = [&](u32x4 (&f)[TT], int buf, int odd, int j) { f[j] = win[buf * SLOT + b_idx[odd] + j * 128]; };
+        auto rd_raw = [&](int buf, int odd, int i) {
+            raw[i] = reinterpret_cast<const u32x2 *>(win + buf * SLOT)[a_idx + odd * 512 * PR + (M32 ? (i >> 1) * 128 + (i & 1) * 32 : i * 64)];
+        };
+        auto rd_b = [&](u32x4 (&f)[TT], int buf, int odd, int j) {
+            f[j] = win[buf * SLOT + (M32 ? b_idx[2 * odd + (j & 1)] + (j >> 1) * 256 : b_idx[odd] + j * 128)];
+        };
         auto widen = [&](u32x4 &o, int i) {
             const float s = sc[NS == 2 ? i / PR : 0];
             uint32_t x0, x1, x2, x3;
@@ -314,7 +334,15 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
         // pairs past the end are fetched as copies of the last one and never multiplied
         auto issue_a = [&](int p, int buf, int i) { issue_a1(src, wave, min(pair0 + p, last), buf, i); };
         auto issue_b = [&](int p, int buf, int i) { Tok::issue1(src, wave, win + buf * SLOT + RAW_PAIR, min(pair0 + p, last), i); };
-        constexpr int NM = RT * TT, BLOCKS = NM / 8;
+        constexpr int NM = M32 ? 2 * PR * TB : RT * TT, SIZE = M32 ? 4 : 8, BLOCKS = NM / SIZE;
+        auto product = [&](const u32x4 (&x)[RT], const u32x4 (&y)[TT], int m) {
+            if constexpr (M32) {
+                const int hs = m / (PR * TB), pr = m / TB % PR, tb = m % TB;
+                out.acc[pr][tb] = T::mfma32(x[2 * pr + hs], y[2 * tb + hs], out.acc[pr][tb]);
+            } else {
+                out.acc[m / TT][m % TT] = T::mfma(x[m / TT], y[m % TT], out.acc[m / TT][m % TT]);
+            }
+        };
 #pragma unroll
         for (int p = 0; p < RP; ++p) {
 #pragma unroll
@@ -323,7 +351,6 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
             for (int i = 0; i < PR; ++i)
                 if (p < RP - 1) issue_a(p, p, i);
         }
-        auto &acc = out.acc;
         out.zero();
         wait_vmcnt_le<(RP - 1) * TB + (RP - 2) * PR>();            // pair 0
         bare_barrier();
@@ -340,7 +367,7 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
             const int nxt = cur == RP - 1 ? 0 : cur + 1, prv = cur == 0 ? RP - 1 : cur - 1;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                // block blk multiplies its eight products, reads part of the next slab's operands and widens the tiles read before it
+                // block blk multiplies, reads part of the next slab's operands and widens the tiles read before it
                 if (h == 1) scales(p + 1);
                 const int buf = h ? nxt : cur;
 #pragma unroll
@@ -348,7 +375,7 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
 #pragma unroll
                 for (int blk = 0; blk < BLOCKS; ++blk) {
 #pragma unroll
-                    for (int m = blk * 8; m < blk * 8 + 8; ++m) acc[m / TT][m % TT] = T::mfma(a[h][m / TT], b[h][m % TT], acc[m / TT][m % TT]);
+                    for (int m = blk * SIZE; m < (blk + 1) * SIZE; ++m) product(a[h], b[h], m);
 #pragma unroll
                     for (int i = 0; i < RT; ++i)
                         if (i * BLOCKS / RT == blk) widen(a[1 - h][i], i);
@@ -365,7 +392,7 @@ struct Panel8LoopFp8 : P8TokenPairs<TB> {
                             if ((i * BLOCKS + BLOCKS / 2) / TB == blk) issue_b(p + RP, cur, i);
                     }
                 }
-                p8_spread_slab<BLOCKS, 8, (RT + TT + BLOCKS - 1) / BLOCKS, (18 * RT + NM - 1) / NM>();
+                p8_spread_slab<BLOCKS, SIZE, (RT + TT + BLOCKS - 1) / BLOCKS, (18 * RT + NM - 1) / NM>();
                 __builtin_amdgcn_sched_barrier(0);
                 if (h == 0) {
                     wait_vmcnt_le<(RP - 2) * (TB + PR)>();         // this wave's loads of pair p + 1 have landed
