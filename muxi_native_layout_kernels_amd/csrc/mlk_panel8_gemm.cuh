@@ -38,6 +38,7 @@ struct Panel8Args {
     int row_tiles, token_tiles;
     int cols;            // tokens of a slot: 64 tb, or the call's tokens in blocks of 16 where one token tile holds them all (32 to 48
                          // tokens in slices are then no larger than the narrow kernels' partial sums)
+    bool rows_first;     // one line: the row tiles of a token tile are neighbours, else the token tiles of a row tile
     int band, chunk;     // groups of eight row tiles and token tiles that neighbouring workgroups of an XCD cover
     int panels;          // of the longest line
     int whole, deal;     // of one line
@@ -60,8 +61,9 @@ __device__ __forceinline__ bool p8_panel(const Panel8Args &p, int line, int u, i
         rt = (band * RB + w / tc) * 8 + line;
         return rt < p.row_tiles;
     }
-    rt = u / p.token_tiles;
-    tt = u - rt * p.token_tiles;
+    const int inner = p.rows_first ? p.row_tiles : p.token_tiles, a = u / inner, b = u - a * inner;
+    rt = p.rows_first ? b : a;
+    tt = p.rows_first ? a : b;
     return rt < p.row_tiles;
 }
 

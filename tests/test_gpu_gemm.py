@@ -651,6 +651,34 @@ def test_gemm_eight_wave_rings(mlk, kind, p1, p2, k, p3):
     assert torch.equal(c.cpu(), want.float().to(x.dtype))
 
 
+@pytest.mark.parametrize("kind,native", [("bf16", False), ("bf16", True), ("fp8", False)])
+@pytest.mark.parametrize("n,m,k,p1,p2,p3", [
+    (384, 1008, 256, 2, 2, 1),         # three row tiles, eight token tiles, the last one short
+    (1040, 1600, 384, 2, 4, 2),        # nine row tiles, the last one ragged, in slices
+    (400, 2064, 256, 4, 1, 3),         # two row tiles, 33 token tiles, more slices than windows of some
+    (640, 1504, 640, 2, 3, 1),
+    (640, 144, 640, 2, 3, 1),          # one token tile: either order
+    (128, 1040, 128, 2, 1, 2),         # one row tile
+])
+def test_gemm_eight_wave_row_tiles_first(mlk, kind, native, n, m, k, p1, p2, p3):
+    """One line of panels with more activations than weights: the row tiles of a token tile side by side.  Whole numbers, one value in
+    any order of the sums."""
+    g = torch.Generator().manual_seed(37)
+    x = torch.randint(-3, 4, (m, k), generator=g).to(torch.bfloat16)
+    w = torch.randint(-2, 3, (n, k), generator=g)
+    want = (x.double() @ w.double().t()).float().to(x.dtype)
+    kw = dict(kernelParam1=p1, kernelParam2=p2, kernelParam3=p3, kernelId=8)
+    if kind == "fp8":
+        scale = torch.ones((n + 127) // 128, k // 128)
+        a = pack_a(w.float().to(torch.float8_e4m3fn).view(torch.uint8)).cuda()
+        c = mlk.gemm_layoutA_soft_fp8_wapper(a, scale.cuda(), x.cuda(), n, m, k, **kw)
+    elif native:
+        c = mlk.gemm_layoutAB_ContinuousC_wapper(pack_a(w.to(x.dtype)).cuda(), mlk.layoutB(x.cuda()), n, m, k, **kw)
+    else:
+        c = mlk.gemm_layoutA_wapper(pack_a(w.to(x.dtype)).cuda(), x.cuda(), n, m, k, **kw)
+    assert torch.equal(c.cpu(), want)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 @pytest.mark.parametrize("n,m,k,p1,p2", [(4352, 4100, 256, 4, 4), (2304, 1984, 256, 2, 1), (8448, 1000, 128, 2, 2)])
 def test_gemm_eight_wave_panels_several_rounds(mlk, kind, n, m, k, p1, p2):
