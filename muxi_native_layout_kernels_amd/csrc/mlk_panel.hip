@@ -211,28 +211,40 @@ size_t panel_partial_bytes(int m, int n, int sk) {
 }
 
 // Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
-// rounds).  Fitted to the times of all shapes of this kernel on 24 weight shapes (512 to 32000 rows, K 640 to 18944) at 19 token counts from
-// 20 to 3000, bf16 and soft-FP8.  On 950 other products of 65 to 4096 tokens the launch it picks is 1.8 % (soft-FP8 1.2 %) slower than the best one in
-// the geometric mean, 11 % (8 %) at the 95th percentile.  What it does not know: 16-bit panels of 192 and 256 tokens are slower where all token tiles have one length
-// (bf16 4096 x 7936 in panels of 256 x 256: 174 us at 2048 tokens, 141 us at 2049; likely because they walk in step and ask for the same weights at the
-// same time, which a shorter last tile, running ahead, has fetched for the others; 22016 x 4096 at 368 tokens 89 us in the panels of 192 tokens that it picks, 74 us in those of 256).
+// rounds).  Fitted to the times of 2300 products (512 to 37888 rows, K 512 to 18432, 65 to 4096 tokens; bf16 and soft-FP8, up to the 18 likeliest
+// launches of each), to the times and to how much slower than the best the launch is that it picks.  On as many other products that is 1.8 %
+// (soft-FP8 1.0 %) in the geometric mean, 9.5 % (6.4 %) at the 95th percentile; with the constants of the kernels before these 2.6 % (2.4 %).
+// What it does not know: panels of one row tile are faster where one token tile is shorter than the others, which runs ahead and fetches
+// their weights (11008 x 4096 at 300 tokens in panels of 128 x 192: 192 and 108 tokens 44.0 us, 160 and 140 45.6); and a last round of few
+// panels (11008 x 4096 at 1302 tokens, 258 panels: dealt 114 us, whole 156).
 struct P8Cost {
     // up to one panel per CU: start, store (256 x 256), fold = fold + fold_slice per slice + fold_mb per MB of slots; a k32 slab of a panel
-    // on an idle chip, what a workgroup on every CU adds to it, and the share of that which weights shared by token tiles keep
+    // on an idle chip, what a workgroup on every CU adds to it, and the power of the token tiles that share weights by which that falls
     float start, store, fold, fold_slice, fold_mb, shared, slab[2][4], busy[2][4];
     // several rounds: start, end of a round (256 x 256), what a last round that is not full saves of its empty part, fold, per MB; a slab
     float r_start, r_end, r_empty, r_fold, r_fold_mb, r_slab[2][4];
 };
-static const P8Cost kP8Cost16 = {3.6f, 3.0f, 2.65f, 0.09f, 0.215f, 0.32f,
-                                 {{0.105f, 0.178f, 0.257f, 0.341f}, {0.171f, 0.299f, 0.362f, 0.503f}},
-                                 {{0.222f, 0.223f, 0.210f, 0.229f}, {0.487f, 0.401f, 0.470f, 0.548f}},
-                                 4.5f, 7.2f, 0.47f, 3.6f, 0.244f,
-                                 {{0.207f, 0.290f, 0.398f, 0.498f}, {0.315f, 0.476f, 0.649f, 0.808f}}};
-static const P8Cost kP8Cost8 = {5.3f, 2.8f, 3.0f, 0.1f, 0.197f, 0.68f,
-                                {{0.113f, 0.162f, 0.229f, 0.390f}, {0.196f, 0.257f, 0.531f, 0.462f}},
-                                {{0.096f, 0.136f, 0.152f, 0.152f}, {0.172f, 0.274f, 0.192f, 0.438f}},
-                                5.8f, 8.7f, 0.47f, 4.6f, 0.197f,
-                                {{0.192f, 0.281f, 0.381f, 0.564f}, {0.322f, 0.471f, 0.730f, 0.844f}}};
+static const P8Cost kP8Cost16 = {3.88f, 3.48f, 2.04f, 0.187f, 0.265f, 0.41f,
+                                 {{0.113f, 0.222f, 0.241f, 0.326f}, {0.146f, 0.250f, 0.341f, 0.437f}},
+                                 {{0.151f, 0.087f, 0.140f, 0.078f}, {0.405f, 0.326f, 0.327f, 0.313f}},
+                                 3.85f, 6.85f, 0.34f, 2.08f, 0.417f,
+                                 {{0.217f, 0.294f, 0.350f, 0.428f}, {0.322f, 0.426f, 0.527f, 0.640f}}};
+static const P8Cost kP8Cost8 = {5.15f, 4.06f, 2.82f, 0.168f, 0.213f, 0.02f,
+                                {{0.111f, 0.151f, 0.205f, 0.250f}, {0.185f, 0.222f, 0.325f, 0.406f}},
+                                {{0.053f, 0.100f, 0.144f, 0.154f}, {0.128f, 0.238f, 0.288f, 0.292f}},
+                                3.67f, 9.56f, 0.26f, 2.66f, 0.255f,
+                                {{0.201f, 0.269f, 0.366f, 0.427f}, {0.348f, 0.447f, 0.607f, 0.675f}}};
+// Up to 64 tokens, where the panels compete with the narrow kernels and one token tile holds the call: fitted with those.
+static const P8Cost kP8Few16 = {3.6f, 3.0f, 2.65f, 0.09f, 0.215f, 0.f,
+                                {{0.105f, 0.178f, 0.257f, 0.341f}, {0.171f, 0.299f, 0.362f, 0.503f}},
+                                {{0.222f, 0.223f, 0.210f, 0.229f}, {0.487f, 0.401f, 0.470f, 0.548f}},
+                                4.5f, 7.2f, 0.47f, 3.6f, 0.244f,
+                                {{0.207f, 0.290f, 0.398f, 0.498f}, {0.315f, 0.476f, 0.649f, 0.808f}}};
+static const P8Cost kP8Few8 = {5.3f, 2.8f, 3.00f, 0.10f, 0.197f, 0.f,
+                               {{0.113f, 0.162f, 0.229f, 0.390f}, {0.196f, 0.257f, 0.531f, 0.462f}},
+                               {{0.096f, 0.136f, 0.152f, 0.152f}, {0.172f, 0.274f, 0.192f, 0.438f}},
+                               5.8f, 8.7f, 0.47f, 4.6f, 0.197f,
+                               {{0.192f, 0.281f, 0.381f, 0.564f}, {0.322f, 0.471f, 0.730f, 0.844f}}};
 static double panel8_us(const P8Cost &f, int m, int n, int k, int pr, int tb, int sk) {
     const int cus = device_cus(), rows = (n + 128 * pr - 1) / (128 * pr), tokens = (m + 64 * tb - 1) / (64 * tb), windows = k / 64;
     const int narrow = (m - (tokens - 1) * 64 * tb + 63) / 64;                   // columns / 64 of the last token tile
@@ -240,7 +252,7 @@ static double panel8_us(const P8Cost &f, int m, int n, int k, int pr, int tb, in
     if (panels <= cus) {
         const int t = tokens == 1 ? narrow : tb;
         const double wgs = (double)panels * sk, busy = wgs < cus ? wgs / cus : 1;
-        const double slab = f.slab[pr - 1][t - 1] + f.busy[pr - 1][t - 1] * busy * (f.shared + (1 - f.shared) / tokens);
+        const double slab = f.slab[pr - 1][t - 1] + f.busy[pr - 1][t - 1] * busy * pow(tokens, -f.shared);
         double us = f.start + f.store * pr * t / 8 + 2 * ((windows + sk - 1) / sk) * slab;
         if (sk > 1) us += f.fold + f.fold_slice * sk + f.fold_mb * wgs * pr * t * 0.032768;
         return us;
@@ -329,7 +341,7 @@ static bool p8_rows_first(const Panel8Args &p, int m, int n, int k, bool fp8) {
 
 // Launch parameters (kernel id, p1, p2, p3) that are expected to be fastest for m tokens x n rows x k.
 void gemm_plan(int m, int n, int k, bool fp8, bool b_native, int32_t *out) {
-    const P8Cost &f = fp8 ? kP8Cost8 : kP8Cost16;
+    const P8Cost &f = m <= 64 ? (fp8 ? kP8Few8 : kP8Few16) : fp8 ? kP8Cost8 : kP8Cost16;
     double best = 1e30;
     auto offer = [&](double us, int id, int p1, int p2, int p3) {
         if (us < best) best = us, out[0] = id, out[1] = p1, out[2] = p2, out[3] = p3;
