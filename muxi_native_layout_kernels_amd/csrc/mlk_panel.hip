@@ -212,8 +212,8 @@ size_t panel_partial_bytes(int m, int n, int sk) {
 
 // Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
 // rounds).  Fitted to the times of 2300 products (512 to 37888 rows, K 512 to 18432, 65 to 4096 tokens; bf16 and soft-FP8, up to the 18 likeliest
-// launches of each), to the times and to how much slower than the best the launch is that it picks.  On as many other products that is 1.8 %
-// (soft-FP8 1.0 %) in the geometric mean, 9.5 % (6.4 %) at the 95th percentile; with the constants of the kernels before these 2.6 % (2.4 %).
+// launches of each), to the times and to how much slower than the best the launch is that it picks.  On as many other products that is 1.6 %
+// (soft-FP8 1.0 %) in the geometric mean, 8.7 % (6.5 %) at the 95th percentile; with the constants of the kernels before these 2.6 % (2.4 %).
 // What it does not know: panels of one row tile are faster where one token tile is shorter than the others, which runs ahead and fetches
 // their weights (11008 x 4096 at 300 tokens in panels of 128 x 192: 192 and 108 tokens 44.0 us, 160 and 140 45.6); and a last round of few
 // panels (11008 x 4096 at 1302 tokens, 258 panels: dealt 114 us, whole 156).

@@ -100,28 +100,33 @@ struct P8Acc32 {
 };
 
 // Tokens of two slabs: chunks of 8 tokens x 64 k (128 bytes of a token row, a whole line), TB per wave.  Lane 8 r + j of a chunk's load
-// fetches octet j ^ t of token t = r ^ (chunk & 1), so that the operand reads of 16 tokens meet 16 different bank groups.  Activations in
+// fetches octet j ^ x of token t = r ^ (chunk & 1).  A read of 16 bytes per lane is served for lanes 0..3, 12..15 and 20..27 together, then
+// for 4..11, 16..19 and 28..31, and the upper half alike; x is chosen so that those sixteen meet sixteen different bank groups: t for operands of
+// 32 tokens; for operands of 16 (F16), where lanes 16..31 hold the next octet, t ^ 1 for the tokens 4..11 of a block (with t, every read took
+// twice its time: SQ_LDS_BANK_CONFLICT 2.7e7 in 13824 x 5120 at 3000 tokens).  Activations in
 // layout B lie as operands already: a chunk is one run of 1 KiB, 16 tokens of one slab, block j of slab e chunk 2 j + e.  (What a CU
 // pulls out of L2: 125 GB/s in runs of 1 KiB, 78 GB/s of loads that gather two pieces or more.)
-template <int TB>
+template <int TB, bool F16>
 struct P8TokenPairs {
     static constexpr int NB = TB, B_PAIR = 512 * TB;                    // granules of a pair of slabs
+    // x of token t of a chunk c (its parity)
+    __device__ static __forceinline__ int swizzle(int t, int c) { return F16 ? t ^ (((t >> 2) ^ c) & 1) : t; }
     __device__ static __forceinline__ int chunk(int wave, int i) { return wave * TB + i; }
     __device__ static __forceinline__ int token_in_chunk(int wave, int i, int lane) { return (lane >> 3) ^ (chunk(wave, i) & 1); }
     __device__ static __forceinline__ int token(int wave, int i, int lane) { return chunk(wave, i) * 8 + token_in_chunk(wave, i, lane); }
-    __device__ static __forceinline__ int octet(int wave, int i, int lane) { return (lane & 7) ^ token_in_chunk(wave, i, lane); }
+    __device__ static __forceinline__ int octet(int wave, int i, int lane) { return (lane & 7) ^ swizzle(token_in_chunk(wave, i, lane), chunk(wave, i) & 1); }
     // Granules of a wave's operands; block j of 16 tokens is at + 128 j.
     // 16x16x32: token lane % 16, octet lane / 16 of slab e.
     __device__ static __forceinline__ int operand16(const P8Src &src, int e, int lane) {
         if (src.b_runs) return 64 * e + lane;
         const int t = lane & 7, c = (lane >> 3) & 1;
-        return c * 64 + (t ^ c) * 8 + (((lane >> 4) + 4 * e) ^ t);
+        return c * 64 + (t ^ c) * 8 + (((lane >> 4) + 4 * e) ^ swizzle(t, c));
     }
     // 32x32x16: token lane % 32 of a block of 32, octet 2 h + lane / 32 of the pair
     __device__ static __forceinline__ int operand32(const P8Src &src, int h, int lane) {
         const int i = lane & 31, t = i & 7, c = i >> 3;
         if (src.b_runs) return (c >> 1) * 128 + 32 * h + (lane >> 5) * 16 + (i & 15);
-        return c * 64 + (t ^ (c & 1)) * 8 + ((2 * h + (lane >> 5)) ^ t);
+        return c * 64 + (t ^ (c & 1)) * 8 + ((2 * h + (lane >> 5)) ^ swizzle(t, c & 1));
     }
     __device__ static __forceinline__ void issue1(const P8Src &src, int wave, u32x4 *dst, int pair, int i) {
         __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)src.b, 0, 0xffffffffu, 0x00020000);
@@ -158,8 +163,8 @@ __device__ __forceinline__ void p8_spread_slab() {
 // into the buffer of pair p.  One wait and one barrier per slab publish slab s + 2.  The rings are as deep as LDS allows: with three
 // slabs ahead a 128 x 64 panel ran at 0.34 us a slab whatever it multiplied.
 template <class T, int TB, int PR>
-struct Panel8Loop16 : P8TokenPairs<TB> {
-    using Tok = P8TokenPairs<TB>;
+struct Panel8Loop16 : P8TokenPairs<TB, true> {
+    using Tok = P8TokenPairs<TB, true>;
     static constexpr int A_SLAB = 512 * PR, RT = 2 * PR, TT = 2 * TB;       // granules of a slab of weights; row tiles, token blocks of a wave
     static constexpr size_t ring_bytes(int da, int pb) { return (size_t)((da + 1) * A_SLAB + pb * Tok::B_PAIR) * 16; }
     static constexpr int pairs(int pb) { return ring_bytes(2 * pb, pb + 1) <= kP8MostLds && pb < 6 ? pairs(pb + 1) : pb; }
@@ -273,8 +278,8 @@ struct Panel8Loop16 : P8TokenPairs<TB> {
 // Ring of RP pairs of slabs, weights and tokens.  The last reads of pair p happen in slab 2 p; slab 2 p + 1 issues the tokens of pair
 // p + RP into its place and slab 2 p + 2 the weights, so that one wait and one barrier per pair do, at the end of the even slab.
 template <class T, int TB, int PR>
-struct Panel8LoopFp8 : P8TokenPairs<TB> {
-    using Tok = P8TokenPairs<TB>;
+struct Panel8LoopFp8 : P8TokenPairs<TB, PR == 1> {
+    using Tok = P8TokenPairs<TB, PR == 1>;
     static constexpr int RAW_PAIR = 512 * PR, SLOT = RAW_PAIR + Tok::B_PAIR, RT = 2 * PR, TT = 2 * TB;
     static constexpr size_t ring_bytes(int rp) { return (size_t)rp * SLOT * 16; }
     static constexpr int RP = ring_bytes(4) <= kP8MostLds ? 4 : 3;

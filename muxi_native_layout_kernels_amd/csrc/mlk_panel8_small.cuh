@@ -23,8 +23,8 @@ namespace mlk {
 // v_mfma_f32_32x32x16 here: these panels are bound by the issue of vector instructions, and the 16 x 16 form takes twice as many (measured 8 to 10 %
 // slower: 4096 x 14336, 200 tokens in panels of 256 x 128 153 -> 172 us, of 128 x 64 76 -> 83).
 template <class T, int TB, int PR>
-struct Panel8SmallFp8 : P8TokenPairs<TB> {
-    using Tok = P8TokenPairs<TB>;
+struct Panel8SmallFp8 : P8TokenPairs<TB, false> {
+    using Tok = P8TokenPairs<TB, false>;
     static constexpr int RAW_PAIR = 512 * PR, SLOT = RAW_PAIR + Tok::B_PAIR, TB2 = 2 * TB, NH = 2 * PR;     // k16 steps per trip
     static constexpr size_t ring_bytes(int d) { return (size_t)(d + 1) * SLOT * 16; }
     static constexpr int deepest(int d) { return ring_bytes(d + 1) <= kP8MostLds && d < 8 ? deepest(d + 1) : d; }
