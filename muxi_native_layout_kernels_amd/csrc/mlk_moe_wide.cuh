@@ -22,12 +22,11 @@
 // 836 -> 798, soft-FP8 770 -> 710.
 //
 // What bounds it: neither the matrix cores' peak nor memory.  8 experts, top-2, H 4096, I 14336, bf16, 2048 tokens: gate/up 962
-// GFLOP in 935 us (1.03 PFLOP/s), down 481 GFLOP in 555 us (0.87), where the same loop reaches 1.36 PFLOP/s on a dense 8192 x
-// 8192 product of 4096 tokens.  Counted: 6 to 8 % of the products are columns that pad a task; the matrix cores are busy 56 % (down:
-// 44 %) of the cycles, at a clock that power holds at 1.87 (2.0) GHz; a CU holds waves 91 % (81 %: 2.5 rounds of long items) of the
-// time, a wave waits a third of its life, and a workgroup's first slabs and its epilogue have nothing
-// beside them on the CU; the L2s serve 77 % of the requests.  With a workgroup per item, and so equal numbers of items of unequal widths per XCD, a CU
-// held waves 79 % (73 %) of the time and the two took 1066 and 599 us.  fp32 partial products of the down projection are 4 H bytes per
+// GFLOP in about 800 us (1.2 PFLOP/s), down 481 GFLOP in 465 us (1.03), where the same loop reaches 1.46 PFLOP/s on a dense 8192 x
+// 8192 product of 4096 tokens; the layer 1529 -> 1335 us with the 16 x 16 products and whole-line tokens of mlk_panel8.cuh.  Counted: 6 to 8 % of the products are
+// columns that pad a task; the matrix cores are busy 67 % (down: 52 %) of the cycles, at a clock that power holds at 1.87 (2.0) GHz; a CU holds
+// waves 93 % (82 %: 2.5 rounds of long items) of the time, and a workgroup's first slabs and its epilogue have nothing
+// beside them on the CU.  fp32 partial products of the down projection are 4 H bytes per
 // routed pair and slice, written and read once (the sum over them: 26 us).
 #pragma once
 
