@@ -241,7 +241,7 @@ __device__ __forceinline__ int moe_down_wide(const MoeArgs &p, float *__restrict
     const int32_t *sorted = p.sorted + tk.block0 * 16;
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
-        acc.each(lane, [&](int row, int token, f32x4 v) {
+        acc.each(lane, [](int) {}, [&](int row, int token, f32x4 v) {
             if (row >> 5 == pr) *reinterpret_cast<f32x4 *>(out + token * kWideDownPitch + (row & 31) * 4) = v;
         });
         wave_lds_sync();

@@ -43,8 +43,9 @@ struct P8Src {
     bool b_runs;           // layout B
 };
 
-// The sums of a wave, its 32 PR rows x 32 TB tokens, as its loop leaves them.  each(lane, f): f(row, token, the sums of rows row .. row + 3),
-// each_half(lane, f), PR = 2: f(row, token, sums of rows row .. + 3, sums of rows 32 + row .. + 3).
+// The sums of a wave, its 32 PR rows x 32 TB tokens, as its loop leaves them.  each(lane, rows, f): f(row, token, the sums of rows row ..
+// row + 3), and rows(row) once ahead of the tokens of four rows; each_half(lane, f), PR = 2: f(row, token, sums of rows row .. + 3,
+// sums of rows 32 + row .. + 3).
 template <int PR, int TB>
 struct P8Acc16 {
     f32x4 acc[2 * PR][2 * TB];                                 // v_mfma_f32_16x16x32: row tiles, blocks of 16 tokens
@@ -54,12 +55,14 @@ struct P8Acc16 {
 #pragma unroll
             for (int j = 0; j < 2 * TB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    template <class F>
-    __device__ __forceinline__ void each(int lane, F f) const {
+    template <class R, class F>
+    __device__ __forceinline__ void each(int lane, R rows, F f) const {
 #pragma unroll
-        for (int i = 0; i < 2 * PR; ++i)
+        for (int i = 0; i < 2 * PR; ++i) {
+            rows(16 * i + 4 * (lane >> 4));
 #pragma unroll
             for (int j = 0; j < 2 * TB; ++j) f(16 * i + 4 * (lane >> 4), 16 * j + (lane & 15), acc[i][j]);
+        }
     }
     template <class F>
     __device__ __forceinline__ void each_half(int lane, F f) const {
@@ -81,14 +84,16 @@ struct P8Acc32 {
                 for (int e = 0; e < 16; ++e) acc[pr][tb][e] = 0.f;
     }
     __device__ static __forceinline__ f32x4 quad(const f32x16 &v, int g) { return f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}; }
-    template <class F>
-    __device__ __forceinline__ void each(int lane, F f) const {
+    template <class R, class F>
+    __device__ __forceinline__ void each(int lane, R rows, F f) const {
 #pragma unroll
         for (int pr = 0; pr < PR; ++pr)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
+            for (int g = 0; g < 4; ++g) {
+                rows(32 * pr + 8 * g + 4 * (lane >> 5));
 #pragma unroll
                 for (int tb = 0; tb < TB; ++tb) f(32 * pr + 8 * g + 4 * (lane >> 5), 32 * tb + (lane & 31), quad(acc[pr][tb], g));
+            }
     }
     template <class F>
     __device__ __forceinline__ void each_half(int lane, F f) const {
