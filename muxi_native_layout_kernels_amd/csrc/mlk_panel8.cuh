@@ -165,18 +165,23 @@ __device__ __forceinline__ void p8_spread_slab() {
 // 16-bit weights.  Ring of DA + 1 slabs of weights and of PB pairs of slabs of tokens.  While slab s is multiplied, the operands of slab
 // s + 1 are read into a second set of registers.  Slab s issues the loads of the weights of slab s + DA into the buffer that slab s - 1 has
 // left; the last operands of pair p are read during slab 2 p, so slab 2 p + 1 issues, ahead of its weights, the tokens of pair p + PB
-// into the buffer of pair p.  One wait and one barrier per slab publish slab s + 2.  The rings are as deep as LDS allows: with three
-// slabs ahead a 128 x 64 panel ran at 0.34 us a slab whatever it multiplied.
+// into the buffer of pair p.  One wait and one barrier per slab publish slab s + 2.  The rings hold at most three pairs of slabs: what is
+// fetched past the end of K has to land before LDS is given up, which in short products is much of their time, and a deeper ring brings
+// nothing in long ones (panels of 128 x 192, five pairs -> three: 25 products of 5 to 12 us 4 % faster, K 2048 to 8192 level; with two
+// pairs 128 x 64 takes 1.3 times as long).  128 x 64 then needs 80 KB, and two workgroups share a CU: grids of several rounds 1.2 times as fast.
+// With one or two accumulator tiles in each direction a slab has too few products to spread its instructions under: the reads go in front, the loads
+// between the two halves of the products (128 x 64 at K 512 5.9 -> 5.4 us with both changes, 4096 x 4096 at 64 tokens in eight slices 14.8 -> 14.3).
 template <class T, int TB, int PR>
 struct Panel8Loop16 : P8TokenPairs<TB, true> {
     using Tok = P8TokenPairs<TB, true>;
     static constexpr int A_SLAB = 512 * PR, RT = 2 * PR, TT = 2 * TB;       // granules of a slab of weights; row tiles, token blocks of a wave
     static constexpr size_t ring_bytes(int da, int pb) { return (size_t)((da + 1) * A_SLAB + pb * Tok::B_PAIR) * 16; }
-    static constexpr int pairs(int pb) { return ring_bytes(2 * pb, pb + 1) <= kP8MostLds && pb < 6 ? pairs(pb + 1) : pb; }
+    static constexpr int pairs(int pb) { return ring_bytes(2 * pb, pb + 1) <= kP8MostLds && pb < 3 ? pairs(pb + 1) : pb; }
     static constexpr int slabs(int da) { return da > 2 * PB - 2 && ring_bytes(da, PB) > kP8MostLds ? slabs(da - 1) : da; }
     static constexpr int PB = pairs(2), DA = slabs(2 * PB);
     static constexpr size_t lds_bytes = ring_bytes(DA, PB);
     static constexpr int B_AT = (DA + 1) * A_SLAB;
+    static constexpr bool FEW = PR * TB <= 2;
     static_assert(lds_bytes <= kP8MostLds && DA >= 3 && DA >= 2 * PB - 2 && DA <= 2 * PB, "the rings have to fit, the waits below to hold");
 
     __device__ static __forceinline__ int tile(int wave, int i) { return PR * wave + i; }
@@ -244,19 +249,33 @@ struct Panel8Loop16 : P8TokenPairs<TB, true> {
                 if (H && l < TB) issue_b(s - 1 + 2 * PB, bcur, l);
                 else issue_a(s + DA, aprv, l - H * TB);
             };
+            auto product = [&](int m) { acc[m / TT][m % TT] = T::mfma(now.a[m / TT], now.b[m % TT], acc[m / TT][m % TT]); };
+            auto read = [&](int r) { rd(next, anxt, H ? bnxt : bcur, 1 - H, r); };
+            if constexpr (FEW) {
 #pragma unroll
-            for (int blk = 0; blk < BLOCKS; ++blk) {
+                for (int m = 0; m < NM; ++m) product(m);
 #pragma unroll
-                for (int m = blk * SIZE; m < (blk + 1) * SIZE; ++m)
-                    acc[m / TT][m % TT] = T::mfma(now.a[m / TT], now.b[m % TT], acc[m / TT][m % TT]);
+                for (int r = 0; r < NR; ++r) read(r);
 #pragma unroll
-                for (int r = 0; r < NR; ++r)
-                    if (r * BLOCKS / NR == blk) rd(next, anxt, H ? bnxt : bcur, 1 - H, r);
+                for (int l = 0; l < NL; ++l) load(l);
+                __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);                                   // LDS reads
+                __builtin_amdgcn_sched_group_barrier(0x008, NM / 2, 0);                               // products
+                __builtin_amdgcn_sched_group_barrier(0x020, NL, 0);                                   // loads
+                __builtin_amdgcn_sched_group_barrier(0x008, NM / 2, 0);
+            } else {
 #pragma unroll
-                for (int l = 0; l < NL; ++l)
-                    if ((l * BLOCKS + BLOCKS / 2) / NL == blk) load(l);
+                for (int blk = 0; blk < BLOCKS; ++blk) {
+#pragma unroll
+                    for (int m = blk * SIZE; m < (blk + 1) * SIZE; ++m) product(m);
+#pragma unroll
+                    for (int r = 0; r < NR; ++r)
+                        if (r * BLOCKS / NR == blk) read(r);
+#pragma unroll
+                    for (int l = 0; l < NL; ++l)
+                        if ((l * BLOCKS + BLOCKS / 2) / NL == blk) load(l);
+                }
+                p8_spread_slab<BLOCKS, SIZE, (NR + BLOCKS - 1) / BLOCKS, 0>();
             }
-            p8_spread_slab<BLOCKS, SIZE, (NR + BLOCKS - 1) / BLOCKS, 0>();
             __builtin_amdgcn_sched_barrier(0);
             wait_vmcnt_le<H ? ODD : EVEN>();
             // the last operands of the pair have been read, not just asked for: its buffer is loaded over behind this barrier
