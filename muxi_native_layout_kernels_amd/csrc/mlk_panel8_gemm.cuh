@@ -250,10 +250,11 @@ __device__ __forceinline__ void gemm_panel8(const Panel8Args &p, int rt, int tt,
     extern __shared__ u32x4 win[];
     constexpr int WBYTES = FP8 ? 1 : 2;
     using Loop = typename Panel8<T, FP8, TB, PR>::Loop;
-    // taken afresh for every run: what the compiler works out from it in front of the loop over runs is spilled there (soft-FP8 256 x 256:
-    // 20 vector registers)
+    // Taken afresh for every run: what the compiler works out from it in front of the loop over runs is spilled there (soft-FP8 256 x 256:
+    // 9 vector registers).  Not in soft-FP8 panels of 128 x 128 and 128 x 192, which spill nothing either way and whose loop is scheduled
+    // better without (products of 12 to 50 us: 1.4 and 2.9 % faster; the other shapes are level or slower without).
     int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
+    if constexpr (!(FP8 && PR == 1 && (MAXTB == 2 || MAXTB == 3))) asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 3, wt = wave >> 2;

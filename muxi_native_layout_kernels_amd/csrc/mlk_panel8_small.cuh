@@ -4,7 +4,10 @@
 // What a CU pulls.  Distinct weights come at 50 GB/s per CU at most (22 to 25 with all CUs at it: HBM), token rows that lie in L2 at
 // 85 GB/s in whole 128-byte lines and half of that in pieces of 64 bytes (hence P8TokenPairs).
 //
-// The round trip to memory.  The rings are as deep as LDS allows.
+// The round trip to memory.  The ring holds up to five pairs of slabs, four of them ahead: what is fetched past the end of K has to land before LDS
+// is given up, which counts in short products (eight pairs ahead -> four, calls of 6 to 12 us: 128 x 64 3 % faster, 128 x 128 and 128 x 192
+// 2 %; products of 12 to 50 us within 1 %, in slices of K 1 to 2 % faster).  128 x 64 then needs 80 KB, and two workgroups
+// share a CU: grids of several rounds 1.25 times as fast.
 //
 // The round trip to LDS.  A wave multiplies the rows it fetched the weights of, so that it widens its operands in registers and nothing
 // but the tokens is shared.  Widened once per workgroup and handed on through LDS, a slab took 0.28 us (128 x 64) to
@@ -27,7 +30,7 @@ struct Panel8SmallFp8 : P8TokenPairs<TB, false> {
     using Tok = P8TokenPairs<TB, false>;
     static constexpr int RAW_PAIR = 512 * PR, SLOT = RAW_PAIR + Tok::B_PAIR, TB2 = 2 * TB, NH = 2 * PR;     // k16 steps per trip
     static constexpr size_t ring_bytes(int d) { return (size_t)(d + 1) * SLOT * 16; }
-    static constexpr int deepest(int d) { return ring_bytes(d + 1) <= kP8MostLds && d < 8 ? deepest(d + 1) : d; }
+    static constexpr int deepest(int d) { return ring_bytes(d + 1) <= kP8MostLds && d < 4 ? deepest(d + 1) : d; }
     static constexpr int D = deepest(3);                                 // pairs of slabs
     static constexpr size_t lds_bytes = ring_bytes(D);
     static_assert(lds_bytes <= kP8MostLds, "the rings have to fit");
