@@ -306,7 +306,7 @@ struct Panel8LoopFp8 : P8TokenPairs<TB, PR == 1> {
     using Tok = P8TokenPairs<TB, PR == 1>;
     static constexpr int RAW_PAIR = 512 * PR, SLOT = RAW_PAIR + Tok::B_PAIR, RT = 2 * PR, TT = 2 * TB;
     static constexpr size_t ring_bytes(int rp) { return (size_t)rp * SLOT * 16; }
-    static constexpr int RP = ring_bytes(4) <= kP8MostLds ? 4 : 3;
+    static constexpr int RP = 3;
     static constexpr size_t lds_bytes = ring_bytes(RP);
     static_assert(lds_bytes <= kP8MostLds, "the ring has to fit");
 

@@ -242,7 +242,8 @@ __device__ __forceinline__ void p8_store_panel(const Panel8Args &p, const Acc &a
 // bands of p.band groups of eight row tiles in chunks of
 // p.chunk token tiles, so that the 32 workgroups an XCD runs at a time cover 8 x 4 (row tiles x token tiles) and share
 // both operands through its L2; with the token tiles of two row tiles side by side (2 x 16) the same product took
-// 17 % longer (8192 x 8192, 4096 tokens: 491 against 413 us).  A fifth slab of LDS (160 KiB) changed nothing.
+// 17 % longer (8192 x 8192, 4096 tokens, 491 against 413 us; timed on a loop before this one, of 32x32x16 products on tokens in
+// pieces of 64 bytes).
 // In one line, token tiles fastest, for few panels: dealing whole row tiles to XCDs leaves half of them idle at 512 rows.  The
 // workgroups of the line (one per panel, or those that share the k windows) are cut into eight runs, one per XCD.
 template <class T, bool FP8, int PR, int TB, int MAXTB>

@@ -55,23 +55,6 @@ __device__ __forceinline__ void bare_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// Order of a half step for the scheduler: NM products, the ND LDS reads of the next half step two at a time behind the first
-// ones, then the NL loads behind the rest.  The reads come first because the compiler keeps LDS reads and loads that write LDS
-// in program order, and reads that end up behind the last product are waited for in full.
-template <int NM, int ND, int NL>
-__device__ __forceinline__ void spread_half_step() {
-    constexpr int S0 = (ND + 1) / 2 < NM ? (ND + 1) / 2 : NM - 1;      // first slot with loads
-    constexpr int SL = NM - S0, PER = (NL + SL - 1) / SL;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (2 * m + 1 < ND) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        else if (2 * m < ND) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (NL > 0 && m >= S0 && (m - S0) * PER < NL) __builtin_amdgcn_sched_group_barrier(0x020, PER, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 template <bool FP8, int TB, int RING_ = 4>
 struct PanelLdsShape {
     static constexpr int TG = FP8 ? 32 : 64;                 // granules of a weight tile
