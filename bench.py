@@ -410,7 +410,7 @@ def main():
     mfma_only = {}
 
     def mfma_only_tflops(dt):
-        """Matrix-core yardstick: a loop of nothing but v_mfma_f32_32x32x16 on operand values drawn like the
+        """Matrix-core yardstick: a loop of nothing but v_mfma_f32_16x16x32 on operand values drawn like the
         benchmark's (weights 0.02 * N(0, 1), activations N(0, 1)), one workgroup of eight waves per CU, replayed
         like the cases.  The power limit, not the instruction rate, sets what the chip sustains on such values."""
         if dt not in mfma_only:
@@ -423,13 +423,14 @@ def main():
                 _lib.check(lib.mlk_mfma_probe(a.data_ptr(), b.data_ptr(), iters, cus, 0,
                                               torch.cuda.current_stream().cuda_stream), "mfma_probe")
             t = run_graph([call], 10, 3, reps=3, direct_if_short=True)
-            mfma_only[dt] = cus * 8 * iters * 16 * 32768.0 / t["us_median"] / 1e6
+            mfma_only[dt] = cus * 8 * iters * 32 * 16384.0 / t["us_median"] / 1e6
         return mfma_only[dt]
 
     def panel_case(name, n, k, kind, m, steps):
         """Prefill-sized token counts: bound by the matrix cores (or by the weight stream up to ~300 tokens).
         The vendor BLAS on an un-packed 16-bit copy of the same shape is timed beside it, and the rate of a loop
-        that only issues the same MFMA instruction on like-valued operands (`mfma_only_tflops`)."""
+        that only issues the MFMA form of the 16-bit panels on like-valued operands (`mfma_only_tflops`; soft-FP8
+        panels of 256 rows issue 32x32x16, which sustains less)."""
         row = gemm_case(name, n, k, kind, m, steps, 3, copies=2, cpu=False)
         flops = 2.0 * m * n * k
         row["tflops"] = flops / row["us"] / 1e6

@@ -112,7 +112,7 @@ int mlk_stream_read(const void *src, int64_t nbytes, int block_dim_x, int workgr
 
 /* Measurement aid: `workgroups` workgroups of eight waves; every wave reads four 1 KiB operands from `a` and four from
  * `b` (32 KiB each must be readable: 16-bit values, e.g. the head of a weight and of an activation matrix) and issues
- * iters x 16 v_mfma_f32_32x32x16_bf16 on them, nothing else.  flops = workgroups x 8 x iters x 16 x 32768.  Used by
+ * iters x 32 v_mfma_f32_16x16x32_bf16 on them, nothing else.  flops = workgroups x 8 x iters x 32 x 16384.  Used by
  * bench.py to report the matrix-core rate the chip sustains on the benchmark's operand values (the power limit lowers
  * the clock under dense random operands) next to the 2.5 PFLOP/s peak.  No counterpart in the reference. */
 int mlk_mfma_probe(const void *a, const void *b, int iters, int workgroups, void *sink, void *stream);

@@ -129,10 +129,11 @@ __global__ void __launch_bounds__(256) fp8_repack16_kernel(const u32x4 *__restri
     }
 }
 
-// Matrix-core yardstick: every wave takes four 32-row operands from `a` and four from `b` (16 bytes per lane each, read
-// once) and issues iters x 16 v_mfma_f32_32x32x16_bf16 on them, eight waves per workgroup, nothing else in the loop and
+// Matrix-core yardstick: every wave takes four 16-row operands from `a` and four from `b` (16 bytes per lane each, read
+// once) and issues iters x 32 v_mfma_f32_16x16x32_bf16 on them, eight waves per workgroup, nothing else in the loop and
 // nothing stored.  What it measures is the rate the chip sustains on those operand VALUES: with zeros the clock stays at
-// its maximum, with the dense random values of a real product the power limit pulls it down by a third.
+// its maximum, with the dense random values of a real product the power limit pulls it down.  Of the two forms of the
+// instruction the one that sustains more (random values: 2.06 PFLOP/s, 32x32x16 1.80), which the 16-bit panels issue.
 __global__ void __launch_bounds__(512) mfma_probe_kernel(const u32x4 *__restrict__ a, const u32x4 *__restrict__ b, int iters,
                                                          uint32_t *__restrict__ sink) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -142,25 +143,23 @@ __global__ void __launch_bounds__(512) mfma_probe_kernel(const u32x4 *__restrict
         x[i] = a[(wave * 4 + i) * 64 + lane];
         y[i] = b[(wave * 4 + i) * 64 + lane];
     }
-    f32x16 acc[2][4];
+    f32x4 acc[4][4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int it = 0; it < iters; ++it) {
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = BF16::mfma32(x[2 * r + i], y[j], acc[i][j]);
+                for (int j = 0; j < 4; ++j) acc[i][j] = BF16::mfma(x[i], y[j], acc[i][j]);
     }
     mfma_settle();
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) s += acc[i][j][0];
     if (sink != nullptr && __float_as_uint(s) == 0x7fc12345u) *sink = 1;      // a NaN payload the products never make
