@@ -1419,15 +1419,14 @@ static MoePlan moe_plan(int tc, int n_experts, int topk, int hidden, int inter, 
 // ------------------------------------------------------------ passes
 // A call of up to kMoeChunk tokens is one pass of the kernels moe_plan() names.  A longer one goes through the wide kernels
 // (mlk_moe_wide.cuh) in passes of as many tokens as their workspace is allowed for: in passes of kMoeChunk tokens every
-// pass streams the weights of all experts it reaches again.  Measured, passes of kMoeChunk tokens -> wide kernels (us, without
-// the router):
+// pass streams the weights of all experts it reaches again.  Measured, passes of kMoeChunk tokens -> wide kernels (us a layer):
 //                                                  tokens   257          264          272          320
-//   8 experts, top-2, H 4096, I 14336, bf16                 645 -> 524   887 -> 523   940 -> 523   964 -> 538
-//   the same, soft-FP8                                      424 -> 365   550 -> 332   578 -> 374   632 -> 393
-//   256 experts, top-8, H 7168, I 256, bf16                 524 -> 555   603 -> 543   676 -> 543   915 -> 552
-//   the same, soft-FP8                                      327 -> 388   407 -> 385   442 -> 389   578 -> 396
-//   128 experts, top-8, H 2048, I 768, bf16                 240 -> 239   313 -> 234   345 -> 234   417 -> 236
-//   the same, soft-FP8                                      156 -> 163   200 -> 163   225 -> 164   261 -> 165
+//   8 experts, top-2, H 4096, I 14336, bf16                 626 -> 528   945 -> 531   901 -> 533   980 -> 541
+//   the same, soft-FP8                                      431 -> 390   564 -> 392   587 -> 400   644 -> 413
+//   256 experts, top-8, H 7168, I 256, bf16                 529 -> 558   617 -> 554   696 -> 556   919 -> 561
+//   the same, soft-FP8                                      333 -> 402   424 -> 404   458 -> 406   588 -> 409
+//   128 experts, top-8, H 2048, I 768, bf16                 242 -> 240   319 -> 239   354 -> 240   424 -> 244
+//   the same, soft-FP8                                      162 -> 173   216 -> 175   238 -> 175   271 -> 178
 // A few tokens above kMoeChunk, moe_two_passes_pay() keeps the pass of kMoeChunk tokens and its remainder.  A remainder of up to
 // kMoeChunk tokens is a pass of the small kernels again, and a call whose workspace only holds passes of kMoeChunk tokens, or
 // whose operands do not lie on 16 bytes, runs in those.
@@ -1446,9 +1445,11 @@ extern template int launch_moe_wide<F16, false>(const MoeArgs &, int, float *, i
 extern template int launch_moe_wide<BF16, true>(const MoeArgs &, int, float *, int, hipStream_t);
 
 // K slices of the wide down projection: its panels run one per CU in rounds, so a grid of one and a half rounds wastes a
-// quarter of the chip unless the panels are cut.  In units of a k32 slab of a panel (0.75 us): a panel costs its slabs and
-// about eight more to start and to store; a slice costs the write and the read of its partial products (8 experts, bf16,
-// 1, 2, 3 slices: 677, 579, 615 us at 256 tokens, 1782, 1689, 1667 us at 2048).
+// quarter of the chip unless the panels are cut.  In units of a k32 slab of a panel (0.64 us): a panel costs its slabs and
+// 24 more to start and to store; a slice costs the write and the read of its partial products.  Both constants are the best of a grid over
+// 210 layers (8 to 256 experts, both kinds of weights) at 1912 token counts from 257 to 4096, one to four slices timed at each: 28 choices
+// cost more than 3 % against the best (13 % at most), 0.2 % in the mean; with 8 slabs and 0.75 us, fitted to the loops before, 74 and 0.3 %
+// (8 experts, top-2, H 4096, bf16, 1, 2, 3 slices: I 14336 589, 527, 560 us at 257 tokens, 1396, 1309, 1347 at 2004; I 2688 193, 216, 210 at 972).
 static int moe_wide_expert_tasks(int tokens, int n_experts, int topk) {
     const double mean = (double)tokens * topk / n_experts;
     return (int)ceil((mean + 0.5 * sqrt(mean)) / (16 * kWideTaskBlocks));
@@ -1457,12 +1458,12 @@ static int moe_wide_down_slices(int tokens, int n_experts, int topk, int hidden,
     const int cus = device_cus();
     const double pairs = (double)tokens * topk;
     const double tasks = moe_wide_expert_tasks(tokens, n_experts, topk) * (pairs < n_experts ? pairs : n_experts);
-    const double per_slice = pairs * hidden * 8 / 5e6 / 0.75;
+    const double per_slice = pairs * hidden * 8 / 5e6 / 0.64;
     int best = 1;
     double best_cost = 0;
     for (int skd = 1; skd <= 4 && inter / 128 / skd >= 2; ++skd) {
         const double rounds = ceil(tasks * ((hidden + 255) / 256) * skd / cus);
-        const double cost = rounds * (inter / 32.0 / skd + 8) + per_slice * skd;
+        const double cost = rounds * (inter / 32.0 / skd + 24) + per_slice * skd;
         if (skd == 1 || cost < best_cost) best = skd, best_cost = cost;
     }
     return best;
@@ -1526,10 +1527,9 @@ static void moe_share_rows(MoePass *ps, int n_experts, int topk, int hidden, int
 // as the small kernels come to be bound by their products; the remainder costs its launches and the experts it reaches once
 // more.  Where a task is one token block and the decode kernels run it, the down kernel walks all tasks in every workgroup (a share per
 // expert) and its grid of 16 output rows each runs in whole rounds.  The constants (us and MB) are fitted to 44 layers of 8 to 256 experts,
-// both kinds of weights and 257 to 320 tokens (twelve small layers to 512): of 832 choices twelve cost more than 3 % against the better one (10 % at
-// most; 0.1 % in the mean).  Fitted before tasks of one block had the row-shared kernels and the wide kernels their short panels, the choice was
-// wrong by more than 3 % 74 times, by up to 40 % (soft-FP8, 32 experts, top-1, H 4096, I 2048, 268 tokens: two passes 232 us, wide 166 us;
-// 256 experts, top-1, H 2048, I 512, 257 tokens: 129 and 154 us).
+// both kinds of weights and 257 to 320 tokens (twelve small layers to 512).  With the wide kernels as they are, both forms forced, on 210 other
+// layers at ten token counts from 257 to 512: of 2164 choices 34 cost more than 3 % against the better one (21 % at most: bf16, 20 experts, top-1,
+// H 4096, I 384, 257 tokens, two passes 70 us, wide 85), 0.1 % in the mean.
 struct MoeTwoPasses {
     float per_mb, per_mb_mean;     // us that a MB of weights saves in the pass of kMoeChunk tokens; less per token above eight of an expert
     float per_panel;               // us per wide panel on a CU
