@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from muxi_native_layout_kernels_amd import ops
 from oracle import gemm as ogemm, layouts
 from helpers import randn, pack_a, pack_b, fp8_codes, assert_close, bits
 
@@ -613,9 +614,14 @@ def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3, native):
     if kind == "fp8":
         w = fp8_codes((n, k), 33)
         scale = (torch.rand(((n + 127) // 128, k // 128), generator=torch.Generator().manual_seed(34)) * 0.02 + 0.001).float()
-        c = mlk.gemm_layoutA_soft_fp8_wapper(pack_a(w).cuda(), scale.cuda(), x.cuda(), n, m, k, **kw)
+        a, scale_dev = pack_a(w).cuda(), scale.cuda()
+        c = mlk.gemm_layoutA_soft_fp8_wapper(a, scale_dev, x.cuda(), n, m, k, **kw)
         want = ogemm.softfp8_linear_expected(w, scale, x, 0.5, bias)
         assert_close(c, want, RTOL, ATOL, "soft-FP8 panels")
+        if native:                     # no Python entry point takes this pair, the C one does
+            for c_mode, row_major in ((0, lambda c: c), (1, mlk.reLayoutC)):
+                got = ops._gemm_call(a, scale_dev, mlk.layoutB(x.cuda()), n, m, k, 0.5, 0, kw["bias"], 1, c_mode, 8, p1, p2, p3, "gemm")
+                assert torch.equal(row_major(got), c)
         return
     w = randn((n, k), dtype, k ** -0.5, 33)
     a = pack_a(w).cuda()
@@ -631,9 +637,9 @@ def test_gemm_eight_wave_panels(mlk, kind, p1, p2, n, m, k, p3, native):
 @pytest.mark.parametrize("p1,p2", [(p1, p2) for p1 in (2, 4) for p2 in (1, 2, 3, 4)])
 @pytest.mark.parametrize("k,p3", [(128, 2), (256, 1), (384, 2), (640, 1), (768, 5), (896, 1), (1152, 1), (1664, 3), (1920, 1)])
 def test_gemm_eight_wave_rings(mlk, kind, p1, p2, k, p3):
-    """kernelId 8 on full panels: K, and slices of it, shorter than the rings of every shape (one to six pairs of k32 slabs), as long, and
+    """kernelId 8 on full panels: K, and slices of it, shorter than the rings of every shape (two to five pairs of k32 slabs), as long, and
     longer by every remainder.  The weights of neighbouring slabs differ in scale, so that a slab multiplied twice or by its
-    neighbour's tokens shows; whole numbers, so that sums of up to 2^24 have one value in any order."""
+    neighbour's tokens shows; whole numbers, so that sums of up to 2^24 have one value in any order.  Activations row-major and in layout B."""
     n, m = 64 * p1, 64 * p2
     g = torch.Generator().manual_seed(36)
     x = torch.randint(-3, 4, (m, k), generator=g).to(torch.float16 if kind == "fp16" else torch.bfloat16)
@@ -645,24 +651,34 @@ def test_gemm_eight_wave_rings(mlk, kind, p1, p2, k, p3):
         scale = torch.exp2(torch.randint(-2, 3, ((n + 127) // 128, k // 128), generator=g).float())
         want = x.double() @ (w * scale.repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)).double().t()
         a = pack_a(w.float().to(torch.float8_e4m3fn).view(torch.uint8)).cuda()
-        c = mlk.gemm_layoutA_soft_fp8_wapper(a, scale.cuda(), x.cuda(), n, m, k, **kw)
+        scale = scale.cuda()
+        c = mlk.gemm_layoutA_soft_fp8_wapper(a, scale, x.cuda(), n, m, k, **kw)
     else:
-        c = mlk.gemm_layoutA_wapper(pack_a(w.to(x.dtype)).cuda(), x.cuda(), n, m, k, **kw)
-    assert torch.equal(c.cpu(), want.float().to(x.dtype))
+        a, scale = pack_a(w.to(x.dtype)).cuda(), None
+        c = mlk.gemm_layoutA_wapper(a, x.cuda(), n, m, k, **kw)
+    want = want.float().to(x.dtype)
+    assert torch.equal(c.cpu(), want)
+    c = ops._gemm_call(a, scale, mlk.layoutB(x.cuda()), n, m, k, 1, 0, None, 1, 0, 8, p1, p2, p3, "gemm")
+    assert torch.equal(c.cpu(), want)
 
 
 @pytest.mark.parametrize("kind,native", [("bf16", False), ("bf16", True), ("fp8", False)])
-@pytest.mark.parametrize("n,m,k,p1,p2,p3", [
-    (384, 1008, 256, 2, 2, 1),         # three row tiles, eight token tiles, the last one short
-    (1040, 1600, 384, 2, 4, 2),        # nine row tiles, the last one ragged, in slices
-    (400, 2064, 256, 4, 1, 3),         # two row tiles, 33 token tiles, more slices than windows of some
-    (640, 1504, 640, 2, 3, 1),
-    (640, 144, 640, 2, 3, 1),          # one token tile: either order
-    (128, 1040, 128, 2, 1, 2),         # one row tile
+@pytest.mark.parametrize("n,m,k,p1,p2,p3,first", [
+    (384, 1488, 256, 2, 2, 1, True),       # three row tiles, twelve token tiles, the last one short
+    (1040, 1600, 384, 2, 4, 2, True),      # nine row tiles, the last one ragged, in slices
+    (400, 2832, 256, 4, 1, 3, True),       # two row tiles, 45 token tiles, more slices than windows of some
+    (640, 1504, 640, 2, 3, 1, True),
+    (640, 144, 640, 2, 3, 1, False),       # one token tile: either order is the same
+    (128, 1040, 128, 2, 1, 2, False),      # one row tile
 ])
-def test_gemm_eight_wave_row_tiles_first(mlk, kind, native, n, m, k, p1, p2, p3):
+def test_gemm_eight_wave_row_tiles_first(mlk, kind, native, n, m, k, p1, p2, p3, first):
     """One line of panels with more activations than weights: the row tiles of a token tile side by side.  Whole numbers, one value in
     any order of the sums."""
+    weights, tokens = n * (1 if kind == "fp8" else 2), 2 * m
+    row_tiles, token_tiles = -(-n // (64 * p1)), -(-m // (64 * p2))
+    assert row_tiles * token_tiles <= 256                      # one line
+    # the rule of p8_rows_first() in csrc/mlk_panel.hip
+    assert first == (tokens > weights and tokens + weights * min(8, token_tiles) < weights + tokens * min(8, row_tiles))
     g = torch.Generator().manual_seed(37)
     x = torch.randint(-3, 4, (m, k), generator=g).to(torch.bfloat16)
     w = torch.randint(-2, 3, (n, k), generator=g)
