@@ -1,6 +1,7 @@
 // Main loops of the eight-wave panels: 128 PR weight rows x 64 TB tokens (PR = 1, 2; TB = 1..4), both operands through LDS,
-// fetched with loads that write LDS directly, v_mfma_f32_16x16x32.  Panel8Loop16 is for 16-bit weights, Panel8LoopFp8 for the large
-// soft-FP8 panels, Panel8SmallFp8 (mlk_panel8_small.cuh) for the others; Panel8<..>::Loop picks.
+// fetched with loads that write LDS directly.  Panel8Loop16 is for 16-bit weights (v_mfma_f32_16x16x32), Panel8LoopFp8 for the large
+// soft-FP8 panels (16x16x32 with 128 rows, 32x32x16 with 256), Panel8SmallFp8 (mlk_panel8_small.cuh, 32x32x16) for the others;
+// Panel8<..>::Loop picks.
 //
 // What sets the pace of a large panel, measured on 8192 x 8192 bf16 at 4096 tokens (256 x 256 panels, one workgroup per CU; a k32 slab
 // takes 0.43 us of products):
@@ -297,8 +298,7 @@ struct Panel8Loop16 : P8TokenPairs<TB, true> {
 // Soft-FP8 weights of large panels.  The fp8 tiles (512 bytes) come through LDS as they are, and every wave widens the row tiles that it
 // multiplies in registers, a slab ahead, between the products: each weight is widened by both token halves, four vector instructions a
 // pair of them.  Widened once per workgroup and handed on through LDS as 16-bit tiles, as this loop once did, a slab moved 144 KiB
-// through LDS, more than it passes while a slab is multiplied (28672 x 8192 at 1024 tokens 455 -> 400 us, 8192 x 8192 at 4096 tokens 472 -> 424,
-// 128 panels of K 14336 316 -> 290).
+// through LDS, more than it passes while a slab is multiplied (28672 x 8192 at 1024 tokens 456 -> 411 us, in the 16 x 16 form).
 // Ring of RP pairs of slabs, weights and tokens.  The last reads of pair p happen in slab 2 p; slab 2 p + 1 issues the tokens of pair
 // p + RP into its place and slab 2 p + 2 the weights, so that one wait and one barrier per pair do, at the end of the even slab.
 template <class T, int TB, int PR>
@@ -323,9 +323,9 @@ struct Panel8LoopFp8 : P8TokenPairs<TB, PR == 1> {
     }
 
     // As Panel8Loop16::run; srow[0]: block scales of the wave's rows, srow[1] (NS = 2): of its second half of row tiles
-    // 256 rows: the 32 x 32 form, which leaves the vector unit more issue slots for the widening (11008 x 4096 at 512 tokens 89 -> 76 us,
-    // 28672 x 8192 at 1024 454 -> 431, 8192 x 8192 at 4096, where power counts, 445 -> 449).  128 rows, half as many weights a product: the
-    // 16 x 16 form (8192 x 8192 at 2048 tokens 275 -> 246).
+    // 256 rows: the 32 x 32 form, which leaves the vector unit more issue slots for the widening (panels of 256 x 256, 11008 x 4096 at 512
+    // tokens 89 -> 76 us, 4096 x 14336 at 512 285 -> 244, 28672 x 8192 at 1024 411 -> 402).  128 rows, half as many weights a product: the
+    // 16 x 16 form (8192 x 8192 at 2048 tokens in panels of 128 x 256: 32 x 32 275, 16 x 16 246).
     static constexpr bool M32 = PR == 2;
     using Acc = std::conditional_t<M32, P8Acc32<PR, TB>, P8Acc16<PR, TB>>;
     template <int NS>

@@ -23,7 +23,7 @@ namespace mlk {
 // same 32 rows, w the even and w + 4 the odd slabs.  At the end the two waves of a row quarter exchange halves of their sums (PR = 1:
 // and add them), so that every wave holds the sums of its row quarter and token half.  Within a trip the token operands are read a k16 step
 // ahead, the fp8 tiles two, and a step's weights are widened between the products of the step before.
-// v_mfma_f32_32x32x16 here: these panels are bound by the issue of vector instructions, and the 16 x 16 form takes twice as many (measured 8 to 10 %
+// v_mfma_f32_32x32x16 here: these panels are bound by the issue of vector instructions, and the 16 x 16 form takes twice as many (measured 9 to 12 %
 // slower: 4096 x 14336, 200 tokens in panels of 256 x 128 153 -> 172 us, of 128 x 64 76 -> 83).
 template <class T, int TB, int PR>
 struct Panel8SmallFp8 : P8TokenPairs<TB, false> {
