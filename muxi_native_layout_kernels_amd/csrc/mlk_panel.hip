@@ -211,12 +211,15 @@ size_t panel_partial_bytes(int m, int n, int sk) {
 }
 
 // Time in us that m x n x k takes in panels of 128 pr rows x 64 tb tokens with K in sk slices (kP8Deal: only for grids of several
-// rounds).  Fitted to the times of 2300 products (512 to 37888 rows, K 512 to 18432, 65 to 4096 tokens; bf16 and soft-FP8, up to the 18 likeliest
-// launches of each), to the times and to how much slower than the best the launch is that it picks.  On as many other products that is 1.6 %
-// (soft-FP8 1.0 %) in the geometric mean, 8.7 % (6.5 %) at the 95th percentile; with the constants of the kernels before these 2.6 % (2.4 %).
+// rounds).  Fitted to the times of 1449 products (512 to 37888 rows, K 512 to 18432, 65 to 4096 tokens; bf16 and soft-FP8, the 9 to 14 likeliest
+// launches of each), to the times and to how much slower than the best the launch is that it picks.  Each launch was timed twice, on weights that come from
+// memory and on two copies in turn, which the Infinity Cache holds up to 128 MB: they rank launches differently (11008 x 4096 bf16 at 128 tokens, panels of
+// 128 x 64 whole and 128 x 128 in two slices: 35.6 and 33.4 us from memory, 24.8 and 27.1 from the cache), and what is fitted is the geometric mean
+// of both.  On as many other products the launch it picks is 0.8 % (soft-FP8 0.5 %) slower than the best one in the geometric mean, 4.1 % (2.8 %) at
+// the 95th percentile (1.1 % and 6 % from memory or from the cache alone); a margin of 2 to 5 % in favour of launches in one slice picks no better.
 // What it does not know: panels of one row tile are faster where one token tile is shorter than the others, which runs ahead and fetches
-// their weights (11008 x 4096 at 300 tokens in panels of 128 x 192: 192 and 108 tokens 44.0 us, 160 and 140 45.6); and a last round of few
-// panels (11008 x 4096 at 1302 tokens, 258 panels: dealt 114 us, whole 156).
+// their weights (11008 x 4096 at 300 tokens in panels of 128 x 192: 192 and 108 tokens 44.0 us, 160 and 140 45.6); and that a count of
+// slices can be a fifth slower than the next one (512 x 2176 at 446 tokens in four and five: 11.9 and 14.4).
 struct P8Cost {
     // up to one panel per CU: start, store (256 x 256), fold = fold + fold_slice per slice + fold_mb per MB of slots; a k32 slab of a panel
     // on an idle chip, what a workgroup on every CU adds to it, and the power of the token tiles that share weights by which that falls
@@ -224,27 +227,23 @@ struct P8Cost {
     // several rounds: start, end of a round (256 x 256), what a last round that is not full saves of its empty part, fold, per MB; a slab
     float r_start, r_end, r_empty, r_fold, r_fold_mb, r_slab[2][4];
 };
-static const P8Cost kP8Cost16 = {3.88f, 3.48f, 2.04f, 0.187f, 0.265f, 0.41f,
-                                 {{0.113f, 0.222f, 0.241f, 0.326f}, {0.146f, 0.250f, 0.341f, 0.437f}},
-                                 {{0.151f, 0.087f, 0.140f, 0.078f}, {0.405f, 0.326f, 0.327f, 0.313f}},
-                                 3.85f, 6.85f, 0.34f, 2.08f, 0.417f,
-                                 {{0.217f, 0.294f, 0.350f, 0.428f}, {0.322f, 0.426f, 0.527f, 0.640f}}};
-static const P8Cost kP8Cost8 = {5.15f, 4.06f, 2.82f, 0.168f, 0.213f, 0.02f,
-                                {{0.111f, 0.151f, 0.205f, 0.250f}, {0.185f, 0.222f, 0.325f, 0.406f}},
-                                {{0.053f, 0.100f, 0.144f, 0.154f}, {0.128f, 0.238f, 0.288f, 0.292f}},
-                                3.67f, 9.56f, 0.26f, 2.66f, 0.255f,
-                                {{0.201f, 0.269f, 0.366f, 0.427f}, {0.348f, 0.447f, 0.607f, 0.675f}}};
-// Up to 64 tokens, where the panels compete with the narrow kernels and one token tile holds the call: fitted with those.
-static const P8Cost kP8Few16 = {3.6f, 3.0f, 2.65f, 0.09f, 0.215f, 0.f,
-                                {{0.105f, 0.178f, 0.257f, 0.341f}, {0.171f, 0.299f, 0.362f, 0.503f}},
-                                {{0.222f, 0.223f, 0.210f, 0.229f}, {0.487f, 0.401f, 0.470f, 0.548f}},
-                                4.5f, 7.2f, 0.47f, 3.6f, 0.244f,
-                                {{0.207f, 0.290f, 0.398f, 0.498f}, {0.315f, 0.476f, 0.649f, 0.808f}}};
-static const P8Cost kP8Few8 = {5.3f, 2.8f, 3.00f, 0.10f, 0.197f, 0.f,
-                               {{0.113f, 0.162f, 0.229f, 0.390f}, {0.196f, 0.257f, 0.531f, 0.462f}},
-                               {{0.096f, 0.136f, 0.152f, 0.152f}, {0.172f, 0.274f, 0.192f, 0.438f}},
-                               5.8f, 8.7f, 0.47f, 4.6f, 0.197f,
-                               {{0.192f, 0.281f, 0.381f, 0.564f}, {0.322f, 0.471f, 0.730f, 0.844f}}};
+static const P8Cost kP8Cost16 = {3.343f, 4.509f, 3.000f, 0.143f, 0.292f, 0.501f,
+                                 {{0.140f, 0.199f, 0.258f, 0.355f}, {0.224f, 0.297f, 0.395f, 0.515f}},
+                                 {{0.102f, 0.110f, 0.107f, 0.083f}, {0.269f, 0.287f, 0.204f, 0.228f}},
+                                 2.969f, 5.880f, 0.250f, 3.548f, 0.574f,
+                                 {{0.205f, 0.287f, 0.339f, 0.426f}, {0.354f, 0.427f, 0.554f, 0.666f}}};
+static const P8Cost kP8Cost8 = {5.004f, 4.579f, 3.301f, 0.115f, 0.254f, 0.021f,
+                                {{0.132f, 0.179f, 0.265f, 0.317f}, {0.219f, 0.279f, 0.436f, 0.515f}},
+                                {{0.050f, 0.080f, 0.076f, 0.096f}, {0.103f, 0.187f, 0.198f, 0.166f}},
+                                3.996f, 9.576f, 0.208f, 3.131f, 0.384f,
+                                {{0.181f, 0.275f, 0.362f, 0.429f}, {0.351f, 0.451f, 0.613f, 0.649f}}};
+// Up to 64 tokens, where panels of 64 compete with the narrow kernels: fitted to 430 products of 16 to 64 tokens, timed in the same way, with the
+// times that narrow_us() expects beside them.  On as many others the choice between all is 5.0 % (soft-FP8 3.7 %) slower than the best, with the constants of the
+// loops before the 16 x 16 products 5.3 % (4.2 %): what is left is in the narrow kernels.
+static const P8Cost kP8Few16 = {3.446f, 2.918f, 3.334f, 0.101f, 0.269f, 0.f, {{0.121f}, {0.165f}}, {{0.157f}, {0.405f}},
+                                4.762f, 7.372f, 0.463f, 3.750f, 0.248f, {{0.286f}, {0.315f}}};
+static const P8Cost kP8Few8 = {4.351f, 2.866f, 3.136f, 0.094f, 0.259f, 0.f, {{0.137f}, {0.224f}}, {{0.056f}, {0.163f}},
+                               5.817f, 8.709f, 0.468f, 4.593f, 0.197f, {{0.207f}, {0.322f}}};
 static double panel8_us(const P8Cost &f, int m, int n, int k, int pr, int tb, int sk) {
     const int cus = device_cus(), rows = (n + 128 * pr - 1) / (128 * pr), tokens = (m + 64 * tb - 1) / (64 * tb), windows = k / 64;
     const int narrow = (m - (tokens - 1) * 64 * tb + 63) / 64;                   // columns / 64 of the last token tile
@@ -265,13 +264,21 @@ static double panel8_us(const P8Cost &f, int m, int n, int k, int pr, int tb, in
     const double t_full = f.r_slab[pr - 1][tb - 1] * slabs, t_narrow = f.r_slab[pr - 1][narrow - 1] * slabs;
     const double even = (full * t_full + (per_xcd - full) * t_narrow) / round;                   // dealt out evenly
     if (sk == 1) {
+        // The last round is as long as a full panel unless the narrow ones are all that it holds: they stand alone at the end where the last chunk
+        // of token tiles is theirs (11008 x 4096 at 1302 tokens in panels of 256 x 256, 36 on the fullest XCD: 159 us, priced as narrow 125, dealt 116).
+        const long long last = per_xcd - round * (rounds - 1);
+        const bool narrow_last = narrow < tb && last <= ((tokens - 1) % 4 ? 1 : (groups - 1) % 8 + 1);
         const double dealt = even + (double)per_xcd / round * end;
-        const double whole = (rounds - 1) * t_full + (full > round * (rounds - 1) ? t_full : t_narrow) + rounds * end;
+        const double whole = (rounds - 1) * t_full + (narrow_last ? t_narrow : t_full) + rounds * end;
         return f.r_start + dealt + (whole - dealt) * (1 - f.r_empty);
     }
-    if (per_xcd % round == 0) return 1e30;                                                       // nothing is left over
+    const long long rest = per_xcd % round;
+    if (rest == 0) return 1e30;                                                                  // nothing is left over
+    // XCDs that have one group of row tiles less deal less, or nothing
+    const int most = rows - 8 * (groups - 1);
+    const double lines = most + (8 - most) * (rest > tokens ? (double)(rest - tokens) / rest : 0);
     // 3 % in favour of whole panels, which are as good where the two come out alike
-    return 1.03 * (f.r_start + even + (per_xcd / round + 1.2) * end + f.r_fold + f.r_fold_mb * cus * pr * tb * 0.032768);
+    return 1.03 * (f.r_start + even + (per_xcd / round + 1.2) * end + f.r_fold + f.r_fold_mb * round * lines * pr * tb * 0.032768);
 }
 
 // Time in us of the narrow kernels (ids 1 and 4) on up to 64 tokens: what a CU pulls through its memory path (weights, and the

@@ -355,6 +355,23 @@ def test_panel_plan_is_a_shape_the_kernel_takes():
         del table[(4224, 300, 1024)]
 
 
+@pytest.mark.parametrize("a_kind,n,k,m,want", [
+    (1, 11008, 4096, 1302, lambda p1, p2, p3: p3 == 64 or p1 * p2 < 16),      # 36 panels of 256 x 256 on the fullest XCD, two of the last four full
+    (1, 27648, 5120, 578, lambda p1, p2, p3: (p1, p2, p3) != (4, 4, 1)),      # 14 rows of panels of 256, 256 and 66 tokens
+    (1, 11008, 4096, 128, lambda p1, p2, p3: p3 == 1),                        # few weights per CU: no second launch
+    (1, 11008, 4096, 256, lambda p1, p2, p3: p3 == 1),
+    (2, 512, 1408, 86, lambda p1, p2, p3: p3 > 1),
+])
+def test_gemm_plan_choices(a_kind, n, k, m, want):
+    """Choices that cost 10 to 40 % the other way round: a last round that holds full panels is as long as a full panel, a split has
+    to pay for its fold, and a small grid is cut."""
+    import ctypes
+    from muxi_native_layout_kernels_amd import _lib
+    out = (ctypes.c_int32 * 4)()
+    assert _lib.load().mlk_gemm_plan(m, n, k, a_kind, out) == 0
+    assert out[0] == 8 and want(*out[1:]), list(out)
+
+
 def test_shipped_panel_rows_fit_the_documented_workspace():
     """A C caller sizes the K split of a table row with mlk_gemm_workspace_bytes(): enough for the rows of kernel id 8 too, at their own
     token count and at every smaller one that borrows them."""
