@@ -418,15 +418,16 @@ int launch_panel8_gemm(const void *a, const void *b, void *c, int m, int n, int 
     return launch_panel8<BF16, false>(p, pr, tb, s);
 }
 
-// Tokens per panel when the caller leaves the choice open.  Workgroups run one per CU in rounds; a 256-token panel
-// takes 1.3 to 1.5 times as long as a 128-token one for 16-bit weights (eight-wave kernel) and 1.84 times for soft-FP8
-// ones (measured), so the width with the cheaper sum of rounds wins.
-int panel_tokens(int m, int n, bool fp8) {
+// Tokens per panel when the caller leaves the choice open.  Workgroups run one per CU in rounds; a round of 256-token panels (eight-wave
+// kernel) takes 1.35 to 1.6 times as long as one of 128-token panels, and the width with the cheaper sum of rounds wins.  On 500 products of
+// 129 to 4096 tokens, both widths timed, the choice is 1.9 % (soft-FP8 1.2 %) slower than the better one in the geometric mean, the same
+// with any ratio from 1 to 1.4; soft-FP8 weights with the 1.84 of an earlier loop: 2.3 %.
+int panel_tokens(int m, int n) {
     const int cus = device_cus();
     const long long row_tiles = (n + kPanelRowsPerWg - 1) / kPanelRowsPerWg;
     const long long rounds128 = (row_tiles * ((m + 127) / 128) + cus - 1) / cus;
     const long long rounds256 = (row_tiles * ((m + 255) / 256) + cus - 1) / cus;
-    return rounds256 * (fp8 ? 184 : 140) < rounds128 * 100 ? 256 : 128;
+    return rounds256 * 140 < rounds128 * 100 ? 256 : 128;
 }
 
 // a_kind: MLK_F16, MLK_BF16 or MLK_FP8_E4M3 (bf16 activations); width: tokens per panel (128 or 256), anything else =
@@ -449,7 +450,7 @@ int launch_panel(const void *a, const void *b, void *c, int m, int n, int k, int
     p.N = n;
     p.K = k;
     p.alpha = alpha;
-    if (width != 128 && width != 256) width = panel_tokens(m, n, a_kind == MLK_FP8_E4M3);
+    if (width != 128 && width != 256) width = panel_tokens(m, n);
     if (width == 256) rows = 256;
     // the loops that fetch straight into LDS take operands on 16 bytes, and panels of 256 tokens store 16 bytes at a time; others
     // run panels of 128 tokens that fetch through registers
