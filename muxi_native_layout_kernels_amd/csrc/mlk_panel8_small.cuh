@@ -74,6 +74,11 @@ struct Panel8SmallFp8 : P8TokenPairs<TB, false> {
 #pragma unroll
             for (int tb = 0; tb < TB2; ++tb) f[tb] = win[buf * SLOT + (b_idx ^ (h * b_step)) + 256 * tb];
         };
+        // Where a trip's loads go out: in its second step; in the first, one behind each product (128 x 64, whose second step is its last:
+        // 4 to 8 % slower there) or in front of the products (256 x 128, level).  All of them in front of the first step's products:
+        // 128 x 128 1 to 2 % slower, 128 x 192 and 256 x 64 0.5 to 1 %, 128 x 64 1 %.
+        constexpr bool SPREAD = PR * TB == 1;
+        constexpr int LOADS = SPREAD || PR * TB == 4 ? 0 : 1;
         auto widen = [&](u32x4 &o, const u32x2 &r, float sc) {
             uint32_t x0, x1, x2, x3;
             fp8x4_to_bf16x4(r[0], sc, x0, x1);
@@ -101,17 +106,18 @@ struct Panel8SmallFp8 : P8TokenPairs<TB, false> {
                 else rd_b(b[0], nxt, 0);
                 if (h + 2 < NH) rd_raw(raw[h & 1], cur, h + 2);
                 else rd_raw(raw[h & 1], nxt, h + 2 - NH);
-                if (h == 0) issue(src, wave, min(pair0 + p + D, last), prv);
+                if (h == LOADS) issue(src, wave, min(pair0 + p + D, last), prv);
                 widen(op[(h + 1) & 1], raw[(h + 1) & 1], h + 1 < NH ? sc : sc_next);
 #pragma unroll
                 for (int tb = 0; tb < TB2; ++tb) sum[tb] = T::mfma32(op[h & 1], b[h & 1][tb], sum[tb]);
                 constexpr int PER = (18 + TB2 - 1) / TB2;          // conversion instructions per product
                 __builtin_amdgcn_sched_group_barrier(0x100, TB2 + 1, 0);                          // LDS reads
-                if (h == 0) __builtin_amdgcn_sched_group_barrier(0x020, PR + TB, 0);              // loads
+                if (h == LOADS && !SPREAD) __builtin_amdgcn_sched_group_barrier(0x020, PR + TB, 0);   // loads
 #pragma unroll
                 for (int m = 0; m < TB2; ++m) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
+                    if (h == LOADS && SPREAD) __builtin_amdgcn_sched_group_barrier(0x020, (PR + TB + TB2 - 1) / TB2, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
